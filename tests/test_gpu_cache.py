@@ -189,6 +189,34 @@ def test_inline_rope_and_forks_on_the_generic_kernels(dtype, page_size, d, slidi
     m.step([(3, 1), (1, 1)])
 
 
+@pytest.mark.parametrize("page_size,d,hq,hkv,tol", [(16, 128, 8, 2, 4e-3), (16, 64, 8, 8, 4e-3), (32, 256, 4, 2, 4e-3),
+                                                   (16, 96, 36, 18, 4e-3), (24, 80, 8, 4, 4e-3), (128, 112, 9, 1, 4e-3)])
+def test_prefill_steps_of_windowed_caches_over_gathered_keys(page_size, d, hq, hkv, tol):
+    """Prefill steps with enough rows run over keys gathered (and rotated) into one run per sequence: windows of one and
+    several runs of 16 keys, with and without sinks, a sequence that is new, one that decodes beside the chunks, chunks
+    longer than the window, more kv heads than one workgroup takes, every head dim, small and large pages."""
+    layers = 2
+    cache = GpuCache([8, 4096, 1024, page_size, 1], layers, hq, hkv, d, d, rope_mode=S.ROPE_INLINE)
+    sc = S.Scenario(cache, layers, hq, hkv, d, rope_mode=S.ROPE_INLINE, seed=4, tol=tol)
+    for sid, (window, sink) in enumerate([(40, 0), (130, 4), (257, 30)]):
+        sc.add_with_window(sid, window, sink)
+    for batch in ([(0, 17), (1, 128), (2, 200)], [(0, 70), (1, 1), (2, 130)], [(3, 65), (2, 90), (0, 40)],
+                  [(0, 33), (1, 129), (2, 1), (3, 16)], [(0, 1), (1, 1), (2, 1), (3, 1)], [(1, 64), (2, 63)]):
+        sc.step(list(batch))
+
+
+@pytest.mark.parametrize("page_size,d,rope_mode", [(24, 128, 1), (5, 64, 1), (12, 256, 1), (40, 96, 0), (16, 128, 2), (16, 112, 2)])
+def test_prefill_steps_of_other_caches_over_gathered_keys(page_size, d, rope_mode):
+    """The same for caches without windows: pages the tuned kernels do not walk (keys kept rotated or never rotated) and
+    RoPE inside the kernels, next to decode steps and forks, against the oracle cache."""
+    m = Mirror([8, 2048, 512, page_size, 0], 2, 8, 2, d, rope_mode=rope_mode)
+    m.step([(0, 60), (1, 88), (2, 17)])
+    m.step([(0, 64), (1, 1), (2, 130)])
+    m.step([(0, 1), (1, 1), (2, 1)])
+    m.step([(0, 15), (1, 90), (3, 33)])
+    m.step([((4, 1, 40), 25), (0, 2)])
+
+
 def test_short_chunk_against_a_long_cached_sequence():
     """A chunk of a few tokens against thousands of cached ones is one or two row tiles per kv head: the
     launch splits their keys over several workgroups and merges the states.  Through the cache's one-pass

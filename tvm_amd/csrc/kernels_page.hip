@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void transpose_append_kernel(half_t* __restric
                                                                const half_t* __restrict__ v_data,
                                                                const int32_t* __restrict__ position_map,
                                                                int64_t ntoken, int num_kv_heads, int page_size,
-                                                               int head_dim) {
+                                                               int head_dim, int64_t token_stride) {
   const int chunks = head_dim / 8;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const int c = gid % chunks;
@@ -179,8 +179,9 @@ __global__ __launch_bounds__(256) void transpose_append_kernel(half_t* __restric
   const int64_t head_stride = static_cast<int64_t>(page_size) * head_dim;
   half_t* kdst = pages + ((page * 2 + 0) * num_kv_heads + h) * head_stride + slot * head_dim + c * 8;
   half_t* vdst = kdst + num_kv_heads * head_stride;
-  st16(kdst, ld16(k_data + row * head_dim + c * 8));
-  st16(vdst, ld16(v_data + row * head_dim + c * 8));
+  const int64_t src = i * token_stride + h * head_dim + c * 8;
+  st16(kdst, ld16(k_data + src));
+  st16(vdst, ld16(v_data + src));
 }
 
 __global__ __launch_bounds__(256) void transpose_append_mla_kernel(half_t* __restrict__ pages,
@@ -427,6 +428,157 @@ __global__ __launch_bounds__(256) void merge_state_inplace_f32_kernel(float* __r
   if (lane_in_row == 0) s[row] = log2f(s_val + s_other_val) + s_max;
 }
 
+// ------------------------------------------------------------------------------------------
+// gather_kv: cached and new keys / values of a step as contiguous rows, keys (and queries) rotated on the way.
+//
+// RoPE inside an attention kernel is redone by every row tile that reads a key, on the vector ALU in front of the
+// matrix work: a prefill step of a sliding-window cache (6 sequences, 2047 cached + 100-1000 new tokens each, 32 heads
+// of dim 96) spent 721 us in each of its two attention launches per layer, 1525 us with everything around them against 363
+// us now.  Here every key is rotated once, window and
+// sinks become one run of logical keys, and the plain ragged kernel does the rest; any page size ends in the same
+// layout.  The pass is bound by HBM: K and V of the step in and out once.
+//
+// A workgroup owns 16 consecutive destination rows and a run of heads.  The first 16 threads find the source of a row
+// each (a binary search over kv_indptr, one page-table lookup), all 256 fill the 16 x d/2 table of (cos, sin), which the
+// heads share, and then a thread moves the two 16-byte pieces of a rotated pair (or two pieces of a v row) at a time.
+// ------------------------------------------------------------------------------------------
+struct GatherParams {
+  const half_t* pages;
+  const int32_t* page_indptr;
+  const int32_t* page_values;
+  const int32_t* last_page_len;
+  const int32_t* window_offset;  // NULL: not a sliding-window cache
+  const int32_t* sink_size;
+  const int32_t* k_rope_pos_offset;
+  const int32_t* q_indptr;
+  const int32_t* kv_indptr;
+  const int32_t* q_rope_position;
+  const half_t* q_new;
+  const half_t* k_new;
+  const half_t* v_new;
+  int64_t q_stride, kv_stride;
+  half_t* k_out;
+  half_t* v_out;
+  half_t* q_out;  // NULL: the queries are left alone
+  int64_t kv_rows;
+  int batch, h_q, h_kv, d, page_size, rotate;
+  int kv_groups;  // blockIdx.y < kv_groups: kGatherHeads kv heads; behind them: kGatherHeads query heads of the new rows
+  float rope_scale;
+};
+constexpr int kGatherRows = 16, kGatherHeads = 8;
+
+__global__ __launch_bounds__(256) void gather_kv_kernel(GatherParams p, InlineRopeTable rope) {
+  extern __shared__ float angle_lds[];  // [rows][width] cos, then [rows][width] sin; width = d / 2, or d when the halves differ
+  __shared__ const half_t* src_lds[kGatherRows][3];  // k row of head 0, v row of head 0, q row of head 0 (NULL: not a new token)
+  __shared__ int64_t head_stride_lds[kGatherRows];   // elements between the heads of the k / v row
+  __shared__ float pos_lds[kGatherRows];
+  __shared__ int q_row_lds[kGatherRows];
+  const int tid = threadIdx.x;
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kGatherRows;
+  const int rows = static_cast<int>(min(static_cast<int64_t>(kGatherRows), p.kv_rows - row0));
+  const bool queries = static_cast<int>(blockIdx.y) >= p.kv_groups;
+  if (tid < rows) {
+    const int row = static_cast<int>(row0) + tid;
+    int lo = 0, hi = p.batch - 1;  // the last sequence whose rows start at or before this one
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (p.kv_indptr[mid] <= row) lo = mid; else hi = mid - 1;
+    }
+    const int b = lo;
+    const int t = row - p.kv_indptr[b];
+    const int q0 = p.q_indptr[b];
+    const int cached = p.kv_indptr[b + 1] - p.kv_indptr[b] - (p.q_indptr[b + 1] - q0);
+    float pos;
+    if (t < cached) {
+      int phys = t;
+      if (p.window_offset != nullptr) {
+        const int sink = p.sink_size[b];
+        if (t >= sink) phys = t - sink + p.window_offset[b];
+      }
+      const int entry = phys / p.page_size;
+      const int64_t page = p.page_values[p.page_indptr[b] + entry];
+      const int64_t page_elems = static_cast<int64_t>(p.page_size) * p.d;
+      const half_t* k = p.pages + page * 2 * p.h_kv * page_elems + (phys - entry * p.page_size) * p.d;
+      src_lds[tid][0] = k;
+      src_lds[tid][1] = k + p.h_kv * page_elems;
+      src_lds[tid][2] = nullptr;
+      head_stride_lds[tid] = page_elems;
+      q_row_lds[tid] = -1;
+      pos = static_cast<float>((p.k_rope_pos_offset != nullptr ? p.k_rope_pos_offset[b] : 0) + t);
+    } else {
+      const int i = q0 + t - cached;
+      src_lds[tid][0] = p.k_new + i * p.kv_stride;
+      src_lds[tid][1] = p.v_new + i * p.kv_stride;
+      src_lds[tid][2] = p.q_new != nullptr ? p.q_new + i * p.q_stride : nullptr;
+      head_stride_lds[tid] = p.d;
+      q_row_lds[tid] = i;
+      pos = p.rotate ? static_cast<float>(p.q_rope_position[i]) : 0.f;
+    }
+    pos_lds[tid] = pos * p.rope_scale;
+  }
+  __syncthreads();
+  if (queries) {  // uniform: nothing to do unless one of the rows is a new token
+    bool any = false;
+    for (int r = 0; r < rows; ++r) any |= q_row_lds[r] >= 0;
+    if (!any) return;
+  }
+  const int d = p.d, half_d = d / 2;
+  const int width = rope.halves_differ ? d : half_d;
+  float* cs_lds = angle_lds;
+  float* sn_lds = angle_lds + kGatherRows * width;
+  if (p.rotate) {
+    for (int i = tid; i < rows * width; i += 256) {
+      const int r = i / width, f = i - r * width;
+      float sn, cs;
+      sincos_reduced(rope.inverse ? pos_lds[r] * rope.v[f] : pos_lds[r] / rope.v[f], sn, cs);
+      cs_lds[i] = cs * rope.magnitude;
+      sn_lds[i] = sn * rope.magnitude;
+    }
+    __syncthreads();
+  }
+  const int pairs = d / 16;  // pairs of 16-byte pieces of a row
+  const int hi_off = rope.halves_differ ? half_d : 0;
+  auto rotate = [&](Vec16& lo, Vec16& hi, int r, int c) {
+    const float* cs = cs_lds + r * width + c * 8;
+    const float* sn = sn_lds + r * width + c * 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float xl = static_cast<float>(lo.h8[e]), xh = static_cast<float>(hi.h8[e]);
+      lo.h8[e] = static_cast<half_t>(cs[e] * xl + sn[e] * (-xh));
+      hi.h8[e] = static_cast<half_t>(cs[hi_off + e] * xh + sn[hi_off + e] * xl);
+    }
+  };
+  const int head0 = (queries ? static_cast<int>(blockIdx.y) - p.kv_groups : static_cast<int>(blockIdx.y)) * kGatherHeads;
+  const int heads = min(kGatherHeads, (queries ? p.h_q : p.h_kv) - head0);
+  const int per_row = heads * pairs;
+  // piece fastest, then the head: consecutive threads write consecutive pieces of a destination row
+  for (int i = tid; i < rows * per_row; i += 256) {
+    const int r = i / per_row, rest = i - r * per_row;
+    const int h = head0 + rest / pairs, c = rest % pairs;
+    if (queries) {
+      if (q_row_lds[r] < 0) continue;
+      const half_t* src = src_lds[r][2] + static_cast<int64_t>(h) * d + c * 8;
+      Vec16 lo = ld16(src), hi = ld16(src + half_d);
+      if (p.rotate) rotate(lo, hi, r, c);
+      half_t* dst = p.q_out + (static_cast<int64_t>(q_row_lds[r]) * p.h_q + h) * d + c * 8;
+      st16(dst, lo);
+      st16(dst + half_d, hi);
+      continue;
+    }
+    const int64_t src_off = h * head_stride_lds[r] + c * 8;
+    const half_t* ksrc = src_lds[r][0] + src_off;
+    const half_t* vsrc = src_lds[r][1] + src_off;
+    Vec16 lo = ld16(ksrc), hi = ld16(ksrc + half_d);
+    const Vec16 vlo = ld16(vsrc), vhi = ld16(vsrc + half_d);
+    if (p.rotate) rotate(lo, hi, r, c);
+    const int64_t dst = ((row0 + r) * p.h_kv + h) * d + c * 8;
+    st16(p.k_out + dst, lo);
+    st16(p.k_out + dst + half_d, hi);
+    st16(p.v_out + dst, vlo);
+    st16(p.v_out + dst + half_d, vhi);
+  }
+}
+
 inline dim3 grid_for(int64_t threads, int block = 256) { return dim3(static_cast<unsigned>((threads + block - 1) / block)); }
 
 }  // namespace tvmkv
@@ -650,9 +802,8 @@ static void check_slot_layout(const char* what, int32_t page_size, int32_t head_
   KV_CHECK(head_dim > 0 && head_dim % 8 == 0) << what << ": feature dim " << head_dim << " must be a multiple of 8";
 }
 
-int tvmkv_kv_cache_transpose_append(void* pages, const void* k_data, const void* v_data,
-                                    const int32_t* position_map, int64_t ntoken, int64_t num_pages,
-                                    int32_t num_kv_heads, int32_t page_size, int32_t head_dim, void* stream) {
+static int append_impl(void* pages, const void* k_data, const void* v_data, int64_t token_stride, const int32_t* position_map,
+                       int64_t ntoken, int64_t num_pages, int32_t num_kv_heads, int32_t page_size, int32_t head_dim, void* stream) {
   KV_API_BEGIN();
   check_slot_layout("transpose_append", page_size, head_dim);
   KV_CHECK(ntoken >= 0 && num_kv_heads > 0) << "transpose_append: bad shape";
@@ -662,9 +813,16 @@ int tvmkv_kv_cache_transpose_append(void* pages, const void* k_data, const void*
   const int64_t threads = ntoken * num_kv_heads * (head_dim / 8);
   hipLaunchKernelGGL(transpose_append_kernel, grid_for(threads), dim3(256), 0, as_stream(stream),
                      static_cast<half_t*>(pages), static_cast<const half_t*>(k_data),
-                     static_cast<const half_t*>(v_data), position_map, ntoken, num_kv_heads, page_size, head_dim);
+                     static_cast<const half_t*>(v_data), position_map, ntoken, num_kv_heads, page_size, head_dim, token_stride);
   KV_LAUNCH_CHECK();
   KV_API_END();
+}
+
+int tvmkv_kv_cache_transpose_append(void* pages, const void* k_data, const void* v_data,
+                                    const int32_t* position_map, int64_t ntoken, int64_t num_pages,
+                                    int32_t num_kv_heads, int32_t page_size, int32_t head_dim, void* stream) {
+  return append_impl(pages, k_data, v_data, static_cast<int64_t>(num_kv_heads) * head_dim, position_map, ntoken, num_pages,
+                     num_kv_heads, page_size, head_dim, stream);
 }
 
 int tvmkv_kv_cache_transpose_append_mla(void* pages, const void* kv_data, const int32_t* position_map,
@@ -803,6 +961,66 @@ int typed_merge_state_inplace(int elem_bits, void* v, float* s, const void* v_ot
   const int64_t rows = n * h;
   hipLaunchKernelGGL(merge_state_inplace_f32_kernel, grid_for(rows * lanes_per_row), dim3(256), 0, as_stream(stream),
                      static_cast<float*>(v), s, static_cast<const float*>(v_other), s_other, rows, d, lanes_per_row);
+  KV_LAUNCH_CHECK();
+  KV_API_END();
+}
+
+int append_strided(void* pages, const void* k_data, const void* v_data, int64_t token_stride, const int32_t* position_map,
+                   int64_t ntoken, int64_t num_pages, int32_t num_kv_heads, int32_t page_size, int32_t head_dim, void* stream) {
+  return append_impl(pages, k_data, v_data, token_stride, position_map, ntoken, num_pages, num_kv_heads, page_size, head_dim, stream);
+}
+
+int gather_kv(const GatherKV& a, void* stream) {
+  KV_API_BEGIN();
+  KV_CHECK(a.batch > 0 && a.h_q > 0 && a.h_kv > 0 && a.d > 0 && a.d <= kMaxHeadDim && a.d % 16 == 0 && a.page_size > 0)
+      << "gather_kv: bad shape";
+  KV_CHECK(a.kv_rows >= 0 && a.kv_rows < (int64_t{1} << 31)) << "gather_kv: too many rows";
+  if (a.kv_rows == 0) return TVMKV_OK;
+  KV_CHECK(a.pages && a.page_indptr && a.length_info && a.q_indptr && a.kv_indptr && a.k_new && a.v_new && a.k_out && a.v_out)
+      << "gather_kv: NULL tensor";
+  KV_CHECK(!a.rotate || a.q_rope_position) << "gather_kv: NULL positions";
+  KV_CHECK((a.q_out == nullptr) == (a.q_new == nullptr)) << "gather_kv: q_new and q_out come together";
+  GatherParams p{};
+  p.pages = static_cast<const half_t*>(a.pages);
+  p.page_indptr = a.page_indptr;
+  p.page_values = a.page_values;
+  p.last_page_len = a.length_info;
+  p.window_offset = a.sliding ? a.length_info + a.batch : nullptr;
+  p.sink_size = a.sliding ? a.length_info + 2 * static_cast<int64_t>(a.batch) : nullptr;
+  p.k_rope_pos_offset = a.k_rope_pos_offset;
+  p.q_indptr = a.q_indptr;
+  p.kv_indptr = a.kv_indptr;
+  p.q_rope_position = a.q_rope_position;
+  p.q_new = static_cast<const half_t*>(a.q_new);
+  p.k_new = static_cast<const half_t*>(a.k_new);
+  p.v_new = static_cast<const half_t*>(a.v_new);
+  p.q_stride = a.q_stride;
+  p.kv_stride = a.kv_stride;
+  p.k_out = static_cast<half_t*>(a.k_out);
+  p.v_out = static_cast<half_t*>(a.v_out);
+  p.q_out = static_cast<half_t*>(a.q_out);
+  p.kv_rows = a.kv_rows;
+  p.batch = a.batch;
+  p.h_q = a.h_q;
+  p.h_kv = a.h_kv;
+  p.d = a.d;
+  p.page_size = a.page_size;
+  p.rotate = a.rotate != 0;
+  p.rope_scale = static_cast<float>(a.rope_scale);
+  p.kv_groups = (a.h_kv + kGatherHeads - 1) / kGatherHeads;
+  InlineRopeTable rope{};
+  rope.magnitude = 1.0f;
+  if (p.rotate) {
+    const InlineRopeHost table = inline_rope_table(a.rope_scaling, a.d, a.rope_theta);
+    for (int i = 0; i < a.d; ++i) rope.v[i] = table.v[i];
+    rope.inverse = table.inverse;
+    rope.halves_differ = table.halves_differ;
+    rope.magnitude = table.magnitude;
+  }
+  const int q_groups = p.q_out != nullptr ? (a.h_q + kGatherHeads - 1) / kGatherHeads : 0;
+  const size_t lds = p.rotate ? 2 * kGatherRows * (rope.halves_differ ? a.d : a.d / 2) * sizeof(float) : 0;  // 32 KiB at most
+  hipLaunchKernelGGL(gather_kv_kernel, dim3(static_cast<unsigned>((a.kv_rows + kGatherRows - 1) / kGatherRows), p.kv_groups + q_groups),
+                     dim3(256), lds, as_stream(stream), p, rope);
   KV_LAUNCH_CHECK();
   KV_API_END();
 }

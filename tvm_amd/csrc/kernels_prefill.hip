@@ -230,7 +230,8 @@ __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 
   // number of logical keys -> physical end of the tokens that hold them
   auto to_phys = [&](int n) { return (!EXT || n <= sink) ? n : n - sink + win_lo; };
   __shared__ float div_lds[DQK > 256 ? 256 : DQK];
-  const bool q_rope = (EXT && p.rotary) || (BOTH && p.q_inline_rope != 0);  // uniform over the launch
+  // uniform over the launch
+  const bool q_rope = (EXT && p.rotary) || (!EXT && !PAGED && !PAD && DQK == DV && p.q_inline_rope != 0);
   if (q_rope) {
     if (tid < DQK && tid < 256) div_lds[tid] = div.v[tid];
     __syncthreads();
@@ -983,6 +984,47 @@ static void launch_prefill_padded(PrefillParams p, int64_t total_q, int d, bool 
 }  // namespace tvmkv
 
 using namespace tvmkv;
+
+int tvmkv::prefill_over_gathered_kv(const void* q, int64_t q_token_stride, const int32_t* q_rope_position, int64_t apply_rope,
+                                    double rope_scale, double rope_theta, const int32_t* q_indptr, const void* k, const void* v,
+                                    const int32_t* kv_indptr, void* output, float* lse, double sm_scale, int32_t batch_size,
+                                    int64_t total_q, int32_t h_q, int32_t h_kv, int32_t d, void* stream) {
+  KV_API_BEGIN();
+  KV_CHECK(batch_size > 0 && total_q > 0 && h_q > 0 && h_kv > 0 && h_q % h_kv == 0) << "prefill_over_gathered_kv: bad shape";
+  KV_CHECK(q && q_indptr && k && v && kv_indptr && output && lse) << "prefill_over_gathered_kv: NULL tensor";
+  KV_CHECK(!apply_rope || (q_rope_position && !padded_head_dim(d))) << "prefill_over_gathered_kv: rotation of the queries";
+  PrefillParams p{};
+  p.q = static_cast<const half_t*>(q);
+  p.q_token_stride = q_token_stride;
+  p.q_inline_rope = apply_rope != 0;
+  p.q_rope_position = q_rope_position;
+  p.rope_scale = static_cast<float>(rope_scale);
+  p.q_indptr = q_indptr;
+  p.k = static_cast<const half_t*>(k);
+  p.v = static_cast<const half_t*>(v);
+  p.kv_indptr = kv_indptr;
+  p.output = static_cast<half_t*>(output);
+  p.lse = lse;
+  p.batch_size = batch_size;
+  p.h_q = h_q;
+  p.h_kv = h_kv;
+  p.group = h_q / h_kv;
+  p.causal = 1;
+  p.scale_log2 = static_cast<float>(sm_scale) * kLog2e;
+  hipStream_t s = as_stream(stream);
+  if (d == 128) {
+    launch_prefill<128, 128, kRagged, 16>(p, total_q, false, rope_theta, s);
+  } else if (d == 64) {
+    launch_prefill<64, 64, kRagged, 16>(p, total_q, false, rope_theta, s);
+  } else if (d == 256) {
+    launch_prefill<256, 256, kRagged, 16>(p, total_q, false, rope_theta, s);
+  } else {
+    KV_UNSUPPORTED(!padded_head_dim(d)) << "prefill_over_gathered_kv: head_dim " << d;
+    launch_prefill_padded<kRagged>(p, total_q, d, false, "prefill_over_gathered_kv", s);
+  }
+  KV_LAUNCH_CHECK();
+  KV_API_END();
+}
 
 extern "C" {
 

@@ -86,6 +86,10 @@ class PagedKVCache {
           << "multiple of " << (elem_bits_ == 32 ? 8 : 16) << ", got " << head_dim;
       KV_UNSUPPORTED(qk_head_dim_ != v_head_dim_) << "the generic kernels need equal qk and v head dims";
     }
+    // Prefill steps that the tuned kernels take only with RoPE, a window or an odd page size inside them: fp16 storage, a
+    // tuned head dim, and what GatheredPrefillApplies() asks of the step.
+    gather_capable_ = has_mha_layer && !has_mla && elem_bits_ == 16 && qk_head_dim_ == v_head_dim_ && tuned_head_dim(head_dim) &&
+                      (support_sliding_window_ || rope_mode_ == TVMKV_ROPE_INLINE || !tuned_page_size(static_cast<int>(page_size_)));
     KV_CHECK(static_cast<int64_t>(attn_kinds_.size()) >= layer_end)
         << "attn_kinds must cover every layer id up to " << layer_end;
     for (int64_t kind : attn_kinds_) {
@@ -147,10 +151,11 @@ class PagedKVCache {
       const int next = aux_slot_ ^ 1;
       // this slot's staging memory was last read by the upload two steps ago
       if (aux_slot_used_[next]) HIP_CHECK(hipEventSynchronize(aux_copied_[next]));
-      book_->SetStepBuffer(static_cast<int32_t*>(aux_staging_[next]), aux_capacity_);
+      book_->SetStepBuffer(static_cast<int32_t*>(aux_staging_[next]) + extras_capacity_, aux_capacity_);
       aux_needs_upload_ = false;
       book_->BeginForward(seq_ids, append_lengths, batch_size, token_tree_parent_ptr, n_tree);
       aux_slot_ = next;
+      PlanStep();
       aux_needs_upload_ = true;
     } else {
       book_->BeginForward(seq_ids, append_lengths, batch_size, token_tree_parent_ptr, n_tree);
@@ -183,6 +188,11 @@ class PagedKVCache {
     const StepLayout& s = book_->step();
     const bool rope_normal = rope_mode_ == TVMKV_ROPE_NORMAL;
 
+    if (gathered_rows_ > 0 && attn_kinds_[layer_id] == TVMKV_ATTN_MHA) {
+      GatheredPrefill(local_layer_id, qkv, out, total_seq_length, sm_scale);
+      RecordComputeEvent();
+      return;
+    }
     // A chunked-prefill step of a plain cache in two launches: k is rotated and the new k / v rows go
     // into their page slots (part 2 without q, part 3), then one pass over the cached and the new
     // tokens that reads the queries from qkv and rotates them itself (parts 2 and 5).
@@ -501,7 +511,11 @@ class PagedKVCache {
   }
   // Device address of an array of the current step (nullptr when the step does not have it).
   const int32_t* Dev(const AuxSpan& span) const {
-    return span.present() ? static_cast<const int32_t*>(aux_device_[aux_slot_]) + span.offset : nullptr;
+    return span.present() ? static_cast<const int32_t*>(aux_device_[aux_slot_]) + extras_capacity_ + span.offset : nullptr;
+  }
+  // The same for the plan of the step (PlanStep): `offset` elements into extras_.
+  const int32_t* DevExtra(int64_t offset) const {
+    return static_cast<const int32_t*>(aux_device_[aux_slot_]) + extras_capacity_ - static_cast<int64_t>(extras_.size()) + offset;
   }
 
   void InitDevice() {
@@ -523,9 +537,15 @@ class PagedKVCache {
       HIP_CHECK(hipMalloc(&temp_lse_, prefill_chunk_size_ * num_qo_heads_ * sizeof(float)));
       HIP_CHECK(hipMalloc(&merged_lse_, prefill_chunk_size_ * num_qo_heads_ * sizeof(float)));
       aux_capacity_ = book_->RequiredCapacity();
+      extras_capacity_ = (reserved_num_seqs_ + 1 + 3) / 4 * 4;
+      if (gather_capable_) {
+        const int64_t row_bytes = 2 * num_kv_heads_ * qk_head_dim_ * static_cast<int64_t>(sizeof(uint16_t));
+        gather_capacity_ = std::min(num_total_pages_ * page_size_ + prefill_chunk_size_, kGatherBytes / row_bytes);
+        HIP_CHECK(hipMalloc(&gather_, gather_capacity_ * row_bytes));
+      }
       for (int i = 0; i < 2; ++i) {
-        HIP_CHECK(hipMalloc(&aux_device_[i], aux_capacity_ * sizeof(int32_t)));
-        HIP_CHECK(hipHostMalloc(&aux_staging_[i], aux_capacity_ * sizeof(int32_t), hipHostMallocDefault));
+        HIP_CHECK(hipMalloc(&aux_device_[i], (extras_capacity_ + aux_capacity_) * sizeof(int32_t)));
+        HIP_CHECK(hipHostMalloc(&aux_staging_[i], (extras_capacity_ + aux_capacity_) * sizeof(int32_t), hipHostMallocDefault));
         HIP_CHECK(hipEventCreateWithFlags(&aux_copied_[i], hipEventDisableTiming));
         HIP_CHECK(hipEventCreateWithFlags(&aux_consumed_[i], hipEventDisableTiming));
       }
@@ -548,7 +568,7 @@ class PagedKVCache {
     (void)hipSetDevice(device_);
     for (void* p : pages_) (void)hipFree(p);
     pages_.clear();
-    for (void** p : {&temp_q_, &temp_k_, &temp_v_, &temp_out_}) {
+    for (void** p : {&temp_q_, &temp_k_, &temp_v_, &temp_out_, &gather_}) {
       (void)hipFree(*p);
       *p = nullptr;
     }
@@ -681,6 +701,109 @@ class PagedKVCache {
     return !generic_ && !s.append_before_attn && s.num_depths == 1 && s.is_chain[0] && !s.use_decode_kernel[0] &&
            s.page_indices[0].size > 0 && !support_sliding_window_ && attn_kinds_[layer_id] == TVMKV_ATTN_MHA &&
            rope_mode_ != TVMKV_ROPE_INLINE && qk_head_dim_ == v_head_dim_ && (qk_head_dim_ == 64 || qk_head_dim_ == 128);
+  }
+
+  // What the kernels of this step need beside the bookkeeper's arrays, written in front of them in the staging buffer.
+  void PlanStep() {
+    extras_.clear();
+    gathered_rows_ = 0;
+    const StepLayout& s = book_->step();
+    const int64_t batch = book_->batch_size();
+    if (gather_capable_ && rope_ext_factors_ == nullptr && s.num_depths == 1 && s.is_chain[0] && !s.append_before_attn &&
+        !s.use_decode_kernel[0] &&
+        s.total_append_length * (num_qo_heads_ / num_kv_heads_) >=
+            batch * (rope_mode_ == TVMKV_ROPE_INLINE ? kGatherMinRowsRotated : kGatherMinRows)) {
+      const int32_t* host = book_->step_buffer();
+      const int32_t* page_indptr = host + s.page_indptr[0].offset;
+      const int32_t* last_len = host + s.last_page_len[0].offset;
+      const int32_t* window_offset = host + s.sliding_window_offset[0].offset;
+      const int32_t* sink = host + s.sink_size[0].offset;
+      const int32_t* append_indptr = host + s.cur_append_lengths_indptr.offset;
+      extras_.assign((batch + 1 + 3) / 4 * 4, 0);
+      int64_t rows = 0;
+      for (int64_t b = 0; b < batch; ++b) {
+        const int64_t pages = page_indptr[b + 1] - page_indptr[b];
+        if (pages > 0) {
+          rows += (pages - 1) * page_size_ + last_len[b];
+          if (support_sliding_window_) rows += sink[b] - window_offset[b];
+        }
+        rows += append_indptr[b + 1] - append_indptr[b];
+        extras_[b + 1] = static_cast<int32_t>(std::min<int64_t>(rows, INT32_MAX));
+      }
+      if (rows <= gather_capacity_) gathered_rows_ = rows; else extras_.clear();
+    }
+    if (!extras_.empty()) {
+      std::memcpy(static_cast<int32_t*>(aux_staging_[aux_slot_]) + extras_capacity_ - extras_.size(), extras_.data(),
+                  extras_.size() * sizeof(int32_t));
+    }
+  }
+
+  // A prefill step of a cache with sliding windows, RoPE inside attention or pages that the tuned kernels do not walk:
+  // cached and new keys become one run of logical keys per sequence, rotated on the way where the cache keeps them
+  // unrotated, and the plain ragged kernel attends to them in one pass (parts 2 and 5); the rows go into their page
+  // slots behind it (part 6), where a cache without windows has had them written already.
+  void GatheredPrefill(int64_t local_layer_id, const void* qkv, void* out, int64_t total_seq_length, double sm_scale) {
+    const StepLayout& s = book_->step();
+    const bool inline_rope = rope_mode_ == TVMKV_ROPE_INLINE;
+    const int64_t d = qk_head_dim_, fused_stride = (num_qo_heads_ + 2 * num_kv_heads_) * d;
+    const uint16_t* rows = static_cast<const uint16_t*>(qkv);
+    GatherKV g;
+    g.pages = pages_[local_layer_id];
+    g.page_indptr = Dev(s.page_indptr[0]);
+    g.page_values = Dev(s.page_indices[0]);
+    g.length_info = Dev(s.length_info[0]);
+    g.k_rope_pos_offset = Dev(s.k_rope_pos_offset[0]);
+    g.q_indptr = Dev(s.cur_append_lengths_indptr);
+    g.kv_indptr = DevExtra(0);
+    g.q_rope_position = Dev(s.q_rope_position_map);
+    g.k_out = gather_;
+    g.v_out = static_cast<uint16_t*>(gather_) + gathered_rows_ * num_kv_heads_ * d;
+    g.kv_rows = gathered_rows_;
+    g.batch = static_cast<int32_t>(book_->batch_size());
+    g.h_q = static_cast<int32_t>(num_qo_heads_);
+    g.h_kv = static_cast<int32_t>(num_kv_heads_);
+    g.d = static_cast<int32_t>(d);
+    g.page_size = static_cast<int32_t>(page_size_);
+    g.sliding = support_sliding_window_;
+    g.rotate = inline_rope;
+    g.rope_scale = rotary_scale_;
+    g.rope_theta = rotary_theta_;
+    g.rope_scaling = InlineScaling();
+    const void* q = qkv;
+    int64_t q_stride = fused_stride;
+    bool rotate_q = inline_rope;  // inside the attention kernel, for the head dims and frequencies it is built for
+    const bool rows_from_qkv = rope_mode_ != TVMKV_ROPE_NORMAL;
+    if (rows_from_qkv) {
+      g.k_new = rows + num_qo_heads_ * d;
+      g.v_new = rows + (num_qo_heads_ + num_kv_heads_) * d;
+      g.kv_stride = fused_stride;
+      if (inline_rope && (g.rope_scaling != nullptr || !(d == 64 || d == 128 || d == 256))) {
+        g.q_new = qkv;
+        g.q_stride = fused_stride;
+        g.q_out = temp_q_;
+        q = temp_q_;
+        q_stride = 0;
+        rotate_q = false;
+      }
+    } else {  // keys are kept rotated (pages of other sizes): split, rotate and append first
+      Launch(typed_fused_rope(elem_bits_, qkv, Dev(s.q_rope_position_map), temp_q_, temp_k_, temp_v_, /*apply_rope=*/1, nullptr,
+                              has_rope_scaling_ ? &rope_scaling_ : nullptr, pages_[local_layer_id], Dev(s.append_position_map),
+                              total_seq_length, num_qo_heads_, num_kv_heads_, qk_head_dim_, num_total_pages_, page_size_,
+                              rotary_scale_, rotary_theta_, compute_stream_));
+      g.k_new = temp_k_;
+      g.v_new = temp_v_;
+      g.kv_stride = num_kv_heads_ * d;
+      q = temp_q_;
+      q_stride = 0;
+    }
+    Launch(gather_kv(g, compute_stream_));
+    Launch(prefill_over_gathered_kv(q, q_stride, Dev(s.q_rope_position_map), rotate_q, rotary_scale_, rotary_theta_,
+                                    Dev(s.cur_append_lengths_indptr), g.k_out, g.v_out, DevExtra(0), out, merged_lse_, sm_scale,
+                                    g.batch, total_seq_length, g.h_q, g.h_kv, g.d, compute_stream_));
+    if (rows_from_qkv) {
+      Launch(append_strided(pages_[local_layer_id], g.k_new, g.v_new, fused_stride, Dev(s.append_position_map), total_seq_length,
+                            num_total_pages_, g.h_kv, g.page_size, g.d, compute_stream_));
+    }
   }
 
   // :2161-2180
@@ -936,7 +1059,10 @@ class PagedKVCache {
         // A host that runs ahead of the device must not overwrite arrays that kernels of the step
         // two uploads ago, still queued on the compute stream, have yet to read.
         if (aux_consumed_recorded_[aux_slot_]) HIP_CHECK(hipStreamWaitEvent(copy_stream_, aux_consumed_[aux_slot_], 0));
-        HIP_CHECK(hipMemcpyAsync(aux_device_[aux_slot_], aux_staging_[aux_slot_], used * sizeof(int32_t),
+        // the plan of the step lies right in front of the bookkeeper's arrays: one copy takes both
+        const int64_t plan = static_cast<int64_t>(extras_.size()), from = extras_capacity_ - plan;
+        HIP_CHECK(hipMemcpyAsync(static_cast<int32_t*>(aux_device_[aux_slot_]) + from,
+                                 static_cast<int32_t*>(aux_staging_[aux_slot_]) + from, (plan + used) * sizeof(int32_t),
                                  hipMemcpyHostToDevice, copy_stream_));
       }
       aux_slot_used_[aux_slot_] = true;
@@ -954,6 +1080,7 @@ class PagedKVCache {
   int64_t num_total_pages_ = 0, prefill_chunk_size_, reserved_num_seqs_ = 0;
   bool support_sliding_window_ = false;
   int elem_bits_ = 16;    // storage type of the MHA layers: 16 (fp16) or 32 (float32)
+  bool gather_capable_ = false;  // prefill steps may run over gathered keys (GatheredPrefill)
   bool generic_ = false;  // the MHA layers run on the typed / generic kernels (typed_kernels.h)
   int64_t layer_sliding_window_size_ = 1024;
   std::vector<int64_t> attn_kinds_;
@@ -983,6 +1110,20 @@ class PagedKVCache {
   void *temp_q_ = nullptr, *temp_k_ = nullptr, *temp_v_ = nullptr, *temp_out_ = nullptr;
   float *temp_lse_ = nullptr, *merged_lse_ = nullptr;
   int64_t aux_capacity_ = 0;
+  // the plan of the current step (PlanStep), held in front of the bookkeeper's arrays in both copies of the buffer
+  std::vector<int32_t> extras_;
+  int64_t extras_capacity_ = 0;
+  // GatheredPrefill: K and V rows of a step, at most kGatherBytes (steps with more keys take the kernels that rotate
+  // inside), and how many rows this step has (0: the step does not run that way)
+  static constexpr int64_t kGatherBytes = int64_t{1} << 30;
+  // Query rows per kv head and sequence, on average, from which the pass over the keys pays.  Measured, us per layer, the
+  // kernels that rotate / look every row's page up inside -> gathered: 32 sequences with windows of 2047 tokens, 32 / 8
+  // heads of dim 128, rows 32: 179 -> 175, 64: 211 -> 177, 128: 226 -> 180; 16 sequences, 32 / 32 heads of dim 96, rows
+  // 16: 255 -> 285, 32: 431 -> 287; pages of 24 tokens, 32 sequences of 1000-4000 tokens, 32 / 8 heads of dim 128,
+  // rows 32: 212 -> 234, 128: 317 -> 243.
+  static constexpr int64_t kGatherMinRowsRotated = 32, kGatherMinRows = 64;
+  void* gather_ = nullptr;
+  int64_t gather_capacity_ = 0, gathered_rows_ = 0;
   void* aux_device_[2] = {nullptr, nullptr};
   void* aux_staging_[2] = {nullptr, nullptr};
   hipEvent_t aux_copied_[2] = {nullptr, nullptr};

@@ -82,6 +82,47 @@ int typed_fused_rope(int elem_bits, const void* qkv, const int32_t* position_map
 int typed_merge_state_inplace(int elem_bits, void* v, float* s, const void* v_other, const float* s_other, int64_t n,
                               int32_t h, int32_t d, void* stream);
 
+// Keys and values of a step as one run of rows per sequence (fp16): the cached tokens of sequence b in logical order
+// (a sliding-window cache's sinks, then its window), then its new tokens, at rows kv_indptr[b] .. kv_indptr[b + 1] of
+// k_out / v_out (rows, h_kv, d).  Keys are rotated on the way when `rotate` (rotate-half over the whole head at
+// k_rope_pos_offset[b] + t for the cached ones, at q_rope_position[i] for the new ones: what the attention kernels
+// do with rotary_mode 1), and q_out, when given, receives the rotated queries (total_q, h_q, d).
+struct GatherKV {
+  const void* pages = nullptr;
+  const int32_t* page_indptr = nullptr;
+  const int32_t* page_values = nullptr;
+  const int32_t* length_info = nullptr;  // (batch) last page lengths, or (3, batch) with `sliding`
+  const int32_t* k_rope_pos_offset = nullptr;
+  const int32_t* q_indptr = nullptr;
+  const int32_t* kv_indptr = nullptr;
+  const int32_t* q_rope_position = nullptr;
+  const void* q_new = nullptr;  // new tokens: rows of consecutive tokens are *_stride elements apart, heads d apart
+  const void* k_new = nullptr;
+  const void* v_new = nullptr;
+  int64_t q_stride = 0, kv_stride = 0;
+  void* k_out = nullptr;
+  void* v_out = nullptr;
+  void* q_out = nullptr;
+  int64_t kv_rows = 0;  // kv_indptr[batch]
+  int32_t batch = 0, h_q = 0, h_kv = 0, d = 0, page_size = 0;
+  int32_t sliding = 0, rotate = 0;
+  double rope_scale = 1.0, rope_theta = 1e4;
+  const tvmkv_rope_scaling* rope_scaling = nullptr;
+};
+int gather_kv(const GatherKV& args, void* stream);
+
+// tvmkv_batch_prefill_ragged_kv (causal, no RoPE inside) over keys that gather_kv laid out; q_token_stride != 0: the
+// queries are read from the fused qkv tensor, rotated at q_rope_position with the default frequencies if apply_rope.
+int prefill_over_gathered_kv(const void* q, int64_t q_token_stride, const int32_t* q_rope_position, int64_t apply_rope,
+                             double rope_scale, double rope_theta, const int32_t* q_indptr, const void* k, const void* v,
+                             const int32_t* kv_indptr, void* output, float* lse, double sm_scale, int32_t batch_size,
+                             int64_t total_q, int32_t h_q, int32_t h_kv, int32_t d, void* stream);
+
+// tvmkv_kv_cache_transpose_append with the k / v rows of consecutive tokens token_stride elements apart (the fused
+// qkv tensor of the step)
+int append_strided(void* pages, const void* k_data, const void* v_data, int64_t token_stride, const int32_t* position_map,
+                   int64_t ntoken, int64_t num_pages, int32_t num_kv_heads, int32_t page_size, int32_t head_dim, void* stream);
+
 // The copy kernels move rows of head_dim elements whatever they hold: float32 rows are fp16 rows of twice
 // the length.
 inline int32_t copy_dim(int elem_bits, int32_t head_dim) { return head_dim * (elem_bits / 16); }
