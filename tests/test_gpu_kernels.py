@@ -367,6 +367,34 @@ def test_decode_sliding_cache_and_inline_rope_other_shapes(hq, hkv, d, rotary):
     assert_close(host(gl), el, atol=2e-3, rtol=1e-4, what="decode (prefill path) lse")
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 128), (8, 2, 64), (4, 2, 256), (20, 1, 128)])
+@pytest.mark.parametrize("page_size", [16, 64])
+def test_decode_inline_rope_over_the_longest_chunks(hq, hkv, d, page_size):
+    """RoPE inside the decode kernel runs its angles on from step to step: the 16 steps of the longest chunk, sinks
+    that end inside a step and on its edge, windows that start inside a page, positions in the thousands."""
+    from tests.test_oracle_kernels import sliding_case
+    rng = np.random.default_rng(27)
+    spec = [(4100, 0, 0), (4097, 4, 37), (2500, 33, 130), (300, 32, 64), (129, 128, 128), (31, 3, 17)]
+    pages, indptr, values, info, ks, _ = sliding_case(rng, spec, hkv, d, npages=sum(n for n, _, _ in spec) // page_size + 20,
+                                                      ps=page_size)
+    b = len(spec)
+    q = rng.standard_normal((b, hq, d)).astype(F16)
+    k_off = np.array([0, 5, 3000, 0, 9000, 1], np.int32)
+    q_pos = np.array([k_off[i] + len(ks[i]) for i in range(b)], np.int32)
+    eo, el = np.zeros((b, hq, d), F16), np.zeros((b, hq), np.float32)
+    ok.decode(q, pages, indptr, values, info, k_off, q_pos, eo, el, 1, 1.0, 1e4, d ** -0.5)
+    prev = tvm_amd.set_option("decode_chunk_pages", 128)
+    try:
+        go = torch.full((b, hq, d), 7.0, dtype=torch.float16, device=DEV)
+        gl = torch.full((b, hq), 7.0, dtype=torch.float32, device=DEV)
+        K.batch_decode_paged_kv(dev(q), dev(pages), i32(indptr), i32(values), i32(info), i32(k_off), i32(q_pos), go, gl,
+                                1, 1.0, 1e4, d ** -0.5)
+    finally:
+        tvm_amd.set_option("decode_chunk_pages", prev)
+    assert_close(host(go), eo, what="long chunk out")
+    assert_close(host(gl), el, atol=2e-3, rtol=1e-4, what="long chunk lse")
+
+
 # ------------------------------------------------------------------------------ prefill
 def _ragged_both(rng, lens, hq, hkv, dqk, dv, causal, scale=1.0):
     n = sum(lens)

@@ -261,6 +261,12 @@ __device__ __forceinline__ int dm_swizzle(int row) {
 struct DecodeRopeDivisors {
   float v[256];
 };
+// The extended kernels with the default frequencies: also cos and sin of the angle between a lane's neighbouring
+// keys of a step (near) and between its last key of a step and its first of the next (far), per feature pair,
+// computed in double
+struct DecodeRopeRunning : DecodeRopeDivisors {
+  float near_cos[128], near_sin[128], far_cos[128], far_sin[128];
+};
 
 // EXT = false: plain cache, q and k already rotated (or no RoPE).  EXT = true adds the sliding-window
 // cache (length_info (3, B): the page table covers `sink` tokens at the front, evicted tokens up to
@@ -285,7 +291,7 @@ struct DecodeRopeDivisors {
 // rotation made every extended launch spill (46-143 registers) while they sat in the same kernel.
 template <bool EXT, int D, bool REREAD, int HB = 1, bool FUSED = false, bool PAD = false, bool VARIANT = false>
 __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void decode_mfma_kernel(DecodeParams p, int group, int num_items,
-                                                             DecodeRopeDivisors div) {
+    std::conditional_t<EXT && !VARIANT, DecodeRopeRunning, DecodeRopeDivisors> div) {
   static_assert(HB == 1 || HB == 2, "head blocks per work item");
   static_assert(!(FUSED && EXT), "the fused step exists for the plain cache");
   static_assert(!PAD || (!EXT && !FUSED), "padded head dims: plain cache, no in-kernel RoPE");
@@ -307,6 +313,9 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   __shared__ float sm_m[4][16];
   __shared__ float sm_l[4][16];
   __shared__ int sm_last;
+  constexpr bool RUNNING = EXT && !VARIANT;  // keys rotate by running angles, see below
+  constexpr int TSTEP = KLINE ? 8 : 16;      // distance of a lane's neighbouring keys
+  __shared__ __attribute__((aligned(16))) float rope_lds[RUNNING ? 5 : 1][RUNNING ? D / 2 : 1];
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
@@ -350,16 +359,42 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   // RoPE divisors of the first halves of this lane's K fragment pairs: features i*32 + g4*8 + e, or
   // with KLINE i*64 + (c16&1)*32 + g4*8 + e
   // (and of the second halves, features + D/2, which differ from the first in some frequency variants)
-  float divr[8 * (NPAIR > 0 ? NPAIR : 1)], divh[VARIANT ? 8 * (NPAIR > 0 ? NPAIR : 1) : 1];
+  auto pair_feature = [&](int i) {
+    return KLINE ? (i >> 3) * 64 + (c16 & 1) * 32 + g4 * 8 + (i & 7) : (i >> 3) * 32 + g4 * 8 + (i & 7);
+  };
+  float divr[VARIANT ? 8 * NPAIR : 1], divh[VARIANT ? 8 * NPAIR : 1];
+  float run_cos[RUNNING ? 8 * NPAIR : 1], run_sin[RUNNING ? 8 * NPAIR : 1];
   float k_pos0 = 0.f;
+  // Angles of the keys.  A lane's keys of a step are TSTEP tokens apart and have the same frequencies, so one sine and
+  // cosine per frequency and work item are enough: the next keys' and the next step's come by rotating (run_cos,
+  // run_sin) by fixed angles.  A division, a reduction and two transcendentals for each of a lane's 32 (key, frequency)
+  // pairs of a step kept the vector ALU busy for longer than the step's 16 KiB take to arrive (64 sequences with
+  // windows of 4096 tokens, 32 / 8 heads of dim 128: 247 us a layer, 206 now).  The fixed angles come from the host in
+  // double, so that after the 16 steps of the longest chunk the drift is a few 2^-24 -- the fp32 angle itself is off by
+  // more.  They wait in LDS: in registers they made every extended launch of head dim 128 spill.
   if (EXT && p.rotary) {
+    k_pos0 = static_cast<float>(p.k_rope_pos_offset[b]);
+    if constexpr (RUNNING) {
+      if (tid < D / 2) {
+        rope_lds[0][tid] = div.v[tid];
+        rope_lds[1][tid] = div.near_cos[tid];
+        rope_lds[2][tid] = div.near_sin[tid];
+        rope_lds[3][tid] = div.far_cos[tid];
+        rope_lds[4][tid] = div.far_sin[tid];
+      }
+      __syncthreads();
+    }
+    const int first = (page_lo + 2 * wave) * PS + (KLINE ? c16 >> 1 : c16);
+    const float pos = (k_pos0 + static_cast<float>(first - win_lo + sink)) * p.rope_scale;
 #pragma unroll
     for (int i = 0; i < 8 * NPAIR; ++i) {
-      const int f = KLINE ? (i >> 3) * 64 + (c16 & 1) * 32 + g4 * 8 + (i & 7) : (i >> 3) * 32 + g4 * 8 + (i & 7);
-      divr[i] = div.v[f];
-      if constexpr (VARIANT) divh[i] = div.v[f + D / 2];
+      if constexpr (RUNNING) {
+        sincos_reduced(pos / rope_lds[0][pair_feature(i)], run_sin[i], run_cos[i]);
+      } else {
+        divr[i] = div.v[pair_feature(i)];
+        divh[i] = div.v[pair_feature(i) + D / 2];
+      }
     }
-    k_pos0 = static_cast<float>(p.k_rope_pos_offset[b]);
   }
 
   // The fused step's append: every work item of the sequence's last chunk writes the new token's k row
@@ -552,7 +587,40 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
     const bool partial = EXT ? !((pi * PS >= win_lo && (pi + 2) * PS <= kv_len) || (pi + 2) * PS <= sink)
                              : (pi + 2) * PS > kv_len;
     auto attended = [&](int t) { return EXT ? (t < sink || (t >= win_lo && t < kv_len)) : t < kv_len; };
-    if (EXT && p.rotary) {
+    if constexpr (RUNNING) {
+      if (p.rotary) {
+        // attention sinks and the keys beside them (wave-uniform): every key by its own angle
+        const bool at_sinks = pi * PS < sink;
+#pragma unroll
+        for (int n = 0; n < 2 * PS / TSTEP; ++n) {  // this lane's keys, TSTEP tokens apart
+          Vec16* frag = KLINE ? r.k[n >> 1] + (n & 1) * TI : r.k[n];
+          const int t = pi * PS + n * TSTEP + (KLINE ? c16 >> 1 : c16);
+          const float pos = (k_pos0 + static_cast<float>(t < sink ? t : t - win_lo + sink)) * p.rope_scale;
+          const int next = n + 1 < 2 * PS / TSTEP ? 1 : 3;  // to the lane's next key, or to its first of the next step
+#pragma unroll
+          for (int i = 0; i < NPAIR; ++i) {
+            const int f = pair_feature(8 * i);
+            if (at_sinks) {
+              rope_pair(frag[i].h8, frag[i + NPAIR].h8, pos, &rope_lds[0][f]);
+            } else {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                const float cs = run_cos[8 * i + e], sn = run_sin[8 * i + e];
+                const float xl = static_cast<float>(frag[i].h8[e]), xh = static_cast<float>(frag[i + NPAIR].h8[e]);
+                frag[i].h8[e] = static_cast<half_t>(cs * xl - sn * xh);
+                frag[i + NPAIR].h8[e] = static_cast<half_t>(cs * xh + sn * xl);
+              }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float cs = run_cos[8 * i + e], sn = run_sin[8 * i + e];
+              run_cos[8 * i + e] = cs * rope_lds[next][f + e] - sn * rope_lds[next + 1][f + e];
+              run_sin[8 * i + e] = sn * rope_lds[next][f + e] + cs * rope_lds[next + 1][f + e];
+            }
+          }
+        }
+      }
+    } else if (EXT && p.rotary) {
       // the key of this lane in page h is physical token (pi+h)*PS + c16 (KLINE: + 8*tile + c16/2);
       // logical index = position
 #pragma unroll
@@ -565,12 +633,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
           Vec16* frag = r.k[h] + (KLINE ? tile * TI : 0);
 #pragma unroll
           for (int i = 0; i < NPAIR; ++i) {
-            if constexpr (VARIANT) {
-              rope_pair_ex(frag[i].h8, frag[i + NPAIR].h8, pos, divr + 8 * i, divh + 8 * i, p.rope_inverse, p.rope_halves_differ,
-                           p.rope_magnitude);
-            } else {
-              rope_pair(frag[i].h8, frag[i + NPAIR].h8, pos, divr + 8 * i);
-            }
+            rope_pair_ex(frag[i].h8, frag[i + NPAIR].h8, pos, divr + 8 * i, divh + 8 * i, p.rope_inverse, p.rope_halves_differ,
+                         p.rope_magnitude);
           }
         }
       }
@@ -894,7 +958,7 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
   const bool fused = static_cast<size_t>(batch_size) * h_kv * head_blocks * sizeof(unsigned long long) <= kArrivalBytes &&
                      option(kOptDecodeSeparateMerge) == 0 && heads_per_item == 16;
   if (fused) p.arrivals = reinterpret_cast<unsigned long long*>(ws.ptr);
-  DecodeRopeDivisors div{};
+  DecodeRopeRunning div{};
   if (p.rotary || (fused_launch && p.apply_rope)) {
     KV_CHECK(k_rope_pos_offset || fused_launch) << "batch_decode_paged_kv: inline RoPE needs the position arrays";
     KV_CHECK(q_rope_position) << "batch_decode_paged_kv: inline RoPE needs the position arrays";
@@ -903,10 +967,22 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
     p.rope_inverse = table.inverse;
     p.rope_halves_differ = table.halves_differ;
     p.rope_magnitude = table.magnitude;
+    if (ext) {
+      // a wave's step is two pages and the next one is eight pages on; a lane's keys are the kernel's TSTEP tokens apart
+      const int near = d == 64 ? 16 : 8, far = (8 - 2) * DM_PS + near;
+      for (int i = 0; i < d / 2; ++i) {
+        const double angle = static_cast<double>(p.rope_scale) / static_cast<double>(div.v[i]);
+        div.near_cos[i] = static_cast<float>(std::cos(near * angle));
+        div.near_sin[i] = static_cast<float>(std::sin(near * angle));
+        div.far_cos[i] = static_cast<float>(std::cos(far * angle));
+        div.far_sin[i] = static_cast<float>(std::sin(far * angle));
+      }
+    }
   }
   if (padded) {
     auto launch_padded = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid_x)), dim3(256), 0, s, p, group, static_cast<int>(num_items), div);
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid_x)), dim3(256), 0, s, p, group, static_cast<int>(num_items),
+                         static_cast<const DecodeRopeDivisors&>(div));
     };
     if (head_blocks > 1) {
       launch_padded(decode_mfma_kernel<false, 128, true, 2, false, true>);
@@ -916,7 +992,11 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
       launch_padded(decode_mfma_kernel<false, 128, false, 1, false, true>);
     }
   }
+  const DecodeRopeDivisors& divisors = div;
   auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid_x)), dim3(256), 0, s, p, group, static_cast<int>(num_items), divisors);
+  };
+  auto launch_running = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid_x)), dim3(256), 0, s, p, group, static_cast<int>(num_items), div);
   };
   // the default frequencies (one divisor per pair, position / divisor) have the kernel without the general rotation
@@ -943,11 +1023,11 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
         launch(decode_mfma_kernel<true, kD, false, 1, false, false, true>);
       }
     } else if (reread) {
-      if (ext) launch(decode_mfma_kernel<true, kD, true, kWide>); else launch(decode_mfma_kernel<false, kD, true, kWide>);
+      if (ext) launch_running(decode_mfma_kernel<true, kD, true, kWide>); else launch(decode_mfma_kernel<false, kD, true, kWide>);
     } else if (wide) {
-      if (ext) launch(decode_mfma_kernel<true, kD, false, kWide>); else launch(decode_mfma_kernel<false, kD, false, kWide>);
+      if (ext) launch_running(decode_mfma_kernel<true, kD, false, kWide>); else launch(decode_mfma_kernel<false, kD, false, kWide>);
     } else {
-      if (ext) launch(decode_mfma_kernel<true, kD, false>); else launch(decode_mfma_kernel<false, kD, false>);
+      if (ext) launch_running(decode_mfma_kernel<true, kD, false>); else launch(decode_mfma_kernel<false, kD, false>);
     }
   };
   if (padded) {
