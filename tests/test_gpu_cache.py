@@ -90,6 +90,8 @@ class Mirror:
         for sid, n in zip(ids, lens):
             self.lengths[sid] += n
             L = self.lengths[sid]
+            if 3 in self.o.attn_kinds:  # debug_get_kv is for caches whose layers are all plain
+                continue
             ek = np.zeros((self.layers, L, self.hkv, self.d), self.dtype)
             ev, gk, gv = np.zeros_like(ek), np.zeros_like(ek), np.zeros_like(ek)
             self.o.debug_get_kv(sid, 0, L, ek, ev)
@@ -215,6 +217,38 @@ def test_prefill_steps_of_other_caches_over_gathered_keys(page_size, d, rope_mod
     m.step([(0, 1), (1, 1), (2, 1)])
     m.step([(0, 15), (1, 90), (3, 33)])
     m.step([((4, 1, 40), 25), (0, 2)])
+
+
+@pytest.mark.parametrize("page_size,d,hq,hkv,window", [(16, 128, 8, 2, 0), (16, 64, 8, 8, 0), (64, 128, 20, 1, 100), (16, 64, 8, 2, 1),
+                                                      (32, 128, 18, 1, 1024), (16, 128, 4, 4, 1200), (128, 64, 4, 1, 33)])
+def test_steps_that_mix_prompts_and_decoding_sequences(page_size, d, hq, hkv, window):
+    """Decoding sequences of a mixed step run on the decode kernel with their new token as one more key: long contexts,
+    one that ends at a page edge, one of a single token, one without any; prompts with and without cached tokens; layers
+    with and without a window (0: none), windows inside one page and longer than some sequences."""
+    m = Mirror([12, 6000, 2048, page_size, 0] + ([window] if window else []), 2 if window else 1, hq, hkv, d,
+               **({"attn_kinds": [3, 0]} if window else {}))
+    m.step([(0, 1300), (1, 64), (2, 300)])
+    m.step([(3, 1), (1, 1)])
+    m.step([(0, 1), (4, 40), (1, 1), (3, 1), (5, 1), (2, 17)])
+    m.step([(2, 1), (0, 1), (6, 130)])
+    m.step([(4, 3), (0, 1), (2, 1)])
+    m.step([(0, 1), (2, 1), (4, 1)])
+
+
+def test_decode_steps_of_windowed_caches_at_the_edges():
+    """A decode step of a sequence-window cache takes the new token as one more key: sequences without cached tokens, of
+    one token, at the edge of a page and beyond their window, with a prompt's first decode among them."""
+    for d, hq, hkv, rope_mode in ((128, 8, 2, 2), (64, 20, 1, 2), (256, 4, 2, 2), (128, 4, 4, 0)):
+        layers = 2
+        cache = GpuCache([8, 4096, 1024, 16, 1], layers, hq, hkv, d, d, rope_mode=rope_mode)
+        sc = S.Scenario(cache, layers, hq, hkv, d, rope_mode=rope_mode, seed=9, tol=4e-3)
+        for sid, (window, sink) in enumerate([(40, 0), (130, 4), (257, 30), (600, 16)]):
+            sc.add_with_window(sid, window, sink)
+        sc.step([(0, 1), (1, 1), (2, 1)])
+        sc.step([(0, 1), (1, 1), (2, 1), (3, 1)])
+        sc.step([(0, 14), (1, 29), (2, 300), (3, 500)])
+        for _ in range(6):
+            sc.step([(0, 1), (1, 1), (2, 1), (3, 1)])
 
 
 def test_short_chunk_against_a_long_cached_sequence():

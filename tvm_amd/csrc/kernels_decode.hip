@@ -46,7 +46,7 @@ struct DecodeParams {
   const int32_t* sink_size;       // (B) attention-sink tokens kept at the front, or NULL
   const int32_t* k_rope_pos_offset;  // (B) position of logical token 0 (inline RoPE)
   const int32_t* q_rope_position;    // (B) position of the query token (inline RoPE)
-  int rotary;                     // 1: rotate q and k inside the kernel
+  int rotary;                     // 1: rotate q and k inside the kernel; 2 (SELF only): the queries alone
   float rope_scale;
   // (batch, h_kv) arrival counters of the fused chunk merge of decode_mfma_kernel, or NULL.  A counter
   // is epoch << 32 | workgroups that have delivered their partial state in the launch with that epoch;
@@ -68,6 +68,15 @@ struct DecodeParams {
   half_t* pages_rw;             // == pages
   const int32_t* append_slot;   // (B) page * page_size + offset, -1 = none
   int apply_rope;               // 0: q and k are used as they come
+  // new-token form (decode_mfma_kernel<..., SELF = true>): the new token of a sequence is not in its page table; its
+  // k / v rows (consecutive tokens new_stride elements apart) are one more key.  Sequence b is token rows[b] of q,
+  // k_new, v_new, q_rope_position and the output (NULL: token b), its pages start at page_values[page_begin[b]]
+  // (page_indptr holds the page counts as sums, so that a step's decoding sequences need no page table of their own).
+  const half_t* k_new;
+  const half_t* v_new;
+  const int32_t* rows;
+  const int32_t* page_begin;
+  int64_t q_stride, new_stride;
   // padded head dims (80, 96, 112 on the head dim 128 kernel): elements per row of q, the pages and the
   // output in memory; 0 = the kernel's head dim
   int d_mem;
@@ -137,7 +146,7 @@ __device__ __forceinline__ void load_partial_row(const float* src, float (&dst)[
 template <int D, bool COHERENT>
 __device__ __forceinline__ void merge_row(const DecodeParams& p, int b, int hq, int nchunks, int lane) {
   constexpr int EPL = D / 64;  // features per lane
-  const int64_t row = static_cast<int64_t>(b) * p.h_q + hq;
+  const int64_t row = static_cast<int64_t>(p.rows != nullptr ? p.rows[b] : b) * p.h_q + hq;
   const int dm = p.d_mem > 0 ? p.d_mem : D;
   half_t* out = p.output + row * dm + lane * EPL;
   const int s0 = slot_begin(p.page_indptr, b, p.chunk_pages);
@@ -222,6 +231,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p, int t
   const int nchunks = (npages + p.chunk_pages - 1) / p.chunk_pages;
   if (nchunks == 1) return;
   if (nchunks == 0) {
+    if (p.k_new != nullptr) return;  // the new token alone: the main kernel wrote it
     empty_row<D>(p, b, hq, lane);
     return;
   }
@@ -289,11 +299,15 @@ struct DecodeRopeRunning : DecodeRopeDivisors {
 // VARIANT (with EXT): the in-kernel RoPE takes a frequency variant (rope_pair_ex: a table entry per element,
 // inverse frequencies, a magnitude).  A kernel of its own: the second set of table entries and the general
 // rotation made every extended launch spill (46-143 registers) while they sat in the same kernel.
-template <bool EXT, int D, bool REREAD, int HB = 1, bool FUSED = false, bool PAD = false, bool VARIANT = false>
+// SELF (with EXT): the new-token form, see DecodeParams.  The wave that starts a sequence's last chunk begins with the
+// state of that one key instead of the empty one, so that a step whose new rows may not be in the pages yet (windows,
+// steps that mix prompts and decoding sequences) needs neither a self-attention launch nor a merge.
+template <bool EXT, int D, bool REREAD, int HB = 1, bool FUSED = false, bool PAD = false, bool VARIANT = false, bool SELF = false>
 __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void decode_mfma_kernel(DecodeParams p, int group, int num_items,
     std::conditional_t<EXT && !VARIANT, DecodeRopeRunning, DecodeRopeDivisors> div) {
   static_assert(HB == 1 || HB == 2, "head blocks per work item");
   static_assert(!(FUSED && EXT), "the fused step exists for the plain cache");
+  static_assert(!SELF || (EXT && !VARIANT), "the new-token form: an extended kernel with the default frequencies");
   static_assert(!PAD || (!EXT && !FUSED), "padded head dims: plain cache, no in-kernel RoPE");
   const int dm = PAD ? p.d_mem : D;  // elements per row in memory
   constexpr int PS = DM_PS;
@@ -339,10 +353,11 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   const int hq0 = kvh * group + hb * HPI;      // first query head of this item
   const int heads = min(HPI, group - hb * HPI);  // and how many
   const int b = find_sequence_wave(p.page_indptr, p.batch_size, cp, slot, lane);
-  const int pbeg = p.page_indptr[b];
-  const int npages = p.page_indptr[b + 1] - pbeg;
+  const int npages = p.page_indptr[b + 1] - p.page_indptr[b];
+  const int pbeg = SELF && p.page_begin != nullptr ? p.page_begin[b] : p.page_indptr[b];
+  const int token = SELF && p.rows != nullptr ? p.rows[b] : b;  // of q and the output
   const int chunk = slot - slot_begin(p.page_indptr, b, cp);
-  const int nchunks = (npages + cp - 1) / cp;
+  const int nchunks = SELF ? max(1, (npages + cp - 1) / cp) : (npages + cp - 1) / cp;
   if (chunk >= nchunks) {  // spare slot (uniform over the workgroup)
     if (p.arrivals != nullptr && npages == 0 && chunk == 0) {  // a sequence without pages: nobody else answers for it
       for (int g = wave; g < heads; g += 4) empty_row<D>(p, b, hq0 + g, lane);
@@ -372,7 +387,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   // windows of 4096 tokens, 32 / 8 heads of dim 128: 247 us a layer, 206 now).  The fixed angles come from the host in
   // double, so that after the 16 steps of the longest chunk the drift is a few 2^-24 -- the fp32 angle itself is off by
   // more.  They wait in LDS: in registers they made every extended launch of head dim 128 spill.
-  if (EXT && p.rotary) {
+  const bool k_rotary = EXT && (SELF ? p.rotary == 1 : p.rotary != 0);
+  if (k_rotary) {
     k_pos0 = static_cast<float>(p.k_rope_pos_offset[b]);
     if constexpr (RUNNING) {
       if (tid < D / 2) {
@@ -440,7 +456,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
 #pragma unroll
   for (int j = 0; j < HB; ++j) {
     const bool head_valid = j * 16 + c16 < heads;
-    const half_t* qrow = FUSED ? p.qkv + (static_cast<int64_t>(b) * (p.h_q + 2 * p.h_kv) + hq0 + j * 16 + c16) * D + g4 * 8
+    const half_t* qrow = SELF ? p.q + token * p.q_stride + (hq0 + j * 16 + c16) * D + g4 * 8
+                         : FUSED ? p.qkv + (static_cast<int64_t>(b) * (p.h_q + 2 * p.h_kv) + hq0 + j * 16 + c16) * D + g4 * 8
                                : p.q + (static_cast<int64_t>(b) * p.h_q + hq0 + j * 16 + c16) * dm + g4 * 8;
     Vec16 qv[KS];
 #pragma unroll
@@ -463,7 +480,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
     }
     if (EXT && p.rotary) {
       // feature f < D/2 rotates with f + D/2: k-step ks with ks + KS/2
-      const float q_pos = static_cast<float>(p.q_rope_position[b]) * p.rope_scale;
+      const float q_pos = static_cast<float>(p.q_rope_position[token]) * p.rope_scale;
 #pragma unroll
       for (int ks = 0; ks < KS / 2; ++ks) {
         float qdiv[8], qdivh[VARIANT ? 8 : 1];
@@ -516,6 +533,42 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   for (int j = 0; j < HB; ++j) {
     m[j] = kNegInit;
     lsum[j] = 0.f;
+  }
+
+  if (SELF && wave == 0 && chunk == nchunks - 1) {
+    const half_t* knew = p.k_new + token * p.new_stride + static_cast<int64_t>(kvh) * D;
+    const half_t* vnew = p.v_new + token * p.new_stride + static_cast<int64_t>(kvh) * D;
+    Vec16 kn[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) kn[ks] = ld16(knew + ks * 32 + g4 * 8);
+    if (k_rotary) {  // at the position of its query
+      const float pos = static_cast<float>(p.q_rope_position[token]) * p.rope_scale;
+#pragma unroll
+      for (int ks = 0; ks < KS / 2; ++ks) {
+        float kdiv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) kdiv[e] = div.v[ks * 32 + g4 * 8 + e];
+        rope_pair(kn[ks].h8, kn[ks + KS / 2].h8, pos, kdiv);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < HB; ++j) {
+      float dot = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = fmaf(static_cast<float>(qf[j][ks][e]), static_cast<float>(kn[ks].h8[e]), dot);
+      }
+      const float score = sum_xor32(sum_xor16(dot)) * p.scale_log2;  // of head c16, in all four lane groups
+      m[j] = fmaxf(kNegInit, score);
+      const float weight = fast_exp2(score - m[j]);
+      lsum[j] = g4 == 0 ? weight : 0.f;  // the lane groups' sums are added at the end
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[j][db][e] = weight * static_cast<float>(vnew[db * 16 + 4 * g4 + e]);
+      }
+    }
   }
 
   // V^T fragment via the transposing read: lane li of a 16-lane group points at 4 features of token
@@ -588,7 +641,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
                              : (pi + 2) * PS > kv_len;
     auto attended = [&](int t) { return EXT ? (t < sink || (t >= win_lo && t < kv_len)) : t < kv_len; };
     if constexpr (RUNNING) {
-      if (p.rotary) {
+      if (k_rotary) {
         // attention sinks and the keys beside them (wave-uniform): every key by its own angle
         const bool at_sinks = pi * PS < sink;
 #pragma unroll
@@ -765,8 +818,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
       const int hq = hq0 + j * 16 + g;
       if (single_chunk) {
         const float denom = lt + fast_exp2(kNegInit - mx);
-        if (!PAD || d < dm) p.output[(static_cast<int64_t>(b) * p.h_q + hq) * dm + d] = static_cast<half_t>(acc / denom);
-        if (d == 0) p.lse[static_cast<int64_t>(b) * p.h_q + hq] = mx + fast_log2(denom);
+        if (!PAD || d < dm) p.output[(static_cast<int64_t>(token) * p.h_q + hq) * dm + d] = static_cast<half_t>(acc / denom);
+        if (d == 0) p.lse[static_cast<int64_t>(token) * p.h_q + hq] = mx + fast_log2(denom);
       } else {
         store_partial(p.part_o + (static_cast<int64_t>(slot) * p.h_q + hq) * D + d, acc);
         if (d == 0) {
@@ -860,12 +913,17 @@ extern "C" int tvmkv_debug_set_scratch_launches(uint64_t launches) {
   KV_API_END();
 }
 
-// The fused step's extra arguments (qkv == nullptr: a plain decode call)
+// The extra arguments of the fused step (qkv == nullptr: a plain decode call) and of the new-token form (k_new)
 struct FusedStep {
   const void* qkv = nullptr;
   const int32_t* append_position_map = nullptr;
   int apply_rope = 0;
   const tvmkv_rope_scaling* rope_scaling = nullptr;  // frequency variant of the in-kernel RoPE of a plain call
+  const void* k_new = nullptr;
+  const void* v_new = nullptr;
+  const int32_t* rows = nullptr;
+  const int32_t* page_begin = nullptr;
+  int64_t q_stride = 0, new_stride = 0;
 };
 
 // Body of the decode entry point.  lease(bytes) hands out the scratch memory of the call: arrival
@@ -879,7 +937,8 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
                          int32_t page_size, int32_t sliding_window, void* stream) {
   KV_CHECK(batch_size >= 0 && nnz_pages >= 0 && h_q > 0 && h_kv > 0 && h_q % h_kv == 0)
       << "batch_decode_paged_kv: bad shape";
-  const bool ext = rotary_mode != 0 || sliding_window != 0;
+  const bool self = fused_step.k_new != nullptr;
+  const bool ext = rotary_mode != 0 || sliding_window != 0 || self;
   KV_UNSUPPORTED(page_size < 16 || page_size > 128 || (page_size & (page_size - 1)) != 0)
       << "batch_decode_paged_kv: page_size " << page_size << " is not built (16, 32, 64, 128)";
   const bool padded = d == 80 || d == 96 || d == 112;  // run on the head dim 128 kernel, rows of d elements
@@ -906,7 +965,7 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
   p.sink_size = sliding_window != 0 ? length_info + 2 * static_cast<int64_t>(batch_size) : nullptr;
   p.k_rope_pos_offset = k_rope_pos_offset;
   p.q_rope_position = q_rope_position;
-  p.rotary = rotary_mode != 0;
+  p.rotary = self ? static_cast<int>(rotary_mode) : rotary_mode != 0;
   p.rope_scale = static_cast<float>(rope_scale);
   p.output = static_cast<half_t*>(output);
   p.lse = lse;
@@ -930,6 +989,12 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
   p.pages_rw = const_cast<half_t*>(p.pages);
   p.append_slot = fused_step.append_position_map;
   p.apply_rope = fused_step.apply_rope;
+  p.k_new = static_cast<const half_t*>(fused_step.k_new);
+  p.v_new = static_cast<const half_t*>(fused_step.v_new);
+  p.rows = fused_step.rows;
+  p.page_begin = fused_step.page_begin;
+  p.q_stride = fused_step.q_stride;
+  p.new_stride = fused_step.new_stride;
   const int64_t slots = nnz_pages / p.chunk_pages + batch_size;
   KV_CHECK(slots < (int64_t{1} << 31)) << "batch_decode_paged_kv: too many chunks";
   const size_t part_o_bytes = static_cast<size_t>(slots) * h_q * dk * sizeof(float);
@@ -960,7 +1025,7 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
   if (fused) p.arrivals = reinterpret_cast<unsigned long long*>(ws.ptr);
   DecodeRopeRunning div{};
   if (p.rotary || (fused_launch && p.apply_rope)) {
-    KV_CHECK(k_rope_pos_offset || fused_launch) << "batch_decode_paged_kv: inline RoPE needs the position arrays";
+    KV_CHECK(k_rope_pos_offset || fused_launch || rotary_mode == 2) << "batch_decode_paged_kv: inline RoPE needs the position arrays";
     KV_CHECK(q_rope_position) << "batch_decode_paged_kv: inline RoPE needs the position arrays";
     const InlineRopeHost table = inline_rope_table(fused_launch ? nullptr : fused_step.rope_scaling, d, rope_theta);
     for (int i = 0; i < d; ++i) div.v[i] = table.v[i];
@@ -1013,6 +1078,14 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
         launch(decode_mfma_kernel<false, kD, false, kWide, true>);
       } else {
         launch(decode_mfma_kernel<false, kD, false, 1, true>);
+      }
+    } else if (self) {
+      if (reread) {
+        launch_running(decode_mfma_kernel<true, kD, true, kWide, false, false, false, true>);
+      } else if (wide) {
+        launch_running(decode_mfma_kernel<true, kD, false, kWide, false, false, false, true>);
+      } else {
+        launch_running(decode_mfma_kernel<true, kD, false, 1, false, false, false, true>);
       }
     } else if (ext && variant) {
       if (reread) {
@@ -1159,6 +1232,26 @@ extern "C" int tvmkv_fused_decode_step(const void* qkv, void* pages, const int32
   decode_entry([&](size_t bytes) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes); }, step, nullptr, pages,
                page_indptr, page_values, last_page_len, nullptr, q_rope_position, output, lse, 0, rope_scale, rope_theta,
                sm_scale, batch_size, nnz_pages, num_pages, h_q, h_kv, d, page_size, 0, stream);
+  KV_API_END();
+}
+
+// Decode attention of tokens whose k / v rows are not in the pages yet (typed_kernels.h)
+int tvmkv::decode_with_new_token(const NewTokenDecode& a, void* stream) {
+  KV_API_BEGIN();
+  hipStream_t s = as_stream(stream);
+  KV_CHECK(a.batch == 0 || (a.q && a.k_new && a.v_new && a.page_indptr)) << "decode_with_new_token: NULL tensor";
+  KV_CHECK(a.rotate >= 0 && a.rotate <= 2) << "decode_with_new_token: bad rotation";
+  FusedStep step;
+  step.k_new = a.k_new;
+  step.v_new = a.v_new;
+  step.rows = a.rows;
+  step.page_begin = a.page_begin;
+  step.q_stride = a.q_stride;
+  step.new_stride = a.new_stride;
+  decode_entry([&](size_t bytes) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes); }, step, a.q, a.pages,
+               a.page_indptr, a.page_values, a.length_info, a.k_rope_pos_offset, a.q_rope_position, a.out, a.lse, a.rotate,
+               a.rope_scale, a.rope_theta, a.sm_scale, a.batch, a.nnz_pages, a.num_pages, a.h_q, a.h_kv, a.d, a.page_size,
+               a.sliding, stream);
   KV_API_END();
 }
 

@@ -139,7 +139,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 
         lk0 = p.kv_indptr[lane];
         lk1 = p.kv_indptr[lane + 1];
       }
-      my_tiles = ((lq1 - lq0) * group + BM - 1) / BM;
+      my_tiles = (p.skip_single && lq1 - lq0 == 1) ? 0 : ((lq1 - lq0) * group + BM - 1) / BM;
       my_key = (lp1 - lp0) * (PS << p.page_shift) + (lk1 - lk0);
     }
     // Row tiles of the sequences ranked before this lane's.  (key, index) is one sortable 32-bit
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 
   const int qo_len = seq_q1 - q_start;
   const int rows = qo_len * group;
   const int n_row_tiles = (rows + BM - 1) / BM;
-  if (local_slot >= n_row_tiles) return;
+  if (local_slot >= n_row_tiles || (p.skip_single && qo_len == 1)) return;
   const int r0 = (n_row_tiles - 1 - local_slot) * BM;
 
   // phys_len: tokens the K/V storage of the sequence covers; kv_len: keys attended to (logical)
@@ -882,11 +882,13 @@ struct KvSplit {
   int splits;
   int merge_into = 0;
   ScratchLease lease{};
-  KvSplit(PrefillParams& p, int64_t total_q, int64_t avg_keys, int dv, hipStream_t stream)
+  // work_q, work_seqs: the query tokens and sequences that the launch works on, where they are not all (skip_single)
+  KvSplit(PrefillParams& p, int64_t total_q, int64_t avg_keys, int dv, hipStream_t stream, int64_t work_q = 0, int64_t work_seqs = 0)
       : output(p.output), lse(p.lse), rows(total_q * p.h_q), splits(1) {
+    if (work_seqs == 0) work_q = total_q, work_seqs = p.batch_size;
     // at most one row tile per (sequence, kv head) on average: the paged kernels stream the K/V rows
-    p.stream_kv = total_q * p.group <= static_cast<int64_t>(p.batch_size) * BM;
-    splits = pick_kv_splits(total_q, p.group, p.batch_size, p.h_kv, avg_keys);
+    p.stream_kv = work_q * p.group <= work_seqs * BM;
+    splits = pick_kv_splits(work_q, p.group, work_seqs, p.h_kv, avg_keys);
     if (dv % 64 != 0) splits = 1;  // padded head dims (80, 96, 112): the merge kernel is not built for their rows
     if (splits <= 1) return;
     const size_t o_bytes = static_cast<size_t>(splits) * rows * dv * sizeof(half_t);
@@ -1021,6 +1023,71 @@ int tvmkv::prefill_over_gathered_kv(const void* q, int64_t q_token_stride, const
   } else {
     KV_UNSUPPORTED(!padded_head_dim(d)) << "prefill_over_gathered_kv: head_dim " << d;
     launch_prefill_padded<kRagged>(p, total_q, d, false, "prefill_over_gathered_kv", s);
+  }
+  KV_LAUNCH_CHECK();
+  KV_API_END();
+}
+
+int tvmkv::prefill_prompts(const PromptPrefill& a, void* stream) {
+  KV_API_BEGIN();
+  KV_CHECK(a.batch > 0 && a.total_q > 0 && a.prompts > 0 && a.h_q > 0 && a.h_kv > 0 && a.h_q % a.h_kv == 0) << "prefill_prompts: bad shape";
+  const int page_shift = paged_page_shift(a.page_size);
+  KV_UNSUPPORTED(page_shift < 0) << "prefill_prompts: page_size " << a.page_size << " is not built (16, 32, 64, 128)";
+  KV_CHECK(a.num_pages < (int64_t{1} << 28)) << "prefill_prompts: page ids must stay below 2^28";
+  KV_CHECK(a.q && a.q_indptr && a.k && a.v && a.pages && a.page_indptr && a.page_values && a.length_info && a.out && a.lse)
+      << "prefill_prompts: NULL tensor";
+  KV_CHECK(!a.apply_rope || (a.q_rope_position && a.layer_window == 0)) << "prefill_prompts: rotation of the queries";
+  PrefillParams p{};
+  p.skip_single = 1;
+  p.page_shift = page_shift;
+  p.q = static_cast<const half_t*>(a.q);
+  p.q_token_stride = a.q_stride;
+  p.q_inline_rope = a.apply_rope != 0;
+  p.q_rope_position = a.q_rope_position;
+  p.rope_scale = static_cast<float>(a.rope_scale);
+  p.q_indptr = a.q_indptr;
+  p.k = static_cast<const half_t*>(a.k);
+  p.v = static_cast<const half_t*>(a.v);
+  p.kv_indptr = a.q_indptr;
+  p.pages = static_cast<const half_t*>(a.pages);
+  p.page_indptr = a.page_indptr;
+  p.page_values = a.page_values;
+  p.last_page_len = a.length_info;
+  p.output = static_cast<half_t*>(a.out);
+  p.lse = a.lse;
+  p.batch_size = a.batch;
+  p.h_q = a.h_q;
+  p.h_kv = a.h_kv;
+  p.group = a.h_q / a.h_kv;
+  p.causal = 1;
+  p.scale_log2 = static_cast<float>(a.sm_scale) * kLog2e;
+  hipStream_t s = as_stream(stream);
+  auto by_dim = [&](auto run) {
+    if (a.d == 128) {
+      run(std::integral_constant<int, 128>{});
+    } else if (a.d == 64) {
+      run(std::integral_constant<int, 64>{});
+    } else {
+      KV_UNSUPPORTED(a.d != 256) << "prefill_prompts: head_dim " << a.d << " is not built (64, 128, 256)";
+      run(std::integral_constant<int, 256>{});
+    }
+    KV_LAUNCH_CHECK();
+  };
+  if (a.layer_window == 0) {
+    const KvSplit split(p, a.total_q, (a.prompt_cached + a.prompt_tokens) / a.prompts, a.d, s, a.prompt_tokens, a.prompts);
+    by_dim([&](auto d) { launch_prefill<d.value, d.value, kBoth, 16>(p, a.total_q, false, a.rope_theta, s); });
+    split.finish(p, a.d, s);
+  } else {
+    by_dim([&](auto d) { launch_prefill<d.value, d.value, kRagged, 16>(p, a.total_q, false, a.rope_theta, s); });
+    if (a.prompt_cached > 0) {
+      p.window_offset = a.length_info + a.batch;
+      p.sink_size = a.length_info + 2 * static_cast<int64_t>(a.batch);
+      p.layer_window = a.layer_window;
+      p.merge_into = 1;
+      const KvSplit split(p, a.total_q, std::min<int64_t>(a.prompt_cached / a.prompts, a.layer_window), a.d, s, a.prompt_tokens, a.prompts);
+      by_dim([&](auto d) { launch_prefill<d.value, d.value, kPaged, 16>(p, a.total_q, true, a.rope_theta, s); });
+      split.finish(p, a.d, s);
+    }
   }
   KV_LAUNCH_CHECK();
   KV_API_END();

@@ -193,9 +193,11 @@ class PagedKVCache {
       RecordComputeEvent();
       return;
     }
-    // A chunked-prefill step of a plain cache in two launches: k is rotated and the new k / v rows go
-    // into their page slots (part 2 without q, part 3), then one pass over the cached and the new
-    // tokens that reads the queries from qkv and rotates them itself (parts 2 and 5).
+    if (new_token_step_ && attn_kinds_[layer_id] == TVMKV_ATTN_MHA) {
+      WindowedDecodeStep(local_layer_id, qkv, out, total_seq_length, sm_scale);
+      RecordComputeEvent();
+      return;
+    }
     if (generic_) {
       // split + RoPE (+ append when the rows may go in before attention), the attention kernels of the step, the
       // append afterwards otherwise: the reference's flow (:1360-1401) on the typed and generic kernels
@@ -251,11 +253,20 @@ class PagedKVCache {
       RecordComputeEvent();
       return;
     }
+    // A chunked-prefill step of a plain cache in two launches: k is rotated and the new k / v rows go
+    // into their page slots (part 2 without q, part 3), then one pass over the cached and the new
+    // tokens that reads the queries from qkv and rotates them itself (parts 2 and 5).
     if (OnePassPrefillApplies(layer_id)) {
       Launch(tvmkv_fused_rope_append(qkv, Dev(s.q_rope_position_map), /*q=*/nullptr, temp_k_, temp_v_, rope_normal,
                                      pages_[local_layer_id], Dev(s.append_position_map), total_seq_length,
                                      num_qo_heads_, num_kv_heads_, qk_head_dim_, num_total_pages_, page_size_,
                                      rotary_scale_, rotary_theta_, compute_stream_));
+      if (RunsMixed()) {
+        MixedAttention(layer_id, qkv, (num_qo_heads_ + 2 * num_kv_heads_) * qk_head_dim_, rope_normal, temp_k_, temp_v_, out,
+                       total_seq_length, sm_scale);
+        RecordComputeEvent();
+        return;
+      }
       Launch(tvmkv_batch_prefill_cached_and_new_kv_fused_q(
           qkv, Dev(s.q_rope_position_map), rope_normal, rotary_scale_, rotary_theta_,
           Dev(s.cur_append_lengths_indptr), temp_k_, temp_v_, pages_[local_layer_id], Dev(s.page_indptr[0]),
@@ -537,7 +548,7 @@ class PagedKVCache {
       HIP_CHECK(hipMalloc(&temp_lse_, prefill_chunk_size_ * num_qo_heads_ * sizeof(float)));
       HIP_CHECK(hipMalloc(&merged_lse_, prefill_chunk_size_ * num_qo_heads_ * sizeof(float)));
       aux_capacity_ = book_->RequiredCapacity();
-      extras_capacity_ = (reserved_num_seqs_ + 1 + 3) / 4 * 4;
+      extras_capacity_ = 12 * ((reserved_num_seqs_ + 1 + 3) / 4 * 4);  // the larger of the plans: MixedStep
       if (gather_capable_) {
         const int64_t row_bytes = 2 * num_kv_heads_ * qk_head_dim_ * static_cast<int64_t>(sizeof(uint16_t));
         gather_capacity_ = std::min(num_total_pages_ * page_size_ + prefill_chunk_size_, kGatherBytes / row_bytes);
@@ -707,8 +718,20 @@ class PagedKVCache {
   void PlanStep() {
     extras_.clear();
     gathered_rows_ = 0;
+    mixed_ = MixedStep{};
+    new_token_step_ = false;
     const StepLayout& s = book_->step();
     const int64_t batch = book_->batch_size();
+    if (batch > reserved_num_seqs_) return;  // the plans are sized for that many
+    const bool tuned_decode = !generic_ && elem_bits_ == 16 && qk_head_dim_ == v_head_dim_ && s.num_depths == 1 &&
+                              s.is_chain[0] && !s.append_before_attn && s.qo_indptr[0].size == batch + 1;
+    new_token_step_ = tuned_decode && support_sliding_window_ && s.use_decode_kernel[0] && rope_mode_ != TVMKV_ROPE_NORMAL &&
+                      !has_rope_scaling_ && rope_ext_factors_ == nullptr &&
+                      (qk_head_dim_ == 64 || qk_head_dim_ == 128 || qk_head_dim_ == 256);
+    if (tuned_decode && !support_sliding_window_ && !s.use_decode_kernel[0] && s.page_indices[0].size > 0 && rope_mode_ != TVMKV_ROPE_INLINE &&
+        (qk_head_dim_ == 64 || qk_head_dim_ == 128)) {
+      PlanMixedStep();
+    }
     if (gather_capable_ && rope_ext_factors_ == nullptr && s.num_depths == 1 && s.is_chain[0] && !s.append_before_attn &&
         !s.use_decode_kernel[0] &&
         s.total_append_length * (num_qo_heads_ / num_kv_heads_) >=
@@ -736,6 +759,189 @@ class PagedKVCache {
       std::memcpy(static_cast<int32_t*>(aux_staging_[aux_slot_]) + extras_capacity_ - extras_.size(), extras_.data(),
                   extras_.size() * sizeof(int32_t));
     }
+  }
+
+  // A step of prompts and decoding sequences.  In one prefill launch a decoding sequence is a row tile of few rows whose
+  // workgroup walks all its keys alone: the longest of them decides how long the launch takes (32 decoding sequences of up
+  // to 6000 tokens beside 8 prompts, 32 / 8 heads of dim 64, every other layer with a window: 886 us for 8 layers, 590 now).  So the prompts run without
+  // them, and the decode kernel, which splits the keys, takes them with the new token as one more key.  What the decode
+  // kernel reads of them is written here, for the pages of the plain layers and for those of the layers with a window.
+  void PlanMixedStep() {
+    const StepLayout& s = book_->step();
+    const int64_t batch = book_->batch_size();
+    const int32_t* host = book_->step_buffer();
+    const int32_t* tokens = host + s.cur_append_lengths_indptr.offset;
+    const bool windows = s.page_indptr_sw[0].present() && s.layer_sw_length_info[0].present();
+    MixedStep plan;
+    const int32_t* page_indptr = host + s.page_indptr[0].offset;
+    const int32_t* last_len = host + s.length_info[0].offset;
+    auto cached = [&](int64_t b) {
+      const int64_t pages = page_indptr[b + 1] - page_indptr[b];
+      return pages > 0 ? (pages - 1) * page_size_ + last_len[b] : 0;
+    };
+    // What the step takes either way, in tiles of 64 keys by 128 rows that a workgroup walks one after the other (about
+    // 1 us each at head dim 128, 0.6 at 64, and 8 tiles' time before the first): the longest walk, or all of them on
+    // the workgroups the chip holds.  The decode kernel: 10 us and the K / V rows at 6 TB/s.
+    const bool wide = qk_head_dim_ == 128;
+    const double tile_us = wide ? 1.0 : 0.6, resident = 256 * (wide ? 2 : 3);
+    const int64_t group = num_qo_heads_ / num_kv_heads_;
+    double walk_decode = 0, walk_prompt = 0, work_decode = 0, work_prompt = 0, decode_bytes = 0;
+    for (int64_t b = 0; b < batch; ++b) {
+      const int64_t n = tokens[b + 1] - tokens[b], keys = cached(b);
+      const double walk = 8.0 + static_cast<double>((keys + n + 63) / 64);
+      if (n == 1) {
+        ++plan.decoding;
+        walk_decode = std::max(walk_decode, walk);
+        work_decode += walk * num_kv_heads_;
+        decode_bytes += 4.0 * keys * num_kv_heads_ * qk_head_dim_;
+      } else {
+        ++plan.prompts;
+        plan.prompt_tokens += n;
+        plan.prompt_cached += keys;
+        walk_prompt = std::max(walk_prompt, walk);
+        work_prompt += (8.0 + static_cast<double>(keys + n / 2) / 64) * num_kv_heads_ * ((n * group + 127) / 128);
+      }
+    }
+    if (plan.decoding == 0 || plan.prompts == 0) return;
+    const double together = tile_us * std::max({walk_decode, walk_prompt, (work_decode + work_prompt) / resident});
+    const double apart = tile_us * std::max(walk_prompt, work_prompt / resident) + 10.0 + decode_bytes / 6e6;
+    if (apart > together) return;
+    auto place = [&](int64_t n) {
+      const int64_t at = static_cast<int64_t>(extras_.size());
+      extras_.resize(at + (n + 3) / 4 * 4, 0);
+      return at;
+    };
+    plan.rows = place(plan.decoding);
+    for (int set = 0; set < (windows ? 2 : 1); ++set) {
+      const int32_t* indptr = host + (set ? s.page_indptr_sw[0] : s.page_indptr[0]).offset;
+      const int32_t* info = host + (set ? s.layer_sw_length_info[0] : s.length_info[0]).offset;
+      const int64_t n = plan.decoding;
+      const int64_t at_indptr = plan.page_indptr[set] = place(n + 1);
+      const int64_t at_begin = plan.page_begin[set] = place(n);
+      const int64_t at_info = plan.length_info[set] = place(3 * n);
+      int64_t i = 0;
+      for (int64_t b = 0; b < batch; ++b) {
+        if (tokens[b + 1] - tokens[b] != 1) continue;
+        const int32_t pages = indptr[b + 1] - indptr[b];
+        extras_[plan.rows + i] = tokens[b];
+        extras_[at_begin + i] = indptr[b];
+        extras_[at_indptr + i + 1] = extras_[at_indptr + i] + pages;
+        extras_[at_info + i] = info[b];
+        if (set && pages > 0) {
+          // the window layer's mask: the new token sees the last window - 1 cached keys (_kernel_common.py:138-144)
+          const int64_t end = (pages - 1) * page_size_ + info[b];
+          extras_[at_info + n + i] = static_cast<int32_t>(
+              std::max<int64_t>(info[batch + b], end - std::max<int64_t>(layer_sliding_window_size_ - 1, 0)));
+        }
+        ++i;
+      }
+      plan.nnz_pages[set] = extras_[at_indptr + n];
+    }
+    mixed_ = plan;
+  }
+
+  // A step that is being captured keeps the launches that need no scratch memory of the decode kernel's.
+  bool RunsMixed() const { return mixed_.decoding > 0 && !stream_is_capturing(static_cast<hipStream_t>(compute_stream_)); }
+
+  void MixedAttention(int64_t layer_id, const void* q, int64_t q_stride, bool rotate_q, const void* k, const void* v, void* out,
+                      int64_t total_seq_length, double sm_scale) {
+    const StepLayout& s = book_->step();
+    const int64_t local_layer_id = layer_id - layer_id_begin_offset_;
+    const bool window = attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING;
+    PromptPrefill a;
+    a.q = q;
+    a.q_stride = q_stride;
+    a.q_rope_position = Dev(s.q_rope_position_map);
+    a.apply_rope = rotate_q;
+    a.rope_scale = rotary_scale_;
+    a.rope_theta = rotary_theta_;
+    a.sm_scale = sm_scale;
+    a.q_indptr = Dev(s.cur_append_lengths_indptr);
+    a.k = k;
+    a.v = v;
+    a.pages = pages_[local_layer_id];
+    a.page_indptr = Dev(window ? s.page_indptr_sw[0] : s.page_indptr[0]);
+    a.page_values = Dev(window ? s.page_indices_sw[0] : s.page_indices[0]);
+    a.length_info = Dev(window ? s.layer_sw_length_info[0] : s.length_info[0]);
+    a.layer_window = window ? static_cast<int32_t>(layer_sliding_window_size_) : 0;
+    a.out = out;
+    a.lse = merged_lse_;
+    a.batch = static_cast<int32_t>(book_->batch_size());
+    a.h_q = static_cast<int32_t>(num_qo_heads_);
+    a.h_kv = static_cast<int32_t>(num_kv_heads_);
+    a.d = static_cast<int32_t>(qk_head_dim_);
+    a.page_size = static_cast<int32_t>(page_size_);
+    a.total_q = total_seq_length;
+    a.num_pages = num_total_pages_;
+    a.prompts = mixed_.prompts;
+    a.prompt_tokens = mixed_.prompt_tokens;
+    a.prompt_cached = mixed_.prompt_cached;
+    Launch(prefill_prompts(a, compute_stream_));
+    NewTokenDecode d;
+    d.q = q;
+    d.q_stride = q_stride;
+    d.k_new = k;
+    d.v_new = v;
+    d.new_stride = num_kv_heads_ * qk_head_dim_;
+    d.rows = DevExtra(mixed_.rows);
+    d.pages = a.pages;
+    d.page_indptr = DevExtra(mixed_.page_indptr[window]);
+    d.page_begin = DevExtra(mixed_.page_begin[window]);
+    d.page_values = a.page_values;
+    d.length_info = DevExtra(mixed_.length_info[window]);
+    d.q_rope_position = a.q_rope_position;
+    d.out = out;
+    d.lse = merged_lse_;
+    d.rotate = rotate_q ? 2 : 0;  // the keys have been rotated already
+    d.rope_scale = rotary_scale_;
+    d.rope_theta = rotary_theta_;
+    d.sm_scale = sm_scale;
+    d.nnz_pages = mixed_.nnz_pages[window];
+    d.num_pages = num_total_pages_;
+    d.batch = mixed_.decoding;
+    d.h_q = a.h_q;
+    d.h_kv = a.h_kv;
+    d.d = a.d;
+    d.page_size = a.page_size;
+    d.sliding = window;
+    Launch(decode_with_new_token(d, compute_stream_));  // behind the prompts: their launch may leave anything in these rows
+  }
+
+  // A decode step of a cache with sequence windows in two launches: the decode kernel rotates and takes the new token as
+  // one more key, and the new rows go into their page slots behind it (another sequence may still attend to what lies
+  // there).  Split, self-attention, decode, merge and append were five (64 sequences with windows of 4096 tokens, 32 / 8
+  // heads of dim 128: 26 of 232 us a layer; the step of four layers and two tokens 1880 -> 1705 us).
+  void WindowedDecodeStep(int64_t local_layer_id, const void* qkv, void* out, int64_t total_seq_length, double sm_scale) {
+    const StepLayout& s = book_->step();
+    const int64_t d = qk_head_dim_;
+    NewTokenDecode a;
+    a.q = qkv;
+    a.q_stride = a.new_stride = (num_qo_heads_ + 2 * num_kv_heads_) * d;
+    a.k_new = static_cast<const uint16_t*>(qkv) + num_qo_heads_ * d;
+    a.v_new = static_cast<const uint16_t*>(qkv) + (num_qo_heads_ + num_kv_heads_) * d;
+    a.pages = pages_[local_layer_id];
+    a.page_indptr = Dev(s.page_indptr[0]);
+    a.page_values = Dev(s.page_indices[0]);
+    a.length_info = Dev(s.length_info[0]);
+    a.k_rope_pos_offset = Dev(s.k_rope_pos_offset[0]);
+    a.q_rope_position = Dev(s.q_rope_position_map);
+    a.out = out;
+    a.lse = merged_lse_;
+    a.rotate = rope_mode_ == TVMKV_ROPE_INLINE;
+    a.rope_scale = rotary_scale_;
+    a.rope_theta = rotary_theta_;
+    a.sm_scale = sm_scale;
+    a.nnz_pages = s.page_indices[0].size;
+    a.num_pages = num_total_pages_;
+    a.batch = static_cast<int32_t>(book_->batch_size());
+    a.h_q = static_cast<int32_t>(num_qo_heads_);
+    a.h_kv = static_cast<int32_t>(num_kv_heads_);
+    a.d = static_cast<int32_t>(d);
+    a.page_size = static_cast<int32_t>(page_size_);
+    a.sliding = 1;
+    Launch(decode_with_new_token(a, compute_stream_));
+    Launch(append_strided(pages_[local_layer_id], a.k_new, a.v_new, a.new_stride, Dev(s.append_position_map), total_seq_length,
+                          num_total_pages_, a.h_kv, a.page_size, a.d, compute_stream_));
   }
 
   // A prefill step of a cache with sliding windows, RoPE inside attention or pages that the tuned kernels do not walk:
@@ -811,6 +1017,10 @@ class PagedKVCache {
                          int64_t total_seq_length, double sm_scale) {
     const int64_t local_layer_id = layer_id - layer_id_begin_offset_;
     const StepLayout& s = book_->step();
+    if (RunsMixed()) {
+      MixedAttention(layer_id, q, num_qo_heads_ * qk_head_dim_, /*rotate_q=*/false, k, v, output, total_seq_length, sm_scale);
+      return;
+    }
     // A chunked-prefill step of a plain cache: self-attention over the new tokens, attention over the
     // cached ones and their merge (:2169-2177, :2285-2292) in one pass over both key sets.
     if (OnePassPrefillApplies(layer_id)) {
@@ -1113,6 +1323,15 @@ class PagedKVCache {
   // the plan of the current step (PlanStep), held in front of the bookkeeper's arrays in both copies of the buffer
   std::vector<int32_t> extras_;
   int64_t extras_capacity_ = 0;
+  // MixedAttention: what its launches need of the step (offsets into extras_; [1]: the layers with a window);
+  // decoding == 0: the step does not run that way
+  struct MixedStep {
+    int32_t decoding = 0;
+    int64_t prompts = 0, prompt_tokens = 0, prompt_cached = 0;
+    int64_t rows = 0, page_indptr[2] = {0, 0}, page_begin[2] = {0, 0}, length_info[2] = {0, 0}, nnz_pages[2] = {0, 0};
+  };
+  MixedStep mixed_;
+  bool new_token_step_ = false;  // the step runs as WindowedDecodeStep
   // GatheredPrefill: K and V rows of a step, at most kGatherBytes (steps with more keys take the kernels that rotate
   // inside), and how many rows this step has (0: the step does not run that way)
   static constexpr int64_t kGatherBytes = int64_t{1} << 30;

@@ -55,6 +55,7 @@ struct PrefillParams {
   int kv_splits;
   int64_t split_rows;
   int page_shift;   // pages hold 16 << page_shift tokens; the kernel walks them as runs of 16-token pages
+  int skip_single;  // != 0: sequences with one query token are passed over (they have no row tiles)
   int stream_kv;    // != 0: every K/V row is read by one row tile only: copy it with the streaming hint
   int d_mem;        // padded head dims (prefill_kernel<..., PAD = true>): elements per row in memory
   // how the entries of the RoPE table are used (InlineRopeTable): position * entry instead of position /

@@ -58,6 +58,8 @@ __global__ void zero_words_kernel(unsigned long long* words, size_t count) {
   }
 }
 
+}  // namespace
+
 bool stream_is_capturing(hipStream_t stream) {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (stream != nullptr && hipStreamIsCapturing(stream, &capture) != hipSuccess) {
@@ -66,8 +68,6 @@ bool stream_is_capturing(hipStream_t stream) {
   }
   return capture != hipStreamCaptureStatusNone;
 }
-
-}  // namespace
 
 int64_t option(Option id) { return g_options.value[id].load(std::memory_order_relaxed); }
 

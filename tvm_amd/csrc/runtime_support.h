@@ -23,6 +23,7 @@ enum Option {
   kOptNoFusedDecodeStep,      // != 0: the cache object runs a decode step as split+RoPE+append and decode, two launches
   kNumOptions
 };
+bool stream_is_capturing(hipStream_t stream);
 int64_t option(Option id);
 
 // Scratch memory of a split-KV launch.  A buffer belongs to one (device, stream, user): launches on

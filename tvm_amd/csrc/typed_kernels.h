@@ -118,6 +118,60 @@ int prefill_over_gathered_kv(const void* q, int64_t q_token_stride, const int32_
                              const int32_t* kv_indptr, void* output, float* lse, double sm_scale, int32_t batch_size,
                              int64_t total_q, int32_t h_q, int32_t h_kv, int32_t d, void* stream);
 
+// Decode attention (fp16, head dims 64 / 128 / 256, tuned page sizes) of sequences whose new token is not in the pages
+// the table names: its k / v row is one more key.  rows (NULL: 0 .. batch - 1): the sequences' tokens in q, k_new,
+// v_new, q_rope_position, out and lse; page_begin (NULL: page_indptr): where their pages start in page_values, with
+// page_indptr[b + 1] - page_indptr[b] pages each.  rotate 1: q, the cached keys and the new one are rotated at their
+// positions (default frequencies); 2: the queries alone; 0: nothing.
+struct NewTokenDecode {
+  const void* q = nullptr;
+  const void* k_new = nullptr;
+  const void* v_new = nullptr;
+  int64_t q_stride = 0, new_stride = 0;  // elements between consecutive tokens
+  const int32_t* rows = nullptr;
+  const void* pages = nullptr;
+  const int32_t* page_indptr = nullptr;
+  const int32_t* page_begin = nullptr;
+  const int32_t* page_values = nullptr;
+  const int32_t* length_info = nullptr;  // (batch), or (3, batch) with `sliding`
+  const int32_t* k_rope_pos_offset = nullptr;
+  const int32_t* q_rope_position = nullptr;
+  void* out = nullptr;
+  float* lse = nullptr;
+  int64_t rotate = 0;
+  double rope_scale = 1.0, rope_theta = 1e4, sm_scale = 1.0;
+  int64_t nnz_pages = 0, num_pages = 0;  // nnz_pages: page_indptr[batch]
+  int32_t batch = 0, h_q = 0, h_kv = 0, d = 0, page_size = 0;
+  int32_t sliding = 0;
+};
+int decode_with_new_token(const NewTokenDecode& args, void* stream);
+
+// Prefill attention (fp16, head dims 64 / 128 / 256, tuned page sizes) of a step's sequences with more than one new token:
+// cached keys, then the new ones under the causal mask.  Sequences with one new token are passed over; their rows of
+// out / lse hold nothing of use afterwards.  layer_window 0: one pass over both key sets, the queries read from q with
+// q_stride and rotated if apply_rope; else the per-layer window mask over the length_info (3, batch) of such a layer.
+struct PromptPrefill {
+  const void* q = nullptr;
+  int64_t q_stride = 0;  // elements between consecutive tokens, 0: h_q * d
+  const int32_t* q_rope_position = nullptr;
+  int32_t apply_rope = 0;
+  double rope_scale = 1.0, rope_theta = 1e4, sm_scale = 1.0;
+  const int32_t* q_indptr = nullptr;
+  const void* k = nullptr;
+  const void* v = nullptr;
+  const void* pages = nullptr;
+  const int32_t* page_indptr = nullptr;
+  const int32_t* page_values = nullptr;
+  const int32_t* length_info = nullptr;
+  int32_t layer_window = 0;
+  void* out = nullptr;
+  float* lse = nullptr;
+  int32_t batch = 0, h_q = 0, h_kv = 0, d = 0, page_size = 0;
+  int64_t total_q = 0, num_pages = 0;
+  int64_t prompts = 0, prompt_tokens = 0, prompt_cached = 0;  // sequences with more than one new token: their number, new and cached tokens
+};
+int prefill_prompts(const PromptPrefill& args, void* stream);
+
 // tvmkv_kv_cache_transpose_append with the k / v rows of consecutive tokens token_stride elements apart (the fused
 // qkv tensor of the step)
 int append_strided(void* pages, const void* k_data, const void* v_data, int64_t token_stride, const int32_t* position_map,
