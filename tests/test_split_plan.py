@@ -67,6 +67,19 @@ def test_chunk_size_follows_the_work():
     assert tvm_amd.decode_split_plan([0, 100, 250, 400, 457], 457, 8)[0] == 24          # (457 / 24 + 4) * 8 = 184 items
 
 
+def test_chunks_of_a_handful_of_sequences():
+    # one step of 8 pages up to 96 pages a sequence, two for one or two sequences up to 320; one chunk up to 24
+    for n, want in ((24, 24), (25, 8), (96, 8), (97, 16), (320, 16), (321, 24)):
+        assert tvm_amd.decode_split_plan([0, n], n, 8)[0] == want
+    assert tvm_amd.decode_split_plan([0, 97, 194], 194, 8)[0] == 16
+    assert tvm_amd.decode_split_plan([0, 97, 194, 291], 291, 8)[0] == 24
+    many = [40 * i for i in range(17)]
+    assert tvm_amd.decode_split_plan(many, 640, 8)[0] == 8   # (80 + 16) * 8 = 768 workgroups
+    assert tvm_amd.decode_split_plan(many[:15] + [561], 561, 8)[0] == 8
+    many = [40 * i for i in range(18)]
+    assert tvm_amd.decode_split_plan(many, 680, 8)[0] == 16  # 8 pages would not fit
+
+
 def test_options_round_trip_and_reject_unknown_names():
     assert tvm_amd.set_option("mla_chunk_tokens", 256) == 0
     assert tvm_amd.set_option("mla_chunk_tokens", 0) == 256

@@ -206,10 +206,19 @@ int decode_pick_chunk_pages(int64_t nnz_pages, int h_kv, int batch, int head_dim
     //   64 x U[64,512]                        16: 23.4  32: 20.0   40*: 20.9  128: 19.4          [16]
     //   32 x U[100,2000]                      16: 34.6  32: 32.5   40*: 34.2  64: 36.2           [32]
     //   1 x 131072                            64: 102.3 120: 100.8 128*: 88.1                    [128]
+    // A handful of sequences: a workgroup's steps of 8 pages are a chain of round trips to memory (~2 us each) and most
+    // of the chip is idle, so chunks of one step while a sequence has no more than 12 of them to merge, for one or two
+    // sequences of two steps while they have no more than 20; sequences that fit one chunk of three steps keep it
+    // (nothing to merge).  Measured, us a layer, 32 / 8 heads of dim 128, 8 / 16 / 24 pages, * = this rule:
+    //   1 x 300       12.2 / 14.5 / 13.6*   1 x 1117           13.6* / 15.4 / 17.9   1 x 2500         16.5 / 16.0* / 18.1
+    //   1 x 4000      19.0 / 17.0* / 18.4   1 x 8000           26.9 / 21.5 / 21.2*   2 x U[500,1500]  13.6* / 16.0 / 18.4
+    //   4 x U[1000,2000]  16.8* / 16.5 / 18.8   16 x U[100,1000]  18.2* / 19.1 / 19.5   8 x U[500,3000]  30.2 / 23.7 / 23.8*
+    // Head dim 256 holds one workgroup per compute unit: 4 x U[1000,1500], 16 / 8 heads  28.3 / 21.2* / 24.3.
+    const int shortest = per_sequence <= 24 ? 24 : per_sequence <= 96 ? 8 : per_sequence <= 320 && batch <= 2 ? 16 : 24;
     int cp = 128;
-    for (int c = 24; c <= 128; c += 8) {
+    for (int c = shortest; c <= 128; c += 8) {
       if (camps(c, h_kv, head_dim)) continue;
-      if ((nnz_pages / c + batch) * h_kv <= 768) {
+      if ((nnz_pages / c + batch) * h_kv <= (c < 24 && head_dim > 128 ? 256 : 768)) {
         cp = c;
         break;
       }
