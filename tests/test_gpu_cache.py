@@ -235,17 +235,44 @@ def test_steps_that_mix_prompts_and_decoding_sequences(page_size, d, hq, hkv, wi
     m.step([(0, 1), (2, 1), (4, 1)])
 
 
+@pytest.mark.parametrize("dtype,page_size,d,hq,hkv,window", [(np.float32, 16, 128, 8, 2, 0), (np.float32, 24, 64, 4, 4, 70),
+                                                            (np.float32, 16, 256, 20, 1, 0), (np.float16, 20, 72, 6, 2, 0),
+                                                            (np.float32, 16, 96, 4, 2, 1)])
+def test_mixed_steps_on_the_generic_kernels(dtype, page_size, d, hq, hkv, window):
+    """The same for storage types, pages and head dims of the generic kernels, whose launches merge into the state of the
+    new tokens."""
+    m = Mirror([12, 4000, 1024, page_size, 0] + ([window] if window else []), 2 if window else 1, hq, hkv, d, dtype=dtype,
+               **({"attn_kinds": [3, 0]} if window else {}))
+    m.step([(0, 700), (1, 64), (2, 200)])
+    m.step([(0, 1), (4, 40), (1, 1), (3, 1), (5, 1), (2, 17)])
+    m.step([(2, 1), (0, 1), (6, 30)])
+    m.step([(4, 3), (0, 1), (2, 1), (3, 1)])
+    m.step([(0, 1), (2, 1), (4, 1)])
+
+
 def test_decode_steps_of_windowed_caches_at_the_edges():
     """A decode step of a sequence-window cache takes the new token as one more key: sequences without cached tokens, of
     one token, at the edge of a page and beyond their window, with a prompt's first decode among them."""
     for d, hq, hkv, rope_mode in ((128, 8, 2, 2), (64, 20, 1, 2), (256, 4, 2, 2), (128, 4, 4, 0)):
         layers = 2
+        # the pool is what an earlier cache of the same size left: NaN in every slot
+        used = GpuCache([8, 4096, 1024, 16, 1], layers, hq, hkv, d, d, rope_mode=rope_mode)
+        for sid in range(4):
+            used.add_sequence(sid)
+        for _ in range(4):
+            used.begin_forward([0, 1, 2, 3], [255] * 4)
+            for layer in range(layers):
+                used.attention_with_fused_qkv(layer, 1.0, np.full((1020, hq + 2 * hkv, d), np.nan, np.float16),
+                                              np.zeros((1020, hq, d), np.float16))
+            used.end_forward()
+        del used
         cache = GpuCache([8, 4096, 1024, 16, 1], layers, hq, hkv, d, d, rope_mode=rope_mode)
         sc = S.Scenario(cache, layers, hq, hkv, d, rope_mode=rope_mode, seed=9, tol=4e-3)
         for sid, (window, sink) in enumerate([(40, 0), (130, 4), (257, 30), (600, 16)]):
             sc.add_with_window(sid, window, sink)
         sc.step([(0, 1), (1, 1), (2, 1)])
         sc.step([(0, 1), (1, 1), (2, 1), (3, 1)])
+        # (a chunk longer than its window leaves slots behind the sinks that nothing ever writes)
         sc.step([(0, 14), (1, 29), (2, 300), (3, 500)])
         for _ in range(6):
             sc.step([(0, 1), (1, 1), (2, 1), (3, 1)])

@@ -760,6 +760,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
     // vmcnt reaches 0, and the reads below are done before the MFMAs that use them are issued,
     // which is before the next step's copies in program order.
     wait_vmcnt<0>();
+    const bool gap = EXT && __builtin_amdgcn_readfirstlane(pi * PS < win_lo && (pi + 2) * PS > sink);
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
       const half_t* vb = Vt + v_lane_off + (((db * 2 + v_piece) ^ v_swz) * 8);
@@ -768,6 +769,13 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
       half8_t a;
       a[0] = lo[0]; a[1] = lo[1]; a[2] = lo[2]; a[3] = lo[3];
       a[4] = hi[0]; a[5] = hi[1]; a[6] = hi[2]; a[7] = hi[3];
+      if constexpr (EXT) {
+        // slots between the sinks and the window that a chunk longer than the window was never written to
+        if (gap) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) a[i] = attended((pi + i / 4) * PS + token_of(i % 4)) ? a[i] : static_cast<half_t>(0.f);
+        }
+      }
 #pragma unroll
       for (int j = 0; j < HB; ++j) o[j][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pf[j], o[j][db], 0, 0, 0);
     }
