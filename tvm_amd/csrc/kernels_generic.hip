@@ -54,6 +54,10 @@ struct GAttn {
   int64_t total_q;
   int batch, h_q, h_kv, d, page_size, causal, splits;
   float scale_log2;
+  const int32_t* rows;        // (batch) one query token per sequence: its place in q, out and lse, or NULL: sequence b is token b
+  const int32_t* page_begin;  // (batch) where a sequence's pages start in page_values, or NULL: page_indptr
+  int skip_single;            // != 0: sequences with one query token are passed over
+  int merge_into;             // != 0: out / lse hold a state of the same rows, and this one is merged into it
   // extended form (generic_attn_kernel<..., EXT = true>)
   const int32_t* window_offset;      // paged, (batch): physical index of the first token of the window, or NULL
   const int32_t* sink_size;          // paged, (batch): attention-sink tokens kept at the front, or NULL
@@ -196,7 +200,8 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
   const int qo_len = q_begin(b + 1) - q_start;
   const int rows = qo_len * group;
   const int r0 = (slot - slot_begin(b)) * ROWS;
-  if (r0 >= rows) return;  // the whole workgroup: a slot beyond the sequence's last row tile
+  if (r0 >= rows || (p.skip_single && qo_len == 1)) return;  // the whole workgroup: a slot beyond the sequence's last row tile
+  const int q_token = p.rows != nullptr ? p.rows[b] : q_start;  // the tile's place in q and out
   const bool rotary = EXT && p.rotary != 0;
   if (EXT && rotary) {
     if (tid < d) rope_lds[tid] = rope.v[tid];
@@ -207,8 +212,8 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
   int kv_len, kv_start = 0, pbeg = 0;
   int sink = 0, window_first = 0;  // logical key t lies at physical index t (t < sink) or t - sink + window_first
   if (paged) {
-    pbeg = p.page_indptr[b];
-    const int npages = p.page_indptr[b + 1] - pbeg;
+    pbeg = p.page_begin != nullptr ? p.page_begin[b] : p.page_indptr[b];
+    const int npages = p.page_indptr[b + 1] - p.page_indptr[b];
     kv_len = npages > 0 ? (npages - 1) * p.page_size + p.last_page_len[b] : 0;  // _kernel_common.py:155-159
     if (EXT && p.window_offset != nullptr && npages > 0) {
       sink = p.sink_size[b];
@@ -265,7 +270,7 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
       const int node = min(max(qi + tree_len - qo_len, 0), tree_len - 1);
       child_first[nb] = p.tree_labels[2 * static_cast<int64_t>(tree_base + node)];
     }
-    const T* qrow = qbase + (static_cast<int64_t>(q_start + qi) * p.h_q + head) * d;
+    const T* qrow = qbase + (static_cast<int64_t>(q_token + qi) * p.h_q + head) * d;
 #pragma unroll
     for (int s = 0; s < QS; ++s) {
       const int f = piece_feature(s);
@@ -281,7 +286,7 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
       }
     }
     if (EXT && rotary && valid) {
-      const float pos = static_cast<float>(p.q_rope_position[q_start + qi]) * p.rope_scale;
+      const float pos = static_cast<float>(p.q_rope_position[q_token + qi]) * p.rope_scale;
 #pragma unroll
       for (int s = 0; s < QS / 2; ++s) {
         if (!piece_inside(s)) continue;
@@ -497,13 +502,26 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
   for (int nb = 0; nb < NB; ++nb) {
     const int row = r0 + nb * 16 + j;
     if (row >= rows) continue;
-    const int64_t out_row = static_cast<int64_t>(q_start + row / group) * p.h_q + kvh * group + row % group;
+    const int64_t out_row = static_cast<int64_t>(q_token + row / group) * p.h_q + kvh * group + row % group;
     const bool any = lsum[nb] > 0.f;
-    const float inv = any ? 1.0f / lsum[nb] : 0.f;
+    float inv = any ? 1.0f / lsum[nb] : 0.f;
     const float s_row = any ? m[nb] + fast_log2(lsum[nb]) : kNoKeys;
     // runs of KS consecutive features: (4 g + r) * KS + fb, fb = 0 .. KS - 1
     if (p.splits == 1) {
       T* dst = static_cast<T*>(p.out) + out_row * d;
+      float mine = 1.f, theirs = 0.f;  // weights of this state and of the one that is there
+      float lse = any ? s_row : kNegInit;
+      if (p.merge_into) {  // the arithmetic of merge_state_inplace
+        const float other = p.lse[out_row];
+        const float top = fmaxf(lse, other);
+        mine = fast_exp2(lse - top);
+        theirs = fast_exp2(other - top);
+        const float sum = mine + theirs;
+        lse = top + fast_log2(sum);
+        mine /= sum;
+        theirs /= sum;
+      }
+      inv *= mine;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
 #pragma unroll
@@ -512,13 +530,20 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
           float run[VP];
 #pragma unroll
           for (int e = 0; e < VP; ++e) run[e] = o[nb][c * VP + e][r] * inv;
-          if (f < d) store_run<T, VP>(dst + f, run);
+          if (f < d) {
+            if (p.merge_into) {
+#pragma unroll
+              for (int e = 0; e < VP; ++e) run[e] += theirs * static_cast<float>(dst[f + e]);
+            }
+            store_run<T, VP>(dst + f, run);
+          }
         }
       }
       // a row without keys: out = 0 and the state the reference's kernels start from, m = -5e4, d = 1
-      if (g == 0) p.lse[out_row] = any ? s_row : kNegInit;
+      if (g == 0) p.lse[out_row] = lse;
     } else {
-      float* dst = p.part_o + (static_cast<int64_t>(split) * p.total_q * p.h_q + out_row) * d;
+      const int64_t part_row = static_cast<int64_t>(q_start + row / group) * p.h_q + kvh * group + row % group;
+      float* dst = p.part_o + (static_cast<int64_t>(split) * p.total_q * p.h_q + part_row) * d;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
 #pragma unroll
@@ -530,30 +555,42 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
           if (f < d) store_run<float, 4>(dst + f, run);
         }
       }
-      if (g == 0) p.part_s[static_cast<int64_t>(split) * p.total_q * p.h_q + out_row] = s_row;
+      if (g == 0) p.part_s[static_cast<int64_t>(split) * p.total_q * p.h_q + part_row] = s_row;
     }
   }
 }
 
-// The shares of a split launch: one workgroup of 64 lanes per (query, head) row.
+// The shares of a split launch: one workgroup of 64 lanes per (query, head) row.  token_rows: GAttn::rows; merge_into: the
+// state in out / lse is one more share.
 template <typename T>
 __global__ __launch_bounds__(64) void generic_merge_kernel(const float* part_o, const float* part_s, T* out, float* lse,
-                                                          int64_t rows, int d, int splits) {
+                                                          int64_t rows, int d, int splits, const int32_t* token_rows, int h_q,
+                                                          int merge_into) {
   const int64_t row = blockIdx.x;
-  float s_max = kNoKeys;
-  for (int z = 0; z < splits; ++z) s_max = fmaxf(s_max, part_s[z * rows + row]);
+  const int64_t out_row = token_rows != nullptr ? static_cast<int64_t>(token_rows[row / h_q]) * h_q + row % h_q : row;
+  // at most 64 shares: lane z holds the weight of share z
+  const int lane = threadIdx.x;
+  const float s_mine = lane < splits ? part_s[lane * rows + row] : kNoKeys;
+  const float s_there = merge_into ? lse[out_row] : kNoKeys;
+  float s_max = s_mine;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s_max = fmaxf(s_max, __shfl_xor(s_max, off, 64));
+  s_max = fmaxf(s_max, s_there);
   const bool any = s_max > 0.5f * kNoKeys;
-  float total = 0.f;
-  for (int z = 0; z < splits; ++z) total += any ? fast_exp2(part_s[z * rows + row] - s_max) : 0.f;
-  for (int f = threadIdx.x; f < d; f += 64) {
-    float acc = 0.f;
-    for (int z = 0; z < splits; ++z) {
-      const float w = any ? fast_exp2(part_s[z * rows + row] - s_max) : 0.f;
-      acc += w * part_o[(z * rows + row) * d + f];
-    }
-    out[row * d + f] = static_cast<T>(any ? acc / total : 0.f);
+  const float w_mine = any ? fast_exp2(s_mine - s_max) : 0.f;
+  const float w_there = any && merge_into ? fast_exp2(s_there - s_max) : 0.f;
+  float total = w_mine;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off, 64);
+  total += w_there;
+  for (int f0 = 0; f0 < d; f0 += 64) {
+    const int f = min(f0 + lane, d - 1);
+    float acc = merge_into ? w_there * static_cast<float>(out[out_row * d + f]) : 0.f;
+#pragma unroll 8
+    for (int z = 0; z < splits; ++z) acc += __shfl(w_mine, z, 64) * part_o[(z * rows + row) * d + f];
+    if (f0 + lane < d) out[out_row * d + f] = static_cast<T>(any ? acc / total : 0.f);
   }
-  if (threadIdx.x == 0) lse[row] = any ? s_max + fast_log2(total) : kNegInit;
+  if (lane == 0) lse[out_row] = any ? s_max + fast_log2(total) : kNegInit;
 }
 
 template <typename T, bool EXT>
@@ -608,6 +645,8 @@ int generic_attention(const GenericAttention& a, void* stream_) {
   } else {
     KV_CHECK(a.k && a.v && a.kv_indptr) << a.what << ": NULL tensor";
   }
+  KV_CHECK((a.rows == nullptr && a.page_begin == nullptr) || (paged && a.q_indptr == nullptr))
+      << a.what << ": rows and page_begin are for decoding sequences";
   KV_CHECK((a.tree_indptr == nullptr) == (a.tree_labels == nullptr)) << a.what << ": tree_indptr and the labels come together";
   KV_CHECK(a.total_q * a.h_q < (int64_t{1} << 31)) << a.what << ": too many rows for one launch";
 
@@ -632,6 +671,10 @@ int generic_attention(const GenericAttention& a, void* stream_) {
   p.d = a.d;
   p.page_size = a.page_size;
   p.causal = a.causal;
+  p.rows = a.rows;
+  p.page_begin = a.page_begin;
+  p.skip_single = a.skip_single;
+  p.merge_into = a.merge_into;
   p.scale_log2 = static_cast<float>(a.sm_scale) * kLog2e;
   // length_info of a sliding-window cache: (3, batch) = last page length, window offset, sink size (attn_utils.h:483-495)
   p.window_offset = sliding ? a.last_page_len + a.batch : nullptr;
@@ -651,15 +694,16 @@ int generic_attention(const GenericAttention& a, void* stream_) {
   }
   const bool ext = sliding || rotary;
   const int group = a.h_q / a.h_kv;
-  const int rows_hint = static_cast<int>(std::min<int64_t>(a.total_q * group / a.batch, 1 << 20));
+  const int64_t work_q = a.work_seqs > 0 ? a.work_q : a.total_q, work_seqs = a.work_seqs > 0 ? a.work_seqs : a.batch;
+  const int rows_hint = static_cast<int>(std::min<int64_t>(work_q * group / work_seqs, 1 << 20));
   // Few row tiles against long page lists: split the keys over workgroups until the chip has ~8 workgroups
   // per compute unit, at least 128 keys (8 blocks) per share on average.  Shapes only: no device read.
   p.splits = 1;
   ScratchLease lease{};
-  if (paged) {
+  if (paged && a.skip_single == 0) {  // (the rows that are passed over have no partial states to merge)
     const int rows_per_tile = 16 * generic_row_blocks(a.d, rows_hint);
-    const int64_t tiles = (a.total_q * group / rows_per_tile + a.batch) * a.h_kv;
-    const int64_t keys_per_seq = a.nnz_pages * a.page_size / a.batch;
+    const int64_t tiles = (work_q * group / rows_per_tile + work_seqs) * a.h_kv;
+    const int64_t keys_per_seq = a.nnz_pages * a.page_size / work_seqs;
     const int64_t want = (f32 ? 8 : 16) * static_cast<int64_t>(compute_units()) / std::max<int64_t>(tiles, 1);
     p.splits = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({want, keys_per_seq / 128, 64})));
   }
@@ -679,10 +723,10 @@ int generic_attention(const GenericAttention& a, void* stream_) {
     const int64_t rows = a.total_q * a.h_q;
     if (f32) {
       hipLaunchKernelGGL(generic_merge_kernel<float>, dim3(static_cast<unsigned>(rows)), dim3(64), 0, stream, p.part_o, p.part_s,
-                         static_cast<float*>(a.out), a.lse, rows, a.d, p.splits);
+                         static_cast<float*>(a.out), a.lse, rows, a.d, p.splits, a.rows, a.h_q, a.merge_into);
     } else {
       hipLaunchKernelGGL(generic_merge_kernel<half_t>, dim3(static_cast<unsigned>(rows)), dim3(64), 0, stream, p.part_o, p.part_s,
-                         static_cast<half_t*>(a.out), a.lse, rows, a.d, p.splits);
+                         static_cast<half_t*>(a.out), a.lse, rows, a.d, p.splits, a.rows, a.h_q, a.merge_into);
     }
     KV_LAUNCH_CHECK();
   }

@@ -723,15 +723,11 @@ class PagedKVCache {
     const StepLayout& s = book_->step();
     const int64_t batch = book_->batch_size();
     if (batch > reserved_num_seqs_) return;  // the plans are sized for that many
-    const bool tuned_decode = !generic_ && elem_bits_ == 16 && qk_head_dim_ == v_head_dim_ && s.num_depths == 1 &&
-                              s.is_chain[0] && !s.append_before_attn && s.qo_indptr[0].size == batch + 1;
-    new_token_step_ = tuned_decode && support_sliding_window_ && s.use_decode_kernel[0] && rope_mode_ != TVMKV_ROPE_NORMAL &&
+    const bool one_level = qk_head_dim_ == v_head_dim_ && s.num_depths == 1 && s.is_chain[0] && !s.append_before_attn &&
+                           s.qo_indptr[0].size == batch + 1;
+    new_token_step_ = one_level && !generic_ && support_sliding_window_ && s.use_decode_kernel[0] && rope_mode_ != TVMKV_ROPE_NORMAL &&
                       !has_rope_scaling_ && rope_ext_factors_ == nullptr &&
                       (qk_head_dim_ == 64 || qk_head_dim_ == 128 || qk_head_dim_ == 256);
-    if (tuned_decode && !support_sliding_window_ && !s.use_decode_kernel[0] && s.page_indices[0].size > 0 && rope_mode_ != TVMKV_ROPE_INLINE &&
-        (qk_head_dim_ == 64 || qk_head_dim_ == 128)) {
-      PlanMixedStep();
-    }
     if (gather_capable_ && rope_ext_factors_ == nullptr && s.num_depths == 1 && s.is_chain[0] && !s.append_before_attn &&
         !s.use_decode_kernel[0] &&
         s.total_append_length * (num_qo_heads_ / num_kv_heads_) >=
@@ -754,6 +750,10 @@ class PagedKVCache {
         extras_[b + 1] = static_cast<int32_t>(std::min<int64_t>(rows, INT32_MAX));
       }
       if (rows <= gather_capacity_) gathered_rows_ = rows; else extras_.clear();
+    }
+    if (gathered_rows_ == 0 && one_level && !support_sliding_window_ && !s.use_decode_kernel[0] && s.page_indices[0].size > 0 &&
+        rope_mode_ != TVMKV_ROPE_INLINE && (generic_ || qk_head_dim_ == 64 || qk_head_dim_ == 128)) {
+      PlanMixedStep();
     }
     if (!extras_.empty()) {
       std::memcpy(static_cast<int32_t*>(aux_staging_[aux_slot_]) + extras_capacity_ - extras_.size(), extras_.data(),
@@ -780,10 +780,12 @@ class PagedKVCache {
       return pages > 0 ? (pages - 1) * page_size_ + last_len[b] : 0;
     };
     // What the step takes either way, in tiles of 64 keys by 128 rows that a workgroup walks one after the other (about
-    // 1 us each at head dim 128, 0.6 at 64, and 8 tiles' time before the first): the longest walk, or all of them on
+    // 1 us each at head dim 128, 0.6 at 64, and 8 tiles' time before the first; 64 keys by 32 rows on the generic kernel,
+    // 3 us in float32 and 1.5 in fp16): the longest walk, or all of them on
     // the workgroups the chip holds.  The decode kernel: 10 us and the K / V rows at 6 TB/s.
     const bool wide = qk_head_dim_ == 128;
-    const double tile_us = wide ? 1.0 : 0.6, resident = 256 * (wide ? 2 : 3);
+    const double tile_us = generic_ ? (elem_bits_ == 32 ? 3.0 : 1.5) : wide ? 1.0 : 0.6, resident = 256 * (wide ? 2 : 3);
+    const int64_t tile_rows = generic_ ? 32 : 128;
     const int64_t group = num_qo_heads_ / num_kv_heads_;
     double walk_decode = 0, walk_prompt = 0, work_decode = 0, work_prompt = 0, decode_bytes = 0;
     for (int64_t b = 0; b < batch; ++b) {
@@ -793,13 +795,13 @@ class PagedKVCache {
         ++plan.decoding;
         walk_decode = std::max(walk_decode, walk);
         work_decode += walk * num_kv_heads_;
-        decode_bytes += 4.0 * keys * num_kv_heads_ * qk_head_dim_;
+        decode_bytes += elem_bits_ / 4.0 * keys * num_kv_heads_ * qk_head_dim_;
       } else {
         ++plan.prompts;
         plan.prompt_tokens += n;
         plan.prompt_cached += keys;
         walk_prompt = std::max(walk_prompt, walk);
-        work_prompt += (8.0 + static_cast<double>(keys + n / 2) / 64) * num_kv_heads_ * ((n * group + 127) / 128);
+        work_prompt += (8.0 + static_cast<double>(keys + n / 2) / 64) * num_kv_heads_ * ((n * group + tile_rows - 1) / tile_rows);
       }
     }
     if (plan.decoding == 0 || plan.prompts == 0) return;
@@ -848,6 +850,10 @@ class PagedKVCache {
     const StepLayout& s = book_->step();
     const int64_t local_layer_id = layer_id - layer_id_begin_offset_;
     const bool window = attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING;
+    if (generic_) {
+      GenericMixedAttention(layer_id, q, k, v, out, total_seq_length, sm_scale);
+      return;
+    }
     PromptPrefill a;
     a.q = q;
     a.q_stride = q_stride;
@@ -905,6 +911,54 @@ class PagedKVCache {
     d.page_size = a.page_size;
     d.sliding = window;
     Launch(decode_with_new_token(d, compute_stream_));  // behind the prompts: their launch may leave anything in these rows
+  }
+
+  // The same on the generic kernel: every sequence's new tokens, then the cached ones of the prompts and those of the
+  // decoding sequences (whose launch splits the keys), merged into that state.
+  void GenericMixedAttention(int64_t layer_id, const void* q, const void* k, const void* v, void* out, int64_t total_seq_length,
+                             double sm_scale) {
+    const StepLayout& s = book_->step();
+    const int64_t local_layer_id = layer_id - layer_id_begin_offset_;
+    const bool window = attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING;
+    GenericRagged(q, k, v, out, merged_lse_, total_seq_length, sm_scale, /*tree=*/false);
+    GenericAttention a;
+    a.what = "cross attention";
+    a.elem_bits = elem_bits_;
+    a.q = q;
+    a.pages = pages_[local_layer_id];
+    a.page_values = Dev(window ? s.page_indices_sw[0] : s.page_indices[0]);
+    a.num_pages = num_total_pages_;
+    a.out = out;
+    a.lse = merged_lse_;
+    a.merge_into = 1;
+    a.h_q = static_cast<int32_t>(num_qo_heads_);
+    a.h_kv = static_cast<int32_t>(num_kv_heads_);
+    a.d = static_cast<int32_t>(qk_head_dim_);
+    a.page_size = static_cast<int32_t>(page_size_);
+    a.sm_scale = sm_scale;
+    a.sliding_window = window;
+    if (mixed_.prompt_cached > 0) {
+      GenericAttention prompts = a;
+      prompts.q_indptr = Dev(s.qo_indptr[0]);
+      prompts.page_indptr = Dev(window ? s.page_indptr_sw[0] : s.page_indptr[0]);
+      prompts.last_page_len = Dev(window ? s.layer_sw_length_info[0] : s.length_info[0]);
+      prompts.total_q = total_seq_length;
+      prompts.batch = static_cast<int32_t>(book_->batch_size());
+      prompts.causal = window;
+      prompts.layer_window = static_cast<int32_t>(layer_sliding_window_size_);
+      prompts.skip_single = 1;
+      prompts.work_q = mixed_.prompt_tokens;
+      prompts.work_seqs = mixed_.prompts;
+      prompts.nnz_pages = mixed_.prompt_cached / page_size_;
+      Launch(generic_attention(prompts, compute_stream_));
+    }
+    a.rows = DevExtra(mixed_.rows);
+    a.page_indptr = DevExtra(mixed_.page_indptr[window]);
+    a.page_begin = DevExtra(mixed_.page_begin[window]);
+    a.last_page_len = DevExtra(mixed_.length_info[window]);
+    a.total_q = a.batch = mixed_.decoding;
+    a.nnz_pages = mixed_.nnz_pages[window];
+    Launch(generic_attention(a, compute_stream_));
   }
 
   // A decode step of a cache with sequence windows in two launches: the decode kernel rotates and takes the new token as

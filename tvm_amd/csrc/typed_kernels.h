@@ -68,6 +68,14 @@ struct GenericAttention {
   const int32_t* k_rope_pos_offset = nullptr;
   double rope_scale = 1.0, rope_theta = 1e4;
   const tvmkv_rope_scaling* rope_scaling = nullptr;
+  // rows, page_begin (paged, q_indptr NULL): sequence b's query is token rows[b] of q, q_rope_position, out and lse (NULL:
+  // b), its pages start at page_values[page_begin[b]] (NULL: page_indptr[b]).  skip_single: sequences with one query
+  // token are passed over; work_q / work_seqs / nnz_pages then describe the others.  merge_into: out / lse hold an
+  // attention state of the rows that are computed, and this one is merged into it.
+  const int32_t* rows = nullptr;
+  const int32_t* page_begin = nullptr;
+  int32_t skip_single = 0, merge_into = 0;
+  int64_t work_q = 0, work_seqs = 0;
 };
 int generic_attention(const GenericAttention& args, void* stream);
 
