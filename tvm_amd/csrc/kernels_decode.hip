@@ -143,10 +143,12 @@ __device__ __forceinline__ void load_partial_row(const float* src, float (&dst)[
   }
 }
 
-template <int D, bool COHERENT>
+// ROWS: the output row may be another than the sequence's (DecodeParams::rows); the plain kernels don't look, the pointer
+// cost them scalar registers (64 sequences of 256-2048 tokens 54.6 -> 57.9 us).
+template <int D, bool COHERENT, bool ROWS>
 __device__ __forceinline__ void merge_row(const DecodeParams& p, int b, int hq, int nchunks, int lane) {
   constexpr int EPL = D / 64;  // features per lane
-  const int64_t row = static_cast<int64_t>(p.rows != nullptr ? p.rows[b] : b) * p.h_q + hq;
+  const int64_t row = static_cast<int64_t>(ROWS && p.rows != nullptr ? p.rows[b] : b) * p.h_q + hq;
   const int dm = p.d_mem > 0 ? p.d_mem : D;
   half_t* out = p.output + row * dm + lane * EPL;
   const int s0 = slot_begin(p.page_indptr, b, p.chunk_pages);
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p, int t
     empty_row<D>(p, b, hq, lane);
     return;
   }
-  merge_row<D, false>(p, b, hq, nchunks, lane);
+  merge_row<D, false, true>(p, b, hq, nchunks, lane);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -864,7 +866,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
     }
     __syncthreads();
     if (sm_last) {
-      for (int g = wave; g < heads; g += 4) merge_row<D, true>(p, b, hq0 + g, nchunks, lane);
+      for (int g = wave; g < heads; g += 4) merge_row<D, true, SELF>(p, b, hq0 + g, nchunks, lane);
     }
   }
   __syncthreads();  // the merge buffers are the next item's V tiles
