@@ -77,6 +77,28 @@ def test_float32_decode_and_paged_prefill(hq, hkv, d, ps):
     del keep
 
 
+@pytest.mark.parametrize("d", [2, 8, 12, 72, 76, 248, 256])
+def test_rope_in_runs_of_four_and_single_elements(d):
+    """float32 rows whose halves hold whole runs of four elements (8, 72, 248, 256) and ones that do not, an odd number of
+    heads, against the arithmetic in 64 bits: an angle below 2 rad is off by 2^-23 of itself at most, its sine and cosine
+    and the two products by a few 2^-24 of the row."""
+    hq, hkv = 3, 1
+    rng = np.random.default_rng(310)
+    pos = np.array([0, 1, 2], np.int32)
+    qkv = rng.standard_normal((3, hq + 2 * hkv, d)).astype(F32)
+    gq, gq_dl = T(np.zeros((3, hq, d), F32))
+    gk, gk_dl = T(np.zeros((3, hkv, d), F32))
+    gv, gv_dl = T(np.zeros((3, hkv, d), F32))
+    dl.call("fused_rope", T(qkv)[1], TI(pos), gq_dl, gk_dl, gv_dl, 1, None, None, 1.0, 1e4)
+    x = qkv.astype(np.float64)
+    angle = pos[:, None, None] / 1e4 ** (2 * (np.arange(d) % (d // 2)) / d)
+    half = np.concatenate([-x[..., d // 2:], x[..., :d // 2]], axis=-1)
+    rotated = np.cos(angle) * x + np.sin(angle) * half
+    assert_close(host(gq), rotated[:, :hq], atol=4e-6, rtol=2e-6, what="q")
+    assert_close(host(gk), rotated[:, hq:hq + hkv], atol=4e-6, rtol=2e-6, what="k")
+    assert np.array_equal(host(gv), qkv[:, hq + hkv:])
+
+
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (8, 2, 64), (4, 4, 100)])
 def test_float32_ragged_tree_merge_and_rope(hq, hkv, d):
     rng = np.random.default_rng(301)

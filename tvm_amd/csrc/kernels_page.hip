@@ -332,10 +332,12 @@ __global__ __launch_bounds__(256) void merge_state_inplace_kernel(half_t* __rest
 }
 
 // The split-rotary kernel for what the vectorised one above is not built for: float32 storage and head dims
-// outside its list (any even head dim up to kMaxHeadDim).  The same tables and the same arithmetic, one
-// element per thread and step: element e of a rotating head becomes cos * x[e] + sin * partner(e), the partner
+// outside its list (any even head dim up to kMaxHeadDim).  The same tables and the same arithmetic, RUN
+// consecutive elements per thread and step -- 4 where a run and its partners are aligned and lie in one half of the
+// rotated part, else 1 (1500 tokens of 32 / 8 heads of dim 128 in float32: 48 us with single elements, whose index
+// division and narrow accesses bounded it, 19 with runs): element e of a rotating head becomes cos * x[e] + sin * partner(e), the partner
 // being -x[e + R/2] / x[e - R/2], or -x[e + 1] / x[e - 1] for the gptj pairing.
-template <typename T, bool APPEND>
+template <typename T, bool APPEND, int RUN>
 __global__ __launch_bounds__(256) void fused_rope_any_kernel(const T* __restrict__ qkv, const int32_t* __restrict__ position_map,
                                                              T* __restrict__ q, T* __restrict__ k, T* __restrict__ v,
                                                              int num_q_heads, int num_kv_heads, int D, int apply_rope,
@@ -369,31 +371,35 @@ __global__ __launch_bounds__(256) void fused_rope_any_kernel(const T* __restrict
     __syncthreads();
   }
   const int32_t slot = APPEND ? append_position_map[s] : -1;
-  const int first = q == nullptr ? num_q_heads * D : 0;  // q == NULL: the q rows are left alone
-  for (int idx = first + threadIdx.x; idx < fused_heads * D; idx += 256) {
-    const int h = idx / D, e = idx - h * D;
+  typedef T run_t __attribute__((ext_vector_type(RUN)));
+  const int runs = D / RUN;
+  const int first = q == nullptr ? num_q_heads * runs : 0;  // q == NULL: the q rows are left alone
+  for (int idx = first + threadIdx.x; idx < fused_heads * runs; idx += 256) {
+    const int h = idx / runs, e = (idx - h * runs) * RUN;
     const T* row = qkv + (s * fused_heads + h) * D;
-    float x = static_cast<float>(row[e]);
-    T result = row[e];
+    run_t result = *reinterpret_cast<const run_t*>(row + e);
     if (apply_rope > 0 && h < num_q_heads + num_kv_heads && e < R) {
-      float other;
-      if (interleaved) {
-        other = (e & 1) == 0 ? -static_cast<float>(row[e + 1]) : static_cast<float>(row[e - 1]);
-      } else {
-        other = e < R / 2 ? -static_cast<float>(row[e + R / 2]) : static_cast<float>(row[e - R / 2]);
+      const bool pairs = RUN == 1 && interleaved;
+      const bool low = pairs ? (e & 1) == 0 : e < R / 2;
+      const int partner = pairs ? (low ? e + 1 : e - 1) : (low ? e + R / 2 : e - R / 2);
+      const run_t there = *reinterpret_cast<const run_t*>(row + partner);
+#pragma unroll
+      for (int i = 0; i < RUN; ++i) {
+        const float other = low ? -static_cast<float>(there[i]) : static_cast<float>(there[i]);
+        result[i] = static_cast<T>(cs_lds[e + i] * static_cast<float>(result[i]) + sn_lds[e + i] * other);
       }
-      result = static_cast<T>(cs_lds[e] * x + sn_lds[e] * other);
     }
     if (h < num_q_heads) {
-      q[(s * num_q_heads + h) * D + e] = result;
+      *reinterpret_cast<run_t*>(q + (s * num_q_heads + h) * D + e) = result;
       continue;
     }
     const int kv = h >= num_q_heads + num_kv_heads;
     const int head = h - num_q_heads - kv * num_kv_heads;
-    (kv ? v : k)[(s * num_kv_heads + head) * D + e] = result;
+    *reinterpret_cast<run_t*>((kv ? v : k) + (s * num_kv_heads + head) * D + e) = result;
     if (APPEND && slot != -1) {
-      pages[((static_cast<int64_t>(slot / page_size) * 2 + kv) * num_kv_heads + head) * (static_cast<int64_t>(page_size) * D) +
-            static_cast<int64_t>(slot % page_size) * D + e] = result;
+      *reinterpret_cast<run_t*>(pages + ((static_cast<int64_t>(slot / page_size) * 2 + kv) * num_kv_heads + head) *
+                                            (static_cast<int64_t>(page_size) * D) +
+                                static_cast<int64_t>(slot % page_size) * D + e) = result;
     }
   }
 }
@@ -732,12 +738,25 @@ static int fused_rope_impl(const void* qkv, const int32_t* position_map, void* q
                        page_size, rotary_dim, static_cast<int>(scaling != nullptr && scaling->rope_type == TVMKV_ROPE_FREQ_GPTJ));
   };
   if (!vectorised) {
-    if (elem_bits == 32) {
-      if (append) launch_any(fused_rope_any_kernel<float, true>, static_cast<float*>(nullptr));
-      else launch_any(fused_rope_any_kernel<float, false>, static_cast<float*>(nullptr));
+    const int64_t run_bytes = 4 * (elem_bits / 8);
+    bool runs = head_dim % 4 == 0 && rotary_dim % 8 == 0 && !(scaling != nullptr && scaling->rope_type == TVMKV_ROPE_FREQ_GPTJ);
+    for (const void* p : {qkv, static_cast<const void*>(q), static_cast<const void*>(k), static_cast<const void*>(v), static_cast<const void*>(pages)}) {
+      runs = runs && reinterpret_cast<uintptr_t>(p) % run_bytes == 0;
+    }
+    auto launch_runs = [&](auto append_c, auto run_c) {
+      constexpr bool kAppend = decltype(append_c)::value;
+      constexpr int kRun = decltype(run_c)::value;
+      if (elem_bits == 32) {
+        launch_any(fused_rope_any_kernel<float, kAppend, kRun>, static_cast<float*>(nullptr));
+      } else {
+        launch_any(fused_rope_any_kernel<half_t, kAppend, kRun>, static_cast<half_t*>(nullptr));
+      }
+    };
+    using std::integral_constant;
+    if (append) {
+      if (runs) launch_runs(std::true_type{}, integral_constant<int, 4>{}); else launch_runs(std::true_type{}, integral_constant<int, 1>{});
     } else {
-      if (append) launch_any(fused_rope_any_kernel<half_t, true>, static_cast<half_t*>(nullptr));
-      else launch_any(fused_rope_any_kernel<half_t, false>, static_cast<half_t*>(nullptr));
+      if (runs) launch_runs(std::false_type{}, integral_constant<int, 4>{}); else launch_runs(std::false_type{}, integral_constant<int, 1>{});
     }
   } else if (head_dim == 64) {
     if (append) launch(fused_rope_kernel<64, true>); else launch(fused_rope_kernel<64, false>);
