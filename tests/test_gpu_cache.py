@@ -250,6 +250,25 @@ def test_mixed_steps_on_the_generic_kernels(dtype, page_size, d, hq, hkv, window
     m.step([(0, 1), (2, 1), (4, 1)])
 
 
+@pytest.mark.parametrize("d,lengths", [(128, (1500, 90)), (64, (1500, 90)), (128, (1200, 1100))])
+def test_tree_steps_over_sequences_of_unlike_lengths(d, lengths):
+    """A verify step whose row tiles are full and whose longest sequence is well above the mean walks its keys in two
+    shares (64 kv heads here: one round of workgroups); the tree's own state is merged with both."""
+    hq, hkv, nodes = 64, 64, 70
+    m = Mirror([8, 4096, 1600, 16, 0], 1, hq, hkv, d)
+    m.step([(0, lengths[0])])
+    m.step([(1, lengths[1])])
+    parents = [(i - 1) // 2 if i else -1 for i in range(nodes)]
+    m.o.begin_forward([0, 1], [nodes, nodes], parents * 2)
+    m.g.begin_forward([0, 1], [nodes, nodes], parents * 2)
+    qkv = m.rng.standard_normal((2 * nodes, hq + 2 * hkv, d)).astype(np.float16)
+    eo = np.zeros((2 * nodes, hq, d), np.float16)
+    go = np.zeros_like(eo)
+    m.o.attention_with_fused_qkv(0, d ** -0.5, qkv, eo)
+    m.g.attention_with_fused_qkv(0, d ** -0.5, qkv, go)
+    assert_close(go, eo, what="tree step over unlike lengths")
+
+
 def test_decode_steps_of_windowed_caches_at_the_edges():
     """A decode step of a sequence-window cache takes the new token as one more key: sequences without cached tokens, of
     one token, at the edge of a page and beyond their window, with a prompt's first decode among them."""

@@ -858,7 +858,11 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(const half_t* 
 //    2000-6000 keys, 512 workgroups: 0.171 ms unsplit, 0.183 with 2 shares; a 63-node tree per sequence,
 //    1008 workgroups, matrix-bound: 0.409 against 0.442).
 // No share shorter than 8 tiles on average, at most 64 shares.
-static int pick_kv_splits(int64_t total_q, int group, int batch, int h_kv, int64_t avg_keys) {
+// longest: the keys of the longest sequence where the caller knows them, else 0.  One round of full row tiles lasts as
+// long as its longest walk: two shares each when that is well above the mean (us a layer, 64 sequences with a 31-node
+// tree, 32 / 8 heads, unsplit -> two shares: U[1024,8192] cached tokens 311 -> 286 at head dim 128, 233 -> 186 at 64;
+// U[4000,5000], where the walks are alike, 267 -> 283).
+static int pick_kv_splits(int64_t total_q, int group, int batch, int h_kv, int64_t avg_keys, int64_t longest) {
   const int64_t forced = option(kOptPrefillKvSplits);
   if (forced > 0) return static_cast<int>(std::min<int64_t>(forced, 64));
   const int64_t resident = static_cast<int64_t>(compute_units()) * 2;
@@ -867,7 +871,7 @@ static int pick_kv_splits(int64_t total_q, int group, int batch, int h_kv, int64
   int64_t want = 1;
   if (workgroups * 2 <= resident) {
     want = (2 * resident + workgroups - 1) / workgroups;
-  } else if (workgroups <= resident && total_q * group * 2 <= tiles * BM) {
+  } else if (workgroups <= resident && (total_q * group * 2 <= tiles * BM || longest * 10 >= avg_keys * 14)) {
     want = 2;
   }
   const int64_t by_length = avg_keys / (8 * BN);
@@ -883,12 +887,13 @@ struct KvSplit {
   int merge_into = 0;
   ScratchLease lease{};
   // work_q, work_seqs: the query tokens and sequences that the launch works on, where they are not all (skip_single)
-  KvSplit(PrefillParams& p, int64_t total_q, int64_t avg_keys, int dv, hipStream_t stream, int64_t work_q = 0, int64_t work_seqs = 0)
+  KvSplit(PrefillParams& p, int64_t total_q, int64_t avg_keys, int dv, hipStream_t stream, int64_t work_q = 0, int64_t work_seqs = 0,
+          int64_t longest = 0)
       : output(p.output), lse(p.lse), rows(total_q * p.h_q), splits(1) {
     if (work_seqs == 0) work_q = total_q, work_seqs = p.batch_size;
     // at most one row tile per (sequence, kv head) on average: the paged kernels stream the K/V rows
     p.stream_kv = work_q * p.group <= work_seqs * BM;
-    splits = pick_kv_splits(work_q, p.group, work_seqs, p.h_kv, avg_keys);
+    splits = pick_kv_splits(work_q, p.group, work_seqs, p.h_kv, avg_keys, longest);
     if (dv % 64 != 0) splits = 1;  // padded head dims (80, 96, 112): the merge kernel is not built for their rows
     if (splits <= 1) return;
     const size_t o_bytes = static_cast<size_t>(splits) * rows * dv * sizeof(half_t);
@@ -1200,7 +1205,7 @@ static int paged_prefill(const void* q, const int32_t* q_indptr, const void* pag
                          int32_t batch_size, int64_t total_q, int64_t nnz_pages, int64_t num_pages, int32_t h_q,
                          int32_t h_kv, int32_t d, int32_t page_size, int32_t sliding_window,
                          int32_t sliding_window_size, bool merge_into, void* stream,
-                         const tvmkv_rope_scaling* scaling = nullptr) {
+                         const tvmkv_rope_scaling* scaling = nullptr, int64_t longest = 0) {
   // pages other than 16 / 32 / 64 / 128 tokens, other head dims (80 / 96 / 112 with a sliding-window cache or RoPE
   // inside the kernel among them): the generic matrix-core kernel (its caller merges states with merge_state_inplace)
   const bool plain = rotary_mode == 0 && sliding_window == 0;
@@ -1275,7 +1280,7 @@ static int paged_prefill(const void* q, const int32_t* q_indptr, const void* pag
   }
   const bool ext = p.rotary != 0 || sliding_window != 0;
   hipStream_t s = as_stream(stream);
-  const KvSplit split(p, total_q, nnz_pages * page_size / batch_size, d, s);
+  const KvSplit split(p, total_q, nnz_pages * page_size / batch_size, d, s, 0, 0, longest);
   if (d == 128) {
     launch_prefill<128, 128, kPaged, 16>(p, total_q, ext, rope_theta, s, scaling);
   } else if (d == 64) {
@@ -1334,6 +1339,22 @@ int tvmkv_batch_prefill_paged_kv_scaled(const void* q, const int32_t* q_indptr, 
                        nnz_pages, num_pages, h_q, h_kv, d, page_size, sliding_window, sliding_window_size,
                        merge_into != 0, stream, rope_scaling);
 }
+
+}  // extern "C"
+
+int tvmkv::prefill_paged_with_lengths(const void* q, const int32_t* q_indptr, const void* pages, const int32_t* page_indptr,
+                                      const int32_t* page_values, const int32_t* length_info, const int32_t* k_rope_pos_offset,
+                                      const int32_t* q_rope_position, void* output, float* lse, int64_t causal, int64_t rotary_mode,
+                                      double rope_scale, double rope_theta, double sm_scale, int32_t batch_size, int64_t total_q,
+                                      int64_t nnz_pages, int64_t num_pages, int32_t h_q, int32_t h_kv, int32_t d, int32_t page_size,
+                                      int32_t sliding_window, int32_t sliding_window_size, int32_t merge_into,
+                                      const tvmkv_rope_scaling* rope_scaling, int64_t longest, void* stream) {
+  return paged_prefill(q, q_indptr, pages, page_indptr, page_values, length_info, k_rope_pos_offset, q_rope_position, output, lse,
+                       causal, rotary_mode, rope_scale, rope_theta, sm_scale, batch_size, total_q, nnz_pages, num_pages, h_q, h_kv, d,
+                       page_size, sliding_window, sliding_window_size, merge_into != 0, stream, rope_scaling, longest);
+}
+
+extern "C" {
 
 static int cached_and_new(const void* q, int64_t q_token_stride, const int32_t* q_rope_position, int64_t apply_rope,
                           double rope_scale, double rope_theta, const int32_t* q_indptr, const void* k, const void* v,

@@ -722,6 +722,15 @@ class PagedKVCache {
     new_token_step_ = false;
     const StepLayout& s = book_->step();
     const int64_t batch = book_->batch_size();
+    for (int set = 0; set < 2; ++set) {
+      for (int d = 0; d < s.num_depths; ++d) {
+        const AuxSpan& span = set ? s.page_indptr_sw[d] : s.page_indptr[d];
+        longest_pages_[set][d] = 0;
+        if (s.use_decode_kernel[d] || !span.present()) continue;
+        const int32_t* indptr = book_->step_buffer() + span.offset;
+        for (int64_t e = 0; e + 1 < span.size; ++e) longest_pages_[set][d] = std::max(longest_pages_[set][d], indptr[e + 1] - indptr[e]);
+      }
+    }
     if (batch > reserved_num_seqs_) return;  // the plans are sized for that many
     const bool one_level = qk_head_dim_ == v_head_dim_ && s.num_depths == 1 && s.is_chain[0] && !s.append_before_attn &&
                            s.qo_indptr[0].size == batch + 1;
@@ -1204,6 +1213,7 @@ class PagedKVCache {
       const int32_t* q_pos = Dev(s.q_rope_position_map);
       const int64_t entries = s.qo_indptr[d].size - 1;
       const int64_t nnz_pages = page_indices_span.size;
+      const int64_t longest = longest_pages_[sliding_layer ? 1 : 0][d] * page_size_;
       if (generic_) {
         GenericAttention a;
         a.what = "cross attention";
@@ -1258,21 +1268,21 @@ class PagedKVCache {
       } else if (!is_first_kernel) {
         // The prefill kernel merges its state into (o, lse) in its epilogue: one launch for the
         // kernel and the merge of :2285-2292, and no temporary output.
-        Launch(tvmkv_batch_prefill_paged_kv_scaled(q, qo_indptr, pages_[local_layer_id], page_indptr, page_indices,
+        Launch(prefill_paged_with_lengths(q, qo_indptr, pages_[local_layer_id], page_indptr, page_indices,
                                                    length_info, k_rope_pos, q_pos, o, lse, causal, rotary_mode, rotary_scale,
                                                    rotary_theta, sm_scale, entries, total_seq_length, nnz_pages,
                                                    num_total_pages_, num_qo_heads_, num_kv_heads_, qk_head_dim_, page_size_,
                                                    sliding_window, layer_sliding_window_size_, /*merge_into=*/1,
-                                                   InlineScaling(), compute_stream_));
+                                                   InlineScaling(), longest, compute_stream_));
         cross_attn_computed = true;
         continue;
       } else {
-        Launch(tvmkv_batch_prefill_paged_kv_scaled(q, qo_indptr, pages_[local_layer_id], page_indptr, page_indices,
+        Launch(prefill_paged_with_lengths(q, qo_indptr, pages_[local_layer_id], page_indptr, page_indices,
                                                    length_info, k_rope_pos, q_pos, attn_output, attn_lse, causal, rotary_mode,
                                                    rotary_scale, rotary_theta, sm_scale, entries, total_seq_length, nnz_pages,
                                                    num_total_pages_, num_qo_heads_, num_kv_heads_, qk_head_dim_, page_size_,
                                                    sliding_window, layer_sliding_window_size_, /*merge_into=*/0,
-                                                   InlineScaling(), compute_stream_));
+                                                   InlineScaling(), longest, compute_stream_));
       }
       if (!is_first_kernel) {
         Launch(typed_merge_state_inplace(elem_bits_, o, lse, temp_out_, temp_lse_, total_seq_length, num_qo_heads_,
@@ -1385,6 +1395,7 @@ class PagedKVCache {
     int64_t rows = 0, page_indptr[2] = {0, 0}, page_begin[2] = {0, 0}, length_info[2] = {0, 0}, nnz_pages[2] = {0, 0};
   };
   MixedStep mixed_;
+  int32_t longest_pages_[2][kMaxBlockDepth] = {};  // of the entries of each depth ([1]: in the layers with a window)
   bool new_token_step_ = false;  // the step runs as WindowedDecodeStep
   // GatheredPrefill: K and V rows of a step, at most kGatherBytes (steps with more keys take the kernels that rotate
   // inside), and how many rows this step has (0: the step does not run that way)

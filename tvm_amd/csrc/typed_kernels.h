@@ -180,6 +180,15 @@ struct PromptPrefill {
 };
 int prefill_prompts(const PromptPrefill& args, void* stream);
 
+// tvmkv_batch_prefill_paged_kv_scaled for a caller that knows the keys of its longest sequence (0: not known)
+int prefill_paged_with_lengths(const void* q, const int32_t* q_indptr, const void* pages, const int32_t* page_indptr,
+                               const int32_t* page_values, const int32_t* length_info, const int32_t* k_rope_pos_offset,
+                               const int32_t* q_rope_position, void* output, float* lse, int64_t causal, int64_t rotary_mode,
+                               double rope_scale, double rope_theta, double sm_scale, int32_t batch_size, int64_t total_q,
+                               int64_t nnz_pages, int64_t num_pages, int32_t h_q, int32_t h_kv, int32_t d, int32_t page_size,
+                               int32_t sliding_window, int32_t sliding_window_size, int32_t merge_into,
+                               const tvmkv_rope_scaling* rope_scaling, int64_t longest, void* stream);
+
 // tvmkv_kv_cache_transpose_append with the k / v rows of consecutive tokens token_stride elements apart (the fused
 // qkv tensor of the step)
 int append_strided(void* pages, const void* k_data, const void* v_data, int64_t token_stride, const int32_t* position_map,
