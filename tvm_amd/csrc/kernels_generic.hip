@@ -200,8 +200,8 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
   const int qo_len = q_begin(b + 1) - q_start;
   const int rows = qo_len * group;
   const int r0 = (slot - slot_begin(b)) * ROWS;
-  if (r0 >= rows || (p.skip_single && qo_len == 1)) return;  // the whole workgroup: a slot beyond the sequence's last row tile
-  const int q_token = p.rows != nullptr ? p.rows[b] : q_start;  // the tile's place in q and out
+  if (r0 >= rows || (!EXT && p.skip_single && qo_len == 1)) return;  // the whole workgroup: a slot beyond the sequence's last row tile
+  const int q_token = !EXT && p.rows != nullptr ? p.rows[b] : q_start;  // the tile's place in q and out
   const bool rotary = EXT && p.rotary != 0;
   if (EXT && rotary) {
     if (tid < d) rope_lds[tid] = rope.v[tid];
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
   int kv_len, kv_start = 0, pbeg = 0;
   int sink = 0, window_first = 0;  // logical key t lies at physical index t (t < sink) or t - sink + window_first
   if (paged) {
-    pbeg = p.page_begin != nullptr ? p.page_begin[b] : p.page_indptr[b];
+    pbeg = !EXT && p.page_begin != nullptr ? p.page_begin[b] : p.page_indptr[b];
     const int npages = p.page_indptr[b + 1] - p.page_indptr[b];
     kv_len = npages > 0 ? (npages - 1) * p.page_size + p.last_page_len[b] : 0;  // _kernel_common.py:155-159
     if (EXT && p.window_offset != nullptr && npages > 0) {
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
       T* dst = static_cast<T*>(p.out) + out_row * d;
       float mine = 1.f, theirs = 0.f;  // weights of this state and of the one that is there
       float lse = any ? s_row : kNegInit;
-      if (p.merge_into) {  // the arithmetic of merge_state_inplace
+      if (!EXT && p.merge_into) {  // the arithmetic of merge_state_inplace
         const float other = p.lse[out_row];
         const float top = fmaxf(lse, other);
         mine = fast_exp2(lse - top);
@@ -531,7 +531,7 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
 #pragma unroll
           for (int e = 0; e < VP; ++e) run[e] = o[nb][c * VP + e][r] * inv;
           if (f < d) {
-            if (p.merge_into) {
+            if (!EXT && p.merge_into) {
 #pragma unroll
               for (int e = 0; e < VP; ++e) run[e] += theirs * static_cast<float>(dst[f + e]);
             }
@@ -542,7 +542,7 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
       // a row without keys: out = 0 and the state the reference's kernels start from, m = -5e4, d = 1
       if (g == 0) p.lse[out_row] = lse;
     } else {
-      const int64_t part_row = static_cast<int64_t>(q_start + row / group) * p.h_q + kvh * group + row % group;
+      const int64_t part_row = EXT ? out_row : static_cast<int64_t>(q_start + row / group) * p.h_q + kvh * group + row % group;
       float* dst = p.part_o + (static_cast<int64_t>(split) * p.total_q * p.h_q + part_row) * d;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -693,6 +693,8 @@ int generic_attention(const GenericAttention& a, void* stream_) {
     rope.magnitude = table.magnitude;
   }
   const bool ext = sliding || rotary;
+  KV_CHECK(!ext || (a.rows == nullptr && a.page_begin == nullptr && a.skip_single == 0 && a.merge_into == 0))
+      << a.what << ": the extended form computes every sequence of the call";
   const int group = a.h_q / a.h_kv;
   const int64_t work_q = a.work_seqs > 0 ? a.work_q : a.total_q, work_seqs = a.work_seqs > 0 ? a.work_seqs : a.batch;
   const int rows_hint = static_cast<int>(std::min<int64_t>(work_q * group / work_seqs, 1 << 20));

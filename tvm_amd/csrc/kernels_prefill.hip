@@ -79,6 +79,8 @@ constexpr size_t prefill_lds_bytes(int dqk, int dv) {
 template <int DQK, int DV, int SRC, int PS, bool EXT, bool STREAM = false, bool PAD = false, bool VARIANT = false>
 __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 64 ? 3 : 2)) void prefill_kernel(PrefillParams p, PrefillRopeDivisors div) {
   constexpr bool PAGED = SRC == kPaged, BOTH = SRC == kBoth;
+  // the kernels that prefill_prompts launches; in the others the test alone cost head dim 256 0.6 %
+  constexpr bool SKIPS = DQK == DV && DQK <= 128 && !PAD && !VARIANT && (BOTH || PAGED == EXT);
   static_assert(!PAD || (!EXT && !BOTH && DQK == DV), "padded head dims: plain ragged and paged kernels");
   const int dqm = PAD ? p.d_mem : DQK;  // elements per q / k row in memory
   const int dvm = PAD ? p.d_mem : DV;   // elements per v / output row in memory
@@ -139,7 +141,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 
         lk0 = p.kv_indptr[lane];
         lk1 = p.kv_indptr[lane + 1];
       }
-      my_tiles = (p.skip_single && lq1 - lq0 == 1) ? 0 : ((lq1 - lq0) * group + BM - 1) / BM;
+      my_tiles = (SKIPS && p.skip_single && lq1 - lq0 == 1) ? 0 : ((lq1 - lq0) * group + BM - 1) / BM;
       my_key = (lp1 - lp0) * (PS << p.page_shift) + (lk1 - lk0);
     }
     // Row tiles of the sequences ranked before this lane's.  (key, index) is one sortable 32-bit
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 
   const int qo_len = seq_q1 - q_start;
   const int rows = qo_len * group;
   const int n_row_tiles = (rows + BM - 1) / BM;
-  if (local_slot >= n_row_tiles || (p.skip_single && qo_len == 1)) return;
+  if (local_slot >= n_row_tiles || (SKIPS && p.skip_single && qo_len == 1)) return;
   const int r0 = (n_row_tiles - 1 - local_slot) * BM;
 
   // phys_len: tokens the K/V storage of the sequence covers; kv_len: keys attended to (logical)
@@ -230,8 +232,8 @@ __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 
   // number of logical keys -> physical end of the tokens that hold them
   auto to_phys = [&](int n) { return (!EXT || n <= sink) ? n : n - sink + win_lo; };
   __shared__ float div_lds[DQK > 256 ? 256 : DQK];
-  // uniform over the launch
-  const bool q_rope = (EXT && p.rotary) || (!EXT && !PAGED && !PAD && DQK == DV && p.q_inline_rope != 0);
+  // uniform over the launch (the ragged kernel of head dim 256 spills with a rotation of its own, 60 -> 96 bytes a lane)
+  const bool q_rope = (EXT && p.rotary) || (!EXT && !PAGED && !PAD && DQK == DV && (BOTH || DQK < 256) && p.q_inline_rope != 0);
   if (q_rope) {
     if (tid < DQK && tid < 256) div_lds[tid] = div.v[tid];
     __syncthreads();
@@ -999,7 +1001,7 @@ int tvmkv::prefill_over_gathered_kv(const void* q, int64_t q_token_stride, const
   KV_API_BEGIN();
   KV_CHECK(batch_size > 0 && total_q > 0 && h_q > 0 && h_kv > 0 && h_q % h_kv == 0) << "prefill_over_gathered_kv: bad shape";
   KV_CHECK(q && q_indptr && k && v && kv_indptr && output && lse) << "prefill_over_gathered_kv: NULL tensor";
-  KV_CHECK(!apply_rope || (q_rope_position && !padded_head_dim(d))) << "prefill_over_gathered_kv: rotation of the queries";
+  KV_CHECK(!apply_rope || (q_rope_position && (d == 64 || d == 128))) << "prefill_over_gathered_kv: rotation of the queries";
   PrefillParams p{};
   p.q = static_cast<const half_t*>(q);
   p.q_token_stride = q_token_stride;
@@ -1068,13 +1070,11 @@ int tvmkv::prefill_prompts(const PromptPrefill& a, void* stream) {
   p.scale_log2 = static_cast<float>(a.sm_scale) * kLog2e;
   hipStream_t s = as_stream(stream);
   auto by_dim = [&](auto run) {
+    KV_UNSUPPORTED(a.d != 64 && a.d != 128) << "prefill_prompts: head_dim " << a.d << " is not built (64, 128)";
     if (a.d == 128) {
       run(std::integral_constant<int, 128>{});
-    } else if (a.d == 64) {
-      run(std::integral_constant<int, 64>{});
     } else {
-      KV_UNSUPPORTED(a.d != 256) << "prefill_prompts: head_dim " << a.d << " is not built (64, 128, 256)";
-      run(std::integral_constant<int, 256>{});
+      run(std::integral_constant<int, 64>{});
     }
     KV_LAUNCH_CHECK();
   };

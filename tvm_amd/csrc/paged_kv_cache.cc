@@ -261,7 +261,7 @@ class PagedKVCache {
                                      pages_[local_layer_id], Dev(s.append_position_map), total_seq_length,
                                      num_qo_heads_, num_kv_heads_, qk_head_dim_, num_total_pages_, page_size_,
                                      rotary_scale_, rotary_theta_, compute_stream_));
-      if (RunsMixed()) {
+      if (RunsMixed(layer_id)) {
         MixedAttention(layer_id, qkv, (num_qo_heads_ + 2 * num_kv_heads_) * qk_head_dim_, rope_normal, temp_k_, temp_v_, out,
                        total_seq_length, sm_scale);
         RecordComputeEvent();
@@ -851,8 +851,12 @@ class PagedKVCache {
     mixed_ = plan;
   }
 
-  // A step that is being captured keeps the launches that need no scratch memory of the decode kernel's.
-  bool RunsMixed() const { return mixed_.decoding > 0 && !stream_is_capturing(static_cast<hipStream_t>(compute_stream_)); }
+  // A step that is being captured keeps the launches that need no scratch memory of the decode kernel's; the generic
+  // kernel's extended form, which the layers with a window take, has no index of sequences (it spills with one).
+  bool RunsMixed(int64_t layer_id) const {
+    return mixed_.decoding > 0 && !(generic_ && attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING) &&
+           !stream_is_capturing(static_cast<hipStream_t>(compute_stream_));
+  }
 
   void MixedAttention(int64_t layer_id, const void* q, int64_t q_stride, bool rotate_q, const void* k, const void* v, void* out,
                       int64_t total_seq_length, double sm_scale) {
@@ -928,14 +932,13 @@ class PagedKVCache {
                              double sm_scale) {
     const StepLayout& s = book_->step();
     const int64_t local_layer_id = layer_id - layer_id_begin_offset_;
-    const bool window = attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING;
     GenericRagged(q, k, v, out, merged_lse_, total_seq_length, sm_scale, /*tree=*/false);
     GenericAttention a;
     a.what = "cross attention";
     a.elem_bits = elem_bits_;
     a.q = q;
     a.pages = pages_[local_layer_id];
-    a.page_values = Dev(window ? s.page_indices_sw[0] : s.page_indices[0]);
+    a.page_values = Dev(s.page_indices[0]);
     a.num_pages = num_total_pages_;
     a.out = out;
     a.lse = merged_lse_;
@@ -945,16 +948,13 @@ class PagedKVCache {
     a.d = static_cast<int32_t>(qk_head_dim_);
     a.page_size = static_cast<int32_t>(page_size_);
     a.sm_scale = sm_scale;
-    a.sliding_window = window;
     if (mixed_.prompt_cached > 0) {
       GenericAttention prompts = a;
       prompts.q_indptr = Dev(s.qo_indptr[0]);
-      prompts.page_indptr = Dev(window ? s.page_indptr_sw[0] : s.page_indptr[0]);
-      prompts.last_page_len = Dev(window ? s.layer_sw_length_info[0] : s.length_info[0]);
+      prompts.page_indptr = Dev(s.page_indptr[0]);
+      prompts.last_page_len = Dev(s.length_info[0]);
       prompts.total_q = total_seq_length;
       prompts.batch = static_cast<int32_t>(book_->batch_size());
-      prompts.causal = window;
-      prompts.layer_window = static_cast<int32_t>(layer_sliding_window_size_);
       prompts.skip_single = 1;
       prompts.work_q = mixed_.prompt_tokens;
       prompts.work_seqs = mixed_.prompts;
@@ -962,11 +962,11 @@ class PagedKVCache {
       Launch(generic_attention(prompts, compute_stream_));
     }
     a.rows = DevExtra(mixed_.rows);
-    a.page_indptr = DevExtra(mixed_.page_indptr[window]);
-    a.page_begin = DevExtra(mixed_.page_begin[window]);
-    a.last_page_len = DevExtra(mixed_.length_info[window]);
+    a.page_indptr = DevExtra(mixed_.page_indptr[0]);
+    a.page_begin = DevExtra(mixed_.page_begin[0]);
+    a.last_page_len = DevExtra(mixed_.length_info[0]);
     a.total_q = a.batch = mixed_.decoding;
-    a.nnz_pages = mixed_.nnz_pages[window];
+    a.nnz_pages = mixed_.nnz_pages[0];
     Launch(generic_attention(a, compute_stream_));
   }
 
@@ -1046,7 +1046,7 @@ class PagedKVCache {
       g.k_new = rows + num_qo_heads_ * d;
       g.v_new = rows + (num_qo_heads_ + num_kv_heads_) * d;
       g.kv_stride = fused_stride;
-      if (inline_rope && (g.rope_scaling != nullptr || !(d == 64 || d == 128 || d == 256))) {
+      if (inline_rope && (g.rope_scaling != nullptr || !(d == 64 || d == 128))) {
         g.q_new = qkv;
         g.q_stride = fused_stride;
         g.q_out = temp_q_;
@@ -1080,7 +1080,7 @@ class PagedKVCache {
                          int64_t total_seq_length, double sm_scale) {
     const int64_t local_layer_id = layer_id - layer_id_begin_offset_;
     const StepLayout& s = book_->step();
-    if (RunsMixed()) {
+    if (RunsMixed(layer_id)) {
       MixedAttention(layer_id, q, num_qo_heads_ * qk_head_dim_, /*rotate_q=*/false, k, v, output, total_seq_length, sm_scale);
       return;
     }

@@ -68,6 +68,7 @@ struct GenericAttention {
   const int32_t* k_rope_pos_offset = nullptr;
   double rope_scale = 1.0, rope_theta = 1e4;
   const tvmkv_rope_scaling* rope_scaling = nullptr;
+  // Not in the extended form:
   // rows, page_begin (paged, q_indptr NULL): sequence b's query is token rows[b] of q, q_rope_position, out and lse (NULL:
   // b), its pages start at page_values[page_begin[b]] (NULL: page_indptr[b]).  skip_single: sequences with one query
   // token are passed over; work_q / work_seqs / nnz_pages then describe the others.  merge_into: out / lse hold an
@@ -154,7 +155,7 @@ struct NewTokenDecode {
 };
 int decode_with_new_token(const NewTokenDecode& args, void* stream);
 
-// Prefill attention (fp16, head dims 64 / 128 / 256, tuned page sizes) of a step's sequences with more than one new token:
+// Prefill attention (fp16, head dims 64 / 128, tuned page sizes) of a step's sequences with more than one new token:
 // cached keys, then the new ones under the causal mask.  Sequences with one new token are passed over; their rows of
 // out / lse hold nothing of use afterwards.  layer_window 0: one pass over both key sets, the queries read from q with
 // q_stride and rotated if apply_rope; else the per-layer window mask over the length_info (3, batch) of such a layer.
