@@ -250,23 +250,33 @@ def test_mixed_steps_on_the_generic_kernels(dtype, page_size, d, hq, hkv, window
     m.step([(0, 1), (2, 1), (4, 1)])
 
 
-@pytest.mark.parametrize("d,lengths", [(128, (1500, 90)), (64, (1500, 90)), (128, (1200, 1100))])
-def test_tree_steps_over_sequences_of_unlike_lengths(d, lengths):
-    """A verify step whose row tiles are full and whose longest sequence is well above the mean walks its keys in two
-    shares (64 kv heads here: one round of workgroups); the tree's own state is merged with both."""
-    hq, hkv, nodes = 64, 64, 70
-    m = Mirror([8, 4096, 1600, 16, 0], 1, hq, hkv, d)
-    m.step([(0, lengths[0])])
-    m.step([(1, lengths[1])])
+@pytest.mark.parametrize("d,page_size", [(128, 16), (64, 16), (64, 64)])
+def test_tree_steps_over_sequences_of_unlike_lengths(d, page_size):
+    """A verify step of one round of full row tiles whose longest sequence is well above the mean walks its keys in two
+    shares; the same step unsplit differs by the fp16 rounding of the shares' states (2^-11 of values below 1, twice)."""
+    heads, nodes, batch = 32, 66, 9
+    rng = np.random.default_rng(12)
+    cache = GpuCache([batch, 16384, 2600, page_size, 0], 1, heads, heads, d, d)
+    qkv = rng.standard_normal((2600, 3 * heads, d)).astype(np.float16)
+    for b in range(batch):
+        cache.add_sequence(b)
+        n = 2600 if b == 4 else 900
+        cache.begin_forward([b], [n])
+        cache.attention_with_fused_qkv(0, d ** -0.5, qkv[:n], np.zeros((n, heads, d), np.float16))
+        cache.end_forward()
     parents = [(i - 1) // 2 if i else -1 for i in range(nodes)]
-    m.o.begin_forward([0, 1], [nodes, nodes], parents * 2)
-    m.g.begin_forward([0, 1], [nodes, nodes], parents * 2)
-    qkv = m.rng.standard_normal((2 * nodes, hq + 2 * hkv, d)).astype(np.float16)
-    eo = np.zeros((2 * nodes, hq, d), np.float16)
-    go = np.zeros_like(eo)
-    m.o.attention_with_fused_qkv(0, d ** -0.5, qkv, eo)
-    m.g.attention_with_fused_qkv(0, d ** -0.5, qkv, go)
-    assert_close(go, eo, what="tree step over unlike lengths")
+    cache.begin_forward(list(range(batch)), [nodes] * batch, parents * batch)
+    outs = []
+    for splits in (0, 1):
+        prev = tvm_amd.set_option("prefill_kv_splits", splits)
+        try:
+            out = np.zeros((batch * nodes, heads, d), np.float16)
+            cache.attention_with_fused_qkv(0, d ** -0.5, qkv[:batch * nodes], out)
+            outs.append(out)
+        finally:
+            tvm_amd.set_option("prefill_kv_splits", prev)
+    assert not np.array_equal(outs[0], outs[1]), "the step did not split"
+    assert_close(outs[0], outs[1], atol=1e-3, rtol=1e-3, what="two shares")
 
 
 def test_decode_steps_of_windowed_caches_at_the_edges():
