@@ -65,6 +65,15 @@ def test_version_and_error_channel():
     rc = lib.tvmkv_batch_decode_paged_kv(None, None, None, None, None, None, None, None, None, 0, 1.0, 1e4, 1.0,
                                          1, 1, 1, 8, 2, 128, 16, 0, None)
     assert rc == -1 and b"NULL tensor" in lib.tvmkv_last_error()
+    # every rotary_mode but 0 rotates the cached keys: without their positions the call is refused, also for mode 2 (the
+    # cache's ROPE_INLINE); the addresses are never read
+    some = 4096
+    for mode in (1, 2, 3):
+        for k_offset, q_position in ((None, some), (some, None)):
+            args = (some, some, some, some, some, k_offset, q_position, some, some, mode, 1.0, 1e4, 1.0, 1, 1, 1, 8, 2, 128, 16, 0)
+            for entry in (lambda: lib.tvmkv_batch_decode_paged_kv(*args, None), lambda: lib.tvmkv_batch_decode_paged_kv_noalloc(*args, None),
+                          lambda: lib.tvmkv_batch_decode_paged_kv_scaled(*args, None, None)):
+                assert entry() == -1 and b"position arrays" in lib.tvmkv_last_error()
     rc = lib.tvmkv_merge_state_inplace(None, None, None, None, 1, 1, 100, None)
     assert rc == -2 and b"head dim 100" in lib.tvmkv_last_error()
     rc = lib.tvmkv_fused_rope(None, None, None, None, None, 1, 0, 8, 2, 128, 1.0, 1e4, None)

@@ -962,6 +962,9 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
   KV_CHECK((q || fused_launch) && pages && page_indptr && length_info && output && lse) << "batch_decode_paged_kv: NULL tensor";
   KV_CHECK(!fused_launch || (!ext && fused_step.append_position_map && q_rope_position))
       << "fused decode step: plain cache only, and it needs the append slots and the positions";
+  // rotary_mode 2 leaves the keys alone in the new-token form only; the other entry points rotate them for any mode but 0
+  KV_CHECK(rotary_mode == 0 || (q_rope_position && (k_rope_pos_offset || (self && rotary_mode == 2))))
+      << "batch_decode_paged_kv: inline RoPE needs the position arrays";
   KV_CHECK(nnz_pages == 0 || page_values) << "batch_decode_paged_kv: NULL page table";
   hipStream_t s = as_stream(stream);
 
@@ -1035,8 +1038,6 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
   if (fused) p.arrivals = reinterpret_cast<unsigned long long*>(ws.ptr);
   DecodeRopeRunning div{};
   if (p.rotary || (fused_launch && p.apply_rope)) {
-    KV_CHECK(k_rope_pos_offset || fused_launch || rotary_mode == 2) << "batch_decode_paged_kv: inline RoPE needs the position arrays";
-    KV_CHECK(q_rope_position) << "batch_decode_paged_kv: inline RoPE needs the position arrays";
     const InlineRopeHost table = inline_rope_table(fused_launch ? nullptr : fused_step.rope_scaling, d, rope_theta);
     for (int i = 0; i < d; ++i) div.v[i] = table.v[i];
     p.rope_inverse = table.inverse;
