@@ -585,6 +585,49 @@ def test_paged_kernels_with_other_page_sizes(page_size, hq, hkv, d):
     assert_close(host(gl), el, atol=2e-3, rtol=1e-4, what=f"one-pass chunked prefill lse, page size {ps}")
 
 
+@pytest.mark.parametrize("page_size", [16, 24, 128])
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 128), (8, 8, 64), (4, 2, 256), (8, 4, 96)])
+def test_slots_between_sinks_and_window_are_never_read(page_size, hq, hkv, d):
+    """A chunk longer than its window leaves slots between the attention sinks and the window that nothing has written:
+    with NaN in them the windowed forms of prefill and decode (gaps inside a run of keys, across runs and tiles, whole
+    runs of a large page) return what the oracle does over a pool without them."""
+    from tests.test_oracle_kernels import sliding_case
+    rng = np.random.default_rng(77)
+    spec = [(100, 4, 20), (257, 0, 7), (330, 16, 48), (33, 2, 3), (200, 30, 127), (2300, 8, 100), (40, 0, 31)]
+    lens = [7, 64, 33, 2, 1, 40, 3]
+    pages, pindptr, pvalues, info, k_log, _ = sliding_case(rng, spec, hkv, d, ps=page_size,
+                                                           npages=8 + sum(x[0] // page_size + 1 for x in spec))
+
+    poisoned = pages.copy()
+    for i, (_, sink, off) in enumerate(spec):
+        for t in range(sink, off):
+            poisoned[pvalues[pindptr[i] + t // page_size], :, :, t % page_size] = np.nan
+
+    b, n = len(spec), sum(lens)
+    qindptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    q = rng.standard_normal((n, hq, d)).astype(F16)
+    k_off = rng.integers(0, 200, size=b).astype(np.int32)
+    q_pos = np.concatenate([k_off[i] + len(k_log[i]) - lens[i] + np.arange(lens[i]) for i in range(b)]).astype(np.int32)
+    for causal, window, rotary in ((0, 0, 1), (0, 0, 0), (1, 40, 0), (1, 0, 1)):
+        eo, el = np.zeros((n, hq, d), F16), np.zeros((n, hq), np.float32)
+        ok.prefill_paged(q, qindptr, pages, pindptr, pvalues, info, k_off, q_pos, eo, el, causal, rotary, 1.0, 1e4,
+                         d ** -0.5, sliding_window_size=window)
+        go, gl = torch.full((n, hq, d), 7.0, dtype=torch.float16, device=DEV), torch.full((n, hq), 7.0, device=DEV)
+        K.batch_prefill_paged_kv(dev(q), i32(qindptr), dev(poisoned), i32(pindptr), i32(pvalues), i32(info), i32(k_off),
+                                 i32(q_pos), go, gl, causal, rotary, 1.0, 1e4, d ** -0.5, sliding_window_size=window)
+        assert_close_where_keys(host(go), host(gl), eo, el, rows_without_keys(lens, causal, window), 2e-3,
+                                f"prefill, causal {causal}, window {window}, rotary {rotary}")
+    last = [qindptr[i + 1] - 1 for i in range(b)]
+    for rotary in (0, 1):
+        eo, el = np.zeros((b, hq, d), F16), np.zeros((b, hq), np.float32)
+        ok.decode(q[last], pages, pindptr, pvalues, info, k_off, q_pos[last], eo, el, rotary, 1.0, 1e4, d ** -0.5)
+        go, gl = torch.full((b, hq, d), 7.0, dtype=torch.float16, device=DEV), torch.full((b, hq), 7.0, device=DEV)
+        K.batch_decode_paged_kv(dev(q[last]), dev(poisoned), i32(pindptr), i32(pvalues), i32(info), i32(k_off),
+                                i32(q_pos[last]), go, gl, rotary, 1.0, 1e4, d ** -0.5)
+        assert_close(host(go), eo, what=f"decode, rotary {rotary}")
+        assert_close(host(gl), el, atol=2e-3, rtol=1e-4, what=f"decode lse, rotary {rotary}")
+
+
 @pytest.mark.parametrize("hq,hkv,d,splits", [(16, 4, 128, 0), (16, 4, 128, 3), (8, 2, 64, 5), (8, 2, 64, 64), (8, 2, 256, 2)])
 def test_prefill_split_over_the_keys(hq, hkv, d, splits):
     """Launches with few row tiles split every row tile's keys over several workgroups and merge the

@@ -556,6 +556,18 @@ __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 
     } else {
       wait_vmcnt<0>();
     }
+    if (EXT && PAGED && kv0 < win_lo && kv0 + BN > sink) {  // wave-uniform
+      // Slots between the sinks and the window may never have been written (a chunk longer than its window).  Their
+      // probabilities are 0; the wave that copied their V rows makes them 0 as well (0 times an unwritten page's NaN
+      // would reach the output).
+#pragma unroll 1
+      for (int row = wave_u * RPW; row < wave_u * RPW + RPW; ++row) {
+        if (kv0 + row < sink || kv0 + row >= win_lo) continue;
+        uint32_t* dst = reinterpret_cast<uint32_t*>(lds_tiles + (tile % NSTAGE) * STAGE + BN * DQK + row * VW) + lane % (VW / 2);
+#pragma unroll
+        for (int blk = 0; blk < VBLK; ++blk) dst[blk * (BN * VW / 2)] = 0;
+      }
+    }
     __syncthreads();
     // no prefetch across a 64-tile window of page ids: the ids held are those of the last copy issued
     const int next = tile + NSTAGE - 1;  // the tile whose copy this iteration issues
