@@ -762,6 +762,17 @@ __global__ __launch_bounds__(NW * 64, (NW == 8 || DQK + DV > 320) ? 1 : (DQK == 
         }
       }
       if (half == 0) *lse_ptr = fast_log2(w_prev + w_mine) + s_max;
+    } else if (SRC != kRagged && DQK == DV && !PAD && p.split_f32) {
+      float* share = reinterpret_cast<float*>(p.output) + out_row * DV + half * 4;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+#pragma unroll
+        for (int j4 = 0; j4 < 4; ++j4) {
+          *reinterpret_cast<float4*>(share + db * 32 + j4 * 8) =
+              make_float4(o[db][j4 * 4] * inv, o[db][j4 * 4 + 1] * inv, o[db][j4 * 4 + 2] * inv, o[db][j4 * 4 + 3] * inv);
+        }
+      }
+      if (half == 0) *lse_ptr = my_lse;
     } else {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
@@ -808,12 +819,13 @@ static void launch_prefill_ext(const PrefillParams& p, int64_t total_q, const Pr
 // A launch with few row tiles and long key ranges (a token tree or a short chunk against long cached
 // sequences) neither fills the chip nor balances it: a row tile is one workgroup that walks all its
 // keys.  Such a launch is split: kv_splits workgroups share a row tile, each writes the attention state
-// of its share of the key tiles (normalised output in fp16, lse) to scratch memory, and a second kernel
+// of its share of the key tiles (normalised output, lse) to scratch memory, and a second kernel
 // merges the states of a row with the arithmetic of merge_state_inplace
 // (python/tvm/relax/frontend/nn/llm/_decode_kernels.py:441-450) over kv_splits states at once.  A row
 // whose states are all empty (lse = -5e4) stays the empty state: out 0, lse -5e4.
-template <int DV>
-__global__ __launch_bounds__(256) void prefill_split_merge_kernel(const half_t* __restrict__ part_o,
+// T: the type of the shares' outputs, half_t or float (KvSplit).
+template <typename T, int DV>
+__global__ __launch_bounds__(256) void prefill_split_merge_kernel(const T* __restrict__ part_o,
                                                                   const float* __restrict__ part_lse, half_t* __restrict__ output,
                                                                   float* __restrict__ lse, int64_t rows, int splits,
                                                                   int merge_into) {
@@ -845,10 +857,11 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(const half_t* 
 #pragma unroll 8
     for (int i = 0; i < splits; ++i) {
       const float w = fast_exp2(part_lse[i * rows + row] - s_max);
-      const Vec16 v = ld16(part_o + (i * rows + row) * DV + piece * 8);
+      typedef T share_t __attribute__((ext_vector_type(8)));
+      const share_t v = *reinterpret_cast<const share_t*>(part_o + (i * rows + row) * DV + piece * 8);
       w_sum += w;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] += w * static_cast<float>(v.h8[e]);
+      for (int e = 0; e < 8; ++e) acc[e] += w * static_cast<float>(v[e]);
     }
   }
   const float inv = w_sum > 0.f ? 1.0f / w_sum : 0.f;
@@ -859,40 +872,17 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(const half_t* 
   if (piece == 0) lse[row] = w_sum > 0.f ? s_max + fast_log2(w_sum) : kNegInit;
 }
 
-// How many ways to split the keys of a launch of total_q query tokens in `batch` sequences whose
-// sequences hold avg_keys keys on average (shapes only: no read of the index arrays).  The launch has at
-// least max(total_q * group / BM, batch) row tiles, times h_kv workgroups, and the chip holds two
-// workgroups per compute unit.
-//  * Less than half a round of workgroups: as many shares as fill two rounds.
-//  * Up to one round, of row tiles that are at most half full (a draft chain or a small tree per
-//    sequence): the K/V stream decides and two shares balance it (64 sequences of 1024-8192 keys with a
-//    4-token chain each: 0.241 ms unsplit, 0.217 with 2 shares, 0.226 with 4, 0.239 with 8).
-//  * Otherwise none: workgroups that end early leave their compute unit to the one that shares it, and
-//    shares only add start-up, epilogue and merge traffic (16 sequences with 128-token chunks on
-//    2000-6000 keys, 512 workgroups: 0.171 ms unsplit, 0.183 with 2 shares; a 63-node tree per sequence,
-//    1008 workgroups, matrix-bound: 0.409 against 0.442).
-// No share shorter than 8 tiles on average, at most 64 shares.
-// longest: the keys of the longest sequence where the caller knows them, else 0.  One round of full row tiles lasts as
-// long as its longest walk: two shares each when that is well above the mean (us a layer, 64 sequences with a 31-node
-// tree, 32 / 8 heads, unsplit -> two shares: U[1024,8192] cached tokens 311 -> 286 at head dim 128, 233 -> 186 at 64;
-// U[4000,5000], where the walks are alike, 267 -> 283).
-static int pick_kv_splits(int64_t total_q, int group, int batch, int h_kv, int64_t avg_keys, int64_t longest) {
-  const int64_t forced = option(kOptPrefillKvSplits);
-  if (forced > 0) return static_cast<int>(std::min<int64_t>(forced, 64));
-  const int64_t resident = static_cast<int64_t>(compute_units()) * 2;
-  const int64_t tiles = std::max<int64_t>((total_q * group + BM - 1) / BM, batch);
-  const int64_t workgroups = tiles * h_kv;
-  int64_t want = 1;
-  if (workgroups * 2 <= resident) {
-    want = (2 * resident + workgroups - 1) / workgroups;
-  } else if (workgroups <= resident && (total_q * group * 2 <= tiles * BM || longest * 10 >= avg_keys * 14)) {
-    want = 2;
-  }
-  const int64_t by_length = avg_keys / (8 * BN);
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(std::min(want, by_length), 64)));
-}
-
-// Redirects the launch described by p to scratch memory when it is to be split; finish() merges.
+// Redirects the launch described by p to scratch memory when it is to be split (prefill_kv_splits); finish() merges.
+// The shares' outputs are fp16 where the launch has always been split, and float32 where it would otherwise run whole:
+//  * float_shares: the prompts of a step whose decoding sequences run elsewhere (prefill_prompts);
+//  * longest, the keys of the longest sequence where the caller knows them, else 0: one round of full row tiles lasts as
+//    long as its longest walk, so two shares each where that is well above the mean.  How much it has to be above is what
+//    the shares' traffic costs, and how many workgroups share a compute unit (one that ends early leaves its unit to the
+//    others): 1.4 times the mean and 1024 keys more at head dim 64, 1.75 times and 2048 more at 128, and at 256, one
+//    workgroup per unit in two rounds, none.  Measured, time whole / time in two shares, 260-512 workgroups, lengths
+//    around means of 1500-8000 keys evenly spread or one long among equal ones, longest / mean 1.3 | 1.4 | 1.6 | 1.8 | 2.0:
+//      64    0.87-1.10 | 0.91-1.18 | 0.96-1.24 | 1.06-1.30 | 1.20-1.34       256 (1.1-1.9)    0.84-0.94
+//      128   0.82-1.06 | 0.81-1.10 | 0.84-1.16 | 0.85-1.23 | 1.00-1.34, from 2048 keys above the mean on 0.97-1.34 at 1.75-2.0
 struct KvSplit {
   half_t* output;
   float* lse;
@@ -901,16 +891,23 @@ struct KvSplit {
   int merge_into = 0;
   ScratchLease lease{};
   // work_q, work_seqs: the query tokens and sequences that the launch works on, where they are not all (skip_single)
-  KvSplit(PrefillParams& p, int64_t total_q, int64_t avg_keys, int dv, hipStream_t stream, int64_t work_q = 0, int64_t work_seqs = 0,
-          int64_t longest = 0)
+  KvSplit(PrefillParams& p, int64_t total_q, int64_t avg_keys, int dv, hipStream_t stream, int64_t longest = 0, int64_t work_q = 0,
+          int64_t work_seqs = 0, bool float_shares = false)
       : output(p.output), lse(p.lse), rows(total_q * p.h_q), splits(1) {
     if (work_seqs == 0) work_q = total_q, work_seqs = p.batch_size;
     // at most one row tile per (sequence, kv head) on average: the paged kernels stream the K/V rows
     p.stream_kv = work_q * p.group <= work_seqs * BM;
-    splits = pick_kv_splits(work_q, p.group, work_seqs, p.h_kv, avg_keys, longest);
+    splits = prefill_kv_splits(work_q, p.group, work_seqs, p.h_kv, avg_keys, compute_units());
+    const bool unlike = dv == 64 ? longest * 10 >= avg_keys * 14 && longest - avg_keys >= 1024
+                                 : dv == 128 && longest * 4 >= avg_keys * 7 && longest - avg_keys >= 2048;
+    if (splits == 1 && unlike && avg_keys >= 2 * kMinShareKeys && option(kOptPrefillKvSplits) == 0 &&
+        prefill_workgroups(work_q, p.group, work_seqs, p.h_kv) <= 2 * static_cast<int64_t>(compute_units())) {
+      splits = 2;
+      float_shares = true;
+    }
     if (dv % 64 != 0) splits = 1;  // padded head dims (80, 96, 112): the merge kernel is not built for their rows
     if (splits <= 1) return;
-    const size_t o_bytes = static_cast<size_t>(splits) * rows * dv * sizeof(half_t);
+    const size_t o_bytes = static_cast<size_t>(splits) * rows * dv * (float_shares ? sizeof(float) : sizeof(half_t));
     const size_t lse_bytes = static_cast<size_t>(splits) * rows * sizeof(float);
     lease = lease_scratch(kScratchPrefill, stream, o_bytes + lse_bytes, 0);  // held until the merge is enqueued
     char* ws = lease.ptr;
@@ -918,6 +915,7 @@ struct KvSplit {
     p.lse = reinterpret_cast<float*>(ws + o_bytes);
     p.kv_splits = splits;
     p.split_rows = rows;
+    p.split_f32 = float_shares;
     merge_into = p.merge_into;  // the shares write plain states; the merge kernel folds the caller's state in
     p.merge_into = 0;
   }
@@ -926,12 +924,23 @@ struct KvSplit {
     KV_LAUNCH_CHECK();
     const unsigned rows_per_block = 256 / (dv / 8);
     const dim3 grid(static_cast<unsigned>((rows + rows_per_block - 1) / rows_per_block));
+    auto merge = [&](auto kernel, const auto* shares) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, shares, p.lse, output, lse, rows, splits, merge_into);
+    };
+    auto merge_dim = [&](auto dim) {
+      constexpr int kD = decltype(dim)::value;
+      if (p.split_f32) {
+        merge(prefill_split_merge_kernel<float, kD>, reinterpret_cast<const float*>(p.output));
+      } else {
+        merge(prefill_split_merge_kernel<half_t, kD>, static_cast<const half_t*>(p.output));
+      }
+    };
     if (dv == 128) {
-      hipLaunchKernelGGL(prefill_split_merge_kernel<128>, grid, dim3(256), 0, stream, p.output, p.lse, output, lse, rows, splits, merge_into);
+      merge_dim(std::integral_constant<int, 128>{});
     } else if (dv == 64) {
-      hipLaunchKernelGGL(prefill_split_merge_kernel<64>, grid, dim3(256), 0, stream, p.output, p.lse, output, lse, rows, splits, merge_into);
+      merge_dim(std::integral_constant<int, 64>{});
     } else {
-      hipLaunchKernelGGL(prefill_split_merge_kernel<256>, grid, dim3(256), 0, stream, p.output, p.lse, output, lse, rows, splits, merge_into);
+      merge_dim(std::integral_constant<int, 256>{});
     }
   }
 };
@@ -1091,7 +1100,7 @@ int tvmkv::prefill_prompts(const PromptPrefill& a, void* stream) {
     KV_LAUNCH_CHECK();
   };
   if (a.layer_window == 0) {
-    const KvSplit split(p, a.total_q, (a.prompt_cached + a.prompt_tokens) / a.prompts, a.d, s, a.prompt_tokens, a.prompts);
+    const KvSplit split(p, a.total_q, (a.prompt_cached + a.prompt_tokens) / a.prompts, a.d, s, 0, a.prompt_tokens, a.prompts, true);
     by_dim([&](auto d) { launch_prefill<d.value, d.value, kBoth, 16>(p, a.total_q, false, a.rope_theta, s); });
     split.finish(p, a.d, s);
   } else {
@@ -1101,7 +1110,8 @@ int tvmkv::prefill_prompts(const PromptPrefill& a, void* stream) {
       p.sink_size = a.length_info + 2 * static_cast<int64_t>(a.batch);
       p.layer_window = a.layer_window;
       p.merge_into = 1;
-      const KvSplit split(p, a.total_q, std::min<int64_t>(a.prompt_cached / a.prompts, a.layer_window), a.d, s, a.prompt_tokens, a.prompts);
+      const KvSplit split(p, a.total_q, std::min<int64_t>(a.prompt_cached / a.prompts, a.layer_window), a.d, s, 0, a.prompt_tokens,
+                          a.prompts, true);
       by_dim([&](auto d) { launch_prefill<d.value, d.value, kPaged, 16>(p, a.total_q, true, a.rope_theta, s); });
       split.finish(p, a.d, s);
     }
@@ -1292,7 +1302,7 @@ static int paged_prefill(const void* q, const int32_t* q_indptr, const void* pag
   }
   const bool ext = p.rotary != 0 || sliding_window != 0;
   hipStream_t s = as_stream(stream);
-  const KvSplit split(p, total_q, nnz_pages * page_size / batch_size, d, s, 0, 0, longest);
+  const KvSplit split(p, total_q, nnz_pages * page_size / batch_size, d, s, longest);
   if (d == 128) {
     launch_prefill<128, 128, kPaged, 16>(p, total_q, ext, rope_theta, s, scaling);
   } else if (d == 64) {

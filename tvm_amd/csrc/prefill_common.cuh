@@ -54,6 +54,7 @@ struct PrefillParams {
   // its own attention state: output / lse then point at kv_splits arrays of split_rows rows each
   int kv_splits;
   int64_t split_rows;
+  int split_f32;    // != 0: the shares' outputs are float32 (output points at floats)
   int page_shift;   // pages hold 16 << page_shift tokens; the kernel walks them as runs of 16-token pages
   int skip_single;  // != 0: sequences with one query token are passed over (they have no row tiles)
   int stream_kv;    // != 0: every K/V row is read by one row tile only: copy it with the streaming hint

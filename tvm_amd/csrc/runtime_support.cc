@@ -272,6 +272,36 @@ int decode_pick_chunk_pages_wide(int64_t nnz_pages, int h_kv, int batch, int hea
   return 128;
 }
 
+int64_t prefill_workgroups(int64_t work_q, int group, int64_t work_seqs, int h_kv) {
+  constexpr int64_t kRows = 128;  // query rows of a workgroup
+  return std::max<int64_t>((work_q * group + kRows - 1) / kRows, work_seqs) * h_kv;
+}
+
+// How many ways to split the keys of a prefill launch (shapes only: no read of the index arrays).  The chip holds two
+// workgroups per compute unit.
+//  * Less than half a round of workgroups: as many shares as fill two rounds.
+//  * Up to one round, of row tiles that are at most half full (a draft chain or a small tree per
+//    sequence): the K/V stream decides and two shares balance it (64 sequences of 1024-8192 keys with a
+//    4-token chain each: 0.241 ms unsplit, 0.217 with 2 shares, 0.226 with 4, 0.239 with 8).
+//  * Otherwise none: workgroups that end early leave their compute unit to the one that shares it, and
+//    shares only add start-up, epilogue and merge traffic (16 sequences with 128-token chunks on
+//    2000-6000 keys, 512 workgroups: 0.171 ms unsplit, 0.183 with 2 shares; a 63-node tree per sequence,
+//    1008 workgroups, matrix-bound: 0.409 against 0.442).
+// No share shorter than 8 tiles on average, at most 64 shares.
+int prefill_kv_splits(int64_t work_q, int group, int64_t work_seqs, int h_kv, int64_t avg_keys, int cus) {
+  const int64_t forced = option(kOptPrefillKvSplits);
+  if (forced > 0) return static_cast<int>(std::min<int64_t>(forced, 64));
+  const int64_t resident = static_cast<int64_t>(cus) * 2;
+  const int64_t workgroups = prefill_workgroups(work_q, group, work_seqs, h_kv);
+  int64_t want = 1;
+  if (workgroups * 2 <= resident) {
+    want = (2 * resident + workgroups - 1) / workgroups;
+  } else if (workgroups <= resident && work_q * group * h_kv * 2 <= workgroups * 128) {
+    want = 2;
+  }
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(std::min(want, avg_keys / kMinShareKeys), 64)));
+}
+
 }  // namespace tvmkv
 
 extern "C" {

@@ -69,6 +69,12 @@ int decode_pick_chunk_pages(int64_t nnz_pages, int h_kv, int batch, int head_dim
 // the same for launches whose work items carry 32 query heads (GQA groups above 16)
 int decode_pick_chunk_pages_wide(int64_t nnz_pages, int h_kv, int batch, int head_blocks, int resident_items);
 
+// Shares of the keys of a paged prefill launch (work_q query tokens in work_seqs sequences of avg_keys keys on average,
+// group query heads per kv head) on a device of `cus` compute units, and the workgroups that it has unsplit.
+constexpr int64_t kMinShareKeys = 512;  // eight tiles of 64 keys
+int64_t prefill_workgroups(int64_t work_q, int group, int64_t work_seqs, int h_kv);
+int prefill_kv_splits(int64_t work_q, int group, int64_t work_seqs, int h_kv, int64_t avg_keys, int cus);
+
 }  // namespace tvmkv
 
 #endif  // TVMKV_CSRC_RUNTIME_SUPPORT_H_
