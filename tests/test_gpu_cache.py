@@ -339,6 +339,32 @@ def test_prompts_of_mixed_steps_lose_no_precision_when_their_keys_are_split(d):
     assert split <= 1.02 * whole
 
 
+def test_captured_tree_step_needs_no_scratch_memory():
+    """Under capture the same step runs unsplit: the two shares need scratch memory that a stream without any cannot get
+    there."""
+    d = 128
+    cache, rows, _ = _tree_step_over_unlike_lengths(d, 16)
+    eager = _attend(cache, rows, d)
+    prev = tvm_amd.set_option("prefill_kv_splits", 1)
+    try:
+        whole = _attend(cache, rows, d)
+    finally:
+        tvm_amd.set_option("prefill_kv_splits", prev)
+    out = torch.zeros_like(whole)
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    cache.cache.set_stream(stream.cuda_stream)
+    with torch.cuda.graph(graph, stream=stream):
+        gf("vm.builtin.attention_kv_cache_attention_with_fused_qkv")(cache.cache, 0, d ** -0.5, rows, out)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, whole) and not torch.equal(out, eager)
+        (rows * 2).sum()  # work of the program's own between the replays
+
+
 def test_decode_steps_of_windowed_caches_at_the_edges():
     """A decode step of a sequence-window cache takes the new token as one more key: sequences without cached tokens, of
     one token, at the edge of a page and beyond their window, with a prompt's first decode among them."""

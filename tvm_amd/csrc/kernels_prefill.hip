@@ -1302,7 +1302,8 @@ static int paged_prefill(const void* q, const int32_t* q_indptr, const void* pag
   }
   const bool ext = p.rotary != 0 || sliding_window != 0;
   hipStream_t s = as_stream(stream);
-  const KvSplit split(p, total_q, nnz_pages * page_size / batch_size, d, s, longest);
+  // (a launch under capture keeps the scratch memory that it has always needed)
+  const KvSplit split(p, total_q, nnz_pages * page_size / batch_size, d, s, stream_is_capturing(s) ? 0 : longest);
   if (d == 128) {
     launch_prefill<128, 128, kPaged, 16>(p, total_q, ext, rope_theta, s, scaling);
   } else if (d == 64) {
