@@ -435,6 +435,9 @@ int tvmkv_compact_kv_copy(void* pages, const int32_t* copy_length_indptr,
  *                          split the keys of every row tile over this many workgroups (at most 64) and merge
  *                          the states in a second launch; 0 = derived from the shapes (launches with few row
  *                          tiles and long cached sequences are split, all others are not)
+ *   step_route             > 0: the route of the cache object's prefill steps instead of the one that an estimate
+ *                          from the lengths prefers, where a step can take it: 1 the general launches, 2 prompts
+ *                          and decoding sequences apart, 3 over gathered keys (tests, measurements).
  *   no_fused_decode_step   != 0: the cache object runs a plain decode step as two launches (split + RoPE +
  *                          append, then decode attention) instead of tvmkv_fused_decode_step */
 int tvmkv_set_option(const char* name, int64_t value);
@@ -598,7 +601,10 @@ int tvmkv_cache_get_aux(tvmkv_cache* cache, const char* name, int32_t depth, con
                         int64_t* size);
 /* flags[0]=num_depths, [1]=append_before_attn, [2]=is_decode_request,
  * [3..4]=use_decode_kernel per depth, [5..6]=is_chain per depth, [7]=num_total_pages,
- * [8]=rope_mode in effect. */
+ * [8]=rope_mode in effect, [9]=how the plain MHA layers of the step run: 0 the general launches,
+ * 1 over gathered keys, 2 a decode step with the new token as one more key, 3 prompts and decoding
+ * sequences apart, [10]=the same of layers with a window of their own (0 or 3).  A step under graph
+ * capture runs 0 instead of 3. */
 int tvmkv_cache_get_flags(tvmkv_cache* cache, int64_t* flags, int32_t n_flags);
 /* Serialises the pool into `buf` (int64): [n_free_pages, pages..., n_free_blocks, blocks...,
  * n_blocks, {n_pages, pages..., seq_length, start_pos, sink_length, sliding_window_offset,

@@ -2,6 +2,8 @@
 HIP-backed cache, checked (a) against the numpy closed form the reference's own test uses,
 (b) against the CPU oracle cache on identical seeded inputs, with page tables / append
 indices / pool state compared bit for bit."""
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -27,6 +29,16 @@ def test_reference_scenarios_on_the_gpu(runner, d, rope_mode):
     cache = GpuCache([32, 2048, 512, 16, 0], layers, hq, hkv, d, d, rope_mode=rope_mode)
     sc = S.Scenario(cache, layers, hq, hkv, d, rope_mode=rope_mode, seed=5, tol=4e-3)
     runner(sc)
+
+
+@contextlib.contextmanager
+def step_route(route):
+    """Steps take this route wherever they can: 1 the general launches, 2 prompts and decoding sequences apart, 3 gathered keys."""
+    prev = tvm_amd.set_option("step_route", route)
+    try:
+        yield
+    finally:
+        tvm_amd.set_option("step_route", prev)
 
 
 class Mirror:
@@ -58,7 +70,8 @@ class Mirror:
         assert [tuple(b) for b in sg["blocks"]] == [tuple(b) for b in so["blocks"]] and sg["seqs"] == so["seqs"]
         assert c.copy_log() == self.o.host.copies
 
-    def step(self, batch):
+    def step(self, batch, routes=None):
+        """routes: what flags() has to say of the step's plain layers and of those with a window."""
         ids, lens = [], []
         for item, n in batch:
             if isinstance(item, tuple):
@@ -77,6 +90,9 @@ class Mirror:
         self.o.begin_forward(ids, lens)
         self.g.begin_forward(ids, lens)
         self.compare_bookkeeping()
+        if routes is not None:
+            flags = self.g.cache.flags()
+            assert (flags["plain_route"], flags["window_route"]) == routes
         total = sum(lens)
         for layer in range(self.layers):
             qkv = self.rng.standard_normal((total, self.hq + 2 * self.hkv, self.d)).astype(self.dtype)
@@ -197,14 +213,17 @@ def test_prefill_steps_of_windowed_caches_over_gathered_keys(page_size, d, hq, h
     """Prefill steps with enough rows run over keys gathered (and rotated) into one run per sequence: windows of one and
     several runs of 16 keys, with and without sinks, a sequence that is new, one that decodes beside the chunks, chunks
     longer than the window, more kv heads than one workgroup takes, every head dim, small and large pages."""
-    layers = 2
+    layers, tuned = 2, page_size != 24 and d in (64, 128, 256)
     cache = GpuCache([8, 4096, 1024, page_size, 1], layers, hq, hkv, d, d, rope_mode=S.ROPE_INLINE)
     sc = S.Scenario(cache, layers, hq, hkv, d, rope_mode=S.ROPE_INLINE, seed=4, tol=tol)
     for sid, (window, sink) in enumerate([(40, 0), (130, 4), (257, 30)]):
         sc.add_with_window(sid, window, sink)
     for batch in ([(0, 17), (1, 128), (2, 200)], [(0, 70), (1, 1), (2, 130)], [(3, 65), (2, 90), (0, 40)],
                   [(0, 33), (1, 129), (2, 1), (3, 16)], [(0, 1), (1, 1), (2, 1), (3, 1)], [(1, 64), (2, 63)]):
-        sc.step(list(batch))
+        with step_route(3):
+            sc.step(list(batch))
+        decode = all(n == 1 for _, n in batch)
+        assert cache.cache.flags()["plain_route"] == ((2 if tuned else 0) if decode else 1)
 
 
 @pytest.mark.parametrize("page_size,d,rope_mode", [(24, 128, 1), (5, 64, 1), (12, 256, 1), (40, 96, 0), (16, 128, 2), (16, 112, 2)])
@@ -212,11 +231,24 @@ def test_prefill_steps_of_other_caches_over_gathered_keys(page_size, d, rope_mod
     """The same for caches without windows: pages the tuned kernels do not walk (keys kept rotated or never rotated) and
     RoPE inside the kernels, next to decode steps and forks, against the oracle cache."""
     m = Mirror([8, 2048, 512, page_size, 0], 2, 8, 2, d, rope_mode=rope_mode)
-    m.step([(0, 60), (1, 88), (2, 17)])
-    m.step([(0, 64), (1, 1), (2, 130)])
-    m.step([(0, 1), (1, 1), (2, 1)])
-    m.step([(0, 15), (1, 90), (3, 33)])
-    m.step([((4, 1, 40), 25), (0, 2)])
+    with step_route(3):
+        m.step([(0, 60), (1, 88), (2, 17)], (1, 0))
+        m.step([(0, 64), (1, 1), (2, 130)], (1, 0))
+        m.step([(0, 1), (1, 1), (2, 1)], (0, 0))
+        m.step([(0, 15), (1, 90), (3, 33)], (1, 0))
+        m.step([((4, 1, 40), 25), (0, 2)], (0, 0))
+
+
+@pytest.mark.parametrize("page_size,d", [(16, 128), (24, 64), (16, 96)])
+def test_inline_rope_chunks_behind_long_contexts(page_size, d):
+    """A chunk of few row tiles behind a long context, by the launch that splits its keys and over gathered keys."""
+    for route in (1, 3):
+        m = Mirror([4, 2000, 800, page_size, 0], 1, 2, 1, d, rope_mode=S.ROPE_INLINE)
+        m.step([(0, 600)])
+        m.step([(0, 500), (1, 7)])
+        with step_route(route):
+            m.step([(0, 33)], (int(route == 3), 0))
+            m.step([(0, 3), (1, 20)], (int(route == 3), 0))
 
 
 @pytest.mark.parametrize("page_size,d,hq,hkv,window", [(16, 128, 8, 2, 0), (16, 64, 8, 8, 0), (64, 128, 20, 1, 100), (16, 64, 8, 2, 1),
@@ -227,12 +259,14 @@ def test_steps_that_mix_prompts_and_decoding_sequences(page_size, d, hq, hkv, wi
     with and without a window (0: none), windows inside one page and longer than some sequences."""
     m = Mirror([12, 6000, 2048, page_size, 0] + ([window] if window else []), 2 if window else 1, hq, hkv, d,
                **({"attn_kinds": [3, 0]} if window else {}))
-    m.step([(0, 1300), (1, 64), (2, 300)])
-    m.step([(3, 1), (1, 1)])
-    m.step([(0, 1), (4, 40), (1, 1), (3, 1), (5, 1), (2, 17)])
-    m.step([(2, 1), (0, 1), (6, 130)])
-    m.step([(4, 3), (0, 1), (2, 1)])
-    m.step([(0, 1), (2, 1), (4, 1)])
+    apart = (3, 3 if window else 0)
+    with step_route(2):
+        m.step([(0, 1300), (1, 64), (2, 300)], (0, 0))
+        m.step([(3, 1), (1, 1)], (0, 0))
+        m.step([(0, 1), (4, 40), (1, 1), (3, 1), (5, 1), (2, 17)], apart)
+        m.step([(2, 1), (0, 1), (6, 130)], apart)
+        m.step([(4, 3), (0, 1), (2, 1)], apart)
+        m.step([(0, 1), (2, 1), (4, 1)], (0, 0))
 
 
 @pytest.mark.parametrize("dtype,page_size,d,hq,hkv,window", [(np.float32, 16, 128, 8, 2, 0), (np.float32, 24, 64, 4, 4, 70),
@@ -243,11 +277,12 @@ def test_mixed_steps_on_the_generic_kernels(dtype, page_size, d, hq, hkv, window
     new tokens."""
     m = Mirror([12, 4000, 1024, page_size, 0] + ([window] if window else []), 2 if window else 1, hq, hkv, d, dtype=dtype,
                **({"attn_kinds": [3, 0]} if window else {}))
-    m.step([(0, 700), (1, 64), (2, 200)])
-    m.step([(0, 1), (4, 40), (1, 1), (3, 1), (5, 1), (2, 17)])
-    m.step([(2, 1), (0, 1), (6, 30)])
-    m.step([(4, 3), (0, 1), (2, 1), (3, 1)])
-    m.step([(0, 1), (2, 1), (4, 1)])
+    with step_route(2):
+        m.step([(0, 700), (1, 64), (2, 200)], (0, 0))
+        m.step([(0, 1), (4, 40), (1, 1), (3, 1), (5, 1), (2, 17)], (3, 0))
+        m.step([(2, 1), (0, 1), (6, 30)], (3, 0))
+        m.step([(4, 3), (0, 1), (2, 1), (3, 1)], (3, 0))
+        m.step([(0, 1), (2, 1), (4, 1)], (0, 0))
 
 
 def _exact(rows, cached, starts, mask, heads, kv_heads):

@@ -148,7 +148,7 @@ constexpr int generic_workgroups(int elem_bytes, int dmax, int nb) {
 // (sequence, kv head) has more than 16 rows on average.  Three and four blocks (fp16 storage, one workgroup fewer
 // per CU) measured slower: causal self-attention of 4 x 2048 tokens at head dim 72 173 against 195 TFLOP/s, at
 // head dim 48 144 against 197; only calls that rotate inside the kernel gained (head dim 96: 99 against 90).
-inline int generic_row_blocks(int d, int rows_hint) { return d > 128 || rows_hint <= 16 ? 1 : 2; }
+inline int generic_row_blocks(int d, int rows_hint) { return generic_row_tile(d, rows_hint) / 16; }
 // Also measured and not kept: a form for prefill-shaped calls whose four waves take rows of their own and share
 // stages of 32 keys through LDS (a K / V row fetched and rotated once per 128 query rows).  Plain calls ran slower
 // (head dim 72: 156 against 196 TFLOP/s, with the next stage's loads held in registers during the matrix work 109:
@@ -698,16 +698,10 @@ int generic_attention(const GenericAttention& a, void* stream_) {
   const int group = a.h_q / a.h_kv;
   const int64_t work_q = a.work_seqs > 0 ? a.work_q : a.total_q, work_seqs = a.work_seqs > 0 ? a.work_seqs : a.batch;
   const int rows_hint = static_cast<int>(std::min<int64_t>(work_q * group / work_seqs, 1 << 20));
-  // Few row tiles against long page lists: split the keys over workgroups until the chip has ~8 workgroups
-  // per compute unit, at least 128 keys (8 blocks) per share on average.  Shapes only: no device read.
   p.splits = 1;
   ScratchLease lease{};
   if (paged && a.skip_single == 0) {  // (the rows that are passed over have no partial states to merge)
-    const int rows_per_tile = 16 * generic_row_blocks(a.d, rows_hint);
-    const int64_t tiles = (work_q * group / rows_per_tile + work_seqs) * a.h_kv;
-    const int64_t keys_per_seq = a.nnz_pages * a.page_size / work_seqs;
-    const int64_t want = (f32 ? 8 : 16) * static_cast<int64_t>(compute_units()) / std::max<int64_t>(tiles, 1);
-    p.splits = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({want, keys_per_seq / 128, 64})));
+    p.splits = generic_kv_splits(a.elem_bits, a.d, work_q, group, work_seqs, a.h_kv, a.nnz_pages * a.page_size / work_seqs, compute_units());
   }
   if (p.splits > 1) {
     const size_t o_bytes = static_cast<size_t>(p.splits) * a.total_q * a.h_q * a.d * sizeof(float);

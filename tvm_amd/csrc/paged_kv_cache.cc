@@ -12,6 +12,7 @@
 #include "common.h"
 #include "kv_bookkeeping.h"
 #include "runtime_support.h"
+#include "step_estimate.h"
 #include "typed_kernels.h"
 
 namespace tvmkv {
@@ -56,6 +57,7 @@ class PagedKVCache {
     // paged_kv_cache.cc:335-344
     const bool has_layer_sliding =
         std::find(attn_kinds_.begin(), attn_kinds_.end(), TVMKV_ATTN_MHA_SLIDING) != attn_kinds_.end();
+    has_window_layers_ = has_layer_sliding;
     support_sliding_window_ = has_layer_sliding ? false : support_sliding_window;
     rope_mode_ = (support_sliding_window && rope_mode != TVMKV_ROPE_NONE) ? TVMKV_ROPE_INLINE : rope_mode;
     KV_CHECK(layer_sliding_window_size_ > 0) << "Per-layer sliding window size must be positive.";
@@ -74,6 +76,7 @@ class PagedKVCache {
     // windows or rotates inside the attention kernels (the tuned kernels have those head dims in their plain form).
     bool has_mha_layer = false;
     for (int64_t kind : attn_kinds_) has_mha_layer |= (kind != TVMKV_ATTN_MLA);
+    const bool has_plain_layer = std::find(attn_kinds_.begin(), attn_kinds_.end(), TVMKV_ATTN_MHA) != attn_kinds_.end();
     const bool extended = support_sliding_window_ || has_layer_sliding || rope_mode_ == TVMKV_ROPE_INLINE;
     const int head_dim = static_cast<int>(qk_head_dim_);
     const bool tuned_dim = extended ? (head_dim == 64 || head_dim == 128 || head_dim == 256) : tuned_head_dim(head_dim);
@@ -86,10 +89,10 @@ class PagedKVCache {
           << "multiple of " << (elem_bits_ == 32 ? 8 : 16) << ", got " << head_dim;
       KV_UNSUPPORTED(qk_head_dim_ != v_head_dim_) << "the generic kernels need equal qk and v head dims";
     }
-    // Prefill steps that the tuned kernels take only with RoPE, a window or an odd page size inside them: fp16 storage, a
-    // tuned head dim, and what GatheredPrefillApplies() asks of the step.
-    gather_capable_ = has_mha_layer && !has_mla && elem_bits_ == 16 && qk_head_dim_ == v_head_dim_ && tuned_head_dim(head_dim) &&
-                      (support_sliding_window_ || rope_mode_ == TVMKV_ROPE_INLINE || !tuned_page_size(static_cast<int>(page_size_)));
+    // Prefill steps that rotate inside attention or that the tuned kernels do not take (odd pages; windows at head dims 80 /
+    // 96 / 112): fp16 storage and a head dim of the ragged kernels; PlanStep() decides for each step.
+    gather_capable_ = has_plain_layer && !has_mla && elem_bits_ == 16 && qk_head_dim_ == v_head_dim_ && tuned_head_dim(head_dim) &&
+                      (rope_mode_ == TVMKV_ROPE_INLINE || (generic_ && (support_sliding_window_ || !tuned_page_size(static_cast<int>(page_size_)))));
     KV_CHECK(static_cast<int64_t>(attn_kinds_.size()) >= layer_end)
         << "attn_kinds must cover every layer id up to " << layer_end;
     for (int64_t kind : attn_kinds_) {
@@ -108,6 +111,8 @@ class PagedKVCache {
     config.first_layer_is_mla = !attn_kinds_.empty() && attn_kinds_[0] == TVMKV_ATTN_MLA;
     book_ = std::make_unique<KVBookkeeper>(config);
     reserved_num_seqs_ = reserved_num_seqs;
+    extras_capacity_ = 12 * ((reserved_num_seqs_ + 1 + 3) / 4 * 4);  // the larger of the plans: MixedStep
+    if (gather_capable_) gather_capacity_ = std::min(num_total_pages_ * page_size_ + prefill_chunk_size_, kGatherBytes / GatherRowBytes());
     if (device_ >= 0) InitDevice();
   }
 
@@ -159,6 +164,7 @@ class PagedKVCache {
       aux_needs_upload_ = true;
     } else {
       book_->BeginForward(seq_ids, append_lengths, batch_size, token_tree_parent_ptr, n_tree);
+      PlanStep();
     }
   }
 
@@ -447,7 +453,9 @@ class PagedKVCache {
 
   void GetFlags(int64_t* flags, int n) const {
     const StepLayout& s = book_->step();
-    const int64_t all[9] = {s.num_depths,
+    // how the plain layers and those with a window run
+    const int64_t plain = gathered_rows_ > 0 ? 1 : new_token_step_ ? 2 : mixed_.run[0] ? 3 : 0, window = mixed_.run[1] ? 3 : 0;
+    const int64_t all[11] = {s.num_depths,
                             s.append_before_attn,
                             s.is_decode_request,
                             s.num_depths > 0 ? s.use_decode_kernel[0] : 0,
@@ -455,8 +463,10 @@ class PagedKVCache {
                             s.is_chain[0],
                             s.is_chain[1],
                             num_total_pages_,
-                            rope_mode_};
-    for (int i = 0; i < n && i < 9; ++i) flags[i] = all[i];
+                            rope_mode_,
+                            plain,
+                            window};
+    for (int i = 0; i < n && i < 11; ++i) flags[i] = all[i];
   }
 
   std::vector<int64_t> DumpState() const { return book_->DumpState(); }
@@ -548,12 +558,8 @@ class PagedKVCache {
       HIP_CHECK(hipMalloc(&temp_lse_, prefill_chunk_size_ * num_qo_heads_ * sizeof(float)));
       HIP_CHECK(hipMalloc(&merged_lse_, prefill_chunk_size_ * num_qo_heads_ * sizeof(float)));
       aux_capacity_ = book_->RequiredCapacity();
-      extras_capacity_ = 12 * ((reserved_num_seqs_ + 1 + 3) / 4 * 4);  // the larger of the plans: MixedStep
-      if (gather_capable_) {
-        const int64_t row_bytes = 2 * num_kv_heads_ * qk_head_dim_ * static_cast<int64_t>(sizeof(uint16_t));
-        gather_capacity_ = std::min(num_total_pages_ * page_size_ + prefill_chunk_size_, kGatherBytes / row_bytes);
-        HIP_CHECK(hipMalloc(&gather_, gather_capacity_ * row_bytes));
-      }
+      if (gather_capable_) HIP_CHECK(hipMalloc(&gather_, gather_capacity_ * GatherRowBytes()));
+      HIP_CHECK(hipDeviceGetAttribute(&compute_units_, hipDeviceAttributeMultiprocessorCount, device_));
       for (int i = 0; i < 2; ++i) {
         HIP_CHECK(hipMalloc(&aux_device_[i], (extras_capacity_ + aux_capacity_) * sizeof(int32_t)));
         HIP_CHECK(hipHostMalloc(&aux_staging_[i], (extras_capacity_ + aux_capacity_) * sizeof(int32_t), hipHostMallocDefault));
@@ -714,7 +720,25 @@ class PagedKVCache {
            rope_mode_ != TVMKV_ROPE_INLINE && qk_head_dim_ == v_head_dim_ && (qk_head_dim_ == 64 || qk_head_dim_ == 128);
   }
 
-  // What the kernels of this step need beside the bookkeeper's arrays, written in front of them in the staging buffer.
+  // K and V of one token and all kv heads as the ragged kernel reads them
+  int64_t GatherRowBytes() const { return 2 * num_kv_heads_ * qk_head_dim_ * static_cast<int64_t>(sizeof(uint16_t)); }
+
+  // A sequence of the step: keys that its layers' pages hold for it and new tokens
+  struct StepSequence {
+    int64_t cached, tokens;
+  };
+
+  // MixedAttention: what its launches need of the step (offsets into extras_; [1]: the layers with a window);
+  // run: whether the plain layers and those with a window run that way
+  struct MixedStep {
+    bool run[2] = {false, false};
+    int32_t decoding = 0;
+    int64_t prompts = 0, prompt_tokens = 0, prompt_cached = 0;
+    int64_t rows = 0, page_indptr[2] = {0, 0}, page_begin[2] = {0, 0}, length_info[2] = {0, 0}, nnz_pages[2] = {0, 0};
+  };
+
+  // How the step runs, and what its kernels need beside the bookkeeper's arrays, written in front of them in the staging
+  // buffer.  (A cache without a device plans as well: the tests look at the routes.)
   void PlanStep() {
     extras_.clear();
     gathered_rows_ = 0;
@@ -737,93 +761,166 @@ class PagedKVCache {
     new_token_step_ = one_level && !generic_ && support_sliding_window_ && s.use_decode_kernel[0] && rope_mode_ != TVMKV_ROPE_NORMAL &&
                       !has_rope_scaling_ && rope_ext_factors_ == nullptr &&
                       (qk_head_dim_ == 64 || qk_head_dim_ == 128 || qk_head_dim_ == 256);
-    if (gather_capable_ && rope_ext_factors_ == nullptr && s.num_depths == 1 && s.is_chain[0] && !s.append_before_attn &&
-        !s.use_decode_kernel[0] &&
-        s.total_append_length * (num_qo_heads_ / num_kv_heads_) >=
-            batch * (rope_mode_ == TVMKV_ROPE_INLINE ? kGatherMinRowsRotated : kGatherMinRows)) {
-      const int32_t* host = book_->step_buffer();
-      const int32_t* page_indptr = host + s.page_indptr[0].offset;
-      const int32_t* last_len = host + s.last_page_len[0].offset;
-      const int32_t* window_offset = host + s.sliding_window_offset[0].offset;
-      const int32_t* sink = host + s.sink_size[0].offset;
-      const int32_t* append_indptr = host + s.cur_append_lengths_indptr.offset;
-      extras_.assign((batch + 1 + 3) / 4 * 4, 0);
-      int64_t rows = 0;
-      for (int64_t b = 0; b < batch; ++b) {
-        const int64_t pages = page_indptr[b + 1] - page_indptr[b];
-        if (pages > 0) {
-          rows += (pages - 1) * page_size_ + last_len[b];
-          if (support_sliding_window_) rows += sink[b] - window_offset[b];
+    if (!one_level || s.use_decode_kernel[0]) return;
+    const int64_t forced = option(kOptStepRoute);
+    const bool may_gather = gather_capable_ && rope_ext_factors_ == nullptr && (forced == 0 || forced == 3);
+    const bool may_mix = (forced == 0 || forced == 2) && !support_sliding_window_ && s.page_indices[0].size > 0 && rope_mode_ != TVMKV_ROPE_INLINE &&
+                         (generic_ || qk_head_dim_ == 64 || qk_head_dim_ == 128);
+    if (!may_gather && !may_mix) return;
+    const std::vector<StepSequence> seqs = StepSequences(/*window=*/false);
+    int64_t gathered = 0;
+    for (const StepSequence& q : seqs) gathered += q.cached + q.tokens;
+    // The other route has to be better than the general one by what the estimate is off (measured on 1169 steps: with no
+    // margin 1.5 % of the steps were up to 1.35 times as long as in the general launches, with it none by more than noise)
+    const double margin = forced > 0 ? 0 : qk_head_dim_ > 128 ? 1.2 : 1.1;
+    const double general_us = GeneralUs(seqs, /*window=*/false);
+    const bool can_gather = may_gather && gathered <= gather_capacity_;
+    const double gathered_us = can_gather ? GatheredUs(seqs, gathered) : 2 * general_us;
+    if (may_mix) {
+      MixedStep plan = CountMixedStep(seqs);
+      if (plan.decoding > 0 && plan.prompts > 0) {
+        const double mixed_us = MixedUs(seqs, plan, /*window=*/false);
+        plan.run[0] = mixed_us * margin < general_us && mixed_us <= gathered_us;
+        if (has_window_layers_ && !generic_) {
+          const std::vector<StepSequence> in_window = StepSequences(/*window=*/true);
+          plan.run[1] = MixedUs(in_window, plan, /*window=*/true) * margin < GeneralUs(in_window, /*window=*/true);
         }
-        rows += append_indptr[b + 1] - append_indptr[b];
-        extras_[b + 1] = static_cast<int32_t>(std::min<int64_t>(rows, INT32_MAX));
+        if (plan.run[0] || plan.run[1]) PlanMixedStep(plan);
       }
-      if (rows <= gather_capacity_) gathered_rows_ = rows; else extras_.clear();
     }
-    if (gathered_rows_ == 0 && one_level && !support_sliding_window_ && !s.use_decode_kernel[0] && s.page_indices[0].size > 0 &&
-        rope_mode_ != TVMKV_ROPE_INLINE && (generic_ || qk_head_dim_ == 64 || qk_head_dim_ == 128)) {
-      PlanMixedStep();
+    if (can_gather && !mixed_.run[0] && gathered_us * margin < general_us) {
+      gathered_rows_ = gathered;
+      extras_.assign((batch + 1 + 3) / 4 * 4, 0);
+      for (int64_t b = 0; b < batch; ++b) extras_[b + 1] = static_cast<int32_t>(extras_[b] + seqs[b].cached + seqs[b].tokens);
     }
-    if (!extras_.empty()) {
+    if (device_ >= 0 && !extras_.empty()) {
       std::memcpy(static_cast<int32_t*>(aux_staging_[aux_slot_]) + extras_capacity_ - extras_.size(), extras_.data(),
                   extras_.size() * sizeof(int32_t));
     }
   }
 
+  // window: as the layers with a window of their own see them
+  std::vector<StepSequence> StepSequences(bool window) const {
+    const StepLayout& s = book_->step();
+    const int64_t batch = book_->batch_size();
+    const int32_t* host = book_->step_buffer();
+    const int32_t* page_indptr = host + (window ? s.page_indptr_sw[0] : s.page_indptr[0]).offset;
+    const int32_t* info = host + (window ? s.layer_sw_length_info[0] : s.length_info[0]).offset;
+    const int32_t* tokens = host + s.cur_append_lengths_indptr.offset;
+    std::vector<StepSequence> seqs(batch);
+    for (int64_t b = 0; b < batch; ++b) {
+      const int64_t pages = page_indptr[b + 1] - page_indptr[b];
+      int64_t cached = pages > 0 ? (pages - 1) * page_size_ + info[b] : 0;
+      if (pages > 0 && (window || support_sliding_window_)) cached += info[2 * batch + b] - info[batch + b];
+      seqs[b] = {cached, tokens[b + 1] - tokens[b]};
+    }
+    return seqs;
+  }
+
+  // The estimates (step_estimate.h) of a layer's attention.  PagedUs: one launch over the cached keys of some sequences,
+  // with the split that it would have.
+  template <class Keep>
+  double PagedUs(const std::vector<StepSequence>& seqs, Keep keep, bool rotating, bool window, bool with_own, bool may_split,
+                 int share_bytes) const {
+    int64_t tokens = 0, cached = 0, own = 0, count = 0;
+    for (const StepSequence& q : seqs) {
+      if (!keep(q)) continue;
+      tokens += q.tokens, cached += q.cached, own += with_own ? q.tokens : 0, ++count;
+    }
+    if (count == 0 || cached + own == 0) return 0;
+    const int group = static_cast<int>(num_qo_heads_ / num_kv_heads_), h_kv = static_cast<int>(num_kv_heads_);
+    const int d = static_cast<int>(qk_head_dim_);
+    int splits = 1;
+    if (may_split) {
+      splits = generic_ ? generic_kv_splits(elem_bits_, d, tokens, group, count, h_kv, cached / count, compute_units_)
+                        : prefill_kv_splits(tokens, group, count, h_kv, (cached + own) / count, compute_units_);
+    }
+    LaunchEstimate launch(generic_ ? generic_costs(elem_bits_, d, rotating, generic_row_tile(d, tokens * group / count))
+                          : window ? tuned_window_costs(d)
+                                   : tuned_costs(d, rotating),
+                          num_qo_heads_, num_kv_heads_, d, elem_bits_, compute_units_, splits, share_bytes);
+    for (const StepSequence& q : seqs) {
+      if (keep(q)) launch.Add(q.cached, with_own ? q.tokens : 0, q.tokens);
+    }
+    return launch.Us();
+  }
+  // The launch over the new tokens alone, where the route has one
+  template <class Keep>
+  double OwnUs(const std::vector<StepSequence>& seqs, Keep keep, bool rotating) const {
+    const int d = static_cast<int>(qk_head_dim_);
+    LaunchCosts costs = generic_ ? generic_own_costs(elem_bits_, d, rotating) : tuned_costs(d, rotating);
+    costs.start = 0;
+    LaunchEstimate launch(costs, num_qo_heads_, num_kv_heads_, d, elem_bits_, compute_units_);
+    for (const StepSequence& q : seqs) {
+      if (keep(q)) launch.Add(0, q.tokens, q.tokens);
+    }
+    return launch.Us();
+  }
+  // The launches that take every step: one pass over cached and new keys, or one over each and their merge
+  double GeneralUs(const std::vector<StepSequence>& seqs, bool window) const {
+    const auto all = [](const StepSequence&) { return true; };
+    const bool rotating = rope_mode_ == TVMKV_ROPE_INLINE;
+    if (generic_) {
+      const double base = qk_head_dim_ > 128 ? 36 : rotating && qk_head_dim_ > 64 ? 43 : 18;
+      return base + OwnUs(seqs, all, rotating) + PagedUs(seqs, all, rotating, window, /*with_own=*/false, /*may_split=*/true, sizeof(float));
+    }
+    if (!rotating && !window && !support_sliding_window_) return 11 + PagedUs(seqs, all, false, false, true, true, sizeof(uint16_t));
+    return (rotating ? 5 : window ? 16 : 11) + OwnUs(seqs, all, rotating) + PagedUs(seqs, all, rotating, window, false, true, sizeof(uint16_t));
+  }
+  // GatheredPrefill
+  double GatheredUs(const std::vector<StepSequence>& seqs, int64_t rows) const {
+    LaunchEstimate launch(gathered_costs(qk_head_dim_), num_qo_heads_, num_kv_heads_, qk_head_dim_, 16, compute_units_);
+    for (const StepSequence& q : seqs) launch.Add(q.cached, q.tokens, q.tokens);
+    return (qk_head_dim_ > 128 ? 2 : 11) + 1.1 * 2 * static_cast<double>(rows) * GatherRowBytes() / 5e6 + launch.Us();
+  }
+  // MixedAttention
+  double MixedUs(const std::vector<StepSequence>& seqs, const MixedStep& plan, bool window) const {
+    const auto prompt = [](const StepSequence& q) { return q.tokens > 1; };
+    const auto decoding = [](const StepSequence& q) { return q.tokens == 1; };
+    if (generic_) {
+      return (qk_head_dim_ > 128 ? 36 : 16) + OwnUs(seqs, [](const StepSequence&) { return true; }, false) +
+             PagedUs(seqs, prompt, false, false, false, /*may_split=*/false, 0) + PagedUs(seqs, decoding, false, false, false, true, sizeof(float));
+    }
+    double keys = 0;
+    for (const StepSequence& q : seqs) keys += decoding(q) ? static_cast<double>(q.cached) : 0;
+    const double prompts = window ? OwnUs(seqs, prompt, false) + PagedUs(seqs, prompt, false, true, false, true, sizeof(float))
+                                  : PagedUs(seqs, prompt, false, false, true, true, sizeof(float));
+    return 11 + prompts + 12 + keys * GatherRowBytes() / 5e6;  // 12 us and the rows: the decode kernel
+  }
+
   // A step of prompts and decoding sequences.  In one prefill launch a decoding sequence is a row tile of few rows whose
-  // workgroup walks all its keys alone: the longest of them decides how long the launch takes (32 decoding sequences of up
-  // to 6000 tokens beside 8 prompts, 32 / 8 heads of dim 64, every other layer with a window: 886 us for 8 layers, 590 now).  So the prompts run without
-  // them, and the decode kernel, which splits the keys, takes them with the new token as one more key.  What the decode
+  // workgroups walk all its keys: the longest of them decides how long the launch takes (32 decoding sequences of up
+  // to 6000 tokens beside 8 prompts, 32 / 8 heads of dim 64, every other layer with a window: 886 us for 8 layers, 590 now), unless
+  // the launch is small enough to be split.  So the prompts run without them, and the decode kernel, which always splits the
+  // keys, takes them with the new token as one more key, where the estimate says that this is faster.  What the decode
   // kernel reads of them is written here, for the pages of the plain layers and for those of the layers with a window.
-  void PlanMixedStep() {
+  MixedStep CountMixedStep(const std::vector<StepSequence>& seqs) const {
+    MixedStep plan;
+    for (const StepSequence& q : seqs) {
+      if (q.tokens == 1) {
+        ++plan.decoding;
+      } else {
+        ++plan.prompts;
+        plan.prompt_tokens += q.tokens;
+        plan.prompt_cached += q.cached;
+      }
+    }
+    return plan;
+  }
+
+  void PlanMixedStep(MixedStep plan) {
     const StepLayout& s = book_->step();
     const int64_t batch = book_->batch_size();
     const int32_t* host = book_->step_buffer();
     const int32_t* tokens = host + s.cur_append_lengths_indptr.offset;
-    const bool windows = s.page_indptr_sw[0].present() && s.layer_sw_length_info[0].present();
-    MixedStep plan;
-    const int32_t* page_indptr = host + s.page_indptr[0].offset;
-    const int32_t* last_len = host + s.length_info[0].offset;
-    auto cached = [&](int64_t b) {
-      const int64_t pages = page_indptr[b + 1] - page_indptr[b];
-      return pages > 0 ? (pages - 1) * page_size_ + last_len[b] : 0;
-    };
-    // What the step takes either way, in tiles of 64 keys by 128 rows that a workgroup walks one after the other (about
-    // 1 us each at head dim 128, 0.6 at 64, and 8 tiles' time before the first; 64 keys by 32 rows on the generic kernel,
-    // 3 us in float32 and 1.5 in fp16): the longest walk, or all of them on
-    // the workgroups the chip holds.  The decode kernel: 10 us and the K / V rows at 6 TB/s.
-    const bool wide = qk_head_dim_ == 128;
-    const double tile_us = generic_ ? (elem_bits_ == 32 ? 3.0 : 1.5) : wide ? 1.0 : 0.6, resident = 256 * (wide ? 2 : 3);
-    const int64_t tile_rows = generic_ ? 32 : 128;
-    const int64_t group = num_qo_heads_ / num_kv_heads_;
-    double walk_decode = 0, walk_prompt = 0, work_decode = 0, work_prompt = 0, decode_bytes = 0;
-    for (int64_t b = 0; b < batch; ++b) {
-      const int64_t n = tokens[b + 1] - tokens[b], keys = cached(b);
-      const double walk = 8.0 + static_cast<double>((keys + n + 63) / 64);
-      if (n == 1) {
-        ++plan.decoding;
-        walk_decode = std::max(walk_decode, walk);
-        work_decode += walk * num_kv_heads_;
-        decode_bytes += elem_bits_ / 4.0 * keys * num_kv_heads_ * qk_head_dim_;
-      } else {
-        ++plan.prompts;
-        plan.prompt_tokens += n;
-        plan.prompt_cached += keys;
-        walk_prompt = std::max(walk_prompt, walk);
-        work_prompt += (8.0 + static_cast<double>(keys + n / 2) / 64) * num_kv_heads_ * ((n * group + tile_rows - 1) / tile_rows);
-      }
-    }
-    if (plan.decoding == 0 || plan.prompts == 0) return;
-    const double together = tile_us * std::max({walk_decode, walk_prompt, (work_decode + work_prompt) / resident});
-    const double apart = tile_us * std::max(walk_prompt, work_prompt / resident) + 10.0 + decode_bytes / 6e6;
-    if (apart > together) return;
     auto place = [&](int64_t n) {
       const int64_t at = static_cast<int64_t>(extras_.size());
       extras_.resize(at + (n + 3) / 4 * 4, 0);
       return at;
     };
     plan.rows = place(plan.decoding);
-    for (int set = 0; set < (windows ? 2 : 1); ++set) {
+    for (int set = 0; set < 2; ++set) {
+      if (!plan.run[set]) continue;
       const int32_t* indptr = host + (set ? s.page_indptr_sw[0] : s.page_indptr[0]).offset;
       const int32_t* info = host + (set ? s.layer_sw_length_info[0] : s.length_info[0]).offset;
       const int64_t n = plan.decoding;
@@ -854,8 +951,7 @@ class PagedKVCache {
   // A step that is being captured keeps the launches that need no scratch memory of the decode kernel's; the generic
   // kernel's extended form, which the layers with a window take, has no index of sequences (it spills with one).
   bool RunsMixed(int64_t layer_id) const {
-    return mixed_.decoding > 0 && !(generic_ && attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING) &&
-           !stream_is_capturing(static_cast<hipStream_t>(compute_stream_));
+    return mixed_.run[attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING] && !stream_is_capturing(static_cast<hipStream_t>(compute_stream_));
   }
 
   void MixedAttention(int64_t layer_id, const void* q, int64_t q_stride, bool rotate_q, const void* k, const void* v, void* out,
@@ -1353,6 +1449,7 @@ class PagedKVCache {
   int64_t num_qo_heads_, num_kv_heads_, qk_head_dim_, v_head_dim_;
   int64_t num_total_pages_ = 0, prefill_chunk_size_, reserved_num_seqs_ = 0;
   bool support_sliding_window_ = false;
+  bool has_window_layers_ = false;  // layers with a window of their own (MHA_SLIDING)
   int elem_bits_ = 16;    // storage type of the MHA layers: 16 (fp16) or 32 (float32)
   bool gather_capable_ = false;  // prefill steps may run over gathered keys (GatheredPrefill)
   bool generic_ = false;  // the MHA layers run on the typed / generic kernels (typed_kernels.h)
@@ -1387,25 +1484,13 @@ class PagedKVCache {
   // the plan of the current step (PlanStep), held in front of the bookkeeper's arrays in both copies of the buffer
   std::vector<int32_t> extras_;
   int64_t extras_capacity_ = 0;
-  // MixedAttention: what its launches need of the step (offsets into extras_; [1]: the layers with a window);
-  // decoding == 0: the step does not run that way
-  struct MixedStep {
-    int32_t decoding = 0;
-    int64_t prompts = 0, prompt_tokens = 0, prompt_cached = 0;
-    int64_t rows = 0, page_indptr[2] = {0, 0}, page_begin[2] = {0, 0}, length_info[2] = {0, 0}, nnz_pages[2] = {0, 0};
-  };
   MixedStep mixed_;
   int32_t longest_pages_[2][kMaxBlockDepth] = {};  // of the entries of each depth ([1]: in the layers with a window)
+  int compute_units_ = 256;
   bool new_token_step_ = false;  // the step runs as WindowedDecodeStep
   // GatheredPrefill: K and V rows of a step, at most kGatherBytes (steps with more keys take the kernels that rotate
   // inside), and how many rows this step has (0: the step does not run that way)
   static constexpr int64_t kGatherBytes = int64_t{1} << 30;
-  // Query rows per kv head and sequence, on average, from which the pass over the keys pays.  Measured, us per layer, the
-  // kernels that rotate / look every row's page up inside -> gathered: 32 sequences with windows of 2047 tokens, 32 / 8
-  // heads of dim 128, rows 32: 179 -> 175, 64: 211 -> 177, 128: 226 -> 180; 16 sequences, 32 / 32 heads of dim 96, rows
-  // 16: 255 -> 285, 32: 431 -> 287; pages of 24 tokens, 32 sequences of 1000-4000 tokens, 32 / 8 heads of dim 128,
-  // rows 32: 212 -> 234, 128: 317 -> 243.
-  static constexpr int64_t kGatherMinRowsRotated = 32, kGatherMinRows = 64;
   void* gather_ = nullptr;
   int64_t gather_capacity_ = 0, gathered_rows_ = 0;
   void* aux_device_[2] = {nullptr, nullptr};

@@ -24,7 +24,7 @@ struct OptionTable {
     static const char* const env_names[] = {"TVMKV_DECODE_CHUNK_PAGES", "TVMKV_DECODE_SEPARATE_MERGE",
                                                        "TVMKV_DECODE_WGS_PER_CU", "TVMKV_MLA_CHUNK_TOKENS",
                                                        "TVMKV_MLA_SEPARATE_MERGE", "TVMKV_PREFILL_KV_SPLITS",
-                                                       "TVMKV_NO_FUSED_DECODE_STEP"};
+                                                       "TVMKV_NO_FUSED_DECODE_STEP", "TVMKV_STEP_ROUTE"};
     static_assert(sizeof(env_names) / sizeof(env_names[0]) == kNumOptions, "one environment variable per option");
     for (int i = 0; i < kNumOptions; ++i) {
       const char* text = std::getenv(env_names[i]);  // once, when the library is loaded
@@ -36,7 +36,7 @@ OptionTable g_options;
 
 const char* const kOptionNames[] = {"decode_chunk_pages", "decode_separate_merge", "decode_wgs_per_cu",
                                                "mla_chunk_tokens", "mla_separate_merge", "prefill_kv_splits",
-                                               "no_fused_decode_step"};
+                                               "no_fused_decode_step", "step_route"};
 static_assert(sizeof(kOptionNames) / sizeof(kOptionNames[0]) == kNumOptions, "one name per option");
 
 struct Scratch {
@@ -300,6 +300,14 @@ int prefill_kv_splits(int64_t work_q, int group, int64_t work_seqs, int h_kv, in
     want = 2;
   }
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(std::min(want, avg_keys / kMinShareKeys), 64)));
+}
+
+// Few row tiles against long page lists: split the keys over workgroups until the chip has ~16 workgroups per compute
+// unit (8 in float32), at least 128 keys (8 blocks) per share on average.  Shapes only: no device read.
+int generic_kv_splits(int elem_bits, int d, int64_t work_q, int group, int64_t work_seqs, int h_kv, int64_t avg_keys, int cus) {
+  const int64_t tiles = (work_q * group / generic_row_tile(d, work_q * group / work_seqs) + work_seqs) * h_kv;
+  const int64_t want = (elem_bits == 32 ? 8 : 16) * static_cast<int64_t>(cus) / std::max<int64_t>(tiles, 1);
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({want, avg_keys / 128, 64})));
 }
 
 }  // namespace tvmkv

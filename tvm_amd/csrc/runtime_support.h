@@ -21,6 +21,8 @@ enum Option {
   kOptMlaSeparateMerge,       // unused (the MLA chunks are always merged in a second launch)
   kOptPrefillKvSplits,        // > 0: split the keys of every row tile of a paged prefill launch this many ways, 0 = derived
   kOptNoFusedDecodeStep,      // != 0: the cache object runs a decode step as split+RoPE+append and decode, two launches
+  kOptStepRoute,              // > 0: the route of the cache object's steps instead of the one that the estimate prefers, where a
+                              // step can take it: 1 the general launches, 2 prompts and decoding sequences apart, 3 gathered keys
   kNumOptions
 };
 bool stream_is_capturing(hipStream_t stream);
@@ -74,6 +76,9 @@ int decode_pick_chunk_pages_wide(int64_t nnz_pages, int h_kv, int batch, int hea
 constexpr int64_t kMinShareKeys = 512;  // eight tiles of 64 keys
 int64_t prefill_workgroups(int64_t work_q, int group, int64_t work_seqs, int h_kv);
 int prefill_kv_splits(int64_t work_q, int group, int64_t work_seqs, int h_kv, int64_t avg_keys, int cus);
+// The same of a launch of the generic kernel, whose workgroups own generic_row_tile() query rows.
+inline int generic_row_tile(int d, int64_t rows_per_sequence) { return d > 128 || rows_per_sequence <= 16 ? 16 : 32; }
+int generic_kv_splits(int elem_bits, int d, int64_t work_q, int group, int64_t work_seqs, int h_kv, int64_t avg_keys, int cus);
 
 }  // namespace tvmkv
 

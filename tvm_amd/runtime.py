@@ -92,10 +92,11 @@ class PagedAttentionKVCache:
         return [data[i] for i in range(size.value)]
 
     def flags(self):
-        buf = (ctypes.c_int64 * 9)()
-        check(lib().tvmkv_cache_get_flags(self.handle, buf, 9))
+        buf = (ctypes.c_int64 * 11)()
+        check(lib().tvmkv_cache_get_flags(self.handle, buf, 11))
         keys = ["num_depths", "append_before_attn", "is_decode_request", "use_decode_kernel_0",
-                "use_decode_kernel_1", "is_chain_0", "is_chain_1", "num_total_pages", "rope_mode"]
+                "use_decode_kernel_1", "is_chain_0", "is_chain_1", "num_total_pages", "rope_mode",
+                "plain_route", "window_route"]
         return dict(zip(keys, (int(v) for v in buf)))
 
     def state(self):
