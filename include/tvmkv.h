@@ -497,6 +497,10 @@ typedef struct tvmkv_cache tvmkv_cache;
  *                 windows or RoPE inside the attention kernels; that rotation needs a head dim that is a
  *                 multiple of 16 (of 8 for float32), and none of this is built for caches with MLA layers
  *                 (TVMKV_EUNSUPPORTED)
+ *                 A fp16 cache with RoPE inside attention, or on the generic kernels at head dims 64 / 80 / 96 / 112 /
+ *                 128 / 256 (odd page sizes, windows at 80 / 96 / 112), allocates the K / V rows of one layer's
+ *                 step, at most 1 GiB, in the first begin_forward whose step runs over gathered keys; without
+ *                 room for them such steps take the general launches
  *   device_id     HIP device ordinal, or -1 for a HOST-ONLY cache: page-pool bookkeeping and
  *                 auxiliary arrays work, anything that touches device memory returns
  *                 TVMKV_ENODEVICE. */

@@ -239,6 +239,33 @@ def test_prefill_steps_of_other_caches_over_gathered_keys(page_size, d, rope_mod
         m.step([((4, 1, 40), 25), (0, 2)], (0, 0))
 
 
+def test_gathered_rows_are_allocated_by_the_first_step_that_wants_them():
+    """A cache takes no memory for gathered keys when it is created, nor for steps that run without them."""
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info(0)[0]
+
+    d, heads, tokens = 128, 8, 65536
+    rows = (tokens + 16 + 4096) * 2 * heads * d * 2  # the pool's slots and a prefill chunk: 272 MiB
+    step = torch.zeros((4096, 3 * heads, d), dtype=torch.float16, device=DEV)
+    before = free()
+    cache = GpuCache([4, tokens, 4096, 16, 0], 1, heads, heads, d, d, rope_mode=S.ROPE_INLINE)
+    created = free()
+    # pages, the chunk's q / k / v / output, the step's arrays; the allocator's granularity
+    assert before - created < tokens * 2 * heads * d * 2 + 4 * 4096 * heads * d * 2 + (24 << 20)
+    cache.add_sequence(0)
+    left = []
+    for route in (1, 1, 3, 3):  # (a kernel's first launch and split keys take memory of their own)
+        with step_route(route):
+            cache.begin_forward([0], [4096])
+        _attend(cache, step, d)
+        cache.end_forward()
+        assert cache.cache.flags()["plain_route"] == int(route == 3)
+        left.append(free())
+    assert left[0] - left[1] < 64 << 20 and left[2] - left[3] < 64 << 20
+    assert rows <= left[1] - left[2] < rows + (64 << 20)
+
+
 @pytest.mark.parametrize("page_size,d", [(16, 128), (24, 64), (16, 96)])
 def test_inline_rope_chunks_behind_long_contexts(page_size, d):
     """A chunk of few row tiles behind a long context, by the launch that splits its keys and over gathered keys."""

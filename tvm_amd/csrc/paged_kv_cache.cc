@@ -558,7 +558,6 @@ class PagedKVCache {
       HIP_CHECK(hipMalloc(&temp_lse_, prefill_chunk_size_ * num_qo_heads_ * sizeof(float)));
       HIP_CHECK(hipMalloc(&merged_lse_, prefill_chunk_size_ * num_qo_heads_ * sizeof(float)));
       aux_capacity_ = book_->RequiredCapacity();
-      if (gather_capable_) HIP_CHECK(hipMalloc(&gather_, gather_capacity_ * GatherRowBytes()));
       HIP_CHECK(hipDeviceGetAttribute(&compute_units_, hipDeviceAttributeMultiprocessorCount, device_));
       for (int i = 0; i < 2; ++i) {
         HIP_CHECK(hipMalloc(&aux_device_[i], (extras_capacity_ + aux_capacity_) * sizeof(int32_t)));
@@ -723,6 +722,19 @@ class PagedKVCache {
   // K and V of one token and all kv heads as the ragged kernel reads them
   int64_t GatherRowBytes() const { return 2 * num_kv_heads_ * qk_head_dim_ * static_cast<int64_t>(sizeof(uint16_t)); }
 
+  // The rows are allocated by the first step that wants them: where the card has no room for them any more, or the stream
+  // is being captured, the general launches run, as they do in caches whose steps never gather.
+  bool HaveGatherBuffer() {
+    if (device_ < 0 || gather_ != nullptr) return true;
+    if (stream_is_capturing(static_cast<hipStream_t>(compute_stream_))) return false;
+    HIP_CHECK(hipSetDevice(device_));
+    if (hipMalloc(&gather_, gather_capacity_ * GatherRowBytes()) == hipSuccess) return true;
+    (void)hipGetLastError();  // not the error of a later call
+    gather_ = nullptr;
+    gather_capacity_ = 0;
+    return false;
+  }
+
   // A sequence of the step: keys that its layers' pages hold for it and new tokens
   struct StepSequence {
     int64_t cached, tokens;
@@ -774,25 +786,23 @@ class PagedKVCache {
     // margin 1.5 % of the steps were up to 1.35 times as long as in the general launches, with it none by more than noise)
     const double margin = forced > 0 ? 0 : qk_head_dim_ > 128 ? 1.2 : 1.1;
     const double general_us = GeneralUs(seqs, /*window=*/false);
-    const bool can_gather = may_gather && gathered <= gather_capacity_;
-    const double gathered_us = can_gather ? GatheredUs(seqs, gathered) : 2 * general_us;
-    if (may_mix) {
-      MixedStep plan = CountMixedStep(seqs);
-      if (plan.decoding > 0 && plan.prompts > 0) {
-        const double mixed_us = MixedUs(seqs, plan, /*window=*/false);
-        plan.run[0] = mixed_us * margin < general_us && mixed_us <= gathered_us;
-        if (has_window_layers_ && !generic_) {
-          const std::vector<StepSequence> in_window = StepSequences(/*window=*/true);
-          plan.run[1] = MixedUs(in_window, plan, /*window=*/true) * margin < GeneralUs(in_window, /*window=*/true);
-        }
-        if (plan.run[0] || plan.run[1]) PlanMixedStep(plan);
-      }
-    }
-    if (can_gather && !mixed_.run[0] && gathered_us * margin < general_us) {
+    MixedStep plan = may_mix ? CountMixedStep(seqs) : MixedStep{};
+    const bool mixes = plan.decoding > 0 && plan.prompts > 0;
+    const double mixed_us = mixes ? MixedUs(seqs, plan, /*window=*/false) : general_us;
+    const double gathered_us = may_gather && gathered <= gather_capacity_ ? GatheredUs(seqs, gathered) : general_us;
+    plan.run[0] = mixes && mixed_us * margin < general_us;
+    if (may_gather && gathered <= gather_capacity_ && gathered_us * margin < general_us && !(plan.run[0] && mixed_us <= gathered_us) &&
+        HaveGatherBuffer()) {
+      plan.run[0] = false;
       gathered_rows_ = gathered;
       extras_.assign((batch + 1 + 3) / 4 * 4, 0);
       for (int64_t b = 0; b < batch; ++b) extras_[b + 1] = static_cast<int32_t>(extras_[b] + seqs[b].cached + seqs[b].tokens);
     }
+    if (mixes && has_window_layers_ && !generic_) {
+      const std::vector<StepSequence> in_window = StepSequences(/*window=*/true);
+      plan.run[1] = MixedUs(in_window, plan, /*window=*/true) * margin < GeneralUs(in_window, /*window=*/true);
+    }
+    if (plan.run[0] || plan.run[1]) PlanMixedStep(plan);
     if (device_ >= 0 && !extras_.empty()) {
       std::memcpy(static_cast<int32_t*>(aux_staging_[aux_slot_]) + extras_capacity_ - extras_.size(), extras_.data(),
                   extras_.size() * sizeof(int32_t));
