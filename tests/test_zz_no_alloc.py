@@ -143,3 +143,36 @@ def test_allocating_entry_point_says_so_under_capture():
     eo, el = torch.empty_like(go), torch.empty_like(gl)
     K.batch_decode_paged_kv(*args, eo, el, 0, 1.0, 1e4, d ** -0.5)
     assert torch.equal(go, eo) and torch.equal(gl, el)
+
+
+def test_a_shorter_decode_launch_is_captured_after_a_longer_one():
+    """Warmed up at their longest, the sequences of a small launch may be cut into more chunks when they are shorter (4 x
+    1611 tokens: 20 chunk slots, 4 x 1131: 39): the scratch memory of the first launch has to hold the second."""
+    rng = np.random.default_rng(35)
+    hq, hkv, d, b = 32, 8, 128, 4
+    plans = [tvm_amd.decode_split_plan([0, n // 4, n // 2, 3 * n // 4, n], n, hkv)[0] for n in (404, 284)]
+    assert plans == [24, 8]
+    z = i32(np.zeros(b, np.int32))
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    calls = []
+    for tokens in (1611, 1131):
+        pages, indptr, values, last, _, _ = build_paged_kv(rng, [tokens] * b, 4 * (tokens // 16 + 2), hkv, 16, d)
+        out = torch.zeros((b, hq, d), dtype=torch.float16, device=DEV), torch.zeros((b, hq), dtype=torch.float32, device=DEV)
+        args = dev(rng.standard_normal((b, hq, d)).astype(F16)), dev(pages), i32(indptr), i32(values), i32(last), z, z
+        calls.append((lambda o, a=args: K.batch_decode_paged_kv(*a, *o, 0, 1.0, 1e4, d ** -0.5), out))
+    (longer, out_longer), (shorter, out_shorter) = calls
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        longer(out_longer)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        shorter(out_shorter)
+    eager = torch.zeros_like(out_shorter[0]), torch.zeros_like(out_shorter[1])
+    shorter(eager)
+    for _ in range(3):
+        out_shorter[0].zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out_shorter[0], eager[0]) and torch.equal(out_shorter[1], eager[1])
+        shorter(eager)

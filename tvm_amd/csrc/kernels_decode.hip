@@ -936,7 +936,7 @@ struct FusedStep {
   int64_t q_stride = 0, new_stride = 0;
 };
 
-// Body of the decode entry point.  lease(bytes) hands out the scratch memory of the call: arrival
+// Body of the decode entry point.  lease(bytes, at_least) hands out the scratch memory of the call: arrival
 // counters in the first kArrivalBytes, partial states behind them.
 template <class Lease>
 static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void* q, const void* pages, const int32_t* page_indptr, const int32_t* page_values,
@@ -1015,7 +1015,12 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
   p.rope_inverse = p.rope_halves_differ = 0;
   p.rope_magnitude = 1.0f;
   const size_t part_ml_bytes = static_cast<size_t>(slots) * h_q * 2 * sizeof(float);
-  const ScratchLease ws = lease(kArrivalBytes + part_o_bytes + part_ml_bytes);
+  // A small launch has up to 768 work items (decode_pick_chunk_pages), and a shorter one may have more of them than a
+  // longer one: the first buffer holds the states of any of them, so that a stream that has run one launch of these heads
+  // can capture the others.
+  const size_t row_bytes = (dk + 2) * sizeof(float);
+  const size_t small_bytes = heads_per_item == 16 ? static_cast<size_t>(768 / h_kv) * h_q * row_bytes : 0;
+  const ScratchLease ws = lease(kArrivalBytes + part_o_bytes + part_ml_bytes, kArrivalBytes + small_bytes);
   p.part_o = reinterpret_cast<float*>(ws.ptr + kArrivalBytes);
   p.part_ml = reinterpret_cast<float*>(ws.ptr + kArrivalBytes + part_o_bytes);
   p.arrivals = nullptr;
@@ -1191,7 +1196,7 @@ extern "C" int tvmkv_batch_decode_paged_kv(const void* q, const void* pages, con
   }
   KV_API_BEGIN();
   hipStream_t s = as_stream(stream);
-  decode_entry([&](size_t bytes) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes); }, FusedStep{}, q, pages, page_indptr, page_values, length_info, k_rope_pos_offset, q_rope_position, output, lse, rotary_mode,
+  decode_entry([&](size_t bytes, size_t at_least) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes, at_least); }, FusedStep{}, q, pages, page_indptr, page_values, length_info, k_rope_pos_offset, q_rope_position, output, lse, rotary_mode,
                rope_scale, rope_theta, sm_scale, batch_size, nnz_pages, num_pages, h_q, h_kv, d, page_size,
                sliding_window, stream);
   KV_API_END();
@@ -1215,7 +1220,7 @@ extern "C" int tvmkv_batch_decode_paged_kv_scaled(const void* q, const void* pag
   hipStream_t s = as_stream(stream);
   FusedStep plain;
   plain.rope_scaling = rope_scaling;
-  decode_entry([&](size_t bytes) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes); }, plain, q, pages,
+  decode_entry([&](size_t bytes, size_t at_least) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes, at_least); }, plain, q, pages,
                page_indptr, page_values, length_info, k_rope_pos_offset, q_rope_position, output, lse, rotary_mode,
                rope_scale, rope_theta, sm_scale, batch_size, nnz_pages, num_pages, h_q, h_kv, d, page_size,
                sliding_window, stream);
@@ -1240,7 +1245,7 @@ extern "C" int tvmkv_fused_decode_step(const void* qkv, void* pages, const int32
   step.qkv = qkv;
   step.append_position_map = append_position_map;
   step.apply_rope = apply_rope != 0;
-  decode_entry([&](size_t bytes) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes); }, step, nullptr, pages,
+  decode_entry([&](size_t bytes, size_t at_least) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes, at_least); }, step, nullptr, pages,
                page_indptr, page_values, last_page_len, nullptr, q_rope_position, output, lse, 0, rope_scale, rope_theta,
                sm_scale, batch_size, nnz_pages, num_pages, h_q, h_kv, d, page_size, 0, stream);
   KV_API_END();
@@ -1259,7 +1264,7 @@ int tvmkv::decode_with_new_token(const NewTokenDecode& a, void* stream) {
   step.page_begin = a.page_begin;
   step.q_stride = a.q_stride;
   step.new_stride = a.new_stride;
-  decode_entry([&](size_t bytes) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes); }, step, a.q, a.pages,
+  decode_entry([&](size_t bytes, size_t at_least) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes, at_least); }, step, a.q, a.pages,
                a.page_indptr, a.page_values, a.length_info, a.k_rope_pos_offset, a.q_rope_position, a.out, a.lse, a.rotate,
                a.rope_scale, a.rope_theta, a.sm_scale, a.batch, a.nnz_pages, a.num_pages, a.h_q, a.h_kv, a.d, a.page_size,
                a.sliding, stream);
@@ -1279,7 +1284,7 @@ extern "C" int tvmkv_batch_decode_paged_kv_noalloc(const void* q, const void* pa
                                                    int32_t d, int32_t page_size, int32_t sliding_window,
                                                    void* stream) {
   KV_API_BEGIN();
-  decode_entry([&](size_t bytes) { return lease_static_scratch(bytes, as_stream(stream)); }, FusedStep{}, q, pages, page_indptr, page_values,
+  decode_entry([&](size_t bytes, size_t) { return lease_static_scratch(bytes, as_stream(stream)); }, FusedStep{}, q, pages, page_indptr, page_values,
                length_info, k_rope_pos_offset, q_rope_position, output, lse, rotary_mode, rope_scale, rope_theta,
                sm_scale, batch_size, nnz_pages, num_pages, h_q, h_kv, d, page_size, sliding_window, stream);
   KV_API_END();

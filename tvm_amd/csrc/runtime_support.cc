@@ -88,7 +88,7 @@ void zero_scratch_counters(char* ptr, size_t counter_bytes, hipStream_t stream) 
   HIP_CHECK(hipGetLastError());
 }
 
-ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, size_t counter_bytes) {
+ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, size_t counter_bytes, size_t at_least) {
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
   // held by the lease until the caller has enqueued its launch: a thread that grows (and frees) this
@@ -113,7 +113,7 @@ ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, s
       }
       s = Scratch{};
     }
-    const size_t want = bytes + bytes / 2;
+    const size_t want = std::max(bytes + bytes / 2, at_least);
     void* ptr = nullptr;
     HIP_CHECK(hipMalloc(&ptr, want));
     s.ptr = static_cast<char*>(ptr);

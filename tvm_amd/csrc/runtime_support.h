@@ -44,7 +44,8 @@ struct ScratchLease {
   std::unique_lock<std::mutex> lock;
 };
 enum ScratchUser { kScratchDecode = 0, kScratchMla = 1, kScratchPrefill = 2, kScratchGeneric = 3 };
-ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, size_t counter_bytes);
+// at_least: what a buffer that has to be allocated gets in any case
+ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, size_t counter_bytes, size_t at_least = 0);
 // Frees the buffers of (current device, stream) after synchronising the stream; a buffer whose address
 // a graph under capture has recorded is kept until the process ends instead.
 void release_scratch(hipStream_t stream);
