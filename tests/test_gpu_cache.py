@@ -427,6 +427,43 @@ def test_captured_tree_step_needs_no_scratch_memory():
         (rows * 2).sum()  # work of the program's own between the replays
 
 
+@pytest.mark.parametrize("kinds,dtype", [([0], np.float16), ([3], np.float16), ([0], np.float32)])
+def test_a_mixed_step_can_be_captured_once_it_has_run(kinds, dtype):
+    """Under capture the general launches run; their scratch memory is there when the step has run eagerly on that stream."""
+    d, hq, hkv, lengths, new = 128, 8, 2, [3000, 2500], [1, 40]
+    config = [2, 8192, 3000, 16, 0] + ([4096] if 3 in kinds else [])
+    qkv = dev(np.random.default_rng(14).standard_normal((3000, hq + 2 * hkv, d)).astype(dtype))
+    attend = gf("vm.builtin.attention_kv_cache_attention_with_fused_qkv")
+    outs = []
+    for route in (1, 2):
+        cache = GpuCache(config, 1, hq, hkv, d, d, attn_kinds=kinds, dtype=dtype)
+        for b, n in enumerate(lengths):
+            cache.add_sequence(b)
+            cache.begin_forward([b], [n])
+            attend(cache.cache, 0, d ** -0.5, qkv[:n], torch.zeros((n, hq, d), dtype=qkv.dtype, device=DEV))
+            cache.end_forward()
+        with step_route(route):
+            cache.begin_forward([0, 1], new)
+        out = torch.zeros((sum(new), hq, d), dtype=qkv.dtype, device=DEV)
+        torch.cuda.synchronize()
+        stream = torch.cuda.Stream()
+        cache.cache.set_stream(stream.cuda_stream)
+        attend(cache.cache, 0, d ** -0.5, qkv[:sum(new)], out)
+        torch.cuda.synchronize()
+        outs.append(out.clone())
+    assert not torch.equal(outs[0], outs[1])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        attend(cache.cache, 0, d ** -0.5, qkv[:sum(new)], out)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, outs[0])
+        (outs[1] * 2).sum()
+
+
 def test_decode_steps_of_windowed_caches_at_the_edges():
     """A decode step of a sequence-window cache takes the new token as one more key: sequences without cached tokens, of
     one token, at the edge of a page and beyond their window, with a prompt's first decode among them."""

@@ -964,11 +964,26 @@ class PagedKVCache {
     return mixed_.run[attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING] && !stream_is_capturing(static_cast<hipStream_t>(compute_stream_));
   }
 
+  // What the general launches of the step need is allocated by the mixed ones, as they take the step over under capture,
+  // where it cannot be: a program that has run a step once can capture it.
+  void ReserveGeneralScratch(bool window) const {
+    const StepLayout& s = book_->step();
+    const int64_t batch = book_->batch_size(), tokens = s.total_append_length;
+    const int64_t cached = (window ? s.page_indices_sw[0] : s.page_indices[0]).size * page_size_;
+    const int group = static_cast<int>(num_qo_heads_ / num_kv_heads_), h_kv = static_cast<int>(num_kv_heads_);
+    const int64_t splits = generic_ ? generic_kv_splits(elem_bits_, static_cast<int>(qk_head_dim_), tokens, group, batch, h_kv, cached / batch, compute_units_)
+                                    : prefill_kv_splits(tokens, group, batch, h_kv, (cached + (window ? 0 : tokens)) / batch, compute_units_);
+    if (splits <= 1) return;
+    const size_t row_bytes = qk_head_dim_ * (generic_ ? sizeof(float) : sizeof(uint16_t)) + sizeof(float);
+    lease_scratch(generic_ ? kScratchGeneric : kScratchPrefill, static_cast<hipStream_t>(compute_stream_), splits * tokens * num_qo_heads_ * row_bytes, 0);
+  }
+
   void MixedAttention(int64_t layer_id, const void* q, int64_t q_stride, bool rotate_q, const void* k, const void* v, void* out,
                       int64_t total_seq_length, double sm_scale) {
     const StepLayout& s = book_->step();
     const int64_t local_layer_id = layer_id - layer_id_begin_offset_;
     const bool window = attn_kinds_[layer_id] == TVMKV_ATTN_MHA_SLIDING;
+    ReserveGeneralScratch(window);
     if (generic_) {
       GenericMixedAttention(layer_id, q, k, v, out, total_seq_length, sm_scale);
       return;
