@@ -466,7 +466,8 @@ def test_a_mixed_step_can_be_captured_once_it_has_run(kinds, dtype):
 
 def test_decode_steps_of_windowed_caches_at_the_edges():
     """A decode step of a sequence-window cache takes the new token as one more key: sequences without cached tokens, of
-    one token, at the edge of a page and beyond their window, with a prompt's first decode among them."""
+    one token, at the edge of a page and beyond their window, with a prompt's first decode among them; small prefill steps
+    of such a cache as well."""
     for d, hq, hkv, rope_mode in ((128, 8, 2, 2), (64, 20, 1, 2), (256, 4, 2, 2), (128, 4, 4, 0)):
         layers = 2
         # the pool is what an earlier cache of the same size left: NaN in every slot
@@ -488,8 +489,13 @@ def test_decode_steps_of_windowed_caches_at_the_edges():
         sc.step([(0, 1), (1, 1), (2, 1), (3, 1)])
         # (a chunk longer than its window leaves slots behind the sinks that nothing ever writes)
         sc.step([(0, 14), (1, 29), (2, 300), (3, 500)])
-        for _ in range(6):
+        for _ in range(3):
             sc.step([(0, 1), (1, 1), (2, 1), (3, 1)])
+        # a few tokens, and a short chunk beside decoding sequences, by the launches that read the pages themselves
+        with step_route(1):
+            sc.step([(0, 2), (1, 3), (2, 1), (3, 2)])
+            sc.step([(0, 1), (1, 5), (2, 1), (3, 1)])
+        sc.step([(0, 1), (1, 1), (2, 1), (3, 1)])
 
 
 def test_short_chunk_against_a_long_cached_sequence():

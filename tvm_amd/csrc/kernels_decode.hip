@@ -387,8 +387,10 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   // run_sin) by fixed angles.  A division, a reduction and two transcendentals for each of a lane's 32 (key, frequency)
   // pairs of a step kept the vector ALU busy for longer than the step's 16 KiB take to arrive (64 sequences with
   // windows of 4096 tokens, 32 / 8 heads of dim 128: 247 us a layer, 206 now).  The fixed angles come from the host in
-  // double, so that after the 16 steps of the longest chunk the drift is a few 2^-24 -- the fp32 angle itself is off by
-  // more.  They wait in LDS: in registers they made every extended launch of head dim 128 spill.
+  // double and are rounded once, so that the error of (cos, sin) grows with the 63 rotations of the longest chunk to
+  // 19 x 2^-24 at head dim 64 and 34 x 2^-24 at 128 and 256 (2^-19; an fp32 angle is off by as much from position 70 on,
+  // and the rotated row is rounded at 2^-11).  They wait in LDS: in registers they made every extended launch of head
+  // dim 128 spill.
   const bool k_rotary = EXT && (SELF ? p.rotary == 1 : p.rotary != 0);
   if (k_rotary) {
     k_pos0 = static_cast<float>(p.k_rope_pos_offset[b]);
