@@ -309,8 +309,9 @@ int tvmkv_batch_tree_attn_scaled(const void* q, const int32_t* q_indptr, const v
  * (batch, h_q + 2 h_kv, d) tensor of the step, one new token per sequence.  The kernel reads q from it
  * and rotates it at q_rope_position[b] (apply_rope != 0: rotate-half RoPE with the default frequencies
  * theta^(-2i/d); 0: no rotation); the work items of every sequence's last chunk rotate the new k row the
- * same way and write it and the v row to slot append_position_map[b] (page * page_size + offset, -1 =
- * none) of `pages`, wait for those stores and then attend to the slot like to any cached token.  The
+ * same way, write it and the v row to slot append_position_map[b] (page * page_size + offset, -1 =
+ * none) of `pages` and attend to the token (the slot is the page table's last one; where it is another,
+ * they wait for their stores and attend to the pages as they then are).  The
  * page table must already cover the new token, i.e. the step appends before it attends
  * (paged_kv_cache.cc:990-997).  Results as tvmkv_batch_decode_paged_kv; the same head dims and page
  * sizes; a group of more than 16 query heads per kv head is served by work items of 32 heads. */

@@ -1106,6 +1106,36 @@ def test_fused_decode_step(hq, hkv, d, ps, apply_rope):
     assert_close(host(o1), host(o2), atol=2e-3, rtol=2e-3, what="fused step out vs two launches")
 
 
+@pytest.mark.parametrize("hq,hkv,d,ps", [(32, 8, 128, 16), (8, 2, 64, 32), (16, 8, 256, 16), (64, 1, 128, 16)])
+def test_fused_decode_step_into_other_slots(hq, hkv, d, ps):
+    """A slot that is not the last one of the page table is written before the launch attends to the pages; slot -1 leaves
+    the pool alone and attends to what it holds.  Sequences of one chunk: only the items that write read the slot."""
+    rng = np.random.default_rng(190 + hq + d)
+    kv_lens = [40, 17, 5, 100, 33]
+    b = len(kv_lens)
+    pages, ip, pv, last, _, _ = build_paged_kv(rng, kv_lens, 4 + sum((n + ps - 1) // ps for n in kv_lens), hkv, ps, d)
+    at = [3, -1, 0, 64, 31]
+    slots = np.array([-1 if t < 0 else pv[ip[i] + t // ps] * ps + t % ps for i, t in enumerate(at)], np.int32)
+    q_pos = np.array(kv_lens, np.int32) - 1
+    qkv = dev(rng.standard_normal((b, hq + 2 * hkv, d)).astype(F16))
+    z = i32(np.zeros(b, np.int32))
+    outs, pools = [], []
+    for fused in (True, False):
+        pool = dev(pages)
+        o, l = torch.zeros((b, hq, d), dtype=torch.float16, device=DEV), torch.zeros((b, hq), dtype=torch.float32, device=DEV)
+        if fused:
+            K.fused_decode_step(qkv, pool, i32(ip), i32(pv), i32(last), i32(q_pos), i32(slots), o, l, 1, 1.0, 1e4, d ** -0.5)
+        else:
+            q = torch.zeros((b, hq, d), dtype=torch.float16, device=DEV)
+            k, v = (torch.zeros((b, hkv, d), dtype=torch.float16, device=DEV) for _ in range(2))
+            K.fused_rope_append(qkv, i32(q_pos), q, k, v, 1, pool, i32(slots), 1.0, 1e4)
+            K.batch_decode_paged_kv(q, pool, i32(ip), i32(pv), i32(last), z, z, o, l, 0, 1.0, 1e4, d ** -0.5)
+        outs.append(host(o))
+        pools.append(pool)
+    assert torch.equal(*pools)
+    assert_close(outs[0], outs[1], atol=2e-3, rtol=2e-3, what="fused step out vs two launches")
+
+
 def test_decode_group_of_64_heads():
     """One kv head for 64 query heads: two work items of 32 heads per chunk; 16 kv heads x 64: the same at head dim 64."""
     for hq, hkv, d in ((64, 1, 128), (128, 2, 64)):

@@ -66,6 +66,11 @@ __device__ __forceinline__ float group_sum(float x) {
   return x;
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float x) {
+  return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true)));
+}
+
 // Reductions over the lane pairs (l, l ^ 32) and (l, l ^ 16) with the gfx950 lane-swap
 // instructions (vector ALU; a __shfl_xor goes through LDS and its latency).  With both operands
 // equal to x, v_permlane32_swap leaves x[l & 31] in one result and x[(l & 31) + 32] in the other
@@ -85,6 +90,15 @@ __device__ __forceinline__ float max_xor16(float x) {
 __device__ __forceinline__ float sum_xor16(float x) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Maximum over the wave, in every lane.
+__device__ __forceinline__ float wave_max(float x) {
+  x = dpp_max<kDppXor1>(x);
+  x = dpp_max<kDppXor2>(x);
+  x = dpp_max<kDppRowHalfMirror>(x);
+  x = dpp_max<kDppRowMirror>(x);
+  return max_xor32(max_xor16(x));
 }
 
 // ---- asynchronous global -> LDS copies, transposing LDS reads (gfx950) -----------------------
@@ -190,6 +204,18 @@ __device__ __forceinline__ void rope_pair(half8_t& lo, half8_t& hi, float pos_sc
     lo[i] = static_cast<half_t>(cs * xl + sn * (-xh));
     hi[i] = static_cast<half_t>(cs * xh + sn * xl);
   }
+}
+
+// One element of a rotated row, rounded once: the product of sn and other in fp32, then one fused multiply-add whose
+// result is rounded to fp16.  Spelled out for the kernels that write the same cached row by different routes, whose bits
+// must not depend on how the compiler contracts the expression.
+__device__ __forceinline__ half_t rope_element(float cs, half_t x, float sn, float other) {
+  const float product = sn * other;
+  uint32_t out;
+  asm("v_fma_mixlo_f16 %0, %1, %2, %3 op_sel_hi:[0,1,0]"
+      : "=v"(out)
+      : "v"(cs), "v"(static_cast<uint32_t>(__builtin_bit_cast(uint16_t, x))), "v"(product));
+  return __builtin_bit_cast(half_t, static_cast<uint16_t>(out));
 }
 
 // The table an attention kernel rotates q and k with (in-kernel RoPE, rotate-half pairing over the whole

@@ -63,7 +63,8 @@ struct DecodeParams {
   // fused step (decode_mfma_kernel<..., FUSED = true>): the launch does the split + RoPE + append of the
   // step's new token itself.  q is read from the fused (B, h_q + 2 h_kv, D) tensor and rotated at
   // q_rope_position[b]; the work items of a sequence's last chunk rotate its new k row, write it and the
-  // v row to slot append_slot[b] of the page pool, and then attend to them like to any cached token.
+  // v row to slot append_slot[b] of the page pool and attend to them as one more key (where the slot is not
+  // the page table's last one: in the pages, after the stores).
   const half_t* qkv;
   half_t* pages_rw;             // == pages
   const int32_t* append_slot;   // (B) page * page_size + offset, -1 = none
@@ -87,14 +88,15 @@ struct DecodeParams {
   float rope_magnitude;
 };
 
-// Same answer as find_sequence, computed by one wavefront as a 64-ary search: the lanes probe
-// slot_begin at 64 evenly spaced sequences of the range that is left, and because slot_begin is
+// Same answer as find_sequence for more than 64 sequences, computed by one wavefront as a 64-ary search: the lanes
+// probe slot_begin at 64 evenly spaced sequences of the range that is left, and because slot_begin is
 // increasing the number of lanes that qualify tells which sixty-fourth holds the answer.  One round
 // trip to memory per factor of 64 in the batch size (a linear scan in blocks of 64 sequences cost a
-// launch of 2048 sequences up to 32 dependent round trips per work item).
-__device__ __forceinline__ int find_sequence_wave(const int32_t* page_indptr, int batch, int cp, int slot,
-                                                  int lane) {
-  int lo = 0, n = batch;  // the answer lies in [lo, lo + n), and slot_begin(lo) <= slot
+// launch of 2048 sequences up to 32 dependent round trips per work item).  Returns the first of the (at most 64)
+// sequences that are left.
+__device__ __forceinline__ int narrow_sequences(const int32_t* page_indptr, int batch, int cp, int slot, int lane, int& n) {
+  int lo = 0;  // the answer lies in [lo, lo + n), and slot_begin(lo) <= slot
+  n = batch;
   while (n > 64) {
     const int stride = (n + 63) >> 6;
     const int idx = lo + lane * stride;
@@ -103,8 +105,7 @@ __device__ __forceinline__ int find_sequence_wave(const int32_t* page_indptr, in
     n = min(stride, lo + n - first);
     lo = first;
   }
-  const bool le = lane < n && slot_begin(page_indptr, lo + lane, cp) <= slot;
-  return lo + max(__popcll(__ballot(le)), 1) - 1;
+  return lo;
 }
 
 // Merge of the per-chunk partial states of one (sequence, query head) row by one wavefront.
@@ -119,8 +120,9 @@ __device__ __forceinline__ int find_sequence_wave(const int32_t* page_indptr, in
 __device__ __forceinline__ float load_partial(const float* ptr, bool coherent) {
   return coherent ? __hip_atomic_load(ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *ptr;
 }
-__device__ __forceinline__ void store_partial(float* ptr, float v) {
-  __hip_atomic_store(ptr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void store_partial2(float* ptr, float v0, float v1) {  // ptr: aligned to 8 bytes
+  const unsigned long long two = static_cast<unsigned long long>(__float_as_uint(v1)) << 32 | __float_as_uint(v0);
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(ptr), two, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // EPL consecutive floats of a partial output, with the widest loads that come as device-scope loads
@@ -156,46 +158,46 @@ __device__ __forceinline__ void merge_row(const DecodeParams& p, int b, int hq, 
   float acc[EPL];
 #pragma unroll
   for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
+  // The loads of a batch are all issued before the first is used: the merge is a chain of round trips
+  // to memory (device-scope loads do not hit in this XCD's L2), and what it costs is their number.  The first
+  // batch of outputs is on its way while the maxima come in and are reduced.
+  constexpr int BATCH = 16;  // (32 costs the main loop registers: 166 instead of 136, and 1.2 % of the decode rate)
+  const int64_t stride = static_cast<int64_t>(p.h_q) * D;
   for (int c0 = 0; c0 < nchunks; c0 += 64) {
     const int c = c0 + lane;
+    const int n_here = min(64, nchunks - c0);
+    const float* po = p.part_o + (static_cast<int64_t>(s0 + c0) * p.h_q + hq) * D + lane * EPL;
+    float part[BATCH][EPL];
+    auto load_batch = [&](int k0) {
+#pragma unroll
+      for (int k = 0; k < BATCH; ++k) load_partial_row<EPL, COHERENT>(po + min(k0 + k, n_here - 1) * stride, part[k]);
+    };
     float m_c = kNegInit, l_c = 0.f;
     if (c < nchunks) {
-      const float* ml = p.part_ml + (static_cast<int64_t>(s0 + c) * p.h_q + hq) * 2;
-      m_c = load_partial(ml, COHERENT);
-      l_c = load_partial(ml + 1, COHERENT);
+      float ml[2];
+      load_partial_row<2, COHERENT>(p.part_ml + (static_cast<int64_t>(s0 + c) * p.h_q + hq) * 2, ml);
+      m_c = ml[0];
+      l_c = ml[1];
     }
+    load_batch(0);
     float mx_new = m_c;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mx_new = fmaxf(mx_new, __shfl_xor(mx_new, off, 64));
-    mx_new = fmaxf(mx_new, mx);
+    mx_new = fmaxf(wave_max(mx_new), mx);
     const float rescale_old = fast_exp2(mx - mx_new);
     const float sc = fast_exp2(m_c - mx_new);
-    float lpart = l_c * sc;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) lpart += __shfl_xor(lpart, off, 64);
-    lsum = lsum * rescale_old + lpart;
+    lsum = lsum * rescale_old + sum_xor32(sum_xor16(group_sum<16>(l_c * sc)));
 #pragma unroll
     for (int e = 0; e < EPL; ++e) acc[e] *= rescale_old;
     mx = mx_new;
-    const int n_here = min(64, nchunks - c0);
-    const float* po = p.part_o + (static_cast<int64_t>(s0 + c0) * p.h_q + hq) * D + lane * EPL;
-    const int64_t stride = static_cast<int64_t>(p.h_q) * D;
-    // The loads of a batch are all issued before the first is used: the merge is a chain of round trips
-    // to memory (device-scope loads do not hit in this XCD's L2), and what it costs is their number.
-    constexpr int BATCH = 16;  // (32 costs the main loop registers: 166 instead of 136, and 1.2 % of the decode rate)
-    for (int k0 = 0; k0 < n_here; k0 += BATCH) {
-      float part[BATCH][EPL];
+    for (int k0 = 0;;) {
 #pragma unroll
       for (int k = 0; k < BATCH; ++k) {
-        const float* src = po + min(k0 + k, n_here - 1) * stride;
-        load_partial_row<EPL, COHERENT>(src, part[k]);
-      }
-#pragma unroll
-      for (int k = 0; k < BATCH; ++k) {
-        const float w = k0 + k < n_here ? __shfl(sc, min(k0 + k, 63), 64) : 0.f;
+        const float w = k0 + k < n_here ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sc), min(k0 + k, 63))) : 0.f;
 #pragma unroll
         for (int e = 0; e < EPL; ++e) acc[e] = fmaf(part[k][e], w, acc[e]);
       }
+      k0 += BATCH;
+      if (k0 >= n_here) break;
+      load_batch(k0);
     }
   }
   const float denom = lsum + fast_exp2(kNegInit - mx);
@@ -205,6 +207,17 @@ __device__ __forceinline__ void merge_row(const DecodeParams& p, int b, int hq, 
     if (lane * EPL + e < dm) out[e] = static_cast<half_t>(acc[e] * inv);
   }
   if (lane == 0) p.lse[row] = mx + fast_log2(denom);
+}
+
+// The append of the fused step: a pair of the new k row (elements i and i + D/2), rotated with the arithmetic of
+// fused_rope_kernel.
+__device__ __forceinline__ void rotate_new_pair(bool apply_rope, float pos_scaled, float divisor, half_t& lo, half_t& hi) {
+  if (!apply_rope) return;
+  const float freq = pos_scaled / divisor;
+  const float cs = cosf(freq), sn = sinf(freq);
+  const half_t x = lo, y = hi;
+  lo = rope_element(cs, x, sn, -static_cast<float>(y));
+  hi = rope_element(cs, y, sn, static_cast<float>(x));
 }
 
 // The empty-KV answer out = 0, lse = -5e4 (python/tvm/relax/frontend/nn/llm/_decode_kernels.py:129-130,173-176).
@@ -329,17 +342,12 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   __shared__ float sm_m[4][16];
   __shared__ float sm_l[4][16];
   __shared__ int sm_last;
+  __shared__ __attribute__((aligned(16))) half_t own_lds[FUSED ? 2 * D : 8];  // the new token's rotated k row and its v row
   constexpr bool RUNNING = EXT && !VARIANT;  // keys rotate by running angles, see below
   constexpr int TSTEP = KLINE ? 8 : 16;      // distance of a lane's neighbouring keys
   __shared__ __attribute__((aligned(16))) float rope_lds[RUNNING ? 5 : 1][RUNNING ? D / 2 : 1];
 
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
-  const int c16 = lane & 15;   // MFMA column (query head in group) / A-row (token) / V feature piece
-  const int g4 = lane >> 4;    // lane group 0..3
   const int cp = p.chunk_pages;
-  half_t* Vt = Vt_all[wave];
   const int psh = p.page_shift;  // a page of the table is 1 << psh of the 16-token pages the steps consume
   const int64_t head_stride = static_cast<int64_t>(PS << psh) * dm;
 
@@ -348,53 +356,38 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   constexpr int HPI = 16 * HB;  // query heads per work item
   const int head_blocks = (group + HPI - 1) / HPI;
   for (int item = blockIdx.x; item < num_items; item += gridDim.x) {
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // what is formed from it belongs to an item: kept for the next one, it spills
+  const int wave = tid >> 6;
+  const int lane = tid & 63;
+  const int c16 = lane & 15;   // MFMA column (query head in group) / A-row (token) / V feature piece
+  const int g4 = lane >> 4;    // lane group 0..3
+  half_t* Vt = Vt_all[wave];
   const int slot = item / (p.h_kv * head_blocks);
   const int rest = item - slot * (p.h_kv * head_blocks);
   const int kvh = rest / head_blocks;
   const int hb = rest - kvh * head_blocks;
   const int hq0 = kvh * group + hb * HPI;      // first query head of this item
   const int heads = min(HPI, group - hb * HPI);  // and how many
-  const int b = find_sequence_wave(p.page_indptr, p.batch_size, cp, slot, lane);
-  const int npages = p.page_indptr[b + 1] - p.page_indptr[b];
-  const int pbeg = SELF && p.page_begin != nullptr ? p.page_begin[b] : p.page_indptr[b];
-  const int token = SELF && p.rows != nullptr ? p.rows[b] : b;  // of q and the output
-  const int chunk = slot - slot_begin(p.page_indptr, b, cp);
-  const int nchunks = SELF ? max(1, (npages + cp - 1) / cp) : (npages + cp - 1) / cp;
-  if (chunk >= nchunks) {  // spare slot (uniform over the workgroup)
-    if (p.arrivals != nullptr && npages == 0 && chunk == 0) {  // a sequence without pages: nobody else answers for it
-      for (int g = wave; g < heads; g += 4) empty_row<D>(p, b, hq0 + g, lane);
+  // Divisors of the angles: loads that wait for nothing, in front of all others.  (Loads complete in order: what the
+  // rotations need has to be on its way before the first step's K/V rows, or it is there no sooner than they are.)
+  constexpr int NA = 4 * KS;               // fused step: angles a lane needs
+  constexpr int PER_LANE = (NA + 15) / 16;  // and how many it computes (head dim 256: two), see below
+  constexpr int OWN_PAIRS = (D / 2 + 63) / 64;  // pairs of the new k row per lane
+  float angle_div[FUSED ? PER_LANE : 1], own_div[FUSED ? OWN_PAIRS : 1];
+  if constexpr (FUSED) {
+    if (p.apply_rope) {
+#pragma unroll
+      for (int r = 0; r < PER_LANE; ++r) {
+        const int mine = min(r * 16 + c16, NA - 1);
+        angle_div[r] = div.v[(mine >> 3) * 32 + g4 * 8 + (mine & 7)];
+      }
+#pragma unroll
+      for (int r = 0; r < OWN_PAIRS; ++r) own_div[r] = div.v[min(r * 64 + lane, D / 2 - 1)];
     }
-    continue;
   }
-  const int kv_len = (npages - 1) * (PS << psh) + p.last_page_len[b];  // physical end of the cached tokens
-  // the chunk's 16-token pages (chunks are counted in pages of the table; the last one may be partly filled)
-  const int page_lo = (chunk * cp) << psh;
-  const int page_hi = min(min(chunk * cp + cp, npages) << psh, (kv_len + PS - 1) / PS);
-  // physical token t is attended to iff t < sink or win_lo <= t < kv_len
-  const int sink = EXT && p.sink_size != nullptr ? p.sink_size[b] : 0;
-  const int win_lo = EXT && p.window_offset != nullptr ? p.window_offset[b] : 0;
-  // RoPE divisors of the first halves of this lane's K fragment pairs: features i*32 + g4*8 + e, or
-  // with KLINE i*64 + (c16&1)*32 + g4*8 + e
-  // (and of the second halves, features + D/2, which differ from the first in some frequency variants)
-  auto pair_feature = [&](int i) {
-    return KLINE ? (i >> 3) * 64 + (c16 & 1) * 32 + g4 * 8 + (i & 7) : (i >> 3) * 32 + g4 * 8 + (i & 7);
-  };
-  float divr[VARIANT ? 8 * NPAIR : 1], divh[VARIANT ? 8 * NPAIR : 1];
-  float run_cos[RUNNING ? 8 * NPAIR : 1], run_sin[RUNNING ? 8 * NPAIR : 1];
-  float k_pos0 = 0.f;
-  // Angles of the keys.  A lane's keys of a step are TSTEP tokens apart and have the same frequencies, so one sine and
-  // cosine per frequency and work item are enough: the next keys' and the next step's come by rotating (run_cos,
-  // run_sin) by fixed angles.  A division, a reduction and two transcendentals for each of a lane's 32 (key, frequency)
-  // pairs of a step kept the vector ALU busy for longer than the step's 16 KiB take to arrive (64 sequences with
-  // windows of 4096 tokens, 32 / 8 heads of dim 128: 247 us a layer, 206 now).  The fixed angles come from the host in
-  // double and are rounded once, so that the error of (cos, sin) grows with the 63 rotations of the longest chunk to
-  // 19 x 2^-24 at head dim 64 and 34 x 2^-24 at 128 and 256 (2^-19; an fp32 angle is off by as much from position 70 on,
-  // and the rotated row is rounded at 2^-11).  They wait in LDS: in registers they made every extended launch of head
-  // dim 128 spill.
-  const bool k_rotary = EXT && (SELF ? p.rotary == 1 : p.rotary != 0);
-  if (k_rotary) {
-    k_pos0 = static_cast<float>(p.k_rope_pos_offset[b]);
-    if constexpr (RUNNING) {
+  if constexpr (RUNNING) {
+    if (p.rotary) {
       if (tid < D / 2) {
         rope_lds[0][tid] = div.v[tid];
         rope_lds[1][tid] = div.near_cos[tid];
@@ -404,177 +397,151 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
       }
       __syncthreads();
     }
-    const int first = (page_lo + 2 * wave) * PS + (KLINE ? c16 >> 1 : c16);
-    const float pos = (k_pos0 + static_cast<float>(first - win_lo + sink)) * p.rope_scale;
-#pragma unroll
-    for (int i = 0; i < 8 * NPAIR; ++i) {
-      if constexpr (RUNNING) {
-        sincos_reduced(pos / rope_lds[0][pair_feature(i)], run_sin[i], run_cos[i]);
-      } else {
-        divr[i] = div.v[pair_feature(i)];
-        divh[i] = div.v[pair_feature(i) + D / 2];
-      }
-    }
   }
+  // The sequence of the slot and what the arrays hold for it, by one round trip to memory: a lane per sequence.
+  int left;
+  const int lo = narrow_sequences(p.page_indptr, p.batch_size, cp, slot, lane, left);
+  const int at = lo + min(lane, left - 1);
+  const int page_beg = p.page_indptr[at], page_end = p.page_indptr[at + 1], last_len = p.last_page_len[at];
+  const int append_at = FUSED ? p.append_slot[at] : -1;
+  const int position_at = FUSED && p.apply_rope ? p.q_rope_position[at] : 0;
+  const int sink_at = EXT && p.sink_size != nullptr ? p.sink_size[at] : 0;
+  const int window_at = EXT && p.window_offset != nullptr ? p.window_offset[at] : 0;
+  const bool k_rotary = EXT && (SELF ? p.rotary == 1 : p.rotary != 0);
+  const int k_position_at = k_rotary ? p.k_rope_pos_offset[at] : 0;
+  const int row_at = SELF && p.rows != nullptr ? p.rows[at] : at;
+  const int begin_at = SELF && p.page_begin != nullptr ? p.page_begin[at] : page_beg;
+  const int slot_at = page_beg / cp + at;  // slot_begin
+  const int hit = max(static_cast<int>(__popcll(__ballot(lane < left && slot_at <= slot))), 1) - 1;
+  const int b = lo + hit;
+  const int npages = __builtin_amdgcn_readlane(page_end, hit) - __builtin_amdgcn_readlane(page_beg, hit);
+  const int pbeg = __builtin_amdgcn_readlane(begin_at, hit);
+  const int token = __builtin_amdgcn_readlane(row_at, hit);  // of q and the output
+  const int chunk = slot - __builtin_amdgcn_readlane(slot_at, hit);
+  const int nchunks = SELF ? max(1, (npages + cp - 1) / cp) : (npages + cp - 1) / cp;
+  if (chunk >= nchunks) {  // spare slot (uniform over the workgroup)
+    if (p.arrivals != nullptr && npages == 0 && chunk == 0) {  // a sequence without pages: nobody else answers for it
+      for (int g = wave; g < heads; g += 4) empty_row<D>(p, b, hq0 + g, lane);
+    }
+    continue;
+  }
+  // physical end of the cached tokens
+  int kv_len = (npages - 1) * (PS << psh) + __builtin_amdgcn_readlane(last_len, hit);
 
-  // The fused step's append: every work item of the sequence's last chunk writes the new token's k row
-  // (rotated with the precise sinf / cosf, the arithmetic of fused_rope_kernel) and v row of its kv head
-  // to the page slot, waits until the stores have completed and meets the other waves at a barrier.  All
-  // K/V loads of this workgroup come after that, through the same vector cache and L2 as the stores; the
-  // items of other head blocks of the same kv head write the same bytes.  The loads of the append are
-  // issued here, its arithmetic and stores follow the q fragments below, whose loads are in flight beside them.
+  // The fused step's append belongs to the work items of every sequence's last chunk.  The new token is the last one of
+  // the page table: its rows are written to their slot and attended to from registers (the wave that has least to do
+  // does it, under the other waves' loads), nothing waits for the stores.  Through the pages -- rotate, store, wait,
+  // barrier, then load -- it was 0.6 us of a work item's 11, in front of its first K/V load.
   const bool appends = FUSED && chunk == nchunks - 1;
-  int32_t aslot = -1;
-  float app_xl = 0.f, app_xh = 0.f;
-  Vec16 app_v = zero16();
-  if (appends) {
-    aslot = p.append_slot[b];
-    const half_t* krow = p.qkv + (static_cast<int64_t>(b) * (p.h_q + 2 * p.h_kv) + p.h_q + kvh) * D;
-    if (tid < D / 2) {
-      app_xl = static_cast<float>(krow[tid]);
-      app_xh = static_cast<float>(krow[tid + D / 2]);
-    } else if (tid >= 128 && tid < 128 + D / 8) {
-      app_v = ld16(krow + static_cast<int64_t>(p.h_kv) * D + (tid - 128) * 8);
-    }
-  }
+  const int32_t aslot = appends ? __builtin_amdgcn_readlane(append_at, hit) : -1;
+  bool own = SELF && chunk == nchunks - 1;  // the new token is one more key of this item
+  const int last_page = FUSED && appends ? p.page_values[pbeg + npages - 1] : 0;
+  // the chunk's 16-token pages (chunks are counted in pages of the table; the last one may be partly filled)
+  const int page_lo = (chunk * cp) << psh;
+  int page_hi = min(min(chunk * cp + cp, npages) << psh, (kv_len + PS - 1) / PS);
 
-  // The fused step rotates q itself.  A lane needs the angles of its 8 * KS/2 feature pairs, the same
-  // for every head and so for the 16 lanes of its group: each lane computes ONE of them (pair
-  // (i / 8) * 32 + g4 * 8 + i % 8 for i = c16, and i = 16 + c16 at head dim 256; spare lanes repeat one) and
-  // the group shares them through lane shuffles -- a twentieth of the sin / cos work of every lane
-  // computing all of its own.
-  constexpr int NA = 4 * KS;               // angles a lane needs
-  constexpr int PER_LANE = (NA + 15) / 16;  // angles a lane computes (head dim 256: two)
-  float rope_sn[PER_LANE], rope_cs[PER_LANE];
-  if (FUSED && p.apply_rope) {
-    const float q_pos = static_cast<float>(p.q_rope_position[b]) * p.rope_scale;
+  // Page ids of a step's two pages; a missing second page repeats the first.  Those of the first step are on their way
+  // beside the q rows.  The following ones come beside the K/V rows of the step before (IDS_AHEAD) in the extended
+  // kernels, whose steps are long: two layers' windows of 64 sequences 207 -> 192 us.  The plain kernel loads them in
+  // front of each step's rows: with more loads in flight it is slower (64 sequences of 1024-8192 tokens 206.7 -> 210 us).
+  constexpr bool IDS_AHEAD = EXT;
+  const int first_page = page_lo + 2 * wave;
+  int ids[2] = {0, 0};
+  auto load_ids = [&](int pi) {
 #pragma unroll
-    for (int r = 0; r < PER_LANE; ++r) {
-      const int mine = min(r * 16 + c16, NA - 1);
-      sincos_reduced(q_pos / div.v[(mine >> 3) * 32 + g4 * 8 + (mine & 7)], rope_sn[r], rope_cs[r]);
-    }
-  }
-
-  // Q^T fragments (B operand): column = head c16 of block j of the item, contraction slots = 8 features.
-  half8_t qf[HB][KS];
+    for (int h = 0; h < 2; ++h) ids[h] = p.page_values[pbeg + (min(pi + h, page_hi - 1) >> psh)];
+  };
+  if (first_page < page_hi) load_ids(first_page);
+  // q rows, B operand fragments: column = head c16 of block j of the item, contraction slots = 8 features
+  Vec16 qv[HB][KS];
 #pragma unroll
   for (int j = 0; j < HB; ++j) {
     const bool head_valid = j * 16 + c16 < heads;
     const half_t* qrow = SELF ? p.q + token * p.q_stride + (hq0 + j * 16 + c16) * D + g4 * 8
                          : FUSED ? p.qkv + (static_cast<int64_t>(b) * (p.h_q + 2 * p.h_kv) + hq0 + j * 16 + c16) * D + g4 * 8
                                : p.q + (static_cast<int64_t>(b) * p.h_q + hq0 + j * 16 + c16) * dm + g4 * 8;
-    Vec16 qv[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qv[ks] = (head_valid && (!PAD || ks * 32 + g4 * 8 < dm)) ? ld16(qrow + ks * 32) : zero16();
-    if (FUSED && p.apply_rope) {
-      // the arithmetic of rope_pair with the shared angles: fp32, one rounding to fp16
-#pragma unroll
-      for (int ks = 0; ks < KS / 2; ++ks) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int i = ks * 8 + e;  // angle i sits in lane i % 16 of this lane's group
-          const float cs = __shfl(rope_cs[i / 16], (lane & 48) + (i & 15), 64);
-          const float sn = __shfl(rope_sn[i / 16], (lane & 48) + (i & 15), 64);
-          const float xl = static_cast<float>(qv[ks].h8[e]);
-          const float xh = static_cast<float>(qv[ks + KS / 2].h8[e]);
-          qv[ks].h8[e] = static_cast<half_t>(cs * xl + sn * (-xh));
-          qv[ks + KS / 2].h8[e] = static_cast<half_t>(cs * xh + sn * xl);
-        }
-      }
-    }
-    if (EXT && p.rotary) {
-      // feature f < D/2 rotates with f + D/2: k-step ks with ks + KS/2
-      const float q_pos = static_cast<float>(p.q_rope_position[token]) * p.rope_scale;
-#pragma unroll
-      for (int ks = 0; ks < KS / 2; ++ks) {
-        float qdiv[8], qdivh[VARIANT ? 8 : 1];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          qdiv[e] = div.v[ks * 32 + g4 * 8 + e];
-          if constexpr (VARIANT) qdivh[e] = div.v[D / 2 + ks * 32 + g4 * 8 + e];
-        }
-        if constexpr (VARIANT) {
-          rope_pair_ex(qv[ks].h8, qv[ks + KS / 2].h8, q_pos, qdiv, qdivh, p.rope_inverse, p.rope_halves_differ, p.rope_magnitude);
-        } else {
-          rope_pair(qv[ks].h8, qv[ks + KS / 2].h8, q_pos, qdiv);
-        }
-      }
-    }
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[j][ks] = qv[ks].h8;
+    for (int ks = 0; ks < KS; ++ks) qv[j][ks] = (head_valid && (!PAD || ks * 32 + g4 * 8 < dm)) ? ld16(qrow + ks * 32) : zero16();
   }
-  if (appends) {
-    if (aslot >= 0) {
-      const int page_tokens = PS << psh;
-      half_t* kdst = p.pages_rw + (static_cast<int64_t>(aslot / page_tokens) * 2 * p.h_kv + kvh) * head_stride +
-                     (aslot % page_tokens) * D;
-      half_t* vdst = kdst + static_cast<int64_t>(p.h_kv) * head_stride;
-      if (tid < D / 2) {
-        if (p.apply_rope) {
-          const float freq = static_cast<float>(p.q_rope_position[b]) * p.rope_scale / div.v[tid];
-          const float cs = cosf(freq), sn = sinf(freq);
-          kdst[tid] = static_cast<half_t>(cs * app_xl + sn * (-app_xh));
-          kdst[tid + D / 2] = static_cast<half_t>(cs * app_xh + sn * app_xl);
-        } else {
-          kdst[tid] = static_cast<half_t>(app_xl);
-          kdst[tid + D / 2] = static_cast<half_t>(app_xh);
-        }
-      } else if (tid >= 128 && tid < 128 + D / 8) {
-        st16(vdst + (tid - 128) * 8, app_v);
+  const float q_position = FUSED ? static_cast<float>(__builtin_amdgcn_readlane(position_at, hit))
+                           : EXT && p.rotary ? static_cast<float>(p.q_rope_position[token]) : 0.f;
+  // the new token's rows: FUSED pair by pair (k) and 16 bytes a lane (v), SELF as the fragments of k and the features of v
+  // that meet this lane's in O
+  half_t own_lo[FUSED ? OWN_PAIRS : 1], own_hi[FUSED ? OWN_PAIRS : 1];
+  Vec16 own_v;
+  Vec16 kn[KS];
+  half4_t vn[SELF ? DB : 1];
+  // loaded in front of the K/V rows, where the registers are there for it (behind them the wide items and head dim 256
+  // wait, in front of them they spill 31-39 registers)
+  constexpr bool OWN_EARLY = HB == 1 && D <= 128;
+  auto load_own = [&]() {
+    const half_t* knew = p.k_new + token * p.new_stride + static_cast<int64_t>(kvh) * D;
+    const half_t* vnew = p.v_new + token * p.new_stride + static_cast<int64_t>(kvh) * D;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) kn[ks] = ld16(knew + ks * 32 + g4 * 8);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) vn[db] = *reinterpret_cast<const half4_t*>(vnew + db * 16 + 4 * g4);
+  };
+  if (FUSED && aslot >= 0 && wave == 3) {
+    const half_t* k_row = p.qkv + (static_cast<int64_t>(b) * (p.h_q + 2 * p.h_kv) + p.h_q + kvh) * D;
+#pragma unroll
+    for (int r = 0; r < OWN_PAIRS; ++r) {
+      const int i = min(r * 64 + lane, D / 2 - 1);
+      own_lo[r] = k_row[i];
+      own_hi[r] = k_row[i + D / 2];
+    }
+    own_v = ld16(k_row + static_cast<int64_t>(p.h_kv) * D + min(lane, D / 8 - 1) * 8);
+  }
+  if constexpr (SELF && OWN_EARLY) {
+    if (own && wave == 3) load_own();  // the wave with the fewest steps
+  }
+  // The fused step rotates q itself.  A lane needs the angles of its 8 * KS/2 feature pairs, the same
+  // for every head and so for the 16 lanes of its group: each lane computes ONE of them (pair
+  // (i / 8) * 32 + g4 * 8 + i % 8 for i = c16, and i = 16 + c16 at head dim 256; spare lanes repeat one) and
+  // the group shares them through lane shuffles -- a twentieth of the sin / cos work of every lane
+  // computing all of its own.
+  float rope_sn[PER_LANE], rope_cs[PER_LANE];
+  if (FUSED && p.apply_rope) {
+#pragma unroll
+    for (int r = 0; r < PER_LANE; ++r) sincos_reduced(q_position * p.rope_scale / angle_div[r], rope_sn[r], rope_cs[r]);
+  }
+  // The new k row, rotated, and the v row: to LDS (own_lds[0..D): k, [D..2D): v) and to the page slot.  One wave.
+  auto append_new_token = [&]() {
+#pragma unroll
+    for (int r = 0; r < OWN_PAIRS; ++r) {
+      const int i = r * 64 + lane;
+      rotate_new_pair(p.apply_rope, q_position * p.rope_scale, own_div[r], own_lo[r], own_hi[r]);
+      if (i < D / 2) {
+        own_lds[i] = own_lo[r];
+        own_lds[i + D / 2] = own_hi[r];
       }
     }
+    if (lane < D / 8) st16(own_lds + D + lane * 8, own_v);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int page_tokens = PS << psh;
+    half_t* kdst = p.pages_rw + (static_cast<int64_t>(aslot / page_tokens) * 2 * p.h_kv + kvh) * head_stride + (aslot % page_tokens) * D;
+    if (lane < 2 * (D / 8)) {
+      const int kv = lane / (D / 8), piece = lane % (D / 8);
+      st16(kdst + static_cast<int64_t>(kv) * p.h_kv * head_stride + piece * 8, ld16(own_lds + kv * D + piece * 8));
+    }
+  };
+  if (FUSED && aslot >= 0) {
+    const int page_tokens = PS << psh;
+    own = aslot == __builtin_amdgcn_readfirstlane(last_page) * page_tokens + (kv_len - 1) % page_tokens;
+    if (own) {
+      page_hi = min(page_hi, (--kv_len + PS - 1) / PS);
+      if (first_page + 1 >= page_hi) ids[1] = ids[0];  // the second page held the new token alone
+    }
+  }
+  if (FUSED && aslot >= 0 && !own) {  // not the last slot of the page table: append, then attend to the pages as they are
+    if (wave == 3) append_new_token();
     wait_vmcnt<0>();
     __syncthreads();
   }
-  float4_t o[HB][DB];
-#pragma unroll
-  for (int j = 0; j < HB; ++j) {
-#pragma unroll
-    for (int db = 0; db < DB; ++db) o[j][db] = float4_t{0.f, 0.f, 0.f, 0.f};
-  }
-  float m[HB], lsum[HB];
-#pragma unroll
-  for (int j = 0; j < HB; ++j) {
-    m[j] = kNegInit;
-    lsum[j] = 0.f;
-  }
-
-  if (SELF && wave == 0 && chunk == nchunks - 1) {
-    const half_t* knew = p.k_new + token * p.new_stride + static_cast<int64_t>(kvh) * D;
-    const half_t* vnew = p.v_new + token * p.new_stride + static_cast<int64_t>(kvh) * D;
-    Vec16 kn[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kn[ks] = ld16(knew + ks * 32 + g4 * 8);
-    if (k_rotary) {  // at the position of its query
-      const float pos = static_cast<float>(p.q_rope_position[token]) * p.rope_scale;
-#pragma unroll
-      for (int ks = 0; ks < KS / 2; ++ks) {
-        float kdiv[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) kdiv[e] = div.v[ks * 32 + g4 * 8 + e];
-        rope_pair(kn[ks].h8, kn[ks + KS / 2].h8, pos, kdiv);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < HB; ++j) {
-      float dot = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) dot = fmaf(static_cast<float>(qf[j][ks][e]), static_cast<float>(kn[ks].h8[e]), dot);
-      }
-      const float score = sum_xor32(sum_xor16(dot)) * p.scale_log2;  // of head c16, in all four lane groups
-      m[j] = fmaxf(kNegInit, score);
-      const float weight = fast_exp2(score - m[j]);
-      lsum[j] = g4 == 0 ? weight : 0.f;  // the lane groups' sums are added at the end
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[j][db][e] = weight * static_cast<float>(vnew[db * 16 + 4 * g4 + e]);
-      }
-    }
-  }
-
+  // physical token t is attended to iff t < sink or win_lo <= t < kv_len
+  const int sink = EXT ? __builtin_amdgcn_readlane(sink_at, hit) : 0;
+  const int win_lo = EXT ? __builtin_amdgcn_readlane(window_at, hit) : 0;
   // V^T fragment via the transposing read: lane li of a 16-lane group points at 4 features of token
   // (li >> 2) of the group's 4 tokens and receives feature li of the group's 16 for the 4 tokens
   const uint32_t vt_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)Vt));
@@ -607,7 +574,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int pg = min(pi + h, page_hi - 1);
-      const int page = __builtin_amdgcn_readfirstlane(p.page_values[pbeg + (pg >> psh)]);
+      const int page = __builtin_amdgcn_readfirstlane(IDS_AHEAD || pi == first_page ? ids[h] : p.page_values[pbeg + (pg >> psh)]);
       const half_t* kbase = p.pages + (static_cast<int64_t>(page) * 2 * p.h_kv + kvh) * head_stride +
                             __builtin_amdgcn_readfirstlane(pg & ((1 << psh) - 1)) * (PS * dm);
       const half_t* vbase = kbase + static_cast<int64_t>(p.h_kv) * head_stride;
@@ -638,6 +605,142 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
       }
     }
   };
+  // The first step's rows are on their way while q and the new token are rotated.
+  Regs ra;
+#pragma unroll
+  for (int j = 0; j < HB; ++j) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qv[j][ks].h8));  // arrived: no wait for them behind the K/V loads
+  }
+  if (first_page < page_hi) {
+    issue(first_page, ra);
+    if (IDS_AHEAD) load_ids(first_page + 8);
+  }
+
+  // RoPE divisors of the first halves of this lane's K fragment pairs: features i*32 + g4*8 + e, or
+  // with KLINE i*64 + (c16&1)*32 + g4*8 + e
+  // (and of the second halves, features + D/2, which differ from the first in some frequency variants)
+  auto pair_feature = [&](int i) {
+    return KLINE ? (i >> 3) * 64 + (c16 & 1) * 32 + g4 * 8 + (i & 7) : (i >> 3) * 32 + g4 * 8 + (i & 7);
+  };
+  float divr[VARIANT ? 8 * NPAIR : 1], divh[VARIANT ? 8 * NPAIR : 1];
+  float run_cos[RUNNING ? 8 * NPAIR : 1], run_sin[RUNNING ? 8 * NPAIR : 1];
+  float k_pos0 = 0.f;
+  // Angles of the keys.  A lane's keys of a step are TSTEP tokens apart and have the same frequencies, so one sine and
+  // cosine per frequency and work item are enough: the next keys' and the next step's come by rotating (run_cos,
+  // run_sin) by fixed angles.  A division, a reduction and two transcendentals for each of a lane's 32 (key, frequency)
+  // pairs of a step kept the vector ALU busy for longer than the step's 16 KiB take to arrive (64 sequences with
+  // windows of 4096 tokens, 32 / 8 heads of dim 128: 247 us a layer, 206 now).  The fixed angles come from the host in
+  // double and are rounded once, so that the error of (cos, sin) grows with the 63 rotations of the longest chunk to
+  // 19 x 2^-24 at head dim 64 and 34 x 2^-24 at 128 and 256 (2^-19; an fp32 angle is off by as much from position 70 on,
+  // and the rotated row is rounded at 2^-11).  They wait in LDS: in registers they made every extended launch of head
+  // dim 128 spill.
+  if (k_rotary) {
+    k_pos0 = static_cast<float>(__builtin_amdgcn_readlane(k_position_at, hit));
+    const int first = (page_lo + 2 * wave) * PS + (KLINE ? c16 >> 1 : c16);
+    const float pos = (k_pos0 + static_cast<float>(first - win_lo + sink)) * p.rope_scale;
+#pragma unroll
+    for (int i = 0; i < 8 * NPAIR; ++i) {
+      if constexpr (RUNNING) {
+        sincos_reduced(pos / rope_lds[0][pair_feature(i)], run_sin[i], run_cos[i]);
+      } else {
+        divr[i] = div.v[pair_feature(i)];
+        divh[i] = div.v[pair_feature(i) + D / 2];
+      }
+    }
+  }
+
+  // Q^T fragments
+  half8_t qf[HB][KS];
+#pragma unroll
+  for (int j = 0; j < HB; ++j) {
+    if (FUSED && p.apply_rope) {
+      // the arithmetic of rope_pair with the shared angles: fp32, one rounding to fp16
+#pragma unroll
+      for (int ks = 0; ks < KS / 2; ++ks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int i = ks * 8 + e;  // angle i sits in lane i % 16 of this lane's group
+          const float cs = __shfl(rope_cs[i / 16], (lane & 48) + (i & 15), 64);
+          const float sn = __shfl(rope_sn[i / 16], (lane & 48) + (i & 15), 64);
+          const float xl = static_cast<float>(qv[j][ks].h8[e]);
+          const float xh = static_cast<float>(qv[j][ks + KS / 2].h8[e]);
+          qv[j][ks].h8[e] = static_cast<half_t>(cs * xl + sn * (-xh));
+          qv[j][ks + KS / 2].h8[e] = static_cast<half_t>(cs * xh + sn * xl);
+        }
+      }
+    }
+    if (EXT && p.rotary) {
+      // feature f < D/2 rotates with f + D/2: k-step ks with ks + KS/2
+      const float q_pos = q_position * p.rope_scale;
+#pragma unroll
+      for (int ks = 0; ks < KS / 2; ++ks) {
+        float qdiv[8], qdivh[VARIANT ? 8 : 1];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          qdiv[e] = RUNNING ? rope_lds[0][ks * 32 + g4 * 8 + e] : div.v[ks * 32 + g4 * 8 + e];
+          if constexpr (VARIANT) qdivh[e] = div.v[D / 2 + ks * 32 + g4 * 8 + e];
+        }
+        if constexpr (VARIANT) {
+          rope_pair_ex(qv[j][ks].h8, qv[j][ks + KS / 2].h8, q_pos, qdiv, qdivh, p.rope_inverse, p.rope_halves_differ, p.rope_magnitude);
+        } else {
+          rope_pair(qv[j][ks].h8, qv[j][ks + KS / 2].h8, q_pos, qdiv);
+        }
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[j][ks] = qv[j][ks].h8;
+  }
+  float4_t o[HB][DB];
+#pragma unroll
+  for (int j = 0; j < HB; ++j) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db) o[j][db] = float4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  float m[HB], lsum[HB];
+#pragma unroll
+  for (int j = 0; j < HB; ++j) {
+    m[j] = kNegInit;
+    lsum[j] = 0.f;
+  }
+
+  if (own && wave == 3) {
+    if constexpr (FUSED) {
+      append_new_token();
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kn[ks] = ld16(own_lds + ks * 32 + g4 * 8);
+    }
+    if constexpr (SELF && !OWN_EARLY) load_own();
+    if (SELF && k_rotary) {  // at the position of its query
+      const float pos = q_position * p.rope_scale;
+#pragma unroll
+      for (int ks = 0; ks < KS / 2; ++ks) {
+        float kdiv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) kdiv[e] = rope_lds[0][ks * 32 + g4 * 8 + e];
+        rope_pair(kn[ks].h8, kn[ks + KS / 2].h8, pos, kdiv);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < HB; ++j) {
+      float dot = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = fmaf(static_cast<float>(qf[j][ks][e]), static_cast<float>(kn[ks].h8[e]), dot);
+      }
+      const float score = sum_xor32(sum_xor16(dot)) * p.scale_log2;  // of head c16, in all four lane groups
+      m[j] = fmaxf(kNegInit, score);
+      const float weight = fast_exp2(score - m[j]);
+      lsum[j] = g4 == 0 ? weight : 0.f;  // the lane groups' sums are added at the end
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const half4_t v4 = SELF ? vn[SELF ? db : 0] : *reinterpret_cast<const half4_t*>(own_lds + D + db * 16 + 4 * g4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[j][db][e] = weight * static_cast<float>(v4[e]);
+      }
+    }
+  }
 
   auto consume = [&](int pi, Regs& r) {
     // wave-uniform: some token of the two pages is not attended to (end of the sequence, evicted)
@@ -788,10 +891,12 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   // No software pipelining: three waves per SIMD (twelve per CU, each with 16 KiB of loads in
   // flight while it waits) hide the load latency; four per SIMD measured 4 % slower (more page
   // streams at once than the memory system likes), two about the same.
-  Regs ra;
-  for (int pi = page_lo + 2 * wave; pi < page_hi; pi += 8) {
-    issue(pi, ra);
+  for (int pi = first_page; pi < page_hi;) {
     consume(pi, ra);
+    pi += 8;
+    if (pi >= page_hi) break;
+    issue(pi, ra);
+    if (IDS_AHEAD) load_ids(pi + 8);
   }
 
   // ---- merge the 4 waves through LDS, one head block at a time: o[j][db][e] is feature db*16 + 4*g4 + e
@@ -803,41 +908,47 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
     // the row sums are per lane group: add them up; m is already common
     const float lrow = sum_xor32(sum_xor16(lsum[j]));
     float* sm_o_w = reinterpret_cast<float*>(Vt_all[wave]);
+    const int heads_here = min(16, heads - j * 16);
+    // runs of 4 features, run r of head g at position r ^ (g & 7): rows of whole bank lines, written a head per lane,
+    // met in the same banks (1.1 us of a small launch's 11 together with the sums below in two rounds)
+    int place_of = (g4 ^ (c16 & 7)) * 4;  // of run g4; formed here, not kept in registers through the main loop
+    asm volatile("" : "+v"(place_of));
+    if (c16 < heads_here) {
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sm_o_w[c16 * D + db * 16 + 4 * g4 + e] = o[j][db][e];
+      for (int db = 0; db < DB; ++db) *reinterpret_cast<float4_t*>(sm_o_w + c16 * D + (place_of ^ (db * 16))) = o[j][db];
     }
     if (g4 == 0) {
       sm_m[wave][c16] = m[j];
       sm_l[wave][c16] = lrow;
     }
     __syncthreads();
-    const int heads_here = min(16, heads - j * 16);
-    for (int idx = tid; idx < heads_here * D; idx += 256) {
-      const int g = idx / D;
-      const int d = idx % D;
+    for (int idx = tid; idx < heads_here * (D / 2); idx += 256) {
+      const int g = idx / (D / 2);
+      const int d = idx % (D / 2) * 2;
+      const int place = g * D + (((d >> 2) ^ (g & 7)) << 2) + (d & 3);
       float mx = sm_m[0][g];
 #pragma unroll
       for (int w = 1; w < 4; ++w) mx = fmaxf(mx, sm_m[w][g]);
-      float lt = 0.f, acc = 0.f;
+      float lt = 0.f, acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
         const float sc = fast_exp2(sm_m[w][g] - mx);
+        const float* two = reinterpret_cast<const float*>(Vt_all[w]) + place;
         lt += sm_l[w][g] * sc;
-        acc += reinterpret_cast<const float*>(Vt_all[w])[g * D + d] * sc;
+        acc0 += two[0] * sc;
+        acc1 += two[1] * sc;
       }
       const int hq = hq0 + j * 16 + g;
       if (single_chunk) {
         const float denom = lt + fast_exp2(kNegInit - mx);
-        if (!PAD || d < dm) p.output[(static_cast<int64_t>(token) * p.h_q + hq) * dm + d] = static_cast<half_t>(acc / denom);
+        if (!PAD || d < dm) {
+          *reinterpret_cast<half2_t*>(p.output + (static_cast<int64_t>(token) * p.h_q + hq) * dm + d) =
+              half2_t{static_cast<half_t>(acc0 / denom), static_cast<half_t>(acc1 / denom)};
+        }
         if (d == 0) p.lse[static_cast<int64_t>(token) * p.h_q + hq] = mx + fast_log2(denom);
       } else {
-        store_partial(p.part_o + (static_cast<int64_t>(slot) * p.h_q + hq) * D + d, acc);
-        if (d == 0) {
-          store_partial(p.part_ml + (static_cast<int64_t>(slot) * p.h_q + hq) * 2 + 0, mx);
-          store_partial(p.part_ml + (static_cast<int64_t>(slot) * p.h_q + hq) * 2 + 1, lt);
-        }
+        store_partial2(p.part_o + (static_cast<int64_t>(slot) * p.h_q + hq) * D + d, acc0, acc1);
+        if (d == 0) store_partial2(p.part_ml + (static_cast<int64_t>(slot) * p.h_q + hq) * 2, mx, lt);
       }
     }
   }

@@ -132,10 +132,8 @@ __global__ __launch_bounds__(256) void fused_rope_kernel(const half_t* __restric
       Vec16 out_lo, out_hi;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float xl = static_cast<float>(lo.h[e]);
-        const float xh = static_cast<float>(hi.h[e]);
-        out_lo.h[e] = static_cast<half_t>(cs_lds[c * 8 + e] * xl + sn_lds[c * 8 + e] * (-xh));
-        out_hi.h[e] = static_cast<half_t>(cs_lds[D / 2 + c * 8 + e] * xh + sn_lds[D / 2 + c * 8 + e] * xl);
+        out_lo.h[e] = rope_element(cs_lds[c * 8 + e], lo.h[e], sn_lds[c * 8 + e], -static_cast<float>(hi.h[e]));
+        out_hi.h[e] = rope_element(cs_lds[D / 2 + c * 8 + e], hi.h[e], sn_lds[D / 2 + c * 8 + e], static_cast<float>(lo.h[e]));
       }
       lo = out_lo;
       hi = out_hi;
