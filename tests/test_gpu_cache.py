@@ -312,6 +312,25 @@ def test_mixed_steps_on_the_generic_kernels(dtype, page_size, d, hq, hkv, window
         m.step([(0, 1), (2, 1), (4, 1)], (0, 0))
 
 
+@pytest.mark.parametrize("dtype,page_size,d,hq,hkv,window", [(np.float16, 16, 64, 8, 2, 0), (np.float16, 16, 128, 16, 1, 0), (np.float16, 32, 64, 3, 3, 50),
+                                                            (np.float16, 16, 128, 8, 2, 90), (np.float32, 16, 128, 8, 2, 0), (np.float32, 24, 64, 8, 1, 0),
+                                                            (np.float16, 20, 72, 12, 2, 0), (np.float16, 12, 64, 8, 2, 0)])
+def test_prompts_and_decoding_sequences_in_one_launch(dtype, page_size, d, hq, hkv, window):
+    """Steps whose work of either kind is the shorter one by far, a single item, or no multiple of the eight workgroups that
+    are dealt out together: new prompts, whose launch is not split, beside long and short decoding sequences (the generic
+    kernels': long ones, whose launch is).  The oracle's results, with the bounds of every step of a Mirror."""
+    m = Mirror([16, 5000, 1024, page_size, 0] + ([window] if window else []), 2 if window else 1, hq, hkv, d, dtype=dtype,
+               **({"attn_kinds": [3, 0]} if window else {}))
+    mixed = (3, 3 if window else 0)
+    with step_route(2):
+        m.step([(0, 900), (1, 64)], (0, 0))
+        m.step([(2, 400), (3, 1)], None)
+        m.step([(4, 2), (0, 1)], mixed)  # an item or two of prompts; one sequence
+        m.step([(0, 1), (5, 33), (2, 1), (6, 257), (1, 1), (7, 19)], mixed)
+        m.step([(8, 300), (9, 131), (10, 64), (11, 5), (2, 1)], mixed)  # few decoding items
+        m.step([(12, 17), (0, 1), (1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (8, 1), (9, 1)], mixed)
+
+
 def _exact(rows, cached, starts, mask, heads, kv_heads):
     """Attention in 64 bits of one sequence's new tokens (q, k, v rows) over its cached ones and, under `mask`, the new."""
     q, k, v = rows.double().transpose(0, 1).split([heads, kv_heads, kv_heads])

@@ -24,7 +24,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "kernels_common.cuh"
+#include "prefill_kernel.cuh"
 #include "runtime_support.h"
 #include "typed_kernels.h"
 #include "split_plan.h"
@@ -281,11 +281,7 @@ __device__ __forceinline__ int dm_swizzle(int row) {
   return D >= 128 ? (row & 7) << 1 : ((row >> 1) & 3) << 1;
 }
 
-// One entry per element of the head for in-kernel RoPE (the default: theta^(2i/D) for elements i and
-// i + D/2), computed on the host with the libm call the CPU kernels use; DecodeParams says how they are used
-struct DecodeRopeDivisors {
-  float v[256];
-};
+using DecodeRopeDivisors = PrefillRopeDivisors;
 // The extended kernels with the default frequencies: also cos and sin of the angle between a lane's neighbouring
 // keys of a step (near) and between its last key of a step and its first of the next (far), per feature pair,
 // computed in double
@@ -317,9 +313,20 @@ struct DecodeRopeRunning : DecodeRopeDivisors {
 // SELF (with EXT): the new-token form, see DecodeParams.  The wave that starts a sequence's last chunk begins with the
 // state of that one key instead of the empty one, so that a step whose new rows may not be in the pages yet (windows,
 // steps that mix prompts and decoding sequences) needs neither a self-attention launch nor a merge.
+//
+// decode_items works on items first_item, first_item + stride, ... below num_items.
+template <int D, bool FUSED, bool RUNNING>
+struct DecodeShared {
+  alignas(16) half_t v_tiles[4][2 * DM_PS * D];
+  float m[4][16], l[4][16];
+  int last;
+  alignas(16) half_t own[FUSED ? 2 * D : 8];  // the new token's rotated k row and its v row
+  alignas(16) float rope[RUNNING ? 5 : 1][RUNNING ? D / 2 : 1];
+};
 template <bool EXT, int D, bool REREAD, int HB = 1, bool FUSED = false, bool PAD = false, bool VARIANT = false, bool SELF = false>
-__global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void decode_mfma_kernel(DecodeParams p, int group, int num_items,
-    std::conditional_t<EXT && !VARIANT, DecodeRopeRunning, DecodeRopeDivisors> div) {
+__device__ __forceinline__ void decode_items(const DecodeParams& p, const int group, const int num_items,
+                                             const std::conditional_t<EXT && !VARIANT, DecodeRopeRunning, DecodeRopeDivisors>& div,
+                                             const int first_item, const int stride, DecodeShared<D, FUSED, EXT && !VARIANT>& shared) {
   static_assert(HB == 1 || HB == 2, "head blocks per work item");
   static_assert(!(FUSED && EXT), "the fused step exists for the plain cache");
   static_assert(!SELF || (EXT && !VARIANT), "the new-token form: an extended kernel with the default frequencies");
@@ -338,14 +345,14 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   constexpr int NPAIR = KLINE ? KS / 4 : KS / 2;  // fragment pairs (f, f + D/2) of a K token in one lane
   static_assert(D == 64 || D == 128 || D == 256, "head dim");
   static_assert(DM_VTILE * sizeof(half_t) >= 16 * D * sizeof(float), "the merge buffer aliases the V tile");
-  __shared__ __attribute__((aligned(16))) half_t Vt_all[4][DM_VTILE];
-  __shared__ float sm_m[4][16];
-  __shared__ float sm_l[4][16];
-  __shared__ int sm_last;
-  __shared__ __attribute__((aligned(16))) half_t own_lds[FUSED ? 2 * D : 8];  // the new token's rotated k row and its v row
+  auto& Vt_all = shared.v_tiles;
+  auto& sm_m = shared.m;
+  auto& sm_l = shared.l;
+  auto& sm_last = shared.last;
+  auto& own_lds = shared.own;
   constexpr bool RUNNING = EXT && !VARIANT;  // keys rotate by running angles, see below
   constexpr int TSTEP = KLINE ? 8 : 16;      // distance of a lane's neighbouring keys
-  __shared__ __attribute__((aligned(16))) float rope_lds[RUNNING ? 5 : 1][RUNNING ? D / 2 : 1];
+  auto& rope_lds = shared.rope;
 
   const int cp = p.chunk_pages;
   const int psh = p.page_shift;  // a page of the table is 1 << psh of the 16-token pages the steps consume
@@ -355,7 +362,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   // the grid.  Neighbouring workgroups take the head blocks and kv heads of one slot, i.e. the same pages.
   constexpr int HPI = 16 * HB;  // query heads per work item
   const int head_blocks = (group + HPI - 1) / HPI;
-  for (int item = blockIdx.x; item < num_items; item += gridDim.x) {
+  for (int item = first_item; item < num_items; item += stride) {
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));  // what is formed from it belongs to an item: kept for the next one, it spills
   const int wave = tid >> 6;
@@ -986,6 +993,59 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
   }  // items
 }
 
+template <bool EXT, int D, bool REREAD, int HB = 1, bool FUSED = false, bool PAD = false, bool VARIANT = false, bool SELF = false>
+__global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void decode_mfma_kernel(DecodeParams p, int group, int num_items,
+    std::conditional_t<EXT && !VARIANT, DecodeRopeRunning, DecodeRopeDivisors> div) {
+  __shared__ DecodeShared<D, FUSED, EXT && !VARIANT> shared;
+  decode_items<EXT, D, REREAD, HB, FUSED, PAD, VARIANT, SELF>(p, group, num_items, div, blockIdx.x, gridDim.x, shared);
+}
+
+// The decoding sequences of a step and its prompts in one launch.  Behind each other, the prompts' row tiles wait for the
+// matrix cores and for their own short chains while the memory idles, then the decoding sequences' items wait for the
+// memory while the matrix cores do; both have too few workgroups to fill the chip to their end.  Eight neighbouring
+// workgroups (one per XCD) are of one kind; two such groups of decoding items follow one of prompts until a kind is used
+// up.  32 decoding sequences of up to 6000 tokens beside 8 prompts of up to 777, 32 / 8 heads of dim 64, every other layer with
+// a window: 8 layers 591 -> 478 us; the prompts' groups all in front 541, all behind 500, evenly spread over the grid 513,
+// one to one 491 and one to three 483 (periods of an even number of groups put a kind on the same compute units: 4
+// decoding sequences beside 10 prompts 1 : 1 337, 1 : 2 322, 1 : 3 343, 1 : 4 324 us).  The registers and LDS are those of the
+// prefill kernel (head dim 64: three workgroups per compute unit, 128: two), which leaves as many workgroups as the decode kernel has
+// by itself at 128.
+template <int D, int SRC>
+__global__ __launch_bounds__(256, prefill_waves_per_simd(D, D)) void decode_beside_prefill_kernel(
+    DecodeParams p, int group, DecodeRopeRunning div, PrefillParams prompts, LaunchMix mix) {
+  extern __shared__ __attribute__((aligned(16))) half_t beside_lds[];
+  bool is_prompts;
+  const int item = mix.item(blockIdx.x, is_prompts);
+  if (item < 0) return;
+  if (is_prompts) {
+    const int slot = item / p.h_kv;
+    prefill_row_tile<D, D, SRC, 16, false>(prompts, div, item - slot * p.h_kv, slot, 0, beside_lds,
+                                           reinterpret_cast<float*>(beside_lds + prefill_lds_bytes(D, D) / sizeof(half_t)));
+  } else {
+    decode_items<true, D, false, 1, false, false, false, true>(p, group, mix.other_items, div, item, mix.other_items,
+                                                               *reinterpret_cast<DecodeShared<D, false, true>*>(beside_lds));
+  }
+}
+
+template <int D>
+static void launch_beside_prefill(const DecodeParams& p, int group, int64_t num_items, const DecodeRopeRunning& div,
+                                  const PromptLaunch& prompts, hipStream_t stream) {
+  constexpr size_t lds_bytes = std::max(prefill_lds_bytes(D, D) + D * sizeof(float), sizeof(DecodeShared<D, false, true>));
+  const LaunchMix mix(prompts.slots * p.h_kv, num_items);
+  auto launch = [&](auto kernel) {
+    // per function, not per device
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       static_cast<int>(lds_bytes));
+    HIP_CHECK(attr);
+    hipLaunchKernelGGL(kernel, dim3(mix.grid()), dim3(256), lds_bytes, stream, p, group, div, prompts.p, mix);
+  };
+  if (prompts.src == kBoth) {
+    launch(decode_beside_prefill_kernel<D, kBoth>);
+  } else {
+    launch(decode_beside_prefill_kernel<D, kRagged>);
+  }
+}
+
 constexpr size_t kArrivalBytes = 256 * 1024;  // the first bytes of the scratch buffer: arrival counters
 
 }  // namespace tvmkv
@@ -1047,6 +1107,7 @@ struct FusedStep {
   const int32_t* rows = nullptr;
   const int32_t* page_begin = nullptr;
   int64_t q_stride = 0, new_stride = 0;
+  const PromptLaunch* beside = nullptr;
 };
 
 // Body of the decode entry point.  lease(bytes, at_least) hands out the scratch memory of the call: arrival
@@ -1209,7 +1270,9 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
         launch(decode_mfma_kernel<false, kD, false, 1, true>);
       }
     } else if (self) {
-      if (reread) {
+      if (fused_step.beside != nullptr) {
+        if constexpr (kD <= 128) launch_beside_prefill<kD>(p, group, num_items, div, *fused_step.beside, s);
+      } else if (reread) {
         launch_running(decode_mfma_kernel<true, kD, true, kWide, false, false, false, true>);
       } else if (wide) {
         launch_running(decode_mfma_kernel<true, kD, false, kWide, false, false, false, true>);
@@ -1365,7 +1428,7 @@ extern "C" int tvmkv_fused_decode_step(const void* qkv, void* pages, const int32
 }
 
 // Decode attention of tokens whose k / v rows are not in the pages yet (typed_kernels.h)
-int tvmkv::decode_with_new_token(const NewTokenDecode& a, void* stream) {
+int tvmkv::decode_with_new_token(const NewTokenDecode& a, void* stream, const PromptLaunch* beside) {
   KV_API_BEGIN();
   hipStream_t s = as_stream(stream);
   KV_CHECK(a.batch == 0 || (a.q && a.k_new && a.v_new && a.page_indptr)) << "decode_with_new_token: NULL tensor";
@@ -1377,11 +1440,21 @@ int tvmkv::decode_with_new_token(const NewTokenDecode& a, void* stream) {
   step.page_begin = a.page_begin;
   step.q_stride = a.q_stride;
   step.new_stride = a.new_stride;
+  step.beside = beside;
   decode_entry([&](size_t bytes, size_t at_least) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes, at_least); }, step, a.q, a.pages,
                a.page_indptr, a.page_values, a.length_info, a.k_rope_pos_offset, a.q_rope_position, a.out, a.lse, a.rotate,
                a.rope_scale, a.rope_theta, a.sm_scale, a.batch, a.nnz_pages, a.num_pages, a.h_q, a.h_kv, a.d, a.page_size,
                a.sliding, stream);
   KV_API_END();
+}
+
+// One launch where the decode kernel's work items are of one block of heads; a cap on its grid (a measuring option) and wider
+// groups keep the launches apart.  The decoding sequences go behind the prompts then: a split launch of those merges every row.
+int tvmkv::attend_mixed(const PromptPrefill& a, const NewTokenDecode& d, void* stream) {
+  const bool together = d.batch > 0 && d.h_kv > 0 && mixed_in_one_launch(d.d, d.h_q / d.h_kv) && option(kOptDecodeWgsPerCu) == 0;
+  PromptLaunch prompts;
+  const int code = prefill_prompts(a, together ? &prompts : nullptr, stream);
+  return code != TVMKV_OK ? code : decode_with_new_token(d, stream, prompts.slots > 0 ? &prompts : nullptr);
 }
 
 // The same entry point for callers that must not allocate (code under HIP graph capture, serving

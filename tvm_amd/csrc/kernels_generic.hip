@@ -142,7 +142,7 @@ __device__ __forceinline__ void rotate_pair(half8_t& lo, half8_t& hi, int f, int
 
 // workgroups per CU: the fp16 form holds its operands in half the registers
 constexpr int generic_workgroups(int elem_bytes, int dmax, int nb) {
-  return elem_bytes == 2 ? (dmax > 128 ? 2 : (nb == 1 ? 4 : 3)) : (dmax > 128 ? 1 : (nb == 1 ? 3 : 2));
+  return elem_bytes == 2 ? (dmax > 128 ? 2 : (nb == 1 || dmax <= 64 ? 4 : 3)) : (dmax > 128 ? 1 : (nb == 1 ? 3 : 2));
 }
 // 16-row blocks per row tile: one for decode-shaped calls and for head dims above 128 (registers), two when a
 // (sequence, kv head) has more than 16 rows on average.  Three and four blocks (fp16 storage, one workgroup fewer
@@ -160,8 +160,16 @@ inline int generic_row_blocks(int d, int rows_hint) { return generic_row_tile(d,
 // the masks and RoPE use, _kernel_common.py:155-170), the per-layer sliding-window mask (:138-144) and RoPE inside
 // the kernel with any frequency variant (the table, one entry per element; the halves of a variant whose halves
 // differ are rotated by their own entries).
+template <int DMAX, int NB, bool EXT>
+struct GenericShared {
+  alignas(16) float o[2 * 16 * NB * DMAX];
+  float ml[2 * 16 * NB * 2];
+  float rope[EXT ? kMaxHeadDim : 1];
+};
+// Share `split` of the keys of row tile `slot` and kv head `kvh`
 template <typename T, int DMAX, int NB, bool EXT>
-__global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void generic_attn_kernel(GAttn p, InlineRopeTable rope) {
+__device__ __forceinline__ void generic_row_tile_attn(const GAttn p, const InlineRopeTable& rope, const int slot, const int kvh,
+                                                      const int split, GenericShared<DMAX, NB, EXT>& shared) {
   constexpr bool HALF = sizeof(T) == 2;
   constexpr int ROWS = 16 * NB;
   constexpr int KS = DMAX / 16;  // output feature "blocks": lane (i, g) of the V^T operand owns features i * KS .. + KS - 1
@@ -169,23 +177,20 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
   constexpr int QS = DMAX / (4 * PIECE);                   // load steps of the score product (4 pieces each)
   constexpr int VP = KS < PIECE ? KS : PIECE;              // elements per load of the V^T operand (8 or 16 bytes)
   static_assert(KS % VP == 0 && DMAX % (4 * PIECE) == 0, "head dim vs load width");
-  __shared__ __attribute__((aligned(16))) float o_lds[2 * ROWS * DMAX];
-  __shared__ float ml_lds[2 * ROWS * 2];
-  __shared__ float rope_lds[EXT ? kMaxHeadDim : 1];
+  auto& o_lds = shared.o;
+  auto& ml_lds = shared.ml;
+  auto& rope_lds = shared.rope;
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int j = lane & 15;  // query row of a 16-row block (matrix column) / key of a block / feature of a block
   const int g = lane >> 4;
   const int group = p.h_q / p.h_kv;
-  const int kvh = blockIdx.y;
-  const int split = blockIdx.z;
   const int d = p.d;
 
   // the sequence of this row-tile slot: sequence b owns the slots from (q_start(b) * group) / ROWS + b on
   auto q_begin = [&](int b) { return p.q_indptr != nullptr ? p.q_indptr[b] : b; };
   auto slot_begin = [&](int b) { return static_cast<int>(static_cast<int64_t>(q_begin(b)) * group / ROWS) + b; };
-  const int slot = blockIdx.x;
   int lo = 0, hi = p.batch - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -560,6 +565,35 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
   }
 }
 
+template <typename T, int DMAX, int NB, bool EXT>
+__global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void generic_attn_kernel(GAttn p, InlineRopeTable rope) {
+  __shared__ GenericShared<DMAX, NB, EXT> shared;
+  generic_row_tile_attn<T, DMAX, NB, EXT>(p, rope, blockIdx.x, blockIdx.y, blockIdx.z, shared);
+}
+
+// Two plain launches that do not wait for each other in one: row tiles of 32 rows over the new tokens of a step, which the
+// matrix cores bound, and split shares of its decoding sequences, which the memory bounds (float32, 20 decoding sequences of
+// 200-4000 tokens beside 4 prompts of 50-700, 32 / 8 heads of dim 128: 112 and 84 us behind each other, 31 us less in one; as
+// many workgroups per compute unit as the first kind has by itself)
+template <typename T, int DMAX>
+__global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, 2)) void generic_pair_kernel(GAttn own, GAttn decoding, LaunchMix mix) {
+  __shared__ union {
+    GenericShared<DMAX, 2, false> own;
+    GenericShared<DMAX, 1, false> decoding;
+  } shared;
+  InlineRopeTable none;  // neither rotates
+  bool is_first;
+  const int item = mix.item(blockIdx.x, is_first);
+  if (item < 0) return;
+  if (is_first) {
+    const int slot = item / own.h_kv;
+    generic_row_tile_attn<T, DMAX, 2, false>(own, none, slot, item - slot * own.h_kv, 0, shared.own);
+  } else {
+    const int tile = item / decoding.h_kv, slot = tile / decoding.splits;
+    generic_row_tile_attn<T, DMAX, 1, false>(decoding, none, slot, item - tile * decoding.h_kv, tile - slot * decoding.splits, shared.decoding);
+  }
+}
+
 // The shares of a split launch: one workgroup of 64 lanes per (query, head) row.  token_rows: GAttn::rows; merge_into: the
 // state in out / lse is one more share.
 template <typename T>
@@ -612,11 +646,16 @@ void launch_attention(const GAttn& p, const InlineRopeTable& rope, int rows_hint
   KV_LAUNCH_CHECK();
 }
 
-}  // namespace
+struct GenericLaunch {
+  GAttn p{};
+  InlineRopeTable rope{};
+  bool ext = false;
+  int rows_hint = 0;
+  ScratchLease lease{};  // of a split launch: held until the merge is enqueued
+};
 
-int generic_attention(const GenericAttention& a, void* stream_) {
-  KV_API_BEGIN();
-  hipStream_t stream = as_stream(stream_);
+// Checks a call and lays out its launch; false: there is nothing to do
+bool prepare(const GenericAttention& a, hipStream_t stream, GenericLaunch& launch) {
   const bool f32 = a.elem_bits == 32;
   KV_CHECK(a.elem_bits == 16 || a.elem_bits == 32) << a.what << ": elem_bits must be 16 or 32";
   KV_CHECK(a.batch >= 0 && a.total_q >= 0 && a.h_q > 0 && a.h_kv > 0 && a.h_q % a.h_kv == 0) << a.what << ": bad shape";
@@ -627,7 +666,7 @@ int generic_attention(const GenericAttention& a, void* stream_) {
   KV_UNSUPPORTED(rotary && a.d % (f32 ? 8 : 16) != 0)
       << a.what << ": RoPE inside the generic kernels needs a head dim that is a multiple of " << (f32 ? 8 : 16) << ", got "
       << a.d << " (an element and its partner half a head away are loaded as whole 16-byte pieces)";
-  if (a.batch == 0 || a.total_q == 0) return TVMKV_OK;
+  if (a.batch == 0 || a.total_q == 0) return false;
   const bool paged = a.pages != nullptr;
   KV_CHECK(a.q && a.out && a.lse) << a.what << ": NULL tensor";
   const bool sliding = paged && a.sliding_window != 0;
@@ -650,7 +689,7 @@ int generic_attention(const GenericAttention& a, void* stream_) {
   KV_CHECK((a.tree_indptr == nullptr) == (a.tree_labels == nullptr)) << a.what << ": tree_indptr and the labels come together";
   KV_CHECK(a.total_q * a.h_q < (int64_t{1} << 31)) << a.what << ": too many rows for one launch";
 
-  GAttn p{};
+  GAttn& p = launch.p;
   p.q = a.q;
   p.k = a.k;
   p.v = a.v;
@@ -684,7 +723,7 @@ int generic_attention(const GenericAttention& a, void* stream_) {
   p.q_rope_position = a.q_rope_position;
   p.k_rope_pos_offset = a.k_rope_pos_offset;
   p.rope_scale = static_cast<float>(a.rope_scale);
-  InlineRopeTable rope{};
+  InlineRopeTable& rope = launch.rope;
   if (rotary) {
     const InlineRopeHost table = inline_rope_table(a.rope_scaling, a.d, a.rope_theta);
     for (int i = 0; i < a.d; ++i) rope.v[i] = table.v[i];
@@ -692,40 +731,80 @@ int generic_attention(const GenericAttention& a, void* stream_) {
     rope.halves_differ = table.halves_differ;
     rope.magnitude = table.magnitude;
   }
-  const bool ext = sliding || rotary;
+  const bool ext = launch.ext = sliding || rotary;
   KV_CHECK(!ext || (a.rows == nullptr && a.page_begin == nullptr && a.skip_single == 0 && a.merge_into == 0))
       << a.what << ": the extended form computes every sequence of the call";
   const int group = a.h_q / a.h_kv;
   const int64_t work_q = a.work_seqs > 0 ? a.work_q : a.total_q, work_seqs = a.work_seqs > 0 ? a.work_seqs : a.batch;
-  const int rows_hint = static_cast<int>(std::min<int64_t>(work_q * group / work_seqs, 1 << 20));
+  launch.rows_hint = static_cast<int>(std::min<int64_t>(work_q * group / work_seqs, 1 << 20));
   p.splits = 1;
-  ScratchLease lease{};
   if (paged && a.skip_single == 0) {  // (the rows that are passed over have no partial states to merge)
     p.splits = generic_kv_splits(a.elem_bits, a.d, work_q, group, work_seqs, a.h_kv, a.nnz_pages * a.page_size / work_seqs, compute_units());
   }
   if (p.splits > 1) {
     const size_t o_bytes = static_cast<size_t>(p.splits) * a.total_q * a.h_q * a.d * sizeof(float);
     const size_t s_bytes = static_cast<size_t>(p.splits) * a.total_q * a.h_q * sizeof(float);
-    lease = lease_scratch(kScratchGeneric, stream, o_bytes + s_bytes, 0);  // held until the merge is enqueued
-    p.part_o = reinterpret_cast<float*>(lease.ptr);
-    p.part_s = reinterpret_cast<float*>(lease.ptr + o_bytes);
+    launch.lease = lease_scratch(kScratchGeneric, stream, o_bytes + s_bytes, 0);
+    p.part_o = reinterpret_cast<float*>(launch.lease.ptr);
+    p.part_s = reinterpret_cast<float*>(launch.lease.ptr + o_bytes);
   }
-  if (f32) {
-    if (ext) launch_attention<float, true>(p, rope, rows_hint, stream); else launch_attention<float, false>(p, rope, rows_hint, stream);
+  return true;
+}
+
+// The launch that merges the shares of a split one
+void merge_shares(const GenericAttention& a, const GAttn& p, hipStream_t stream) {
+  if (p.splits == 1) return;
+  const int64_t rows = a.total_q * a.h_q;
+  if (a.elem_bits == 32) {
+    hipLaunchKernelGGL(generic_merge_kernel<float>, dim3(static_cast<unsigned>(rows)), dim3(64), 0, stream, p.part_o, p.part_s,
+                       static_cast<float*>(a.out), a.lse, rows, a.d, p.splits, a.rows, a.h_q, a.merge_into);
   } else {
-    if (ext) launch_attention<half_t, true>(p, rope, rows_hint, stream); else launch_attention<half_t, false>(p, rope, rows_hint, stream);
+    hipLaunchKernelGGL(generic_merge_kernel<half_t>, dim3(static_cast<unsigned>(rows)), dim3(64), 0, stream, p.part_o, p.part_s,
+                       static_cast<half_t*>(a.out), a.lse, rows, a.d, p.splits, a.rows, a.h_q, a.merge_into);
   }
-  if (p.splits > 1) {
-    const int64_t rows = a.total_q * a.h_q;
-    if (f32) {
-      hipLaunchKernelGGL(generic_merge_kernel<float>, dim3(static_cast<unsigned>(rows)), dim3(64), 0, stream, p.part_o, p.part_s,
-                         static_cast<float*>(a.out), a.lse, rows, a.d, p.splits, a.rows, a.h_q, a.merge_into);
-    } else {
-      hipLaunchKernelGGL(generic_merge_kernel<half_t>, dim3(static_cast<unsigned>(rows)), dim3(64), 0, stream, p.part_o, p.part_s,
-                         static_cast<half_t*>(a.out), a.lse, rows, a.d, p.splits, a.rows, a.h_q, a.merge_into);
-    }
-    KV_LAUNCH_CHECK();
+  KV_LAUNCH_CHECK();
+}
+
+}  // namespace
+
+int generic_attention(const GenericAttention& a, void* stream_) {
+  KV_API_BEGIN();
+  hipStream_t stream = as_stream(stream_);
+  GenericLaunch launch;
+  if (!prepare(a, stream, launch)) return TVMKV_OK;
+  auto run = [&](auto type) {
+    using T = decltype(type);
+    if (launch.ext) launch_attention<T, true>(launch.p, launch.rope, launch.rows_hint, stream); else launch_attention<T, false>(launch.p, launch.rope, launch.rows_hint, stream);
+  };
+  if (a.elem_bits == 32) run(float{}); else run(half_t{});
+  merge_shares(a, launch.p, stream);
+  KV_API_END();
+}
+
+// One launch where the second call is split: its shares go to scratch memory, the merge behind them reads the first's rows.
+int generic_attention_pair(const GenericAttention& own, const GenericAttention& decoding, void* stream_) {
+  KV_API_BEGIN();
+  hipStream_t stream = as_stream(stream_);
+  GenericLaunch first, second;
+  const bool some = own.pages == nullptr && decoding.skip_single == 0 && own.d == decoding.d && own.elem_bits == decoding.elem_bits &&
+                    prepare(own, stream, first) && prepare(decoding, stream, second);
+  const int group = own.h_q / std::max(own.h_kv, 1);
+  if (!some || first.ext || second.ext || second.p.splits == 1 || !generic_pair_tiles(own.d, group, first.rows_hint) || decoding.q_indptr != nullptr) {
+    second.lease = {};
+    const int code = generic_attention(own, stream_);
+    return code != TVMKV_OK ? code : generic_attention(decoding, stream_);
   }
+  const int64_t own_items = (own.total_q * group / 32 + own.batch) * own.h_kv;
+  const int64_t other_items = (decoding.total_q * group / 16 + decoding.batch) * decoding.h_kv * second.p.splits;
+  const LaunchMix mix(own_items, other_items);
+  auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(mix.grid()), dim3(256), 0, stream, first.p, second.p, mix); };
+  auto run_type = [&](auto type) {
+    using T = decltype(type);
+    if (own.d <= 64) run(generic_pair_kernel<T, 64>); else run(generic_pair_kernel<T, 128>);
+  };
+  if (own.elem_bits == 32) run_type(float{}); else run_type(half_t{});
+  KV_LAUNCH_CHECK();
+  merge_shares(decoding, second.p, stream);
   KV_API_END();
 }
 

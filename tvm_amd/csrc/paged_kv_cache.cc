@@ -887,20 +887,33 @@ class PagedKVCache {
   double MixedUs(const std::vector<StepSequence>& seqs, const MixedStep& plan, bool window) const {
     const auto prompt = [](const StepSequence& q) { return q.tokens > 1; };
     const auto decoding = [](const StepSequence& q) { return q.tokens == 1; };
+    const int64_t tokens = plan.prompt_tokens + plan.decoding;
+    const int group = static_cast<int>(num_qo_heads_ / num_kv_heads_), h_kv = static_cast<int>(num_kv_heads_), d = static_cast<int>(qk_head_dim_);
     if (generic_) {
-      return (qk_head_dim_ > 128 ? 36 : 16) + OwnUs(seqs, [](const StepSequence&) { return true; }, false) +
-             PagedUs(seqs, prompt, false, false, false, /*may_split=*/false, 0) + PagedUs(seqs, decoding, false, false, false, true, sizeof(float));
+      const double own = OwnUs(seqs, [](const StepSequence&) { return true; }, false);
+      const double rows = PagedUs(seqs, decoding, false, false, false, true, sizeof(float));
+      const bool together = generic_pair_tiles(d, group, tokens * group / static_cast<int64_t>(seqs.size()));
+      return (d > 128 ? 36 : 16) + (together ? std::max(own, rows) + 0.8 * std::min(own, rows) : own + rows) +
+             PagedUs(seqs, prompt, false, false, false, /*may_split=*/false, 0);
     }
     double keys = 0;
     for (const StepSequence& q : seqs) keys += decoding(q) ? static_cast<double>(q.cached) : 0;
     const double prompts = window ? OwnUs(seqs, prompt, false) + PagedUs(seqs, prompt, false, true, false, true, sizeof(float))
                                   : PagedUs(seqs, prompt, false, false, true, true, sizeof(float));
-    return 11 + prompts + 12 + keys * GatherRowBytes() / 5e6;  // 12 us and the rows: the decode kernel
+    const double rows = keys * GatherRowBytes() / 5e6;  // the decode kernel's time grows with them
+    // In one launch, as long as the prompts' is not split.  (As a sum of launches this let steps of a few sequences take the
+    // general ones, which ran 1.1-1.7 times as long; with it 60 steps were within 1.13 of the better route.)
+    const bool together = mixed_in_one_launch(d, group) &&
+                          (window ? plan.prompt_cached == 0
+                                  : prefill_kv_splits(plan.prompt_tokens, group, plan.prompts, h_kv,
+                                                      (plan.prompt_cached + plan.prompt_tokens) / plan.prompts, compute_units_) == 1);
+    if (together) return 8 + std::max(prompts, 8 + rows) + 0.5 * std::min(prompts, 8 + rows);
+    return 11 + prompts + 12 + rows;
   }
 
   // A step of prompts and decoding sequences.  In one prefill launch a decoding sequence is a row tile of few rows whose
   // workgroups walk all its keys: the longest of them decides how long the launch takes (32 decoding sequences of up
-  // to 6000 tokens beside 8 prompts, 32 / 8 heads of dim 64, every other layer with a window: 886 us for 8 layers, 590 now), unless
+  // to 6000 tokens beside 8 prompts, 32 / 8 heads of dim 64, every other layer with a window: 886 us for 8 layers, 479 now), unless
   // the launch is small enough to be split.  So the prompts run without them, and the decode kernel, which always splits the
   // keys, takes them with the new token as one more key, where the estimate says that this is faster.  What the decode
   // kernel reads of them is written here, for the pages of the plain layers and for those of the layers with a window.
@@ -1016,7 +1029,6 @@ class PagedKVCache {
     a.prompts = mixed_.prompts;
     a.prompt_tokens = mixed_.prompt_tokens;
     a.prompt_cached = mixed_.prompt_cached;
-    Launch(prefill_prompts(a, compute_stream_));
     NewTokenDecode d;
     d.q = q;
     d.q_stride = q_stride;
@@ -1044,7 +1056,7 @@ class PagedKVCache {
     d.d = a.d;
     d.page_size = a.page_size;
     d.sliding = window;
-    Launch(decode_with_new_token(d, compute_stream_));  // behind the prompts: their launch may leave anything in these rows
+    Launch(attend_mixed(a, d, compute_stream_));
   }
 
   // The same on the generic kernel: every sequence's new tokens, then the cached ones of the prompts and those of the
@@ -1053,7 +1065,6 @@ class PagedKVCache {
                              double sm_scale) {
     const StepLayout& s = book_->step();
     const int64_t local_layer_id = layer_id - layer_id_begin_offset_;
-    GenericRagged(q, k, v, out, merged_lse_, total_seq_length, sm_scale, /*tree=*/false);
     GenericAttention a;
     a.what = "cross attention";
     a.elem_bits = elem_bits_;
@@ -1069,6 +1080,15 @@ class PagedKVCache {
     a.d = static_cast<int32_t>(qk_head_dim_);
     a.page_size = static_cast<int32_t>(page_size_);
     a.sm_scale = sm_scale;
+    GenericAttention decoding = a;
+    decoding.rows = DevExtra(mixed_.rows);
+    decoding.page_indptr = DevExtra(mixed_.page_indptr[0]);
+    decoding.page_begin = DevExtra(mixed_.page_begin[0]);
+    decoding.last_page_len = DevExtra(mixed_.length_info[0]);
+    decoding.total_q = decoding.batch = mixed_.decoding;
+    decoding.nnz_pages = mixed_.nnz_pages[0];
+    Launch(generic_attention_pair(GenericOwn(q, k, v, out, merged_lse_, total_seq_length, sm_scale, /*tree=*/false), decoding,
+                                  compute_stream_));
     if (mixed_.prompt_cached > 0) {
       GenericAttention prompts = a;
       prompts.q_indptr = Dev(s.qo_indptr[0]);
@@ -1082,13 +1102,6 @@ class PagedKVCache {
       prompts.nnz_pages = mixed_.prompt_cached / page_size_;
       Launch(generic_attention(prompts, compute_stream_));
     }
-    a.rows = DevExtra(mixed_.rows);
-    a.page_indptr = DevExtra(mixed_.page_indptr[0]);
-    a.page_begin = DevExtra(mixed_.page_begin[0]);
-    a.last_page_len = DevExtra(mixed_.length_info[0]);
-    a.total_q = a.batch = mixed_.decoding;
-    a.nnz_pages = mixed_.nnz_pages[0];
-    Launch(generic_attention(a, compute_stream_));
   }
 
   // A decode step of a cache with sequence windows in two launches: the decode kernel rotates and takes the new token as
@@ -1263,6 +1276,10 @@ class PagedKVCache {
   // causal self-attention over the step's new tokens (or the token-tree mask) on the generic kernel
   void GenericRagged(const void* q, const void* k, const void* v, void* o, float* lse, int64_t total_seq_length,
                      double sm_scale, bool tree) {
+    Launch(generic_attention(GenericOwn(q, k, v, o, lse, total_seq_length, sm_scale, tree), compute_stream_));
+  }
+  GenericAttention GenericOwn(const void* q, const void* k, const void* v, void* o, float* lse, int64_t total_seq_length,
+                              double sm_scale, bool tree) {
     const StepLayout& s = book_->step();
     GenericAttention a;
     a.what = "self attention";
@@ -1293,7 +1310,7 @@ class PagedKVCache {
     a.d = static_cast<int32_t>(qk_head_dim_);
     a.causal = 1;
     a.sm_scale = sm_scale;
-    Launch(generic_attention(a, compute_stream_));
+    return a;
   }
 
   // :2216-2299

@@ -79,6 +79,10 @@ struct GenericAttention {
   int64_t work_q = 0, work_seqs = 0;
 };
 int generic_attention(const GenericAttention& args, void* stream);
+// Both calls; the second merges into rows of the first.  One launch where the first has row tiles of 32 rows and the second a
+// split one of 16 (generic_pair_tiles: query rows a sequence and kv head on average).
+inline bool generic_pair_tiles(int d, int group, int64_t own_rows) { return d <= 128 && group <= 16 && own_rows > 16; }
+int generic_attention_pair(const GenericAttention& own, const GenericAttention& decoding, void* stream);
 
 // Slot 24 (and 24 + 13 with pages != NULL) for any even head dim up to 256 and either storage type; the
 // arguments of tvmkv_fused_rope_append_scaled.
@@ -153,7 +157,9 @@ struct NewTokenDecode {
   int32_t batch = 0, h_q = 0, h_kv = 0, d = 0, page_size = 0;
   int32_t sliding = 0;
 };
-int decode_with_new_token(const NewTokenDecode& args, void* stream);
+struct PromptLaunch;
+// beside: prompts to run in the same launch (kernels_decode.hip), or NULL
+int decode_with_new_token(const NewTokenDecode& args, void* stream, const PromptLaunch* beside = nullptr);
 
 // Prefill attention (fp16, head dims 64 / 128, tuned page sizes) of a step's sequences with more than one new token:
 // cached keys, then the new ones under the causal mask.  Sequences with one new token are passed over; their rows of
@@ -179,7 +185,10 @@ struct PromptPrefill {
   int64_t total_q = 0, num_pages = 0;
   int64_t prompts = 0, prompt_tokens = 0, prompt_cached = 0;  // sequences with more than one new token: their number, new and cached tokens
 };
-int prefill_prompts(const PromptPrefill& args, void* stream);
+
+// A step that mixes prompts and decoding sequences: both of the above, in one launch where that is built.
+inline bool mixed_in_one_launch(int d, int group) { return (d == 64 || d == 128) && group <= 16; }
+int attend_mixed(const PromptPrefill& prompts, const NewTokenDecode& decoding, void* stream);
 
 // tvmkv_batch_prefill_paged_kv_scaled for a caller that knows the keys of its longest sequence (0: not known)
 int prefill_paged_with_lengths(const void* q, const int32_t* q_indptr, const void* pages, const int32_t* page_indptr,
