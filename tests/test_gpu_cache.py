@@ -331,6 +331,19 @@ def test_prompts_and_decoding_sequences_in_one_launch(dtype, page_size, d, hq, h
         m.step([(12, 17), (0, 1), (1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (8, 1), (9, 1)], mixed)
 
 
+@pytest.mark.parametrize("page_size,d,hq,hkv,forks,prefix", [(16, 128, 16, 1, 9, 640), (64, 64, 32, 2, 10, 1100), (16, 128, 8, 2, 41, 385),
+                                                            (32, 64, 4, 4, 130, 256), (16, 128, 40, 2, 8, 640)])
+def test_decode_step_over_a_shared_prefix_whose_keys_are_split(page_size, d, hq, hkv, forks, prefix):
+    """The sequences' own tokens and the shares of the prefix in one launch (up to 16 query heads a kv head, the last case keeps
+    two): own parts of one token and of several chunks, a sequence that is the prefix itself."""
+    m = Mirror([forks + 2, prefix + 1500 + forks * 3 * page_size, 1200, page_size, 0], 1, hq, hkv, d)
+    m.step([(0, prefix)])
+    m.step([((b, 0, -1), 1) for b in range(1, forks + 1)])
+    m.step([(1, 500)])
+    m.step([(b, 1) for b in range(1, forks + 1)])
+    m.step([(b, 1) for b in range(forks, 0, -1)])
+
+
 def _exact(rows, cached, starts, mask, heads, kv_heads):
     """Attention in 64 bits of one sequence's new tokens (q, k, v rows) over its cached ones and, under `mask`, the new."""
     q, k, v = rows.double().transpose(0, 1).split([heads, kv_heads, kv_heads])

@@ -1010,20 +1010,26 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
 // decoding sequences beside 10 prompts 1 : 1 337, 1 : 2 322, 1 : 3 343, 1 : 4 324 us).  The registers and LDS are those of the
 // prefill kernel (head dim 64: three workgroups per compute unit, 128: two), which leaves as many workgroups as the decode kernel has
 // by itself at 128.
-template <int D, int SRC>
+// NEW_TOKEN: the new-token form of the decode kernel, else its plain one.  A decode step over a shared prefix has the second
+// beside the split shares of the prefix (SRC kPaged), whose one round of workgroups walked its keys alone: 64 sequences of
+// 256-2048 tokens behind a prompt of 4096, 32 / 8 heads of dim 128, two steps of 8 layers: 1369 -> 1247 us, the same bits.  Over 13
+// other shapes (16-200 sequences, 64-2048 tokens, prompts of 300-6000, 4-8 query heads a kv head) 1.00-1.44 times as fast, most
+// where the prefix is long against the sequences' own tokens; two instead of three workgroups per compute unit for the decoding
+// items cost nothing that could be measured (200 sequences of 1024-2048 tokens: 2014 -> 1998).
+template <int D, int SRC, bool NEW_TOKEN>
 __global__ __launch_bounds__(256, prefill_waves_per_simd(D, D)) void decode_beside_prefill_kernel(
-    DecodeParams p, int group, DecodeRopeRunning div, PrefillParams prompts, LaunchMix mix) {
+    DecodeParams p, int group, std::conditional_t<NEW_TOKEN, DecodeRopeRunning, DecodeRopeDivisors> div, PrefillParams prompts, LaunchMix mix) {
   extern __shared__ __attribute__((aligned(16))) half_t beside_lds[];
   bool is_prompts;
   const int item = mix.item(blockIdx.x, is_prompts);
   if (item < 0) return;
   if (is_prompts) {
-    const int slot = item / p.h_kv;
-    prefill_row_tile<D, D, SRC, 16, false>(prompts, div, item - slot * p.h_kv, slot, 0, beside_lds,
+    const int tile = item / p.h_kv, shares = SRC == kPaged ? prompts.kv_splits : 1, slot = tile / shares;
+    prefill_row_tile<D, D, SRC, 16, false>(prompts, div, item - tile * p.h_kv, slot, tile - slot * shares, beside_lds,
                                            reinterpret_cast<float*>(beside_lds + prefill_lds_bytes(D, D) / sizeof(half_t)));
   } else {
-    decode_items<true, D, false, 1, false, false, false, true>(p, group, mix.other_items, div, item, mix.other_items,
-                                                               *reinterpret_cast<DecodeShared<D, false, true>*>(beside_lds));
+    decode_items<NEW_TOKEN, D, false, 1, false, false, false, NEW_TOKEN>(p, group, mix.other_items, div, item, mix.other_items,
+                                                                         *reinterpret_cast<DecodeShared<D, false, NEW_TOKEN>*>(beside_lds));
   }
 }
 
@@ -1031,18 +1037,20 @@ template <int D>
 static void launch_beside_prefill(const DecodeParams& p, int group, int64_t num_items, const DecodeRopeRunning& div,
                                   const PromptLaunch& prompts, hipStream_t stream) {
   constexpr size_t lds_bytes = std::max(prefill_lds_bytes(D, D) + D * sizeof(float), sizeof(DecodeShared<D, false, true>));
-  const LaunchMix mix(prompts.slots * p.h_kv, num_items);
-  auto launch = [&](auto kernel) {
+  const LaunchMix mix(prompts.slots * p.h_kv * std::max(prompts.p.kv_splits, 1), num_items);
+  auto launch = [&](auto kernel, const auto& divisors) {
     // per function, not per device
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        static_cast<int>(lds_bytes));
     HIP_CHECK(attr);
-    hipLaunchKernelGGL(kernel, dim3(mix.grid()), dim3(256), lds_bytes, stream, p, group, div, prompts.p, mix);
+    hipLaunchKernelGGL(kernel, dim3(mix.grid()), dim3(256), lds_bytes, stream, p, group, divisors, prompts.p, mix);
   };
-  if (prompts.src == kBoth) {
-    launch(decode_beside_prefill_kernel<D, kBoth>);
+  if (prompts.src == kPaged) {
+    launch(decode_beside_prefill_kernel<D, kPaged, false>, static_cast<const DecodeRopeDivisors&>(div));
+  } else if (prompts.src == kBoth) {
+    launch(decode_beside_prefill_kernel<D, kBoth, true>, div);
   } else {
-    launch(decode_beside_prefill_kernel<D, kRagged>);
+    launch(decode_beside_prefill_kernel<D, kRagged, true>, div);
   }
 }
 
@@ -1064,7 +1072,7 @@ struct StaticScratch {
   uint64_t launches = 0;  // the epoch of a launch is the low half
 };
 static StaticScratch g_static_scratch[64];
-static std::mutex g_static_scratch_mutex;
+static std::recursive_mutex g_static_scratch_mutex;
 
 static ScratchLease lease_static_scratch(size_t bytes, hipStream_t stream) {
   int dev = 0;
@@ -1073,7 +1081,7 @@ static ScratchLease lease_static_scratch(size_t bytes, hipStream_t stream) {
   KV_CHECK(bytes <= kStaticScratchBytes)
       << "batch_decode_paged_kv_noalloc: the call needs " << bytes << " bytes of scratch memory, the built-in "
       << "buffer has " << kStaticScratchBytes << "; use tvmkv_batch_decode_paged_kv for this shape";
-  std::unique_lock<std::mutex> lock(g_static_scratch_mutex);
+  std::unique_lock<std::recursive_mutex> lock(g_static_scratch_mutex);
   StaticScratch& s = g_static_scratch[dev];
   if (s.ptr == nullptr) {
     void* ptr = nullptr;
@@ -1091,7 +1099,7 @@ static ScratchLease lease_static_scratch(size_t bytes, hipStream_t stream) {
 extern "C" int tvmkv_debug_set_scratch_launches(uint64_t launches) {
   KV_API_BEGIN();
   debug_set_scratch_launches(launches);
-  std::lock_guard<std::mutex> lock(g_static_scratch_mutex);
+  std::lock_guard<std::recursive_mutex> lock(g_static_scratch_mutex);
   for (auto& s : g_static_scratch) s.launches = launches;
   KV_API_END();
 }
@@ -1261,7 +1269,9 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
     constexpr int kWide = kD <= 128 ? 2 : 1;  // head blocks per item for groups of more than 16 heads
     const bool wide = heads_per_item == 32;
     const bool reread = head_blocks > 1;       // several items read the same K/V rows
-    if (fused_launch) {
+    if (fused_step.beside != nullptr) {
+      if constexpr (kD <= 128) launch_beside_prefill<kD>(p, group, num_items, div, *fused_step.beside, s);
+    } else if (fused_launch) {
       if (reread) {
         launch(decode_mfma_kernel<false, kD, true, kWide, true>);
       } else if (wide) {
@@ -1270,9 +1280,7 @@ static void decode_entry(Lease&& lease, const FusedStep& fused_step, const void*
         launch(decode_mfma_kernel<false, kD, false, 1, true>);
       }
     } else if (self) {
-      if (fused_step.beside != nullptr) {
-        if constexpr (kD <= 128) launch_beside_prefill<kD>(p, group, num_items, div, *fused_step.beside, s);
-      } else if (reread) {
+      if (reread) {
         launch_running(decode_mfma_kernel<true, kD, true, kWide, false, false, false, true>);
       } else if (wide) {
         launch_running(decode_mfma_kernel<true, kD, false, kWide, false, false, false, true>);
@@ -1455,6 +1463,21 @@ int tvmkv::attend_mixed(const PromptPrefill& a, const NewTokenDecode& d, void* s
   PromptLaunch prompts;
   const int code = prefill_prompts(a, together ? &prompts : nullptr, stream);
   return code != TVMKV_OK ? code : decode_with_new_token(d, stream, prompts.slots > 0 ? &prompts : nullptr);
+}
+
+// A decode step behind a shared prefix (typed_kernels.h): the decode launch's items are of one block of heads, as above.
+int tvmkv::decode_with_shared_prefix(const SharedPrefixDecode& a, void* stream) {
+  const auto own = [&](const PromptLaunch* beside) -> int {
+    KV_API_BEGIN();
+    hipStream_t s = as_stream(stream);
+    FusedStep step;
+    step.beside = beside;
+    decode_entry([&](size_t bytes, size_t at_least) { return lease_scratch(kScratchDecode, s, bytes, kArrivalBytes, at_least); }, step, a.q, a.pages,
+                 a.own.page_indptr, a.own.page_values, a.own.length_info, nullptr, nullptr, a.out, a.lse, 0, 1.0, 1e4, a.sm_scale,
+                 a.own.sequences, a.own.nnz_pages, a.num_pages, a.h_q, a.h_kv, a.d, a.page_size, 0, stream);
+    KV_API_END();
+  };
+  return prefill_shared_prefix(a, own, stream);
 }
 
 // The same entry point for callers that must not allocate (code under HIP graph capture, serving

@@ -498,7 +498,8 @@ static int paged_prefill(const void* q, const int32_t* q_indptr, const void* pag
                          int32_t batch_size, int64_t total_q, int64_t nnz_pages, int64_t num_pages, int32_t h_q,
                          int32_t h_kv, int32_t d, int32_t page_size, int32_t sliding_window,
                          int32_t sliding_window_size, bool merge_into, void* stream,
-                         const tvmkv_rope_scaling* scaling = nullptr, int64_t longest = 0) {
+                         const tvmkv_rope_scaling* scaling = nullptr, int64_t longest = 0,
+                         const std::function<int(const PromptLaunch*)>* beside = nullptr) {
   // pages other than 16 / 32 / 64 / 128 tokens, other head dims (80 / 96 / 112 with a sliding-window cache or RoPE
   // inside the kernel among them): the generic matrix-core kernel (its caller merges states with merge_state_inplace)
   const bool plain = rotary_mode == 0 && sliding_window == 0;
@@ -575,6 +576,22 @@ static int paged_prefill(const void* q, const int32_t* q_indptr, const void* pag
   hipStream_t s = as_stream(stream);
   // (a launch under capture keeps the scratch memory that it has always needed)
   const KvSplit split(p, total_q, nnz_pages * page_size / batch_size, d, s, stream_is_capturing(s) ? 0 : longest);
+  if (beside != nullptr) {  // the work that writes the state which this launch merges into
+    const bool together = split.splits > 1 && !p.stream_kv && !ext && (d == 64 || d == 128);
+    PromptLaunch shares;
+    if (together) {
+      shares.p = p;
+      shares.slots = row_tile_slots(p, total_q);
+      shares.src = kPaged;
+    }
+    const int code = (*beside)(together ? &shares : nullptr);
+    if (code != TVMKV_OK) return code;
+    if (together) {
+      split.finish(p, d, s);
+      KV_LAUNCH_CHECK();
+      return TVMKV_OK;
+    }
+  }
   if (d == 128) {
     launch_prefill<128, 128, kPaged, 16>(p, total_q, ext, rope_theta, s, scaling);
   } else if (d == 64) {
@@ -646,6 +663,13 @@ int tvmkv::prefill_paged_with_lengths(const void* q, const int32_t* q_indptr, co
   return paged_prefill(q, q_indptr, pages, page_indptr, page_values, length_info, k_rope_pos_offset, q_rope_position, output, lse,
                        causal, rotary_mode, rope_scale, rope_theta, sm_scale, batch_size, total_q, nnz_pages, num_pages, h_q, h_kv, d,
                        page_size, sliding_window, sliding_window_size, merge_into != 0, stream, rope_scaling, longest);
+}
+
+int tvmkv::prefill_shared_prefix(const SharedPrefixDecode& a, const std::function<int(const PromptLaunch*)>& own, void* stream) {
+  return paged_prefill(a.q, a.prefix_q_indptr, a.pages, a.prefix.page_indptr, a.prefix.page_values, a.prefix.length_info, nullptr, nullptr,
+                       a.out, a.lse, /*causal=*/0, /*rotary_mode=*/0, 1.0, 1e4, a.sm_scale, a.prefix.sequences, a.total_q,
+                       a.prefix.nnz_pages, a.num_pages, a.h_q, a.h_kv, a.d, a.page_size, 0, 0, /*merge_into=*/true, stream, nullptr,
+                       a.longest, &own);
 }
 
 extern "C" {

@@ -1337,6 +1337,37 @@ class PagedKVCache {
         if (merges_itself == (pass == 1)) order[n_order++] = d;
       }
     }
+    // A decode step of sequences with pages of their own behind one level of shared pages: both in one launch
+    const bool plain = !generic_ && rotary_mode == 0 && sliding_window == 0 && option(kOptDecodeWgsPerCu) == 0;
+    if (is_first_kernel && n_order == 2 && plain && mixed_in_one_launch(static_cast<int>(qk_head_dim_), static_cast<int>(num_qo_heads_ / num_kv_heads_)) &&
+        s.use_decode_kernel[order[0]] && !s.use_decode_kernel[order[1]] && !(s.append_before_attn && !(s.is_chain[0] && s.is_chain[1])) &&
+        s.page_indices[0].size > 0 && s.page_indices[1].size > 0) {
+      SharedPrefixDecode a;
+      a.q = q;
+      a.pages = pages_[local_layer_id];
+      a.out = o;
+      a.lse = lse;
+      for (int at = 0; at < 2; ++at) {
+        const int d = order[at];
+        SharedPrefixDecode::Level& level = at == 0 ? a.own : a.prefix;
+        level.page_indptr = Dev(s.page_indptr[d]);
+        level.page_values = Dev(s.page_indices[d]);
+        level.length_info = Dev(s.length_info[d]);
+        level.sequences = static_cast<int32_t>(s.qo_indptr[d].size - 1);
+        level.nnz_pages = s.page_indices[d].size;
+      }
+      a.prefix_q_indptr = Dev(s.qo_indptr[order[1]]);
+      a.longest = longest_pages_[0][order[1]] * page_size_;
+      a.sm_scale = sm_scale;
+      a.total_q = total_seq_length;
+      a.num_pages = num_total_pages_;
+      a.h_q = static_cast<int32_t>(num_qo_heads_);
+      a.h_kv = static_cast<int32_t>(num_kv_heads_);
+      a.d = static_cast<int32_t>(qk_head_dim_);
+      a.page_size = static_cast<int32_t>(page_size_);
+      Launch(decode_with_shared_prefix(a, compute_stream_));
+      return true;
+    }
     for (int at = 0; at < n_order; ++at) {
       const int d = order[at];
       if (s.page_indices[d].size == 0) continue;

@@ -3,6 +3,7 @@
 #ifndef TVMKV_CSRC_PREFILL_KERNEL_CUH_
 #define TVMKV_CSRC_PREFILL_KERNEL_CUH_
 
+#include <functional>
 #include <type_traits>
 
 #include "prefill_common.cuh"
@@ -773,7 +774,8 @@ __global__ __launch_bounds__(NW * 64, prefill_waves_per_simd(DQK, DV)) void pref
   prefill_row_tile<DQK, DV, SRC, PS, EXT, STREAM, PAD, VARIANT>(p, div, blockIdx.x, blockIdx.y, blockIdx.z, lds_tiles, div_lds);
 }
 
-// A launch that its caller is to run beside other work (prefill_prompts): grid (h_kv, slots), SRC kRagged or kBoth, plain.
+// A launch that its caller is to run beside other work (prefill_prompts, prefill_shared_prefix): grid (h_kv, slots,
+// p.kv_splits), plain, SRC kPaged for a prefix.
 struct PromptLaunch {
   PrefillParams p;
   PrefillRopeDivisors div;
@@ -781,6 +783,9 @@ struct PromptLaunch {
   int src = kRagged;
 };
 int prefill_prompts(const PromptPrefill& args, PromptLaunch* leave, void* stream);
+// The prefix's part of decode_with_shared_prefix; `own` is called once, before anything is merged, and runs the launch that it is given
+// beside its own.
+int prefill_shared_prefix(const SharedPrefixDecode& args, const std::function<int(const PromptLaunch*)>& own, void* stream);
 
 }  // namespace tvmkv
 

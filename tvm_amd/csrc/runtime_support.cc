@@ -46,7 +46,7 @@ struct Scratch {
   uint64_t launches = 0;       // launches served from this buffer; the epoch of a launch is its low half
   bool seen_in_capture = false;  // a graph under capture has recorded this buffer's address
 };
-std::mutex g_scratch_mutex;
+std::recursive_mutex g_scratch_mutex;
 std::map<std::tuple<int, hipStream_t, int>, Scratch> g_scratch;
 // Buffers that a captured graph may still name after their entry has grown: kept until the process ends.
 std::vector<char*> g_retired;
@@ -93,7 +93,7 @@ ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, s
   HIP_CHECK(hipGetDevice(&dev));
   // held by the lease until the caller has enqueued its launch: a thread that grows (and frees) this
   // entry's buffer first synchronises the stream, and by then the launch is on it
-  std::unique_lock<std::mutex> lock(g_scratch_mutex);
+  std::unique_lock<std::recursive_mutex> lock(g_scratch_mutex);
   Scratch& s = g_scratch[std::make_tuple(dev, stream, static_cast<int>(user))];
   const bool capturing = stream_is_capturing(stream);
   if (s.bytes < bytes || s.counter_bytes < counter_bytes) {
@@ -135,7 +135,7 @@ ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, s
 void release_scratch(hipStream_t stream) {
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  std::lock_guard<std::recursive_mutex> lock(g_scratch_mutex);
   KV_CHECK(!stream_is_capturing(stream)) << "tvmkv_release_scratch: the stream is being captured";
   bool synced = false;
   for (auto it = g_scratch.begin(); it != g_scratch.end();) {
@@ -157,7 +157,7 @@ void release_scratch(hipStream_t stream) {
 }
 
 void debug_set_scratch_launches(uint64_t launches) {
-  std::lock_guard<std::mutex> lock(g_scratch_mutex);
+  std::lock_guard<std::recursive_mutex> lock(g_scratch_mutex);
   for (auto& entry : g_scratch) entry.second.launches = launches;
 }
 

@@ -41,7 +41,7 @@ int64_t option(Option id);
 struct ScratchLease {
   char* ptr;        // device memory, at least the requested size, 256-byte aligned
   uint32_t epoch;   // never 0
-  std::unique_lock<std::mutex> lock;
+  std::unique_lock<std::recursive_mutex> lock;
 };
 enum ScratchUser { kScratchDecode = 0, kScratchMla = 1, kScratchPrefill = 2, kScratchGeneric = 3 };
 // at_least: what a buffer that has to be allocated gets in any case

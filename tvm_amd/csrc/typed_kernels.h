@@ -199,6 +199,29 @@ int prefill_paged_with_lengths(const void* q, const int32_t* q_indptr, const voi
                                int32_t sliding_window, int32_t sliding_window_size, int32_t merge_into,
                                const tvmkv_rope_scaling* rope_scaling, int64_t longest, void* stream);
 
+// A decode step behind a shared prefix (fp16, plain cache): decode attention over the sequences' own pages, which writes
+// out and lse, and paged prefill attention of all queries over the prefix, merged into them.  One launch and the merge of
+// the prefix's shares where its keys are split.
+struct SharedPrefixDecode {
+  const void* q = nullptr;
+  const void* pages = nullptr;
+  void* out = nullptr;
+  float* lse = nullptr;
+  struct Level {
+    const int32_t* page_indptr = nullptr;
+    const int32_t* page_values = nullptr;
+    const int32_t* length_info = nullptr;
+    int32_t sequences = 0;
+    int64_t nnz_pages = 0;
+  } own, prefix;
+  const int32_t* prefix_q_indptr = nullptr;
+  int64_t longest = 0;  // keys of the longest prefix
+  double sm_scale = 1.0;
+  int64_t total_q = 0, num_pages = 0;
+  int32_t h_q = 0, h_kv = 0, d = 0, page_size = 0;
+};
+int decode_with_shared_prefix(const SharedPrefixDecode& args, void* stream);  // where mixed_in_one_launch
+
 // tvmkv_kv_cache_transpose_append with the k / v rows of consecutive tokens token_stride elements apart (the fused
 // qkv tensor of the step)
 int append_strided(void* pages, const void* k_data, const void* v_data, int64_t token_stride, const int32_t* position_map,
