@@ -902,12 +902,12 @@ class PagedKVCache {
                                   : PagedUs(seqs, prompt, false, false, true, true, sizeof(float));
     const double rows = keys * GatherRowBytes() / 5e6;  // the decode kernel's time grows with them
     // In one launch, as long as the prompts' is not split.  (As a sum of launches this let steps of a few sequences take the
-    // general ones, which ran 1.1-1.7 times as long; with it 60 steps were within 1.13 of the better route.)
-    const bool together = mixed_in_one_launch(d, group) &&
-                          (window ? plan.prompt_cached == 0
-                                  : prefill_kv_splits(plan.prompt_tokens, group, plan.prompts, h_kv,
-                                                      (plan.prompt_cached + plan.prompt_tokens) / plan.prompts, compute_units_) == 1);
-    if (together) return 8 + std::max(prompts, 8 + rows) + 0.5 * std::min(prompts, 8 + rows);
+    // general ones, which ran 1.1-1.7 times as long; with it 60 steps were within 1.13 of the better
+    // route.  A layer with a window walks few keys in the general launches: the sum stays there.)
+    const bool together = !window && mixed_in_one_launch(d, group) &&
+                          prefill_kv_splits(plan.prompt_tokens, group, plan.prompts, h_kv,
+                                            (plan.prompt_cached + plan.prompt_tokens) / plan.prompts, compute_units_) == 1;
+    if (together) return 8 + std::max(prompts, 8 + rows) + 0.8 * std::min(prompts, 8 + rows);
     return 11 + prompts + 12 + rows;
   }
 
