@@ -573,7 +573,7 @@ __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, NB)) void 
 
 // Two plain launches that do not wait for each other in one: row tiles of 32 rows over the new tokens of a step, which the
 // matrix cores bound, and split shares of its decoding sequences, which the memory bounds (float32, 20 decoding sequences of
-// 200-4000 tokens beside 4 prompts of 50-700, 32 / 8 heads of dim 128: 112 and 84 us behind each other, 31 us less in one; as
+// 200-4000 tokens beside 4 prompts of 50-700, 32 / 8 heads of dim 128: 112 and 84 us behind each other, 172 in one; as
 // many workgroups per compute unit as the first kind has by itself)
 template <typename T, int DMAX>
 __global__ __launch_bounds__(256, generic_workgroups(sizeof(T), DMAX, 2)) void generic_pair_kernel(GAttn own, GAttn decoding, LaunchMix mix) {
