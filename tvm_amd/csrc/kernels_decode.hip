@@ -1041,19 +1041,17 @@ static void launch_beside_prefill(const DecodeParams& p, int group, int64_t num_
                                   const PromptLaunch& prompts, hipStream_t stream) {
   constexpr size_t lds_bytes = std::max(prefill_lds_bytes(D, D) + D * sizeof(float), sizeof(DecodeShared<D, false, true>));
   const LaunchMix mix(prompts.slots * p.h_kv * std::max(prompts.p.kv_splits, 1), num_items);
-  auto launch = [&](auto kernel, const auto& divisors) {
-    // per function, not per device
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       static_cast<int>(lds_bytes));
-    HIP_CHECK(attr);
+  auto launch = [&](auto src, auto new_token, const auto& divisors) {
+    constexpr auto kernel = decode_beside_prefill_kernel<D, decltype(src)::value, decltype(new_token)::value>;
+    allow_dynamic_lds<kernel>(lds_bytes);
     hipLaunchKernelGGL(kernel, dim3(mix.grid()), dim3(256), lds_bytes, stream, p, group, divisors, prompts.p, mix);
   };
   if (prompts.src == kPaged) {
-    launch(decode_beside_prefill_kernel<D, kPaged, false>, static_cast<const DecodeRopeDivisors&>(div));
+    launch(std::integral_constant<int, kPaged>{}, std::false_type{}, static_cast<const DecodeRopeDivisors&>(div));
   } else if (prompts.src == kBoth) {
-    launch(decode_beside_prefill_kernel<D, kBoth, true>, div);
+    launch(std::integral_constant<int, kBoth>{}, std::true_type{}, div);
   } else {
-    launch(decode_beside_prefill_kernel<D, kRagged, true>, div);
+    launch(std::integral_constant<int, kRagged>{}, std::true_type{}, div);
   }
 }
 

@@ -1003,14 +1003,8 @@ static int mla_entry(const void* q, const int32_t* q_indptr, const void* pages, 
     p.slot_plan = reinterpret_cast<int4*>(ws + part_o_bytes + part_lse_bytes);
   }
   constexpr size_t lds_bytes = static_cast<size_t>(MLA_STAGES) * MLA_BN * DQK * sizeof(half_t);
-  static bool attr_set = false;
-  if (!attr_set) {
-    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&mla_paged_kernel<DQK, DV, true>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
-    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&mla_paged_kernel<DQK, DV, false>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
-    attr_set = true;
-  }
+  allow_dynamic_lds<mla_paged_kernel<DQK, DV, true>>(lds_bytes);
+  allow_dynamic_lds<mla_paged_kernel<DQK, DV, false>>(lds_bytes);
   hipStream_t s = as_stream(stream);
   KV_CHECK(grid < (int64_t{1} << 31)) << "batch_prefill_paged_kv_mla: too many work items";
   p.page_shift = -1;

@@ -54,12 +54,7 @@ static void launch_prefill_ext(const PrefillParams& p, int64_t total_q, const Pr
                                hipStream_t stream) {
   const int64_t slots = row_tile_slots(p, total_q);
   constexpr size_t lds_bytes = prefill_lds_bytes(DQK, DV);
-  static bool attr_set = false;  // per instantiation; the attribute is per function, not per device
-  if (lds_bytes > 48 * 1024 && !attr_set) {
-    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_kernel<DQK, DV, SRC, PS, EXT, STREAM, PAD, VARIANT>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds_bytes)));
-    attr_set = true;
-  }
+  if constexpr (lds_bytes > 48 * 1024) allow_dynamic_lds<prefill_kernel<DQK, DV, SRC, PS, EXT, STREAM, PAD, VARIANT>>(lds_bytes);
   hipLaunchKernelGGL((prefill_kernel<DQK, DV, SRC, PS, EXT, STREAM, PAD, VARIANT>),
                      dim3(p.h_kv, static_cast<unsigned>(slots), static_cast<unsigned>(std::max(1, p.kv_splits))),
                      dim3(NW * 64), lds_bytes, stream, p, div);

@@ -5,9 +5,12 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <mutex>
+
+#include "common.h"
 
 struct tvmkv_rope_scaling;  // include/tvmkv.h
 
@@ -54,6 +57,17 @@ uint32_t next_scratch_epoch(uint64_t* launches, bool* wrapped);
 void zero_scratch_counters(char* ptr, size_t counter_bytes, hipStream_t stream);
 // Test aid: sets the launch count of every pooled buffer (to run a launch across the epoch wrap).
 void debug_set_scratch_launches(uint64_t launches);
+
+// A kernel that is launched with more dynamic shared memory than every function may have by itself (48 KB): said once per
+// kernel, which is a template argument so that kernels of one type do not share the flag, and again after a call that failed.
+// (The attribute is the function's, not the device's.)
+template <auto kKernel>
+void allow_dynamic_lds(size_t bytes) {
+  static std::atomic<bool> said{false};
+  if (said.load(std::memory_order_acquire)) return;
+  HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kKernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
+  said.store(true, std::memory_order_release);
+}
 
 // The table of an attention kernel's in-kernel RoPE for a frequency variant (NULL: the default
 // frequencies): entries for all head_dim elements, see InlineRopeTable in kernels_common.cuh.  Host
