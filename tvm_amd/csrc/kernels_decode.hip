@@ -1458,9 +1458,11 @@ int tvmkv::decode_with_new_token(const NewTokenDecode& a, void* stream, const Pr
 }
 
 // One launch where the decode kernel's work items are of one block of heads; a cap on its grid (a measuring option) and wider
-// groups keep the launches apart.  The decoding sequences go behind the prompts then: a split launch of those merges every row.
+// groups keep the launches apart, and so would two rotations: the launch has one table, the decoding sequences'.  They go
+// behind the prompts then: a split launch of those merges every row.
 int tvmkv::attend_mixed(const PromptPrefill& a, const NewTokenDecode& d, void* stream) {
-  const bool together = d.batch > 0 && d.h_kv > 0 && mixed_in_one_launch(d.d, d.h_q / d.h_kv) && option(kOptDecodeWgsPerCu) == 0;
+  const bool one_table = !a.apply_rope || (d.rotate != 0 && d.rope_scale == a.rope_scale && d.rope_theta == a.rope_theta);
+  const bool together = d.batch > 0 && d.h_kv > 0 && one_table && mixed_in_one_launch(d.d, d.h_q / d.h_kv) && option(kOptDecodeWgsPerCu) == 0;
   PromptLaunch prompts;
   const int code = prefill_prompts(a, together ? &prompts : nullptr, stream);
   return code != TVMKV_OK ? code : decode_with_new_token(d, stream, prompts.slots > 0 ? &prompts : nullptr);

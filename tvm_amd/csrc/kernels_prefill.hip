@@ -348,14 +348,6 @@ int tvmkv::prefill_prompts(const PromptPrefill& a, PromptLaunch* leave, void* st
   // sequence's; the cached keys behind a window are a second launch, which needs this one's rows)
   auto leave_out = [&](int src) {
     leave->p = p;
-    leave->p.rope_magnitude = 1.0f;
-    if (p.q_inline_rope) {
-      const InlineRopeHost table = inline_rope_table(nullptr, a.d, a.rope_theta);
-      for (int i = 0; i < a.d; ++i) leave->div.v[i] = table.v[i];
-      leave->p.rope_inverse = table.inverse;
-      leave->p.rope_halves_differ = table.halves_differ;
-      leave->p.rope_magnitude = table.magnitude;
-    }
     leave->slots = row_tile_slots(p, a.total_q);
     leave->src = src;
   };

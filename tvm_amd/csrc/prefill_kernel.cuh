@@ -777,8 +777,7 @@ __global__ __launch_bounds__(NW * 64, prefill_waves_per_simd(DQK, DV)) void pref
 // A launch that its caller is to run beside other work (prefill_prompts, prefill_shared_prefix): grid (h_kv, slots,
 // p.kv_splits), plain, SRC kPaged for a prefix.
 struct PromptLaunch {
-  PrefillParams p;
-  PrefillRopeDivisors div;
+  PrefillParams p;  // queries that are rotated: by the default table, which the other work brings
   int64_t slots = 0;  // 0: nothing is left to launch
   int src = kRagged;
 };
