@@ -4,6 +4,7 @@
 #include <cstdlib>
 #include <map>
 #include <set>
+#include <thread>
 
 #include "../../tvm_amd/csrc/runtime_support.h"
 
@@ -49,7 +50,44 @@ static void dynamic_lds_is_allowed_for_every_kernel_of_a_type() {
   REQUIRE(g_lds_bytes[reinterpret_cast<const void*>(kernel_b)] == 66048);
 }
 
+static void a_buffer_is_leased_once() {
+  std::recursive_mutex mutex;
+  bool decode = false, prefill = false;
+  auto hold = [&](bool* buffer) { return tvmkv::ScratchHold(std::unique_lock<std::recursive_mutex>(mutex), buffer); };
+  auto refused = [&](bool* buffer) {
+    try {
+      hold(buffer);
+    } catch (const tvmkv::Error&) {
+      return true;
+    }
+    return false;
+  };
+  auto locked_for_others = [&] {
+    bool got = false;
+    std::thread([&] {
+      got = mutex.try_lock();
+      if (got) mutex.unlock();
+    }).join();
+    return !got;
+  };
+  {
+    tvmkv::ScratchHold outer = hold(&prefill);
+    REQUIRE(refused(&prefill) && prefill);  // the refused one leaves the mark alone
+    {
+      tvmkv::ScratchHold inner = hold(&decode);  // another buffer, the same thread
+      REQUIRE(decode && refused(&decode) && refused(&prefill));
+    }
+    REQUIRE(!decode && prefill && locked_for_others());
+    tvmkv::ScratchHold moved = std::move(outer);
+    REQUIRE(prefill && refused(&prefill) && locked_for_others());
+    moved = {};
+    REQUIRE(!prefill && !refused(&prefill) && !locked_for_others());
+  }
+  REQUIRE(!decode && !prefill && !locked_for_others());
+}
+
 int main() {
+  a_buffer_is_leased_once();
   dynamic_lds_is_allowed_for_every_kernel_of_a_type();
   std::printf("all checks passed\n");
   return 0;

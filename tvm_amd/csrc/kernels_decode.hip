@@ -1071,6 +1071,7 @@ static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 struct StaticScratch {
   char* ptr = nullptr;    // device address of `scratch` on this device
   uint64_t launches = 0;  // the epoch of a launch is the low half
+  bool held = false;      // ScratchHold
 };
 static StaticScratch g_static_scratch[64];
 static std::recursive_mutex g_static_scratch_mutex;
@@ -1084,6 +1085,7 @@ static ScratchLease lease_static_scratch(size_t bytes, hipStream_t stream) {
       << "buffer has " << kStaticScratchBytes << "; use tvmkv_batch_decode_paged_kv for this shape";
   std::unique_lock<std::recursive_mutex> lock(g_static_scratch_mutex);
   StaticScratch& s = g_static_scratch[dev];
+  ScratchHold hold(std::move(lock), &s.held);
   if (s.ptr == nullptr) {
     void* ptr = nullptr;
     HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
@@ -1094,7 +1096,7 @@ static ScratchLease lease_static_scratch(size_t bytes, hipStream_t stream) {
   // 2^32 calls on this device: the epochs start over at 1 from counters cleared by a kernel in stream
   // order (no allocation, no memset node)
   if (wrapped) zero_scratch_counters(s.ptr, kArrivalBytes, stream);
-  return ScratchLease{s.ptr, epoch, std::move(lock)};
+  return ScratchLease{s.ptr, epoch, std::move(hold)};
 }
 
 extern "C" int tvmkv_debug_set_scratch_launches(uint64_t launches) {

@@ -45,6 +45,7 @@ struct Scratch {
   size_t counter_bytes = 0;
   uint64_t launches = 0;       // launches served from this buffer; the epoch of a launch is its low half
   bool seen_in_capture = false;  // a graph under capture has recorded this buffer's address
+  bool held = false;             // ScratchHold
 };
 std::recursive_mutex g_scratch_mutex;
 std::map<std::tuple<int, hipStream_t, int>, Scratch> g_scratch;
@@ -91,10 +92,12 @@ void zero_scratch_counters(char* ptr, size_t counter_bytes, hipStream_t stream) 
 ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, size_t counter_bytes, size_t at_least) {
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
-  // held by the lease until the caller has enqueued its launch: a thread that grows (and frees) this
-  // entry's buffer first synchronises the stream, and by then the launch is on it
+  // held by the lease until the caller has enqueued its launch: another thread that grows (and frees) this
+  // entry's buffer first synchronises the stream, and by then the launch is on it; this thread gets other
+  // users' buffers only
   std::unique_lock<std::recursive_mutex> lock(g_scratch_mutex);
   Scratch& s = g_scratch[std::make_tuple(dev, stream, static_cast<int>(user))];
+  ScratchHold hold(std::move(lock), &s.held);
   const bool capturing = stream_is_capturing(stream);
   if (s.bytes < bytes || s.counter_bytes < counter_bytes) {
     // growing means hipMalloc and hipFree: neither belongs into a graph under capture
@@ -112,6 +115,7 @@ ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, s
         HIP_CHECK(hipFree(s.ptr));
       }
       s = Scratch{};
+      s.held = true;
     }
     const size_t want = std::max(bytes + bytes / 2, at_least);
     void* ptr = nullptr;
@@ -129,7 +133,7 @@ ScratchLease lease_scratch(ScratchUser user, hipStream_t stream, size_t bytes, s
   // their own with a maximum: after the wrap an abandoned launch's word would compare as newer, so the
   // counters start over from zero (a kernel in stream order; recorded into a graph it is harmless).
   if (wrapped) zero_scratch_counters(s.ptr, s.counter_bytes, stream);
-  return ScratchLease{s.ptr, epoch, std::move(lock)};
+  return ScratchLease{s.ptr, epoch, std::move(hold)};
 }
 
 void release_scratch(hipStream_t stream) {
@@ -143,6 +147,7 @@ void release_scratch(hipStream_t stream) {
       ++it;
       continue;
     }
+    KV_CHECK(!it->second.held) << "tvmkv_release_scratch: a launch that uses the memory is being prepared";
     if (it->second.ptr != nullptr) {
       if (it->second.seen_in_capture) {
         g_retired.push_back(it->second.ptr);

@@ -9,6 +9,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <mutex>
+#include <utility>
 
 #include "common.h"
 
@@ -41,10 +42,40 @@ int64_t option(Option id);
 // start over at 1.
 // The lease keeps the pool locked until it is destroyed: hold it until the launch that uses the buffer
 // has been enqueued, so that a second host thread on the same stream cannot free the buffer in between.
+// The lock lets the same thread in again, as one launch may use the buffers of two users; a second lease
+// of the same buffer meanwhile, which would share it or free it, is refused.
+class ScratchHold {
+ public:
+  ScratchHold() = default;
+  // held: the mark of the buffer, which the lock guards
+  ScratchHold(std::unique_lock<std::recursive_mutex> lock, bool* held) : lock_(std::move(lock)) {
+    KV_CHECK(!*held) << "scratch memory is leased while a launch that uses it is being prepared";
+    *held = true;
+    held_ = held;
+  }
+  ScratchHold(ScratchHold&& other) noexcept { *this = std::move(other); }
+  ScratchHold& operator=(ScratchHold&& other) noexcept {
+    if (this != &other) {
+      Release();
+      lock_ = std::move(other.lock_);
+      held_ = std::exchange(other.held_, nullptr);
+    }
+    return *this;
+  }
+  ~ScratchHold() { Release(); }
+
+ private:
+  void Release() {
+    if (held_ != nullptr) *std::exchange(held_, nullptr) = false;  // in front of the unlock
+    if (lock_.owns_lock()) lock_.unlock();
+  }
+  std::unique_lock<std::recursive_mutex> lock_;
+  bool* held_ = nullptr;
+};
 struct ScratchLease {
   char* ptr;        // device memory, at least the requested size, 256-byte aligned
   uint32_t epoch;   // never 0
-  std::unique_lock<std::recursive_mutex> lock;
+  ScratchHold hold;
 };
 enum ScratchUser { kScratchDecode = 0, kScratchMla = 1, kScratchPrefill = 2, kScratchGeneric = 3 };
 // at_least: what a buffer that has to be allocated gets in any case
