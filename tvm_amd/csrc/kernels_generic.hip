@@ -142,7 +142,7 @@ __device__ __forceinline__ void rotate_pair(half8_t& lo, half8_t& hi, int f, int
 
 // workgroups per CU: the fp16 form holds its operands in half the registers
 constexpr int generic_workgroups(int elem_bytes, int dmax, int nb) {
-  return elem_bytes == 2 ? (dmax > 128 ? 2 : (nb == 1 || dmax <= 64 ? 4 : 3)) : (dmax > 128 ? 1 : (nb == 1 ? 3 : 2));
+  return elem_bytes == 2 ? (dmax > 128 ? 2 : (nb == 1 ? 4 : 3)) : (dmax > 128 ? 1 : (nb == 1 ? 3 : 2));
 }
 // 16-row blocks per row tile: one for decode-shaped calls and for head dims above 128 (registers), two when a
 // (sequence, kv head) has more than 16 rows on average.  Three and four blocks (fp16 storage, one workgroup fewer
@@ -182,9 +182,9 @@ __device__ __forceinline__ void generic_row_tile_attn(const GAttn p, const Inlin
   auto& rope_lds = shared.rope;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int j = lane & 15;  // query row of a 16-row block (matrix column) / key of a block / feature of a block
-  const int g = lane >> 4;
+  const int wave = HALF ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6, lane = tid & 63;
+  int j = lane & 15;  // query row of a 16-row block (matrix column) / key of a block / feature of a block
+  int g = lane >> 4;
   const int group = p.h_q / p.h_kv;
   const int d = p.d;
 
@@ -201,12 +201,12 @@ __device__ __forceinline__ void generic_row_tile_attn(const GAttn p, const Inlin
     }
   }
   const int b = lo;
-  const int q_start = q_begin(b);
+  const int q_start = __builtin_amdgcn_readfirstlane(q_begin(b));
   const int qo_len = q_begin(b + 1) - q_start;
   const int rows = qo_len * group;
   const int r0 = (slot - slot_begin(b)) * ROWS;
   if (r0 >= rows || (!EXT && p.skip_single && qo_len == 1)) return;  // the whole workgroup: a slot beyond the sequence's last row tile
-  const int q_token = !EXT && p.rows != nullptr ? p.rows[b] : q_start;  // the tile's place in q and out
+  const int q_token = !EXT && p.rows != nullptr ? __builtin_amdgcn_readfirstlane(p.rows[b]) : q_start;  // the tile's place in q and out
   const bool rotary = EXT && p.rotary != 0;
   if (EXT && rotary) {
     if (tid < d) rope_lds[tid] = rope.v[tid];
@@ -459,6 +459,16 @@ __device__ __forceinline__ void generic_row_tile_attn(const GAttn p, const Inlin
         }
       }
     }
+  }
+  // fp16 storage: the lane's place is formed anew and the wave's number is scalar; in vector registers through the main loop
+  // they spilled (head dims up to 128, two row blocks: 1 register, 4 in generic_pair_kernel, 49 with rotation, now 0, 0 and 37;
+  // causal prompts of 1500-2048 tokens, 32 / 8 heads of dim 128, two layers: 740 -> 726 us).  float32 storage, whose two
+  // workgroups leave registers over, was 1.2 % slower with it.
+  if constexpr (HALF) {
+    int lane_again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+    asm volatile("" : "+v"(lane_again));
+    j = lane_again & 15;
+    g = lane_again >> 4;
   }
   // the row sums of the four lane groups
 #pragma unroll
