@@ -1,11 +1,13 @@
 // Host-side support of the launchers (runtime_support.h, split_plan.h), driven without a GPU: the HIP calls that they make are
 // the ones below.  Exits with the line of the first check that fails.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <map>
 #include <set>
 #include <thread>
 
+#include "../../tvm_amd/csrc/launch_mix.h"
 #include "../../tvm_amd/csrc/runtime_support.h"
 
 #define REQUIRE(cond)                                        \
@@ -86,7 +88,63 @@ static void a_buffer_is_leased_once() {
   REQUIRE(!decode && !prefill && !locked_for_others());
 }
 
+// Every item of either kind has one workgroup, eight neighbours are of one kind, and two groups of the second follow one of the
+// first as long as there are both
+static void two_kinds_of_items_are_dealt_out_once() {
+  const int counts[] = {0, 1, 7, 8, 9, 15, 16, 17, 63, 64, 65, 129, 1000, 2047, 5003};
+  for (int first : counts) {
+    for (int others : counts) {
+      const tvmkv::LaunchMix mix(first, others);
+      std::set<int> seen[2];
+      int in_front = 0;
+      for (unsigned block = 0; block < mix.grid(); ++block) {
+        bool is_first = false, group_is_first = false;
+        const int item = mix.item(static_cast<int>(block), is_first);
+        mix.item(static_cast<int>(block & ~7u), group_is_first);
+        REQUIRE(is_first == group_is_first);
+        if (item < 0) continue;
+        REQUIRE(item < (is_first ? first : others) && item % 8 == static_cast<int>(block % 8));
+        REQUIRE(seen[is_first].insert(item).second);
+        if (!is_first && static_cast<int>(seen[1].size()) < first) in_front = std::max(in_front, item / 8 + 1);
+      }
+      REQUIRE(static_cast<int>(seen[1].size()) == first && static_cast<int>(seen[0].size()) == others);
+      REQUIRE(first == 0 || in_front >= std::min((others + 7) / 8, 2 * ((first + 7) / 8 - 1)));
+    }
+  }
+  for (int64_t bad : {int64_t{-1}, (int64_t{1} << 31) - 16}) {
+    bool threw = false;
+    try {
+      tvmkv::LaunchMix(bad, 0);
+    } catch (const tvmkv::Error&) {
+      threw = true;
+    }
+    REQUIRE(threw);
+  }
+}
+
+// The items of a split launch come in the order of its grid by itself: (kv heads, row tiles, shares), the first fastest
+static void row_tiles_of_one_share_are_neighbours() {
+  for (int h_kv : {1, 3, 8}) {
+    for (int slots : {1, 2, 5}) {
+      for (int shares : {1, 2, 64}) {
+        int item = 0;
+        const int items = h_kv * slots * shares;
+        for (int share = 0; share < shares; ++share) {
+          for (int slot = 0; slot < slots; ++slot) {
+            for (int kvh = 0; kvh < h_kv; ++kvh) {
+              const tvmkv::RowTileItem it(item++, items, h_kv, shares);
+              REQUIRE(it.kvh == kvh && it.slot == slot && it.share == share);
+            }
+          }
+        }
+      }
+    }
+  }
+}
+
 int main() {
+  two_kinds_of_items_are_dealt_out_once();
+  row_tiles_of_one_share_are_neighbours();
   a_buffer_is_leased_once();
   dynamic_lds_is_allowed_for_every_kernel_of_a_type();
   std::printf("all checks passed\n");

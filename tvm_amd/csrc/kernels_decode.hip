@@ -24,6 +24,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "launch_mix.h"
 #include "prefill_kernel.cuh"
 #include "runtime_support.h"
 #include "typed_kernels.h"
@@ -1015,10 +1016,10 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
 // by itself at 128.
 // NEW_TOKEN: the new-token form of the decode kernel, else its plain one.  A decode step over a shared prefix has the second
 // beside the split shares of the prefix (SRC kPaged), whose one round of workgroups walked its keys alone: 64 sequences of
-// 256-2048 tokens behind a prompt of 4096, 32 / 8 heads of dim 128, two steps of 8 layers: 1369 -> 1247 us, the same bits.  Over 13
-// other shapes (16-200 sequences, 64-2048 tokens, prompts of 300-6000, 4-8 query heads a kv head) 1.00-1.44 times as fast, most
-// where the prefix is long against the sequences' own tokens; two instead of three workgroups per compute unit for the decoding
-// items cost nothing that could be measured (200 sequences of 1024-2048 tokens: 2014 -> 1998).
+// 256-2048 tokens behind a prompt of 4096, 32 / 8 heads of dim 128, two steps of 8 layers: 1369 -> 1242 us, the same bits.  Over
+// 271 other shapes (20-200 sequences of 32-32 000 tokens, prefixes of 1100-64 000) 0.96-1.36 times as fast, 1.06 in the mean.  The
+// prefix's items go share by share (RowTileItem): row tile by row tile, each of them had the prefix's keys from memory by itself
+// (36 sequences of 32 tokens behind 64 000: 137 us a layer, in two launches 109, now 100).
 template <int D, int SRC, bool NEW_TOKEN>
 __global__ __launch_bounds__(256, prefill_waves_per_simd(D, D)) void decode_beside_prefill_kernel(
     DecodeParams p, int group, std::conditional_t<NEW_TOKEN, DecodeRopeRunning, DecodeRopeDivisors> div, PrefillParams prompts, LaunchMix mix) {
@@ -1027,8 +1028,8 @@ __global__ __launch_bounds__(256, prefill_waves_per_simd(D, D)) void decode_besi
   const int item = mix.item(blockIdx.x, is_prompts);
   if (item < 0) return;
   if (is_prompts) {
-    const int tile = item / p.h_kv, shares = SRC == kPaged ? prompts.kv_splits : 1, slot = tile / shares;
-    prefill_row_tile<D, D, SRC, 16, false>(prompts, div, item - tile * p.h_kv, slot, tile - slot * shares, beside_lds,
+    const RowTileItem tile(item, mix.first_items, p.h_kv, SRC == kPaged ? prompts.kv_splits : 1);
+    prefill_row_tile<D, D, SRC, 16, false>(prompts, div, tile.kvh, tile.slot, SRC == kPaged ? tile.share : 0, beside_lds,
                                            reinterpret_cast<float*>(beside_lds + prefill_lds_bytes(D, D) / sizeof(half_t)));
   } else {
     decode_items<NEW_TOKEN, D, false, 1, false, false, false, NEW_TOKEN>(p, group, mix.other_items, div, item, mix.other_items,

@@ -29,6 +29,7 @@
 #include <algorithm>
 
 #include "kernels_common.cuh"
+#include "launch_mix.h"
 #include "runtime_support.h"
 #include "typed_kernels.h"
 
