@@ -9,6 +9,7 @@
 
 #include "../../tvm_amd/csrc/launch_mix.h"
 #include "../../tvm_amd/csrc/runtime_support.h"
+#include "../../tvm_amd/csrc/typed_kernels.h"
 
 #define REQUIRE(cond)                                        \
   do {                                                       \
@@ -142,7 +143,24 @@ static void row_tiles_of_one_share_are_neighbours() {
   }
 }
 
+// Decode steps over a shared prefix whose times were measured in one launch and in two
+static void a_prefix_is_walked_beside_the_sequences_where_that_is_faster() {
+  const auto one = [](int d, int hq, int h_kv, int64_t sequences, int64_t own) {
+    return tvmkv::shared_prefix_in_one_launch(d, hq / h_kv, h_kv, sequences, sequences * own, 256);
+  };
+  for (int d : {64, 128}) {
+    for (int64_t own : {32, 1500, 6000, 32000}) REQUIRE(one(d, 32, 8, 64, own) && one(d, 32, 8, 36, own));
+    REQUIRE(one(d, 32, 8, 160, 300) && one(d, 32, 8, 200, 1500) && one(d, 8, 8, 200, 1500) && one(d, 32, 4, 110, 6000));
+  }
+  for (int64_t own : {3000, 6000, 10000}) {
+    REQUIRE(!one(64, 32, 8, 110, own) && !one(64, 8, 8, 140, own) && !one(64, 64, 8, 200, own));
+    REQUIRE(one(128, 32, 8, 110, own) && one(128, 8, 8, 140, own) && one(128, 64, 8, 200, own));
+  }
+  REQUIRE(!one(64, 32, 1, 64, 500) && !one(96, 32, 8, 64, 500) && !one(256, 32, 8, 64, 500));  // not built
+}
+
 int main() {
+  a_prefix_is_walked_beside_the_sequences_where_that_is_faster();
   two_kinds_of_items_are_dealt_out_once();
   row_tiles_of_one_share_are_neighbours();
   a_buffer_is_leased_once();

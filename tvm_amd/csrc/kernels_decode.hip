@@ -1017,8 +1017,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
 // NEW_TOKEN: the new-token form of the decode kernel, else its plain one.  A decode step over a shared prefix has the second
 // beside the split shares of the prefix (SRC kPaged), whose one round of workgroups walked its keys alone: 64 sequences of
 // 256-2048 tokens behind a prompt of 4096, 32 / 8 heads of dim 128, two steps of 8 layers: 1369 -> 1242 us, the same bits.  Over
-// 271 other shapes (20-200 sequences of 32-32 000 tokens, prefixes of 1100-64 000) 0.96-1.36 times as fast, 1.06 in the mean.  The
-// prefix's items go share by share (RowTileItem): row tile by row tile, each of them had the prefix's keys from memory by itself
+// 387 other shapes where it is taken (shared_prefix_in_one_launch; 20-200 sequences of 32-32 000 tokens, prefixes of 1100-64 000)
+// 0.97-1.36 times as fast, 1.07 in the mean.  The prefix's items go share by share (RowTileItem): row tile by row tile, each of them had the prefix's keys from memory by itself
 // (36 sequences of 32 tokens behind 64 000: 137 us a layer, in two launches 109, now 100).
 template <int D, int SRC, bool NEW_TOKEN>
 __global__ __launch_bounds__(256, prefill_waves_per_simd(D, D)) void decode_beside_prefill_kernel(

@@ -1339,9 +1339,10 @@ class PagedKVCache {
     }
     // A decode step of sequences with pages of their own behind one level of shared pages: both in one launch
     const bool plain = !generic_ && rotary_mode == 0 && sliding_window == 0 && option(kOptDecodeWgsPerCu) == 0;
-    if (is_first_kernel && n_order == 2 && plain && mixed_in_one_launch(static_cast<int>(qk_head_dim_), static_cast<int>(num_qo_heads_ / num_kv_heads_)) &&
-        s.use_decode_kernel[order[0]] && !s.use_decode_kernel[order[1]] && !(s.append_before_attn && !(s.is_chain[0] && s.is_chain[1])) &&
-        s.page_indices[0].size > 0 && s.page_indices[1].size > 0) {
+    if (is_first_kernel && n_order == 2 && plain && s.use_decode_kernel[order[0]] && !s.use_decode_kernel[order[1]] &&
+        !(s.append_before_attn && !(s.is_chain[0] && s.is_chain[1])) && s.page_indices[0].size > 0 && s.page_indices[1].size > 0 &&
+        shared_prefix_in_one_launch(static_cast<int>(qk_head_dim_), static_cast<int>(num_qo_heads_ / num_kv_heads_), static_cast<int>(num_kv_heads_),
+                                    s.qo_indptr[order[0]].size - 1, s.page_indices[order[0]].size * page_size_, compute_units_)) {
       SharedPrefixDecode a;
       a.q = q;
       a.pages = pages_[local_layer_id];

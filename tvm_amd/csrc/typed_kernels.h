@@ -220,7 +220,16 @@ struct SharedPrefixDecode {
   int64_t total_q = 0, num_pages = 0;
   int32_t h_q = 0, h_kv = 0, d = 0, page_size = 0;
 };
-int decode_with_shared_prefix(const SharedPrefixDecode& args, void* stream);  // where mixed_in_one_launch
+int decode_with_shared_prefix(const SharedPrefixDecode& args, void* stream);  // where shared_prefix_in_one_launch
+// At head dim 64 the launch of both holds three workgroups per compute unit, the decode kernel by itself five.  Where the
+// sequences alone are that many items, of more than one chunk each, nothing is left to overlap with: 100-200 sequences of
+// 3000-10 000 tokens behind 1100-16 000, 4-8 kv heads with 1-8 query heads each, took 0.96-1.08 times as long in two launches,
+// 1.00 in the mean of 93 shapes (32 / 8 heads, 140 x 6000 behind 4096: 329 us a layer, in two 318).  Fewer or shorter ones, and
+// head dim 128: 0.97-1.36, 1.07 in the mean of 387.
+inline bool shared_prefix_in_one_launch(int d, int group, int h_kv, int64_t sequences, int64_t own_tokens, int cus) {
+  const bool full = d == 64 && sequences * h_kv >= 3 * static_cast<int64_t>(cus) && own_tokens > 2048 * sequences;
+  return mixed_in_one_launch(d, group) && !full;
+}
 
 // tvmkv_kv_cache_transpose_append with the k / v rows of consecutive tokens token_stride elements apart (the fused
 // qkv tensor of the step)
