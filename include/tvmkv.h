@@ -471,6 +471,10 @@ int tvmkv_debug_set_scratch_launches(uint64_t launches);
  * 0); *wrapped = 1 when the epochs started over, which is when the launchers clear the counters. */
 uint32_t tvmkv_debug_next_scratch_epoch(uint64_t* launches, int32_t* wrapped);
 
+/* Test aid (no counterpart in the reference): how many launches of this process ran two kinds of work side by side
+ * (prompts, or the shares of a shared prefix, beside decoding sequences). */
+int tvmkv_debug_joint_launches(uint64_t* launches);
+
 /* ======================================================================================
  * (2) Cache object
  * ====================================================================================== */

@@ -3,6 +3,7 @@ HIP-backed cache, checked (a) against the numpy closed form the reference's own 
 (b) against the CPU oracle cache on identical seeded inputs, with page tables / append
 indices / pool state compared bit for bit."""
 import contextlib
+import ctypes
 
 import numpy as np
 import pytest
@@ -15,6 +16,7 @@ from tests.gpu_util import DEV, GpuCache, dev, host
 from tests.test_host_cache_parity import GLOBAL, PER_DEPTH
 from tests.util import assert_close
 from tvm_amd import get_global_func as gf
+from tvm_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -39,6 +41,23 @@ def step_route(route):
         yield
     finally:
         tvm_amd.set_option("step_route", prev)
+
+
+def joint_launches():
+    """Launches of two kinds of work side by side since the process began."""
+    count = ctypes.c_uint64()
+    check(lib().tvmkv_debug_joint_launches(ctypes.byref(count)))
+    return count.value
+
+
+@contextlib.contextmanager
+def launches_apart():
+    """A cap on the decode grid that none reaches: the same grids, one kind of work a launch."""
+    prev = tvm_amd.set_option("decode_wgs_per_cu", 1 << 20)
+    try:
+        yield
+    finally:
+        tvm_amd.set_option("decode_wgs_per_cu", prev)
 
 
 class Mirror:
@@ -325,23 +344,104 @@ def test_prompts_and_decoding_sequences_in_one_launch(dtype, page_size, d, hq, h
     with step_route(2):
         m.step([(0, 900), (1, 64)], (0, 0))
         m.step([(2, 400), (3, 1)], None)
-        m.step([(4, 2), (0, 1)], mixed)  # an item or two of prompts; one sequence
-        m.step([(0, 1), (5, 33), (2, 1), (6, 257), (1, 1), (7, 19)], mixed)
-        m.step([(8, 300), (9, 131), (10, 64), (11, 5), (2, 1)], mixed)  # few decoding items
-        m.step([(12, 17), (0, 1), (1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (8, 1), (9, 1)], mixed)
+        for batch in ([(4, 2), (0, 1)],  # an item or two of prompts; one sequence
+                      [(0, 1), (5, 33), (2, 1), (6, 257), (1, 1), (7, 19)],
+                      [(8, 300), (9, 131), (10, 64), (11, 5), (2, 1)],  # few decoding items
+                      [(12, 17), (0, 1), (1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (8, 1), (9, 1)]):
+            # the generic kernels: where the new tokens' row tiles are of 32 rows and the cached keys are split
+            cached = [-(-m.lengths[b] // page_size) * page_size for b, n in batch if n == 1]
+            together = dtype == np.float16 and page_size % 16 == 0 or (
+                sum(n for _, n in batch) * (hq // hkv) // len(batch) > 16 and sum(cached) // len(cached) >= 256)
+            before = joint_launches()
+            m.step(batch, mixed)
+            assert joint_launches() - before == (m.layers if together else 0)
 
 
-@pytest.mark.parametrize("page_size,d,hq,hkv,forks,prefix", [(16, 128, 16, 1, 9, 640), (64, 64, 32, 2, 10, 1100), (16, 128, 8, 2, 41, 385),
-                                                            (32, 64, 4, 4, 130, 256), (16, 128, 40, 2, 8, 640)])
-def test_decode_step_over_a_shared_prefix_whose_keys_are_split(page_size, d, hq, hkv, forks, prefix):
-    """The sequences' own tokens and the shares of the prefix in one launch (up to 16 query heads a kv head, the last case keeps
-    two): own parts of one token and of several chunks, a sequence that is the prefix itself."""
+@pytest.mark.parametrize("dtype,page_size,d,hq,hkv,window", [(np.float16, 16, 128, 8, 2, 0), (np.float16, 16, 64, 8, 2, 1300), (np.float32, 16, 64, 8, 2, 0)])
+def test_mixed_steps_of_more_sequences_than_a_wave_has_lanes(dtype, page_size, d, hq, hkv, window):
+    """77 sequences, 70 of them decoding, whose order and work items are looked up in two rounds."""
+    m = Mirror([80, 30000, 2600, page_size, 0] + ([window] if window else []), 2 if window else 1, hq, hkv, d, dtype=dtype,
+               **({"attn_kinds": [3, 0]} if window else {}))
+    with step_route(2):
+        for first in range(0, 70, 7):  # a quarter of them short
+            m.step([(b, 1 + b * 7 % 23 if b % 4 == 0 else 300 + b) for b in range(first, first + 7)])
+        m.step([(3, 900), (66, 300)])
+        before = joint_launches()
+        m.step([(b, 1) for b in range(40)] + [(70 + i, 61 + 50 * i) for i in range(7)] + [(b, 1) for b in range(40, 70)], (3, 3 if window else 0))
+    assert joint_launches() - before == m.layers
+
+
+@pytest.mark.parametrize("page_size,d,hq,hkv,forks,prefix,joint", [(16, 128, 16, 1, 9, 640, 0), (64, 64, 32, 2, 10, 1100, 0), (16, 128, 8, 2, 41, 385, 0),
+                                                                  (32, 64, 4, 4, 130, 256, 0), (16, 128, 40, 2, 8, 640, 0), (16, 128, 16, 1, 33, 1290, 1),
+                                                                  (32, 128, 8, 2, 41, 2400, 1), (64, 128, 4, 4, 130, 1100, 1), (16, 64, 4, 4, 130, 4100, 1),
+                                                                  (64, 64, 32, 2, 33, 1100, 1), (16, 128, 20, 1, 33, 1100, 0)])
+def test_decode_step_over_a_shared_prefix_whose_keys_are_split(page_size, d, hq, hkv, forks, prefix, joint):
+    """The sequences' own tokens and the shares of the prefix in one launch (from 32 sequences on, where the prefix is a level of
+    its own, and 1024 of its keys on, where they are split; up to 16 query heads a kv head): own parts of one token and of
+    several chunks, a sequence that is the prefix itself."""
     m = Mirror([forks + 2, prefix + 1500 + forks * 3 * page_size, 1200, page_size, 0], 1, hq, hkv, d)
-    m.step([(0, prefix)])
+    for first in range(0, prefix, 1200):
+        m.step([(0, min(1200, prefix - first))])
+    before = joint_launches()
     m.step([((b, 0, -1), 1) for b in range(1, forks + 1)])
+    assert joint_launches() - before == joint
     m.step([(1, 500)])
     m.step([(b, 1) for b in range(1, forks + 1)])
+    before = joint_launches()
     m.step([(b, 1) for b in range(forks, 0, -1)])
+    assert joint_launches() - before == joint
+
+
+@pytest.mark.parametrize("d,hq,hkv,page_size", [(128, 32, 8, 16), (64, 16, 2, 32), (128, 4, 4, 64)])
+def test_a_prefix_beside_its_sequences_is_the_same_as_apart_and_under_capture(d, hq, hkv, page_size):
+    """One launch and two write the same bits; so does every replay of a graph of the step."""
+    forks, prefix = 140, 5000
+    cache = GpuCache([forks + 2, 2 * prefix + forks * 900, 8192, page_size, 0], 1, hq, hkv, d, d)
+    rng = np.random.default_rng(33)
+    qkv = dev(rng.standard_normal((forks * 40, hq + 2 * hkv, d)).astype(np.float16))
+    attend = gf("vm.builtin.attention_kv_cache_attention_with_fused_qkv")
+
+    def forward(ids, lens):
+        cache.begin_forward(ids, lens)
+        attend(cache.cache, 0, d ** -0.5, qkv[:sum(lens)], torch.zeros((sum(lens), hq, d), dtype=torch.float16, device=DEV))
+        cache.end_forward()
+
+    cache.add_sequence(0)
+    forward([0], [prefix])
+    ids = list(range(1, forks + 1))
+    for b in ids:
+        cache.fork_sequence(0, b)
+    forward(ids, [1 + 11 * b % 60 for b in ids])
+    forward(ids[:3], [700, 800, 900])
+    cache.begin_forward(ids, [1] * forks)
+    rows = qkv[-forks:]
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    cache.cache.set_stream(stream.cuda_stream)
+    out = torch.zeros((forks, hq, d), dtype=torch.float16, device=DEV)
+    outs = []
+    for apart in (False, True):
+        out.zero_()
+        torch.cuda.synchronize()
+        before = joint_launches()
+        with launches_apart() if apart else contextlib.nullcontext():
+            attend(cache.cache, 0, d ** -0.5, rows, out)
+        assert joint_launches() - before == int(not apart)
+        torch.cuda.synchronize()
+        outs.append(out.clone())
+    assert bool(outs[0].any()) and torch.equal(outs[0], outs[1])
+    graph = torch.cuda.CUDAGraph()
+    before = joint_launches()
+    with torch.cuda.graph(graph, stream=stream):
+        attend(cache.cache, 0, d ** -0.5, rows, out)
+    assert joint_launches() - before == 1
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, outs[0])
+        (rows * 2).sum()  # work of the program's own between the replays
 
 
 def _exact(rows, cached, starts, mask, heads, kv_heads):

@@ -71,6 +71,7 @@ SIGNATURES = {
     "tvmkv_get_option": [ctypes.c_char_p, p_i64],
     "tvmkv_release_scratch": [c_vp],
     "tvmkv_debug_set_scratch_launches": [ctypes.c_uint64],
+    "tvmkv_debug_joint_launches": [c_vp],
     "tvmkv_decode_split_plan": [p_i32, c_i32, c_i64, c_i32, p_i32, p_i64, p_i32, p_i32, c_i64],
     "tvmkv_cache_create": [p_i64, c_i32, p_i64, c_i32, c_i64, c_i64, c_i64, c_i64, p_i64, c_i32, c_i32, c_i32,
                            c_f64, c_f64, c_i32, c_i32, ctypes.POINTER(c_vp)],

@@ -1054,6 +1054,7 @@ static void launch_beside_prefill(const DecodeParams& p, int group, int64_t num_
   } else {
     launch(std::integral_constant<int, kRagged>{}, std::true_type{}, div);
   }
+  count_joint_launch();
 }
 
 constexpr size_t kArrivalBytes = 256 * 1024;  // the first bytes of the scratch buffer: arrival counters

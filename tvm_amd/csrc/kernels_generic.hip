@@ -815,6 +815,7 @@ int generic_attention_pair(const GenericAttention& own, const GenericAttention& 
   };
   if (own.elem_bits == 32) run_type(float{}); else run_type(half_t{});
   KV_LAUNCH_CHECK();
+  count_joint_launch();
   merge_shares(decoding, second.p, stream);
   KV_API_END();
 }

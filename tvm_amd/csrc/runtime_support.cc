@@ -161,6 +161,9 @@ void release_scratch(hipStream_t stream) {
   }
 }
 
+static std::atomic<uint64_t> g_joint_launches{0};
+void count_joint_launch() { g_joint_launches.fetch_add(1, std::memory_order_relaxed); }
+
 void debug_set_scratch_launches(uint64_t launches) {
   std::lock_guard<std::recursive_mutex> lock(g_scratch_mutex);
   for (auto& entry : g_scratch) entry.second.launches = launches;
@@ -337,6 +340,13 @@ uint32_t tvmkv_debug_next_scratch_epoch(uint64_t* launches, int32_t* wrapped) {
   const uint32_t epoch = tvmkv::next_scratch_epoch(launches, &w);
   *wrapped = w ? 1 : 0;
   return epoch;
+}
+
+int tvmkv_debug_joint_launches(uint64_t* launches) {
+  KV_API_BEGIN();
+  KV_CHECK(launches != nullptr) << "tvmkv_debug_joint_launches: NULL argument";
+  *launches = tvmkv::g_joint_launches.load(std::memory_order_relaxed);
+  KV_API_END();
 }
 
 int tvmkv_release_scratch(void* stream) {

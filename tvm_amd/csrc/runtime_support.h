@@ -86,6 +86,8 @@ void release_scratch(hipStream_t stream);
 // The epoch of the next launch from a 64-bit launch count (host arithmetic only).
 uint32_t next_scratch_epoch(uint64_t* launches, bool* wrapped);
 void zero_scratch_counters(char* ptr, size_t counter_bytes, hipStream_t stream);
+// Test aid: launches of two kinds of work (launch_mix.h) since the process began
+void count_joint_launch();
 // Test aid: sets the launch count of every pooled buffer (to run a launch across the epoch wrap).
 void debug_set_scratch_launches(uint64_t launches);
 
