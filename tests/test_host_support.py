@@ -52,3 +52,14 @@ def test_generic_kernels_without_rotation_hold_their_operands_in_registers(tmp_p
              if "generic_pair_kernel" in k[0] or re.search(r"generic_attn_kernelI.*ELb0EE", k[0])]
     assert len(plain) == 14  # 2 storage types x 5 tiles, 2 x 2 pairs
     assert [k for k in plain if k[1] or k[2]] == []
+
+
+def test_prefill_kernels_of_head_dim_256_keep_no_copy_addresses(tmp_path):
+    """The plain ragged and paged forms spill 8 and 10 registers at most; with the addresses of a tile's copies among the
+    values that are kept from tile to tile it was 14 and 16, and their reloads waited for the copies in flight."""
+    library = os.path.join(ROOT, "tvm_amd", "lib", "libtvmkv.so")
+    if not (os.path.exists(READELF) and os.path.exists(library)):
+        pytest.skip("needs the built library and llvm-readelf")
+    plain = [k for k in _kernel_metadata(library, tmp_path) if re.search(r"prefill_kernelILi256ELi256ELi[01]ELi16ELb0E", k[0])]
+    assert len(plain) == 3
+    assert [k for k in plain if k[1] > 10] == []

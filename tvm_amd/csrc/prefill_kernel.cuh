@@ -317,7 +317,11 @@ __device__ __forceinline__ void prefill_row_tile(const PrefillParams& p, const P
     constexpr int FIRST = decltype(first_c)::value;
     constexpr int COUNT = decltype(count_c)::value;
     int l = lane;
-    if (DQK == 192) asm volatile("" : "+v"(l));  // addresses formed anew for every tile: kept, they spill
+    // Addresses formed anew for every tile: kept, they spill, and the wait for a reload between two copies waits for the
+    // copies before it too.  Head dim 256: cached keys of 41 sequences of 235-5734 tokens under trees of 54 nodes, 8 / 8
+    // heads, 370 -> 303 us a layer; chunks of 128-1500 tokens behind up to 4096, 32 / 8 heads, 691 -> 589, their own keys
+    // 229 -> 206.
+    if (DQK >= 192) asm volatile("" : "+v"(l));
     const bool from_pages = BOTH ? tile < prefix_tiles : PAGED;  // wave-uniform
     const int kv0 = tile * BN - (from_pages ? 0 : prefix_pad);
     const int last_row = (BOTH && !from_pages) ? last_new : last_tok;
