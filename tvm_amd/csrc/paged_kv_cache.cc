@@ -892,7 +892,11 @@ class PagedKVCache {
     if (generic_) {
       const double own = OwnUs(seqs, [](const StepSequence&) { return true; }, false);
       const double rows = PagedUs(seqs, decoding, false, false, false, true, sizeof(float));
-      const bool together = generic_pair_tiles(d, group, tokens * group / static_cast<int64_t>(seqs.size()));
+      // fp16: the sum, although they run in one launch there too.  The choice between this route and gathered keys, which only
+      // fp16 has, is closer than this estimate (24 % off, the gathered one 10 %): of 310 steps 3 took another route with the
+      // launch of both priced as one, 1.25, 1.26 and 0.88 times as long as with the sum (24 sequences of head dim 128, 64 / 8 heads,
+      // pages of 12: 510 us for 6 layers instead of 374).
+      const bool together = elem_bits_ == 32 && generic_pair_tiles(d, group, tokens * group / static_cast<int64_t>(seqs.size()));
       return (d > 128 ? 36 : 16) + (together ? std::max(own, rows) + 0.8 * std::min(own, rows) : own + rows) +
              PagedUs(seqs, prompt, false, false, false, /*may_split=*/false, 0);
     }
