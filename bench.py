@@ -352,8 +352,8 @@ def cache_object_shared_prefix_decode(torch, dev, layers=8, seed=5):
     nbytes = layers * ((prefix + float(own.sum()) + B) * TOKEN_BYTES + B * HQ * D * 2 * 2 + B * (HQ + 2 * HKV) * D * 2)
     unshared = layers * ((B * prefix + float(own.sum()) + B) * TOKEN_BYTES + B * HQ * D * 2 * 2)
     return {"workload": f"64 sequences forked from one 4096-token prompt, U[256,2048] tokens of their own, one token each per "
-                        f"step, {layers} layers through the cache object: per layer split + RoPE + append, the shared prefix "
-                        "for all queries in one paged-prefill launch, the sequences' own tokens in the decode kernel, merge",
+                        f"step, {layers} layers through the cache object: per layer split + RoPE + append, the sequences' own "
+                        "tokens with the shared prefix for all queries beside them in one launch, merge",
             "layers": layers, "depths": flags["num_depths"], "ms_per_step": round(ms, 4), "ms_per_layer": round(ms / layers, 4),
             "MB_per_layer": round(nbytes / layers / 1e6, 1), "GBps": round(nbytes / ms / 1e6, 1),
             "frac_of_hbm_peak": round(nbytes / ms / 1e6 / HBM_PEAK_GBPS, 4),

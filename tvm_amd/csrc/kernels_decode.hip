@@ -162,7 +162,9 @@ __device__ __forceinline__ void merge_row(const DecodeParams& p, int b, int hq, 
   // The loads of a batch are all issued before the first is used: the merge is a chain of round trips
   // to memory (device-scope loads do not hit in this XCD's L2), and what it costs is their number.  The first
   // batch of outputs is on its way while the maxima come in and are reduced.
-  constexpr int BATCH = 16;  // (32 costs the main loop registers: 166 instead of 136, and 1.2 % of the decode rate)
+  // (32 make the main loops of head dim 128 spill 55-72 registers: a layer of 64 sequences of 1024-8192 tokens 208 -> 278 us,
+  // one of 1117 tokens 10.1 -> 13.0)
+  constexpr int BATCH = 16;
   const int64_t stride = static_cast<int64_t>(p.h_q) * D;
   for (int c0 = 0; c0 < nchunks; c0 += 64) {
     const int c = c0 + lane;
@@ -1011,7 +1013,9 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : ((EXT || HB > 1) ? 2 : 3)) void 
 // up.  32 decoding sequences of up to 6000 tokens beside 8 prompts of up to 777, 32 / 8 heads of dim 64, every other layer with
 // a window: 8 layers 591 -> 478 us; the prompts' groups all in front 541, all behind 500, evenly spread over the grid 513,
 // one to one 491 and one to three 483 (periods of an even number of groups put a kind on the same compute units: 4
-// decoding sequences beside 10 prompts 1 : 1 337, 1 : 2 322, 1 : 3 343, 1 : 4 324 us).  The registers and LDS are those of the
+// decoding sequences beside 10 prompts 1 : 1 337, 1 : 2 322, 1 : 3 343, 1 : 4 324 us).  Over 200 steps of 2-80 sequences, with and without
+// layers with a window: 0.99-1.53 times as fast as in two launches, 1.22 in the mean; one to one 0.92-1.26 times as long as one to two, one
+// to three 0.90-1.32, 1.01 in the mean either way.  The registers and LDS are those of the
 // prefill kernel (head dim 64: three workgroups per compute unit, 128: two), which leaves as many workgroups as the decode kernel has
 // by itself at 128.
 // NEW_TOKEN: the new-token form of the decode kernel, else its plain one.  A decode step over a shared prefix has the second

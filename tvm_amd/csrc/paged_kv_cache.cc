@@ -782,7 +782,7 @@ class PagedKVCache {
     const std::vector<StepSequence> seqs = StepSequences(/*window=*/false);
     int64_t gathered = 0;
     for (const StepSequence& q : seqs) gathered += q.cached + q.tokens;
-    // The other route has to be better than the general one by what the estimate is off (measured on 1169 steps: with no
+    // The other route has to be better than the general one by what the estimate is off (measured on 1169 steps, before some routes' launches became one: with no
     // margin 1.5 % of the steps were up to 1.35 times as long as in the general launches, with it none by more than noise)
     const double margin = forced > 0 ? 0 : qk_head_dim_ > 128 ? 1.2 : 1.1;
     const double general_us = GeneralUs(seqs, /*window=*/false);
@@ -906,8 +906,9 @@ class PagedKVCache {
                                   : PagedUs(seqs, prompt, false, false, true, true, sizeof(float));
     const double rows = keys * GatherRowBytes() / 5e6;  // the decode kernel's time grows with them
     // In one launch, as long as the prompts' is not split.  (As a sum of launches this let steps of a few sequences take the
-    // general ones, which ran 1.1-1.7 times as long; with it 60 steps were within 1.13 of the better
-    // route.  A layer with a window walks few keys in the general launches: the sum stays there.)
+    // general ones, which ran 1.1-1.7 times as long; with it 100 steps without windows were within 1.19 of the
+    // better route, 1.015 in the mean, and at most 1.03 times as long as in the general launches.  A layer with a window walks few keys in
+    // the general launches: the sum stays there; 100 steps of which every other layer has one: within 1.30, 1.023 in the mean.)
     const bool together = !window && mixed_in_one_launch(d, group) &&
                           prefill_kv_splits(plan.prompt_tokens, group, plan.prompts, h_kv,
                                             (plan.prompt_cached + plan.prompt_tokens) / plan.prompts, compute_units_) == 1;
